@@ -17,6 +17,8 @@
 // operand reads of 16 lanes cover all banks); within a group of 8 k-values lanes 0-31 feed k..k+3 and lanes
 // 32-63 feed k+4..k+7 to four consecutive MFMAs (the order of the k-sum is free, both operands use the same one).
 //
+// Products of 3 GFLOP and more over more than 32 rows go to the bf16 matrix cores instead (gemm_split.hip, split_pays below).
+//
 // Workgroup ids are dealt round-robin to the 8 XCDs; the tile order makes the workgroups that share a tile
 // column of B (all M-tiles of that column) land on the same XCD back to back, so that B is fetched from HBM
 // once and re-read from that XCD's L2.
@@ -24,21 +26,17 @@
 #include <mutex>
 #include <vector>
 #include "dev_common.h"
+#include "gemm_epilogue.h"
 #include "kernels.h"
 
 namespace born {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
 constexpr int GN = 128, GK = 32;
 constexpr int GPITCH = GK + 4;                // floats per LDS tile row ([row][k] layout)
 constexpr int GPITCH_N = GN + 4;              // floats per LDS k-row ([k][n] layout of B when BT = false)
-constexpr int GEMM_THREADS = 256;
 constexpr int LQ = GK / 4;                    // 128-bit loads per tile row and slice
 constexpr int LROWS = GEMM_THREADS / LQ;      // tile rows one pass of the workgroup's loads covers (32)
 constexpr int BPASS = GN / LROWS;             // passes over B per slice (4; also GK / 8 k-rows of the [k][n] form)
-constexpr int NUM_XCD = 8;
 static_assert(GK / 8 == BPASS && LROWS == 32, "loader geometry");
 
 // Four consecutive k-values of one tile row; zero outside the matrix.
@@ -70,185 +68,6 @@ __device__ __forceinline__ f32x4 gemm_load_n4(const float *base, long long ld, i
         }
     }
     return v;
-}
-
-// What a tile does with its results.  EPI 0: adds the bias and stores them.  EPI 1 (greedy decode fused into
-// the LM head): keeps only the largest logit of every row as a packed key, value in the high word, ~column in
-// the low word, merged across tiles with a 64-bit atomic max, so the logits are never written.  The key order
-// is the reference's argmax (internal/nn/cross_entropy.go:241-251): larger value wins, the lower index on equal
-// values (-0 equals +0), a NaN never wins, except at index 0 where the reference returns 0 whatever follows.
-__device__ __forceinline__ u64 gemm_argmax_key(float v, int col) {
-    if (v != v) return col == 0 ? ~0ull : 0ull;
-    v = v == 0.0f ? 0.0f : v;
-    return ((u64)ordkey(v) << 32) | (u64)(0xFFFFFFFFu - (u32)col);
-}
-__device__ __forceinline__ u64 gemm_max_u64(u64 a, u64 b) { return a > b ? a : b; }
-// The keys of consecutive rows sit a cache line apart, and a tile first looks at the key it would have to beat:
-// the value only ever grows, so a tile that does not beat what it reads (however stale) cannot win, and all but
-// the first few tiles of a row skip the atomic.
-constexpr int GEMM_BEST_PITCH = LM_BEST_PITCH; // u64 words between the keys of consecutive rows (a 128-byte line each)
-__device__ __forceinline__ void gemm_offer_key(u64 *best, int row, u64 key) {
-    u64 *p = best + (long long)row * GEMM_BEST_PITCH;
-    if (key > __builtin_nontemporal_load(p)) atomicMax(p, key);
-}
-__device__ __forceinline__ u64 gemm_shfl_xor_u64(u64 x, int o) {
-    const u32 lo = (u32)__shfl_xor((int)(u32)x, o, WAVE), hi = (u32)__shfl_xor((int)(u32)(x >> 32), o, WAVE);
-    return ((u64)hi << 32) | lo;
-}
-
-// EPI 2 (sampling fused into the LM head): every result at or above its row's threshold is appended, value and
-// column, to the row's candidate list (one global atomic per candidate: a few per row and tile); the logits are
-// never written.  A NaN is never listed.  The counter may run past the list's capacity: the reader sees that.
-__device__ __forceinline__ void gemm_offer_candidate(const GemmArgs &g, int row, int col, float v, float thr) {
-    if (v >= thr) {
-        const unsigned pos = atomicAdd(&g.cand_cnt[(long long)row * LM_CAND_PITCH], 1u);
-        if (pos < (unsigned)g.cand_cap) g.cand[(long long)row * g.cand_cap + pos] = make_uint2(__float_as_uint(v), (unsigned)col);
-    }
-}
-
-// 32 x 32 blocks: accumulator v of lane (r, h) is row 8 * (v / 4) + 4 * h + v % 4, column r of its block
-template <int EPI, int IB, int JB>
-__device__ __forceinline__ void gemm_finish32(const GemmArgs &g, const f32x16 (&acc)[IB][JB], int m0, int n0, int wm,
-                                              int wn, int r, int h) {
-    if (EPI == 0) {
-#pragma unroll
-        for (int j = 0; j < JB; j++) {
-            const int col = n0 + (wn * JB + j) * 32 + r;
-            if (col >= g.N) continue;
-            const float bias = g.bias ? g.bias[col] : 0.f;
-#pragma unroll
-            for (int i = 0; i < IB; i++) {
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int row = m0 + (wm * IB + i) * 32 + (v >> 2) * 8 + h * 4 + (v & 3);
-                    if (row < g.M) {
-                        const float sum = acc[i][j][v];
-                        g.c[(long long)row * g.ldc + col] = g.bias ? sum + bias : sum;
-                    }
-                }
-            }
-        }
-    } else if (EPI == 2) {
-        // A candidate's place in its row's list costs a global atomic, and one per candidate where it is met would make
-        // the wave wait for a memory round trip some forty times.  The wave stages its candidates in LDS instead
-        // (ballot + lane rank, no atomics) and then asks for all their places at once.
-        constexpr int STAGE = 192;                                   // a 64 x 64 block of C yields about 70
-        __shared__ uint2 st_vc[GEMM_THREADS / WAVE][STAGE];
-        __shared__ int st_row[GEMM_THREADS / WAVE][STAGE];
-        uint2 *const vc = st_vc[threadIdx.x >> 6];
-        int *const rw = st_row[threadIdx.x >> 6];
-        u32 count = 0;                                               // wave-uniform
-        float bias[JB];
-#pragma unroll
-        for (int j = 0; j < JB; j++) {
-            const int col = n0 + (wn * JB + j) * 32 + r;
-            bias[j] = (g.bias && col < g.N) ? g.bias[col] : 0.f;
-        }
-#pragma unroll
-        for (int i = 0; i < IB; i++) {
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int row = m0 + (wm * IB + i) * 32 + (v >> 2) * 8 + h * 4 + (v & 3);
-                const float thr = row < g.M ? g.thr[row] : INFINITY;
-#pragma unroll
-                for (int j = 0; j < JB; j++) {
-                    const int col = n0 + (wn * JB + j) * 32 + r;
-                    const float sum = acc[i][j][v];
-                    const float val = g.bias ? sum + bias[j] : sum;
-                    const bool pass = col < g.N && val >= thr;       // a NaN never passes; rows past the batch have thr = +inf
-                    const u64 m = __ballot(pass);
-                    if (m) {                                         // wave-uniform
-                        if (pass) {
-                            const u32 pos = count + __builtin_amdgcn_mbcnt_hi((u32)(m >> 32), __builtin_amdgcn_mbcnt_lo((u32)m, 0u));
-                            if (pos < (u32)STAGE) {
-                                vc[pos] = make_uint2(__float_as_uint(val), (unsigned)col);
-                                rw[pos] = row;
-                            } else {
-                                gemm_offer_candidate(g, row, col, val, thr);   // the stage is full: straight to the list
-                            }
-                        }
-                        count += (u32)__popcll(m);
-                    }
-                }
-            }
-        }
-        const int staged = (int)min(count, (u32)STAGE);
-        for (int e = (int)(threadIdx.x & (WAVE - 1)); e < staged; e += WAVE) {   // (the wave's own LDS writes are visible to it in order)
-            const int row = rw[e];
-            const unsigned pos = atomicAdd(&g.cand_cnt[(long long)row * LM_CAND_PITCH], 1u);
-            if (pos < (unsigned)g.cand_cap) g.cand[(long long)row * g.cand_cap + pos] = vc[e];
-        }
-    } else {
-        float bias[JB];
-#pragma unroll
-        for (int j = 0; j < JB; j++) {
-            const int col = n0 + (wn * JB + j) * 32 + r;
-            bias[j] = (g.bias && col < g.N) ? g.bias[col] : 0.f;
-        }
-#pragma unroll
-        for (int i = 0; i < IB; i++) {
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                if (m0 + (wm * IB + i) * 32 + (v >> 2) * 8 + (v & 3) >= g.M) continue;   // past the batch for both h: wave-uniform
-                u64 key = 0ull;
-#pragma unroll
-                for (int j = 0; j < JB; j++) {
-                    const int col = n0 + (wn * JB + j) * 32 + r;
-                    const float sum = acc[i][j][v];
-                    if (col < g.N) key = gemm_max_u64(key, gemm_argmax_key(g.bias ? sum + bias[j] : sum, col));
-                }
-#pragma unroll
-                for (int o = 16; o > 0; o >>= 1) key = gemm_max_u64(key, gemm_shfl_xor_u64(key, o));   // the 32 lanes of this h
-                const int row = m0 + (wm * IB + i) * 32 + (v >> 2) * 8 + h * 4 + (v & 3);
-                if (r == 0 && row < g.M && key) gemm_offer_key(g.best, row, key);
-            }
-        }
-    }
-}
-// 16 x 16 blocks: accumulator v of lane (j, q) is row 4 q + v, column j of its block
-template <int EPI>
-__device__ __forceinline__ void gemm_finish16(const GemmArgs &g, const f32x4 (&acc16)[2], int m0, int n0, int wn, int j16,
-                                              int q16) {
-    if (EPI == 0) {
-#pragma unroll
-        for (int jb = 0; jb < 2; jb++) {
-            const int col = n0 + wn * 32 + jb * 16 + j16;
-            if (col >= g.N) continue;
-            const float bias = g.bias ? g.bias[col] : 0.f;
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int row = m0 + 4 * q16 + v;
-                if (row < g.M) g.c[(long long)row * g.ldc + col] = g.bias ? acc16[jb][v] + bias : acc16[jb][v];
-            }
-        }
-    } else if (EPI == 2) {
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int row = m0 + 4 * q16 + v;
-            if (row >= g.M) continue;
-            const float thr = g.thr[row];
-#pragma unroll
-            for (int jb = 0; jb < 2; jb++) {
-                const int col = n0 + wn * 32 + jb * 16 + j16;
-                if (col < g.N) gemm_offer_candidate(g, row, col, g.bias ? acc16[jb][v] + g.bias[col] : acc16[jb][v], thr);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            if (m0 + v >= g.M) continue;                              // past the batch for every q: wave-uniform
-            u64 key = 0ull;
-#pragma unroll
-            for (int jb = 0; jb < 2; jb++) {
-                const int col = n0 + wn * 32 + jb * 16 + j16;
-                if (col < g.N) key = gemm_max_u64(key, gemm_argmax_key(g.bias ? acc16[jb][v] + g.bias[col] : acc16[jb][v], col));
-            }
-#pragma unroll
-            for (int o = 8; o > 0; o >>= 1) key = gemm_max_u64(key, gemm_shfl_xor_u64(key, o));         // the 16 lanes of this q
-            const int row = m0 + 4 * q16 + v;
-            if (j16 == 0 && row < g.M && key) gemm_offer_key(g.best, row, key);
-        }
-    }
 }
 
 // FAST: every 128-bit load is legal and K is a multiple of the slice, so the loads need no guards (rows past
@@ -357,7 +176,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_f32_kernel(GemmArgs g) {
         }
     };
 
-    f32x4 acc16[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // SMALL: columns wn * 32 + 16 * jb + lane % 16
+    f32x4 acc16[1][2] = {{{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}};  // SMALL: columns wn * 32 + 16 * jb + lane % 16
     const int j16 = lane & 15, q16 = lane >> 4;
     f32x16 acc[IB][JB];
 #pragma unroll
@@ -387,7 +206,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_f32_kernel(GemmArgs g) {
                 for (int kk = 0; kk < 4; kk++)
 #pragma unroll
                     for (int jb = 0; jb < 2; jb++)
-                        acc16[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[kk], bf[jb][kk], acc16[jb], 0, 0, 0);
+                        acc16[0][jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[kk], bf[jb][kk], acc16[0][jb], 0, 0, 0);
             }
             return;
         }
@@ -437,9 +256,9 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_f32_kernel(GemmArgs g) {
     }
 
     if (SMALL)
-        gemm_finish16<EPI>(g, acc16, m0, n0, wn, j16, q16);
+        gemm_finish<EPI, 16, 4>(g, acc16, m0, n0 + wn * 32, Bs);
     else
-        gemm_finish32<EPI, IB, JB>(g, acc, m0, n0, wm, wn, r, h);
+        gemm_finish<EPI, 32, 4>(g, acc, m0 + wm * IB * 32, n0 + wn * JB * 32, Bs);
 }
 
 // The same tile computation for W[N,K] operands whose loads need no guards, with the global loads written
@@ -561,7 +380,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_f32_dma_kernel(GemmArgs g) 
         }
     }
 
-    gemm_finish32<EPI, IB, JB>(g, acc, m0, n0, wm, wn, r, h);
+    gemm_finish<EPI, 32, 4>(g, acc, m0 + wm * IB * 32, n0 + wn * JB * 32, Bs0);
 }
 
 template <bool BT, bool FAST, int EPI>
@@ -598,16 +417,16 @@ __global__ __launch_bounds__(256) void gemm_splitk_sum_kernel(GemmArgs g, long l
     }
 }
 
-// Workspace for the partial products: one buffer per (device, stream) that ever needed one, kept until the process
-// ends (calls on one stream are ordered, so they can share; calls on different streams cannot).  Null when none can be
-// had now (the stream is being captured, too many streams, out of memory): the product is then computed unsplit.
+// Workspace for partial products and packed operands: one small and one large buffer per (device, stream) that ever needed
+// one, kept until the process ends (calls on one stream are ordered, so they can share; calls on different streams cannot;
+// a buffer once handed out stays, so that a graph captured with it stays good).  Null when none can be had now (the stream
+// is being captured, too many streams, out of memory): the product is then computed without.
 constexpr size_t GEMM_WS_MAX = (size_t)64 << 20, GEMM_WS_MIN = (size_t)8 << 20;
 static float *gemm_workspace(hipStream_t st, size_t bytes) {
     struct Entry {
         int dev;
         hipStream_t st;
-        float *p;
-        size_t bytes;
+        float *p[2];                                                 // GEMM_WS_MIN, GEMM_WS_MAX bytes
     };
     static std::mutex mu;
     static std::vector<Entry> cache;
@@ -617,28 +436,21 @@ static float *gemm_workspace(hipStream_t st, size_t bytes) {
     Entry *found = nullptr;
     for (Entry &e : cache)
         if (e.dev == dev && e.st == st) found = &e;
-    if (found && found->bytes >= bytes) return found->p;
+    const int large = bytes > GEMM_WS_MIN;
+    if (found && (found->p[large] || found->p[1])) return found->p[large] ? found->p[large] : found->p[1];
     if (!found && cache.size() >= 16) return nullptr;
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return nullptr;
-    if (found) {                                                     // a larger one: the old buffer may still be in use on the stream
-        if (hipStreamSynchronize(st) != hipSuccess) return nullptr;
-        (void)hipFree(found->p);
-        found->p = nullptr;
-        found->bytes = 0;
-    }
-    const size_t want = bytes < GEMM_WS_MIN ? GEMM_WS_MIN : GEMM_WS_MAX;
     float *p = nullptr;
-    if (hipMalloc((void **)&p, want) != hipSuccess) {
+    if (hipMalloc((void **)&p, large ? GEMM_WS_MAX : GEMM_WS_MIN) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }
-    if (found) {
-        found->p = p;
-        found->bytes = want;
-    } else {
-        cache.push_back(Entry{dev, st, p, want});
+    if (!found) {
+        cache.push_back(Entry{dev, st, {nullptr, nullptr}});
+        found = &cache.back();
     }
+    found->p[large] = p;
     return p;
 }
 
@@ -744,6 +556,23 @@ hipError_t launch_lm_threshold(const float *samp, long long ld, int B, int nsamp
     return hipGetLastError();
 }
 
+static void launch_splitk_sum(const GemmArgs &g, hipStream_t st) {
+    const long long mn = (long long)g.M * g.N;
+    const dim3 sg((unsigned)std::min<long long>((mn + 255) / 256, 4096)), sb(256);
+    if (g.cand) hipLaunchKernelGGL(gemm_splitk_sum_kernel<2>, sg, sb, 0, st, g, mn);
+    else if (g.best) hipLaunchKernelGGL(gemm_splitk_sum_kernel<1>, sg, sb, 0, st, g, mn);
+    else hipLaunchKernelGGL(gemm_splitk_sum_kernel<0>, sg, sb, 0, st, g, mn);
+}
+
+// Whether the product goes to the bf16 matrix cores (gemm_split.hip).  They do an fp32 product's work about twice as fast,
+// after a launch that packs the left operand: below about 3 GFLOP the fp32 tiles, finer and split along K, are level
+// (64 x 4096 -> 4096, 2.1 GFLOP: 33 us against 28; 1024^3 24 against 32; 128 x 4096 -> 4096, 4.3: 72 against 41; 200 x 1056 ->
+// 8272, 3.5: 72 against 45); a batch of up to 32 rows is bound by reading the weights (32 x 4096 -> 32000: 118 against 130 us).
+// A caller that names the tile height keeps it.
+static bool split_pays(const GemmArgs &g) {
+    return !g.bm && g.M > 32 && 2.0 * (double)g.M * (double)g.N * (double)g.K >= 3e9;
+}
+
 hipError_t launch_gemm_f32(const GemmArgs &g, bool b_transposed, hipStream_t st) {
     int bm = g.bm ? g.bm : g.M <= 16 ? 16 : g.M <= 32 ? 32 : g.M <= 64 ? 64 : 128;
     // A product of few tiles leaves most of the device idle (1024 x 1024 x 1024 is 64 tiles of 128 x 128 for 256 CUs):
@@ -763,6 +592,37 @@ hipError_t launch_gemm_f32(const GemmArgs &g, bool b_transposed, hipStream_t st)
     const bool fast = g.vec_a && g.vec_b && g.K % GK == 0 && (b_transposed || (g.N % 4 == 0));
     if (g.cand && (!b_transposed || !g.thr || !g.cand_cnt || g.cand_cap <= 0)) return hipErrorInvalidValue;   // candidate epilogue: W[N,K] form only
     if (g.best && (!b_transposed || !g.tokens)) return hipErrorInvalidValue;                                    // argmax epilogue: W[N,K] form only
+    const SplitPlan plan = gemm_split_plan(g.M, g.N, g.K);
+    if (split_pays(g)) {
+        // the packed operand of a call takes 6 bytes a value of the workspace: rows in chunks that fit beside the partial products
+        const long long chunk_max = plan.slices > 1 ? g.M : std::max<long long>(256, (long long)(GEMM_WS_MAX / 7) / ((g.K + 63) / 64 * 64) / 256 * 256);
+        const long long chunks = (g.M + chunk_max - 1) / chunk_max, rows = ((g.M + chunks - 1) / chunks + 255) / 256 * 256;
+        const long long most = std::min<long long>(rows, g.M);
+        const size_t packed = gemm_split_workspace((int)most, g.K);
+        float *ws = gemm_workspace(st, packed + (plan.slices > 1 ? (size_t)plan.slices * (size_t)g.M * (size_t)g.N * sizeof(float) : 0));
+        if (ws) {
+            for (long long r0 = 0; r0 < g.M; r0 += rows) {
+                GemmArgs gc = g;
+                gc.M = (int)std::min<long long>(rows, g.M - r0);
+                gc.a += r0 * g.lda;
+                if (g.c) gc.c += r0 * g.ldc;
+                if (g.best) gc.best += r0 * LM_BEST_PITCH;
+                if (g.cand) {
+                    gc.thr += r0;
+                    gc.cand_cnt += r0 * LM_CAND_PITCH;
+                    gc.cand += r0 * g.cand_cap;
+                }
+                gc.ksplit = plan.slices > 1 ? plan.slices : 0;
+                gc.kslice = plan.kslice;
+                gc.ws = ws + packed / sizeof(float);
+                const hipError_t e = launch_gemm_split(gc, b_transposed, plan.tile, ws, st);
+                if (e != hipSuccess) return e;
+                if (gc.ksplit > 1) launch_splitk_sum(gc, st);
+            }
+            if (g.best) hipLaunchKernelGGL(argmax_keys_token_kernel, dim3((unsigned)((g.M + 255) / 256)), dim3(256), 0, st, g.best, g.tokens, g.M);
+            return hipGetLastError();
+        }
+    }
     // A product of few tiles and a long K: the slices of K go to workgroups of their own, each writes a partial
     // product to the workspace, and one more launch adds them in order and does what the product's epilogue does.
     GemmArgs gs = g;
@@ -786,11 +646,7 @@ hipError_t launch_gemm_f32(const GemmArgs &g, bool b_transposed, hipStream_t st)
         } else {
             if (fast) launch_gemm_bm<false, true, 0>(gs, bm, st); else launch_gemm_bm<false, false, 0>(gs, bm, st);
         }
-        const long long mn = (long long)g.M * g.N;
-        const dim3 sg((unsigned)std::min<long long>((mn + 255) / 256, 4096)), sb(256);
-        if (g.cand) hipLaunchKernelGGL(gemm_splitk_sum_kernel<2>, sg, sb, 0, st, gs, mn);
-        else if (g.best) hipLaunchKernelGGL(gemm_splitk_sum_kernel<1>, sg, sb, 0, st, gs, mn);
-        else hipLaunchKernelGGL(gemm_splitk_sum_kernel<0>, sg, sb, 0, st, gs, mn);
+        launch_splitk_sum(gs, st);
         if (g.best) hipLaunchKernelGGL(argmax_keys_token_kernel, dim3((unsigned)((g.M + 255) / 256)), dim3(256), 0, st, g.best, g.tokens, g.M);
         return hipGetLastError();
     }

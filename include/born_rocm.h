@@ -244,7 +244,9 @@ int born_rocm_spec_verify_bonus(born_sampler *s, const float *target, int64_t ta
                                 void *stream);
 
 /* The logits producer, fp32 on the matrix cores (fp32 operands, fp32 accumulation; the order of the k-sum
- * differs from the reference's sequential loop, so results agree with it to rounding, not bit for bit).
+ * differs from the reference's sequential loop, so results agree with it to rounding, not bit for bit).  Large
+ * products run on the bf16 matrix cores at fp32 precision: each operand is the exact sum of three bf16 parts, and the
+ * six products of parts that can reach an fp32 rounding of the product are accumulated in fp32.
  *
  * born_rocm_linear: out[batch, out_features] = x[batch, in_features] @ weight^T + bias, weight stored
  * [out_features, in_features] row-major as nn.Linear holds it, bias [out_features] or NULL: Linear.Forward,
@@ -259,9 +261,10 @@ int born_rocm_spec_verify_bonus(born_sampler *s, const float *target, int64_t ta
 int born_rocm_linear(const float *x, int64_t batch, int64_t in_features, int64_t x_stride, const float *weight,
                      int64_t out_features, int64_t w_stride, const float *bias, float *out, int64_t out_stride,
                      void *stream);
-/* (born_rocm_matmul, born_rocm_linear and the fused heads below: a product of few output tiles and a long k is computed in slices of k that are added in a fixed order;
- * the first such call on a stream allocates the library's workspace for that stream, 8 or 64 MiB kept until the process
- * ends - outside a stream capture; a call under capture that finds no workspace computes the product unsplit.) */
+/* (born_rocm_matmul, born_rocm_linear and the fused heads below: a product of few output tiles and a long k is computed
+ * in slices of k that are added in a fixed order, and a large product reads its left operand from a packed copy; the
+ * first such call on a stream allocates the library's workspace for that stream, 8 or 64 MiB kept until the process
+ * ends - outside a stream capture; a call under capture that finds no workspace computes the product without.) */
 int born_rocm_matmul(const float *a, const float *b, float *c, int64_t m, int64_t k, int64_t n, int64_t lda,
                      int64_t ldb, int64_t ldc, void *stream);
 
