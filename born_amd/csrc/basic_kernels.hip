@@ -48,15 +48,15 @@ __global__ __launch_bounds__(256) void argmax_partial_kernel(const float *__rest
     const int row = blockIdx.x / S, seg = blockIdx.x % S;
     const float *x = logits + (long long)row * stride;
     const int base = seg * ARGMAX_SEG;
-    const bool vec = ((stride & 3) == 0) && ((((uintptr_t)logits) & 15) == 0);
     ArgPair best = {-INFINITY, 0x7FFFFFFF};
 #pragma unroll
     for (int it = 0; it < ARGMAX_SEG / (256 * 4); it++) {
         int j = base + (it * 256 + (int)threadIdx.x) * 4;
         float v[4];
-        if (vec && j + 3 < V) {
-            float4 f = *reinterpret_cast<const float4 *>(x + j);
-            v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+        if (j + 3 < V) {
+            const row_f32x4 f = *reinterpret_cast<const row_f32x4 *>(x + j);
+#pragma unroll
+            for (int c = 0; c < 4; c++) v[c] = f[c];
         } else {
 #pragma unroll
             for (int c = 0; c < 4; c++) v[c] = (j + c < V) ? x[j + c] : __uint_as_float(0x7FC00000u);
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(64) void argmax_merge_kernel(const float *__restric
 // (64 rows x 32000: 7.1 us as two launches, of which the second only merges four partials per row).
 // TPR lanes per row by its length: 1024, 256, or one wave (four rows to a workgroup, no LDS and no barrier) - a row of
 // 1024 logits gives 1024 threads one logit each and spends its time in the reduction.
-typedef float argmax_f32x4 __attribute__((ext_vector_type(4)));
+typedef row_f32x4 argmax_f32x4;
 template <int TPR>
 __global__ __launch_bounds__(TPR == 64 ? 256 : TPR) void argmax_row_kernel(const float *__restrict__ logits, int B, int V, long long stride,
                                                                         int *__restrict__ tokens) {
@@ -109,7 +109,6 @@ __global__ __launch_bounds__(TPR == 64 ? 256 : TPR) void argmax_row_kernel(const
     const int tid = TPR == 64 ? lane_id() : (int)threadIdx.x;
     if (row >= B) return;                                            // (whole waves; no barrier where rows share a workgroup)
     const float *x = logits + (long long)row * stride;
-    const bool vec = ((stride & 3) == 0) && ((((uintptr_t)logits) & 15) == 0);
     ArgPair best = {-INFINITY, 0x7FFFFFFF};
     // a thread meets its indices in ascending order, so "strictly greater" keeps the first of equals; NaN compares false
     auto take = [&](float v, int j) {
@@ -118,28 +117,24 @@ __global__ __launch_bounds__(TPR == 64 ? 256 : TPR) void argmax_row_kernel(const
             best.i = j;
         }
     };
-    if (vec) {
-        const int n4 = V >> 2;
-        const argmax_f32x4 *x4 = reinterpret_cast<const argmax_f32x4 *>(x);
-        int i = tid;
-        for (; i + 3 * TPR < n4; i += 4 * TPR) {                      // four loads in flight per thread
-            argmax_f32x4 f[4];
+    const int n4 = V >> 2;
+    const argmax_f32x4 *x4 = reinterpret_cast<const argmax_f32x4 *>(x);
+    int i = tid;
+    for (; i + 3 * TPR < n4; i += 4 * TPR) {                          // four loads in flight per thread
+        argmax_f32x4 f[4];
 #pragma unroll
-            for (int u = 0; u < 4; u++) f[u] = __builtin_nontemporal_load(x4 + i + u * TPR);
+        for (int u = 0; u < 4; u++) f[u] = __builtin_nontemporal_load(x4 + i + u * TPR);
 #pragma unroll
-            for (int u = 0; u < 4; u++)
+        for (int u = 0; u < 4; u++)
 #pragma unroll
-                for (int c = 0; c < 4; c++) take(f[u][c], ((i + u * TPR) << 2) + c);
-        }
-        for (; i < n4; i += TPR) {
-            const argmax_f32x4 f = __builtin_nontemporal_load(x4 + i);
-#pragma unroll
-            for (int c = 0; c < 4; c++) take(f[c], (i << 2) + c);
-        }
-        for (int j = (n4 << 2) + tid; j < V; j += TPR) take(x[j], j);
-    } else {
-        for (int j = tid; j < V; j += TPR) take(x[j], j);
+            for (int c = 0; c < 4; c++) take(f[u][c], ((i + u * TPR) << 2) + c);
     }
+    for (; i < n4; i += TPR) {
+        const argmax_f32x4 f = __builtin_nontemporal_load(x4 + i);
+#pragma unroll
+        for (int c = 0; c < 4; c++) take(f[c], (i << 2) + c);
+    }
+    for (int j = (n4 << 2) + tid; j < V; j += TPR) take(x[j], j);
     best = wave_best(best);
     if (TPR == 64) {
         if (tid == 0) tokens[row] = argmax_token(best, x[0]);
@@ -209,7 +204,7 @@ hipError_t launch_argmax(const float *logits, int B, int V, long long stride, in
 // 64, 256 or 1024 lanes per row by its length, eight 128-bit loads per lane at most; a row of a single wave needs no
 // LDS and no barrier, and four of them share a workgroup.  Longer rows are swept three times by 1024 threads.
 // ---------------------------------------------------------------------------
-typedef float sm_f32x4 __attribute__((ext_vector_type(4)));
+typedef row_f32x4 sm_f32x4;
 // canon() without its last step (-0 -> +0 only matters where z is turned into a sort key)
 __device__ __forceinline__ float sm_canon(float z) { return fminf((z != z) ? -INFINITY : z, 3.402823466e+38f); }
 
@@ -236,12 +231,11 @@ __global__ __launch_bounds__(TPR == 64 ? 256 : TPR) void softmax_resident_kernel
     if (row >= B) return;                                            // (whole waves, and no barrier where rows share a workgroup)
     const float *x = logits + (long long)row * stride;
     float *o = out + (long long)row * V;
-    const bool vin = (((uintptr_t)x) & 15) == 0, vout = (((uintptr_t)o) & 15) == 0;
     float v[U][4];
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const int j = (u * TPR + t) * 4;
-        if (vin && j + 3 < V) {
+        if (j + 3 < V) {
             const sm_f32x4 f = __builtin_nontemporal_load(reinterpret_cast<const sm_f32x4 *>(x + j));
 #pragma unroll
             for (int c = 0; c < 4; c++) v[u][c] = f[c];
@@ -280,7 +274,7 @@ __global__ __launch_bounds__(TPR == 64 ? 256 : TPR) void softmax_resident_kernel
         float r[4];
 #pragma unroll
         for (int c = 0; c < 4; c++) r[c] = LOG ? (float)(((double)v[u][c] - (double)m) - lz) : softmax_quotient(v[u][c], Zd, rZ);
-        if (vout && j + 3 < V) {
+        if (j + 3 < V) {
             sm_f32x4 f;
 #pragma unroll
             for (int c = 0; c < 4; c++) f[c] = r[c];
@@ -345,8 +339,7 @@ __global__ __launch_bounds__(1024) void softmax_sweep_kernel(const float *__rest
     const int row = blockIdx.x, tid = threadIdx.x;
     const float *x = logits + (long long)row * stride;
     float *o = out + (long long)row * V;
-    const bool vin = (((uintptr_t)x) & 15) == 0, vout = (((uintptr_t)o) & 15) == 0;
-    const int n4 = vin ? V >> 2 : 0;                                 // 128-bit blocks of the row; the rest element by element
+    const int n4 = V >> 2;                                           // 128-bit blocks of the row; the rest element by element
     const sm_f32x4 *x4 = reinterpret_cast<const sm_f32x4 *>(x);
     // every element of the row as f(index, value): four blocks in flight, then single blocks, then the ragged end
     auto sweep = [&](auto f) {
@@ -386,12 +379,7 @@ __global__ __launch_bounds__(1024) void softmax_sweep_kernel(const float *__rest
         sm_f32x4 r;
 #pragma unroll
         for (int c = 0; c < 4; c++) r[c] = result(q[c]);
-        if (vout) {
-            __builtin_nontemporal_store(r, reinterpret_cast<sm_f32x4 *>(o + j));
-        } else {
-#pragma unroll
-            for (int c = 0; c < 4; c++) o[j + c] = r[c];
-        }
+        __builtin_nontemporal_store(r, reinterpret_cast<sm_f32x4 *>(o + j));
     });
     for (int j = (n4 << 2) + tid; j < V; j += 1024) o[j] = result(x[j]);
 }

@@ -99,7 +99,6 @@ struct SpecArgs {
     unsigned long long *run_mass; // [B][SPEC_CHUNKS][1024] residual mass of each thread's run of ids
     int *status;
     int mass_shift;
-    int aligned;                  // set by the launcher: every row starts 16-byte aligned and V % 4 == 0
 };
 
 // C[M,N] = A[M,K] * B (+ bias[N]); B is [N,K] (b_transposed, the weight of a linear layer) or [K,N].

@@ -55,12 +55,12 @@ struct NucGeom {
 };
 constexpr int NUC_BLOCK_MAX = 1024;
 
-typedef float nuc_f32x4 __attribute__((ext_vector_type(4)));
+typedef row_f32x4 nuc_f32x4;
 
 struct NucRow {                               // uniform per workgroup
     const float *x;
     int V;
-    bool vec, penal, degenerate;
+    bool penal, degenerate;
     bool masked = false;                      // the visitor replaces every seen logit by `skip`; the seen ids are visited apart
     float skip = 0.0f;
     float T, rcp, rep, m, scale, range, sbin, dcut;        // rcp: RN(1 / T) where the division shortcut is exact, else 0
@@ -84,9 +84,9 @@ __device__ __forceinline__ float nuc_z_shortcut(const NucRow &r, float y) {
     return __fmaf_rn(e, r.rcp, q);
 }
 
-// Visits every element of the row with its penalised logit: aligned rows four at a time as f4(id of the first, y[4]),
-// in stages of U float4 per thread, the next stage's loads in flight while this one is visited; what is left
-// over (and every element of an unaligned row) one at a time as f1(id, y).
+// Visits every element of the row with its penalised logit: four at a time as f4(id of the first, y[4]), in stages of
+// U float4 per thread, the next stage's loads in flight while this one is visited; what is left over one at a time as
+// f1(id, y).
 // AHEAD: the row's partial last stage is loaded ahead like the whole ones (3 % faster on short rows, where the few
 // blocks left over are a third of the row; measured slower on long ones and in the single-sweep kernel).
 // `pre` runs once before the first element is visited, with the first stage's loads already in flight (work that
@@ -144,90 +144,85 @@ __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 
         if (!PLAIN && r.penal && ((bm[j >> 5] >> (j & 31)) & 1u)) y = r.masked ? r.skip : penalise_seen(y, r.rep, r.counts, j, r.freq, r.pres);
         f1(j, y);
     };
-    if (r.vec) {
-        const int n4 = r.V >> 2;
-        constexpr int NUC_U = NucGeom<NUC_BLOCK>::U;
-        if constexpr (!AHEAD) {
-            const int nfull = n4 / (NUC_U * NUC_BLOCK);
-            const nuc_f32x4 *x4 = reinterpret_cast<const nuc_f32x4 *>(r.x);
-            if (nfull > 0) {
-                // Two stages a turn, each loaded while the other is visited, so that no register is copied; the last
-                // one or two stages in a loop of their own.
-                nuc_f32x4 va[NUC_U], vb[NUC_U];
+    const int n4 = r.V >> 2;
+    constexpr int NUC_U = NucGeom<NUC_BLOCK>::U;
+    if constexpr (!AHEAD) {
+        const int nfull = n4 / (NUC_U * NUC_BLOCK);
+        const nuc_f32x4 *x4 = reinterpret_cast<const nuc_f32x4 *>(r.x);
+        if (nfull > 0) {
+            // Two stages a turn, each loaded while the other is visited, so that no register is copied; the last
+            // one or two stages in a loop of their own.
+            nuc_f32x4 va[NUC_U], vb[NUC_U];
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(x4 + u * NUC_BLOCK + tid);
-                pre();
-                int s = 0;
-                for (; s + 2 < nfull; s += 2) {
+            for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(x4 + u * NUC_BLOCK + tid);
+            pre();
+            int s = 0;
+            for (; s + 2 < nfull; s += 2) {
 #pragma unroll
-                    for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4<NT>(x4 + ((s + 1) * NUC_U + u) * NUC_BLOCK + tid);
+                for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4<NT>(x4 + ((s + 1) * NUC_U + u) * NUC_BLOCK + tid);
 #pragma unroll
-                    for (int u = 0; u < NUC_U; u++) visit4(va[u], ((s * NUC_U + u) * NUC_BLOCK + tid) << 2);
+                for (int u = 0; u < NUC_U; u++) visit4(va[u], ((s * NUC_U + u) * NUC_BLOCK + tid) << 2);
 #pragma unroll
-                    for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(x4 + ((s + 2) * NUC_U + u) * NUC_BLOCK + tid);
+                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(x4 + ((s + 2) * NUC_U + u) * NUC_BLOCK + tid);
 #pragma unroll
-                    for (int u = 0; u < NUC_U; u++) visit4(vb[u], (((s + 1) * NUC_U + u) * NUC_BLOCK + tid) << 2);
-                }
-                for (;;) {
-#pragma unroll
-                    for (int u = 0; u < NUC_U; u++) visit4(va[u], ((s * NUC_U + u) * NUC_BLOCK + tid) << 2);
-                    if (++s >= nfull) break;
-#pragma unroll
-                    for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(x4 + (s * NUC_U + u) * NUC_BLOCK + tid);
-                }
-            } else {
-                pre();
+                for (int u = 0; u < NUC_U; u++) visit4(vb[u], (((s + 1) * NUC_U + u) * NUC_BLOCK + tid) << 2);
             }
-            for (int i = nfull * NUC_U * NUC_BLOCK + tid; i < n4; i += NUC_BLOCK) {
-                const nuc_f32x4 q = nuc_load4<NT>(x4 + i);
-                visit4(q, i << 2);
+            for (;;) {
+#pragma unroll
+                for (int u = 0; u < NUC_U; u++) visit4(va[u], ((s * NUC_U + u) * NUC_BLOCK + tid) << 2);
+                if (++s >= nfull) break;
+#pragma unroll
+                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(x4 + (s * NUC_U + u) * NUC_BLOCK + tid);
             }
         } else {
-            const int nst = (n4 + NUC_U * NUC_BLOCK - 1) / (NUC_U * NUC_BLOCK);      // stages, the last one whole or partial
-            const nuc_f32x4 *x4 = reinterpret_cast<const nuc_f32x4 *>(r.x);
-            if (nst > 0) {
-                // Loads are unconditional, of a block index clamped to the row's last block (a load under a condition makes
-                // the compiler wait for every load in flight); only the visits of the last stage ask whether the block exists.
-                nuc_f32x4 va[NUC_U], vb[NUC_U];
-                const int lastb = n4 - 1;
-                if constexpr (!std::is_same<FIRST, NucNoFirst>::value) {
-#pragma unroll
-                    for (int u = 0; u < NUC_U; u++) va[u] = first[u];
-                } else {
-#pragma unroll
-                    for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(x4 + min(u * NUC_BLOCK + tid, lastb));
-                }
-                pre();
-                for (int s = 0; s + 1 < nst; s++) {
-#pragma unroll
-                    for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4<NT>(x4 + min(((s + 1) * NUC_U + u) * NUC_BLOCK + tid, lastb));
-#pragma unroll
-                    for (int u = 0; u < NUC_U; u++) visit4(va[u], ((s * NUC_U + u) * NUC_BLOCK + tid) << 2);
-#pragma unroll
-                    for (int u = 0; u < NUC_U; u++) va[u] = vb[u];
-                }
-#pragma unroll
-                for (int u = 0; u < NUC_U; u++) {
-                    const int i = ((nst - 1) * NUC_U + u) * NUC_BLOCK + tid;
-                    if (i < n4) visit4(va[u], i << 2);
-                }
-            } else {
-                pre();
-            }
+            pre();
         }
-        for (int j = (n4 << 2) + tid; j < r.V; j += NUC_BLOCK) visit1(j);
+        for (int i = nfull * NUC_U * NUC_BLOCK + tid; i < n4; i += NUC_BLOCK) {
+            const nuc_f32x4 q = nuc_load4<NT>(x4 + i);
+            visit4(q, i << 2);
+        }
     } else {
-        pre();
-        for (int j = tid; j < r.V; j += NUC_BLOCK) visit1(j);
+        const int nst = (n4 + NUC_U * NUC_BLOCK - 1) / (NUC_U * NUC_BLOCK);      // stages, the last one whole or partial
+        const nuc_f32x4 *x4 = reinterpret_cast<const nuc_f32x4 *>(r.x);
+        if (nst > 0) {
+            // Loads are unconditional, of a block index clamped to the row's last block (a load under a condition makes
+            // the compiler wait for every load in flight); only the visits of the last stage ask whether the block exists.
+            nuc_f32x4 va[NUC_U], vb[NUC_U];
+            const int lastb = n4 - 1;
+            if constexpr (!std::is_same<FIRST, NucNoFirst>::value) {
+#pragma unroll
+                for (int u = 0; u < NUC_U; u++) va[u] = first[u];
+            } else {
+#pragma unroll
+                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(x4 + min(u * NUC_BLOCK + tid, lastb));
+            }
+            pre();
+            for (int s = 0; s + 1 < nst; s++) {
+#pragma unroll
+                for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4<NT>(x4 + min(((s + 1) * NUC_U + u) * NUC_BLOCK + tid, lastb));
+#pragma unroll
+                for (int u = 0; u < NUC_U; u++) visit4(va[u], ((s * NUC_U + u) * NUC_BLOCK + tid) << 2);
+#pragma unroll
+                for (int u = 0; u < NUC_U; u++) va[u] = vb[u];
+            }
+#pragma unroll
+            for (int u = 0; u < NUC_U; u++) {
+                const int i = ((nst - 1) * NUC_U + u) * NUC_BLOCK + tid;
+                if (i < n4) visit4(va[u], i << 2);
+            }
+        } else {
+            pre();
+        }
     }
+    for (int j = (n4 << 2) + tid; j < r.V; j += NUC_BLOCK) visit1(j);
 }
-// Requests the first stage of an aligned row's next sweep (the same loads the AHEAD visitor starts with): issued at the
+// Requests the first stage of the row's next sweep (the same loads the AHEAD visitor starts with): issued at the
 // end of one sweep, they are in flight through the reductions and scans between the sweeps, which on a batch that leaves
 // CUs idle are otherwise a memory latency each.
 template <int NUC_BLOCK, bool NT>
 __device__ __forceinline__ void nuc_request_first(const NucRow &r, nuc_f32x4 (&first)[NucGeom<NUC_BLOCK>::U]) {
     const int n4 = r.V >> 2;
-    if (r.vec && n4 > 0) {
+    if (n4 > 0) {
         const nuc_f32x4 *x4 = reinterpret_cast<const nuc_f32x4 *>(r.x);
 #pragma unroll
         for (int u = 0; u < NucGeom<NUC_BLOCK>::U; u++) first[u] = nuc_load4<NT>(x4 + min(u * NUC_BLOCK + (int)threadIdx.x, n4 - 1));
@@ -299,7 +294,6 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     NucRow r;
     r.x = a.logits + (long long)row * a.row_stride;
     r.V = V;
-    r.vec = ((a.row_stride & 3) == 0) && ((((uintptr_t)a.logits) & 15) == 0);
     r.T = cfg_T;
     r.rcp = cfg_rcp;
     r.rep = cfg_rep;
@@ -951,7 +945,6 @@ __global__ __launch_bounds__(NUC_BLOCK, 4) void token_logprob_kernel(SampleArgs 
     NucRow r;
     r.x = a.logits + (long long)row * a.row_stride;
     r.V = V;
-    r.vec = ((a.row_stride & 3) == 0) && ((((uintptr_t)a.logits) & 15) == 0);
     r.T = a.T;
     r.rep = a.rep;
     r.scale = 0.0f;
@@ -1087,9 +1080,8 @@ __global__ __launch_bounds__(256) void token_logprob_small_kernel(SampleArgs a, 
         st += (double)term(z, mt);
     };
     if (live) {
-        const bool vec = G == 64 && ((a.row_stride & 3) == 0) && ((((uintptr_t)a.logits) & 15) == 0);
         int done = 0;
-        if (vec) {
+        if (G == 64) {
             const int n4 = V >> 2;
             const nuc_f32x4 *x4 = reinterpret_cast<const nuc_f32x4 *>(x);
             for (int i = gl; i < n4; i += G) {

@@ -21,27 +21,23 @@ constexpr int SPEC_BLOCK = 1024;
 constexpr int SPEC_NF4 = 8;                   // float4 per thread and array that the stats kernel keeps in registers
 constexpr int SPEC_RESIDENT_V = SPEC_NF4 * SPEC_BLOCK * 4;
 
-typedef float spec_f32x4 __attribute__((ext_vector_type(4)));
+typedef row_f32x4 spec_f32x4;
 
 template <class F>
-__device__ __forceinline__ void spec_foreach(const float *x, int V, bool vec, F f) {
-    const int tid = threadIdx.x;
-    if (vec) {
-        const int n4 = V >> 2;
-        const float4 *x4 = reinterpret_cast<const float4 *>(x);
-        for (int i = tid; i < n4; i += SPEC_BLOCK) {
-            float4 q = x4[i];
-            f(q.x); f(q.y); f(q.z); f(q.w);
-        }
-        for (int j = (n4 << 2) + tid; j < V; j += SPEC_BLOCK) f(x[j]);
-    } else {
-        for (int j = tid; j < V; j += SPEC_BLOCK) f(x[j]);
+__device__ __forceinline__ void spec_foreach(const float *x, int V, F f) {
+    const int tid = threadIdx.x, n4 = V >> 2;
+    const spec_f32x4 *x4 = reinterpret_cast<const spec_f32x4 *>(x);
+    for (int i = tid; i < n4; i += SPEC_BLOCK) {
+        const spec_f32x4 q = x4[i];
+#pragma unroll
+        for (int c = 0; c < 4; c++) f(q[c]);
     }
+    for (int j = (n4 << 2) + tid; j < V; j += SPEC_BLOCK) f(x[j]);
 }
 
 // One workgroup per (sequence, position, distribution): blockIdx.x = 2 * row + (0 target | 1 draft).  The two
 // distributions of a position are independent, and twice as many work items spread better over the CUs.
-// RESIDENT: V <= SPEC_RESIDENT_V, V % 4 == 0 and the rows 16-byte aligned.
+// RESIDENT: V <= SPEC_RESIDENT_V.
 // z = canon(x / T); UNIT: T == 1, where the division is the identity and is not computed at all.
 template <bool UNIT>
 __device__ __forceinline__ float spec_z(float x, float T, float rcp) {
@@ -103,6 +99,9 @@ __global__ __launch_bounds__(SPEC_BLOCK) void spec_stats_kernel(SpecArgs a) {
     if (RESIDENT) {
         const int n4 = V >> 2;
         spec_f32x4 t[SPEC_NF4];
+        const int jt = (n4 << 2) + tid;                              // the row's last V % 4 logits, one per thread
+        const float last = jt < V ? x[jt] : -INFINITY;
+        m = fmaxf(m, last);
 #pragma unroll
         for (int i = 0; i < SPEC_NF4; i++) {
             const int j = i * SPEC_BLOCK + tid;
@@ -126,6 +125,7 @@ __global__ __launch_bounds__(SPEC_BLOCK) void spec_stats_kernel(SpecArgs a) {
                     for (int c = 0; c < 4; c++) sum += spec_usual_mass<UNIT>(t[i][c], m, T, rcp, scale32);
                 }
             }
+            if (jt < V) sum += spec_usual_mass<UNIT>(last, m, T, rcp, scale32);
         } else if (m > -INFINITY) {                                  // (uniform) m - z is a number: +inf for a masked logit, no mass
 #pragma unroll
             for (int i = 0; i < SPEC_NF4; i++) {
@@ -134,6 +134,7 @@ __global__ __launch_bounds__(SPEC_BLOCK) void spec_stats_kernel(SpecArgs a) {
                     for (int c = 0; c < 4; c++) sum += qfix(expneg(m - spec_z<UNIT>(t[i][c], T, rcp)), scale);
                 }
             }
+            if (jt < V) sum += qfix(expneg(m - spec_z<UNIT>(last, T, rcp)), scale);
         } else {                                                     // nothing finite: (-inf) - (-inf) := 0 for every logit
 #pragma unroll
             for (int i = 0; i < SPEC_NF4; i++) {
@@ -142,12 +143,12 @@ __global__ __launch_bounds__(SPEC_BLOCK) void spec_stats_kernel(SpecArgs a) {
                     for (int c = 0; c < 4; c++) sum += qfix(emass(spec_z<UNIT>(t[i][c], T, rcp), m), scale);
                 }
             }
+            if (jt < V) sum += qfix(emass(spec_z<UNIT>(last, T, rcp), m), scale);
         }
     } else {
-        const bool vec = a.aligned != 0;
-        spec_foreach(x, V, vec, [&](float v) { m = fmaxf(m, spec_z<UNIT>(v, T, rcp)); });
+        spec_foreach(x, V, [&](float v) { m = fmaxf(m, spec_z<UNIT>(v, T, rcp)); });
         m = block_max_f32<SPEC_BLOCK>(m, &scr);
-        spec_foreach(x, V, vec, [&](float v) { sum += qfix(emass(spec_z<UNIT>(v, T, rcp), m), scale); });
+        spec_foreach(x, V, [&](float v) { sum += qfix(emass(spec_z<UNIT>(v, T, rcp), m), scale); });
     }
     u64 Z;
     block_inclusive_scan_u64<SPEC_BLOCK>(sum, &scr, &Z);
@@ -369,11 +370,8 @@ __global__ __launch_bounds__(SPEC_BLOCK) void spec_pick_kernel(SpecArgs a) {
     }
 }
 
-hipError_t launch_spec_verify(const SpecArgs &args, hipStream_t st) {
-    SpecArgs a = args;
-    a.aligned = (a.V & 3) == 0 && ((((uintptr_t)a.target) | ((uintptr_t)a.draft) | ((uintptr_t)a.bonus)) & 15) == 0 &&
-                ((a.t_seq | a.d_seq | (a.bonus ? a.b_seq : 0)) & 3) == 0;
-    const bool resident = a.V <= SPEC_RESIDENT_V && a.aligned;
+hipError_t launch_spec_verify(const SpecArgs &a, hipStream_t st) {
+    const bool resident = a.V <= SPEC_RESIDENT_V;
     const unsigned stats_grid = (unsigned)(2 * a.B * a.G + (a.bonus ? a.B : 0));
     const dim3 sg(stats_grid), sb(SPEC_BLOCK);
     if (resident) {

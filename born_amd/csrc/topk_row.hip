@@ -88,8 +88,7 @@ static void launch_topk_row_as(const SampleArgs &a, hipStream_t st, const RowCon
 }
 
 hipError_t launch_topk_row(const SampleArgs &a, hipStream_t st, const RowConfigs *rows, bool two_per_cu) {
-    const bool vec = ((a.row_stride & 3) == 0) && ((((uintptr_t)a.logits) & 15) == 0);
-    if (vec) {
+    if (a.V >= 4) {                                                  // a row holds a 128-bit load
         if (a.local_counts) launch_topk_row_as<true, true>(a, st, rows, two_per_cu); else launch_topk_row_as<true, false>(a, st, rows, two_per_cu);
     } else {
         if (a.local_counts) launch_topk_row_as<false, true>(a, st, rows, two_per_cu); else launch_topk_row_as<false, false>(a, st, rows, two_per_cu);

@@ -62,11 +62,11 @@ static_assert(TOPK_MAX_K == 512, "RowGeom<1> and its last wave are sized for 512
 // Entries a raised threshold keeps beyond top_k (what the penalties may push below the bound without losing the proof).
 __device__ __forceinline__ int row_margin(int k) { return k <= TOPK_SMALL_K ? 16 : k >> 3; }
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef row_f32x4 f32x4;
 
-// row_load_any: one stage of ROW_U consecutive blocks of ROW_BLOCK float4 in row order, for the row's ragged end,
-// unaligned rows, and anything past the end (-inf fill).  Used by the sweeps of the exact selection and by rows that
-// 128-bit loads cannot take.
+// row_load_any: one stage of ROW_U consecutive blocks of ROW_BLOCK float4 in row order, for the row's ragged end
+// and anything past the end (-inf fill).  Used by the sweeps of the exact selection and by rows of less than one 128-bit
+// load.
 template <bool VEC>
 __device__ __forceinline__ void row_load_any(f32x4 (&v)[ROW_U], const float *x, int V, int stage, int tid) {
 #pragma unroll
@@ -89,14 +89,28 @@ __device__ __forceinline__ void row_load_fast(f32x4 (&v)[ROW_U], const float *x,
 }
 
 // Block indices clamped into the row: a stage that reaches past the row's end (or lies wholly beyond it) re-reads the
-// row's last block instead of branching around its loads, so that the loads of later stages can stay in flight (a load
-// under a condition makes the compiler wait for every load in flight).  The row starts 16-byte aligned and its pitch
-// is a multiple of four floats (VEC), so the last block lies inside the pitch.
-__device__ __forceinline__ void row_load_clamped(f32x4 (&v)[ROW_U], const float *x, int n4, int stage, int tid) {
+// row's last four elements instead of branching around its loads, so that the loads of later stages can stay in flight (a
+// load under a condition makes the compiler wait for every load in flight).  V >= 4 (VEC).
+__device__ __forceinline__ void row_load_clamped(f32x4 (&v)[ROW_U], const float *x, int V, int stage, int tid) {
 #pragma unroll
     for (int u = 0; u < ROW_U; u++) {
-        const int i4 = min((stage * ROW_U + u) * ROW_BLOCK + tid, n4 - 1);
-        v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(x) + i4);
+        const int j = min(((stage * ROW_U + u) * ROW_BLOCK + tid) << 2, V - 4);
+        v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(x + j));
+    }
+}
+// A row whose length is no multiple of four: its last block was loaded from where the row's last four elements start, and
+// goes to its place here (what lies past the end is masked by whoever looks at the stage).
+__device__ __forceinline__ void row_place_last(f32x4 (&v)[ROW_U], int V, int stage, int tid) {
+    const int over = (4 - V) & 3;                                    // elements of the last block past the row's end
+    if (over == 0) return;                                           // uniform
+#pragma unroll
+    for (int u = 0; u < ROW_U; u++) {
+        if (((stage * ROW_U + u) * ROW_BLOCK + tid) == V >> 2) {
+            const f32x4 q = v[u];
+            v[u][0] = over == 1 ? q[1] : over == 2 ? q[2] : q[3];
+            v[u][1] = over == 1 ? q[2] : q[3];
+            v[u][2] = q[3];
+        }
     }
 }
 
@@ -647,9 +661,9 @@ __device__ __forceinline__ void topk_row_body(SampleArgs &a) {
     auto stage_at = [&](int t) { return !VEC || nstage < 3 || t == 0 ? t : t == 1 ? last : t < nstage ? t - 1 : nstage; };
     f32x4 va[ROW_U], vb[ROW_U], vc[ROW_U];
     if (VEC) {
-        row_load_clamped(va, x, n4, 0, tid);
-        row_load_clamped(vb, x, n4, stage_at(1), tid);               // in flight during the search for the first threshold
-        row_load_clamped(vc, x, n4, stage_at(2), tid);
+        row_load_clamped(va, x, V, 0, tid);
+        row_load_clamped(vb, x, V, stage_at(1), tid);                // in flight during the search for the first threshold
+        row_load_clamped(vc, x, V, stage_at(2), tid);
     } else {
         row_load_any<false>(va, x, V, 0, tid);
     }
@@ -700,6 +714,7 @@ __device__ __forceinline__ void topk_row_body(SampleArgs &a) {
 #pragma unroll
                 for (int c = 0; c < 4; c++) lm = fmaxf(lm, va[u][c]);    // fmaxf drops NaN
         } else {                                                     // the row ends inside the first stage
+            if (VEC) row_place_last(va, V, 0, tid);
 #pragma unroll
             for (int u = 0; u < ROW_U; u++)
 #pragma unroll
@@ -771,29 +786,31 @@ __device__ __forceinline__ void topk_row_body(SampleArgs &a) {
         // va, vb, vc hold places s, s + 1, s + 2 of the order of examination: two stages stay in flight while one is
         // examined.  Only the row's last stage may reach past its end: it is examined under a mask, in place 1 or (short
         // rows) in the last place, which are kept out of the loop (so that the loop's stages are all of one kind).
-        auto examine = [&](const f32x4 (&v)[ROW_U], int t) {
+        auto examine = [&](f32x4 (&v)[ROW_U], int t) {
             const int st = stage_at(t);
+            if (st == last && nfull > 0) row_place_last(v, V, st, tid);   // (a row of one stage that it does not fill: placed above)
             if (st == last) row_stage<G::WCAP, true>(v, tw, twkey, list, count, st, tid, V, want, W);   // wave-uniform
             else row_stage<G::WCAP, false>(v, tw, twkey, list, count, st, tid, V, want, W);
         };
         int s = 0;
         if (nstage > 3) {                                            // (place 1 is the row's last stage, places 0 and 2 are whole)
             row_stage<G::WCAP, false>(va, tw, twkey, list, count, 0, tid, V, want, W);
-            row_load_clamped(va, x, n4, stage_at(3), tid);
+            row_load_clamped(va, x, V, stage_at(3), tid);
+            row_place_last(vb, V, last, tid);
             row_stage<G::WCAP, true>(vb, tw, twkey, list, count, last, tid, V, want, W);
-            row_load_clamped(vb, x, n4, stage_at(4), tid);
+            row_load_clamped(vb, x, V, stage_at(4), tid);
             row_stage<G::WCAP, false>(vc, tw, twkey, list, count, stage_at(2), tid, V, want, W);
-            row_load_clamped(vc, x, n4, stage_at(5), tid);
+            row_load_clamped(vc, x, V, stage_at(5), tid);
             s = 3;
             tighten();
         }
         while (s + 3 < nstage) {                                     // (places s .. s + 2 < nstage - 1: never the row's last stage)
             row_stage<G::WCAP, false>(va, tw, twkey, list, count, stage_at(s), tid, V, want, W);
-            row_load_clamped(va, x, n4, stage_at(s + 3), tid);
+            row_load_clamped(va, x, V, stage_at(s + 3), tid);
             row_stage<G::WCAP, false>(vb, tw, twkey, list, count, stage_at(s + 1), tid, V, want, W);
-            row_load_clamped(vb, x, n4, stage_at(s + 4), tid);
+            row_load_clamped(vb, x, V, stage_at(s + 4), tid);
             row_stage<G::WCAP, false>(vc, tw, twkey, list, count, stage_at(s + 2), tid, V, want, W);
-            row_load_clamped(vc, x, n4, stage_at(s + 5), tid);
+            row_load_clamped(vc, x, V, stage_at(s + 5), tid);
             s += 3;
             tighten();
         }
@@ -802,12 +819,8 @@ __device__ __forceinline__ void topk_row_body(SampleArgs &a) {
         if (s + 1 < nstage) examine(vb, s + 1);
         if (s + 2 < nstage) examine(vc, s + 2);
     } else {
-        // rows that 128-bit loads cannot take: one stage at a time, then one raise of the threshold
+        // a row of less than one 128-bit load: one stage, then one raise of the threshold
         row_stage<G::WCAP, false>(va, tw, twkey, list, count, 0, tid, V, want, W);
-        for (int s = 1; s < nstage; s++) {
-            row_load_any<false>(va, x, V, s, tid);
-            row_stage<G::WCAP, false>(va, tw, twkey, list, count, s, tid, V, want, W);
-        }
         tighten();
     }
     bound();
