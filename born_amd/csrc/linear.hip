@@ -592,8 +592,8 @@ hipError_t launch_gemm_f32(const GemmArgs &g, bool b_transposed, hipStream_t st)
     const bool fast = g.vec_a && g.vec_b && g.K % GK == 0 && (b_transposed || (g.N % 4 == 0));
     if (g.cand && (!b_transposed || !g.thr || !g.cand_cnt || g.cand_cap <= 0)) return hipErrorInvalidValue;   // candidate epilogue: W[N,K] form only
     if (g.best && (!b_transposed || !g.tokens)) return hipErrorInvalidValue;                                    // argmax epilogue: W[N,K] form only
-    const SplitPlan plan = gemm_split_plan(g.M, g.N, g.K);
     if (split_pays(g)) {
+        const SplitPlan plan = gemm_split_plan(g.M, g.N, g.K);
         // the packed operand of a call takes 6 bytes a value of the workspace: rows in chunks that fit beside the partial products
         const long long chunk_max = plan.slices > 1 ? g.M : std::max<long long>(256, (long long)(GEMM_WS_MAX / 7) / ((g.K + 63) / 64 * 64) / 256 * 256);
         const long long chunks = (g.M + chunk_max - 1) / chunk_max, rows = ((g.M + chunks - 1) / chunks + 255) / 256 * 256;
