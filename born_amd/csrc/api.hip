@@ -457,7 +457,7 @@ static int sample_impl(born_sampler *s, const float *logits, int64_t batch, int6
         keep_first(launch_topk_row(a, st, nullptr, s->path == 2));
     } else {
         // the kernels that divide every logit by the temperature take the shortcut where it is exact for this temperature
-        // (host arithmetic only: nothing is launched or waited for; per-row temperatures, above, always divide)
+        // (host arithmetic only: nothing is launched or waited for; per-row temperatures, above, are the kernels' own matter)
         if (a.T != 1.0f) {
             if (s->div_T != a.T) {
                 s->div_rcp = division_shortcut_reciprocal(a.T);

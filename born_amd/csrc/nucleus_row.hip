@@ -78,10 +78,21 @@ __device__ __forceinline__ int nuc_bin(const NucRow &r, float d) {
 }
 // (the magnitude test of the division shortcut and of the unit-temperature path: dev_common.h)
 __device__ __forceinline__ bool nuc_ordinary(float y) { return ordinary_magnitude(y); }
+// ANY_T: a row's own temperature, which the host has not seen.  The first correction's quotient lies within a hair of half
+// an ulp of y / T whatever T is (the start is off by an ulp and a half at most, the correction leaves 2^-23 of that), so
+// the second residual is exact and, with rcp = RN(1 / T), the second correction gives the correctly rounded quotient for every T
+// (Markstein's theorem: a quotient within an ulp, corrected once with a correctly rounded reciprocal).  Five instructions
+// where the division takes eleven and keeps the row from the arithmetic of usual rows.
+template <bool ANY_T>
 __device__ __forceinline__ float nuc_z_shortcut(const NucRow &r, float y) {
-    const float q = __fmul_rn(y, r.rcp);
+    float q = __fmul_rn(y, r.rcp);
+    if (ANY_T) q = __fmaf_rn(__fmaf_rn(-q, r.T, y), r.rcp, q);
     const float e = __fmaf_rn(-q, r.T, y);
     return __fmaf_rn(e, r.rcp, q);
+}
+// RN(1 / T) for ANY_T; 0 where the division is taken: T = 1 needs none, outside [2^-20, 2^20] a residual may underflow.
+__device__ __forceinline__ float nuc_reciprocal(float T) {
+    return T >= 0x1p-20f && T <= 0x1p20f && T != 1.0f ? uniform_f32(1.0f / T) : 0.0f;
 }
 
 // Visits every element of the row with its penalised logit: four at a time as f4(id of the first, y[4]), in stages of
@@ -269,8 +280,9 @@ __device__ __forceinline__ void nuc_range(const NucRow &r, int w, float &ylo, fl
 // cfg_T, cfg_p, cfg_rep: the row's temperature, top_p and repetition penalty (the handle's, or the row's own).
 // COUNTED: a frequency or presence penalty is on (the table of occurrence counts is read for ids the history holds);
 // its own instance, so that the usual one carries none of it.
+// ANY_T: cfg_rcp is the reciprocal of a temperature that the host has not tried the three-instruction quotient on.
 // REQUEST (1024 threads only): the first stage of sweeps 2 and 3 is requested before the reductions between the sweeps.
-template <int NUC_BLOCK, bool COUNTED, bool REQUEST = true>
+template <int NUC_BLOCK, bool COUNTED, bool REQUEST = true, bool ANY_T = false>
 __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const float cfg_T, const float cfg_p, const float cfg_rep,
                                                  const float cfg_dcut, const float cfg_freq, const float cfg_pres,
                                                  const float cfg_rcp) {
@@ -449,7 +461,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     // Beyond d = 80 the specified mass is 0, and so is trunc(exp(x) * 2^S) down to the clamp (S <= 61).  A seen id's
     // stored logit may exceed the penalised maximum: clamped to x = 0, some mass that the correction takes out again.
     const float scale32 = r.scale * 2.3283064365386963e-10f, nsbin = -r.sbin;
-    auto lin_z = [&](float y) { return r.T == 1.0f ? y : nuc_z_shortcut(r, y); };
+    auto lin_z = [&](float y) { return r.T == 1.0f ? y : nuc_z_shortcut<ANY_T>(r, y); };
     auto lin_put = [&](float z, auto minus) {
         const float x = z - r.m;
         const u64 q = qfix32(expneg_core(__builtin_amdgcn_fmed3f(x, -87.0f, 0.0f)), scale32);
@@ -478,7 +490,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     // ---- sweep 2: integer masses by bin
     if (lin) {
         if (r.T == 1.0f) sweep_plain(Cached(), [&](int, float y) { lin_put(y, Plus()); }, first);
-        else sweep_plain(Cached(), [&](int, float y) { lin_put(nuc_z_shortcut(r, y), Plus()); }, first);
+        else sweep_plain(Cached(), [&](int, float y) { lin_put(nuc_z_shortcut<ANY_T>(r, y), Plus()); }, first);
     } else if (r.T == 1.0f && !r.degenerate) {
         sweep(Cached(), [&](int, float y) {
             float z = y;                                             // a logit of ordinary magnitude is its own canonical form
@@ -491,7 +503,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         }, NucNoPre(), first);
     } else if (r.rcp != 0.0f && !r.degenerate) {
         sweep(Cached(), [&](int, float y) {
-            float z = nuc_z_shortcut(r, y);
+            float z = nuc_z_shortcut<ANY_T>(r, y);
             if (!nuc_ordinary(y)) z = nuc_z(r, y);                   // zeros, masked (-inf) and other unusual logits: the division
             const float d = r.m - z;
             atomicAdd(&mass[nuc_bin(r, d)], qfix(expneg(d, r.dcut), r.scale));
@@ -885,7 +897,7 @@ __global__ __launch_bounds__(BLOCK, 4) void nucleus_row_rows_kernel(SampleArgs a
         row_config_reject(a, (int)blockIdx.x);
         return;
     }
-    nucleus_row_body<BLOCK, COUNTED>(a, v.T, v.top_p, v.rep, v.dcut, v.freq, v.pres, 0.0f);   // (a row's own temperature: no shortcut)
+    nucleus_row_body<BLOCK, COUNTED, true, true>(a, v.T, v.top_p, v.rep, v.dcut, v.freq, v.pres, nuc_reciprocal(v.T));
 }
 // Per-row configurations of any kind: the rows without a top-k cut and the rows of the general kernel in one launch (a
 // launch whose workgroups all find their rows to be another kernel's still costs its 7 us at 256 rows).
@@ -900,7 +912,7 @@ __global__ __launch_bounds__(1024) void nucleus_or_general_rows_kernel(SampleArg
     bool invalid;
     if (row_config_values(a, rc, row, ROUTE_NUCLEUS, v, invalid)) {   // workgroup-uniform, before any barrier
         if (invalid) row_config_reject(a, row);
-        else nucleus_row_body<1024, COUNTED>(a, v.T, v.top_p, v.rep, v.dcut, v.freq, v.pres, 0.0f);
+        else nucleus_row_body<1024, COUNTED, true, true>(a, v.T, v.top_p, v.rep, v.dcut, v.freq, v.pres, nuc_reciprocal(v.T));
         return;
     }
     if (!row_config(a, rc, row, ROUTE_GENERAL, invalid)) return;

@@ -74,3 +74,39 @@ def test_sequence_is_the_rounded_quotient_at_the_admitted_magnitudes(shortcut, T
                 assert e == y - q * Tf                            # .. and the residual is representable (denormal at 2^-100)
                 q2 = rn32(q + e * r)
                 assert q2 == rn32(y / Tf), (T, k, int(m), sign)
+
+
+def test_two_corrections_divide_by_any_temperature(tmp_path):
+    """The quotient with two correction steps (rows that bring a temperature of their own) equals the division for every
+    significand, also for divisors whose one-step quotient does not."""
+    src = tmp_path / "two.cpp"
+    src.write_text("""#include <cmath>
+#include <cstdint>
+#include <cstring>
+extern "C" __attribute__((target("avx2,fma"))) int mismatches(float T, int exponent) {
+    const float r = 1.0f / T;
+    int bad = 0;
+    for (uint32_t m = 0; m < (1u << 23); m++) {
+        const uint32_t b = (uint32_t)(127 + exponent) << 23 | m;
+        float y;
+        std::memcpy(&y, &b, 4);
+        float q = y * r;
+        q = __builtin_fmaf(__builtin_fmaf(-q, T, y), r, q);
+        q = __builtin_fmaf(__builtin_fmaf(-q, T, y), r, q);
+        bad += q != y / T;
+    }
+    return bad;
+}
+""")
+    so = tmp_path / "libtwo.so"
+    subprocess.check_call(["g++", "-O3", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", str(src), "-o", str(so)])
+    f = ctypes.CDLL(str(so)).mismatches
+    f.argtypes = [ctypes.c_float, ctypes.c_int]
+    rng = np.random.default_rng(0)
+    hard = [np.float32(2) - np.float32(k) * np.float32(2.0 ** -23) for k in range(1, 8)]     # significands close to 2
+    easy = [np.float32(v) for v in (0.7, 0.8, 1.3, 1.0 + 2.0 ** -23, 1.5, 3.0)] + list(rng.uniform(0.3, 2.0, 8).astype(np.float32))
+    for T in hard + easy:
+        assert f(float(T), 0) == 0, T
+    for T in (hard[0], np.float32(0.7), np.float32(2.0 ** 20), np.float32(2.0 ** -20 * 1.9999999)):
+        for exponent in (-100, 99):                               # the ends of the magnitudes the kernels admit
+            assert f(float(T), exponent) == 0, (T, exponent)
