@@ -8,10 +8,12 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <new>
 #include <vector>
 
+#include "device_pool.h"
 #include "kernels.h"
 
 using namespace born;
@@ -35,6 +37,12 @@ int hip_fail(hipError_t e, const char *what) {
         hipError_t e__ = (expr);                            \
         if (e__ != hipSuccess) return hip_fail(e__, #expr); \
     } while (0)
+
+// (never destroyed: a buffer may come back while the process ends)
+DevicePool &device_pool() {
+    static DevicePool *const pool = new DevicePool;
+    return *pool;
+}
 
 std::once_flag g_cfg_once;
 hipError_t g_cfg_err = hipSuccess;
@@ -121,12 +129,20 @@ int born_rocm_device_name(int32_t device, char *buf, int64_t buf_len) {
 
 int born_rocm_alloc(int64_t bytes, void **dev_ptr) {
     if (!dev_ptr || bytes <= 0) return fail(BORN_ROCM_ERR_ARGUMENT, "sampler: alloc: bytes must be > 0 and the output non-null");
-    HIP_TRY(hipMalloc(dev_ptr, (size_t)bytes));
+    try {
+        HIP_TRY(device_pool().alloc((size_t)bytes, dev_ptr));
+    } catch (const std::exception &e) {
+        return fail(BORN_ROCM_ERR_HIP, "sampler: alloc: %s", e.what());
+    }
     return BORN_ROCM_OK;
 }
 int born_rocm_free(void *dev_ptr) {
     if (!dev_ptr) return BORN_ROCM_OK;
-    HIP_TRY(hipFree(dev_ptr));
+    try {
+        HIP_TRY(device_pool().free(dev_ptr));
+    } catch (const std::exception &e) {
+        return fail(BORN_ROCM_ERR_HIP, "sampler: free: %s", e.what());
+    }
     return BORN_ROCM_OK;
 }
 int born_rocm_h2d(void *dst_dev, const void *src_host, int64_t bytes, void *stream) {
@@ -134,6 +150,7 @@ int born_rocm_h2d(void *dst_dev, const void *src_host, int64_t bytes, void *stre
     if (bytes == 0) return BORN_ROCM_OK;
     HIP_TRY(hipMemcpyAsync(dst_dev, src_host, (size_t)bytes, hipMemcpyHostToDevice, (hipStream_t)stream));
     HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
+    device_pool().waited();
     return BORN_ROCM_OK;
 }
 int born_rocm_d2h(void *dst_host, const void *src_dev, int64_t bytes, void *stream) {
@@ -141,10 +158,12 @@ int born_rocm_d2h(void *dst_host, const void *src_dev, int64_t bytes, void *stre
     if (bytes == 0) return BORN_ROCM_OK;
     HIP_TRY(hipMemcpyAsync(dst_host, src_dev, (size_t)bytes, hipMemcpyDeviceToHost, (hipStream_t)stream));
     HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
+    device_pool().waited();
     return BORN_ROCM_OK;
 }
 int born_rocm_stream_sync(void *stream) {
     HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
+    device_pool().waited();
     return BORN_ROCM_OK;
 }
 
@@ -268,6 +287,7 @@ int born_rocm_sampler_status(born_sampler *s, void *stream) {
 int born_rocm_debug_read_counters(born_sampler *s, void *stream, unsigned long long *out, int64_t n) {
     HIP_TRY(hipMemcpyAsync(out, s->counters, (size_t)n * sizeof(unsigned long long), hipMemcpyDeviceToHost, (hipStream_t)stream));
     HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
+    device_pool().waited();
     return BORN_ROCM_OK;
 }
 #endif

@@ -102,7 +102,7 @@ __device__ __forceinline__ void row_load_clamped(f32x4 (&v)[ROW_U], const float 
 // goes to its place here (what lies past the end is masked by whoever looks at the stage).
 __device__ __forceinline__ void row_place_last(f32x4 (&v)[ROW_U], int V, int stage, int tid) {
     const int over = (4 - V) & 3;                                    // elements of the last block past the row's end
-    if (over == 0) return;                                           // uniform
+    if (__builtin_expect(over == 0, 1)) return;                      // uniform
 #pragma unroll
     for (int u = 0; u < ROW_U; u++) {
         if (((stage * ROW_U + u) * ROW_BLOCK + tid) == V >> 2) {
