@@ -1,12 +1,14 @@
 // Device buffers handed out and taken back by born_rocm_alloc and born_rocm_free.  The backend's operations return a new
 // buffer each: an MNIST network's forward pass makes eleven, and hipMalloc and hipFree (which waits
-// for the device) took most of its time (64 images: 347 us, 154 like this).  A freed buffer of up to POOL_BUFFER_MAX bytes is kept, up to
+// for the device) took most of its time (64 images: 339 us, 170 like this).  A freed buffer of up to POOL_BUFFER_MAX bytes is kept, up to
 // POOL_TOTAL_MAX bytes and POOL_COUNT_MAX buffers in all, the oldest given back first, all of them where memory runs out.
 //
 // A kept buffer may still be in use by work on any stream of its device.  It is handed out again only once the whole device
-// has been waited for after it was freed: what hipFree promises.  One wait serves every buffer freed before it.  Where
-// the program has waited for the device's results since the free (the usual end of a pass) that wait finds the device idle; else a
-// fresh buffer costs less than draining the device, until the pool is full.
+// has been waited for after it was freed.  hipFree does that wait: the smallest kept buffer goes back to the device, and every
+// buffer freed before that call is idle from then on.  (hipDeviceSynchronize would spare that buffer, but it is refused and ends the
+// capture where a stream is being captured in relaxed mode, in which hipMalloc and hipFree are allowed.)  Where the program has waited
+// for the device's results since the free (the usual end of a pass) the wait finds the device idle; else a fresh buffer costs less
+// than draining the device, until the pool is full.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -48,45 +50,21 @@ public:
         int dev = 0;
         if (bytes > POOL_BUFFER_MAX || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= DEVICES) return fresh_or_release(bytes, out);
         const size_t size = (bytes + GRAIN - 1) / GRAIN * GRAIN;
-        Kept got = {nullptr, 0, 0, 0, 0};
-        bool wait = false;
-        uint64_t upto = 0;
-        {
-            std::lock_guard<std::mutex> g(mu);
-            auto best = kept.end();
-            for (auto it = kept.begin(); it != kept.end(); ++it) {   // the oldest of the size: the first to have been waited for
-                if (it->dev == dev && it->bytes == size) {
-                    best = it;
-                    break;
-                }
-            }
-            if (best != kept.end()) {
-                wait = best->freed > idle[dev];
-                if (!wait || best->waits < waits || total + size > POOL_TOTAL_MAX || kept.size() >= POOL_COUNT_MAX) {
-                    got = *best;
-                    kept.erase(best);
-                    total -= size;
-                    upto = frees;
-                    if (!wait) live[got.p] = Live{size, dev};
-                }
-            }
-        }
-        if (got.p && wait) {
-            const hipError_t e = hipDeviceSynchronize();             // (outside the lock: other threads go on)
-            std::lock_guard<std::mutex> g(mu);
+        if (take(dev, size, out)) return hipSuccess;
+        Kept back;
+        uint64_t upto;
+        if (give_back(dev, size, &back, &upto)) {
+            const hipError_t e = hipFree(back.p);                    // (outside the lock: other threads go on)
+            std::unique_lock<std::mutex> g(mu);
             if (e == hipSuccess) {
                 if (upto > idle[dev]) idle[dev] = upto;
-                live[got.p] = Live{size, dev};
-            } else {                                                 // (not now, for instance while a stream is captured: kept on)
+            } else {                                                 // (not now: kept on)
                 (void)hipGetLastError();
-                kept.push_back(got);
-                total += size;
-                got.p = nullptr;
+                kept.push_front(back);
+                total += back.bytes;
             }
-        }
-        if (got.p) {
-            *out = got.p;
-            return hipSuccess;
+            g.unlock();
+            if (take(dev, size, out)) return hipSuccess;
         }
         const hipError_t e = fresh_or_release(size, out);
         if (e == hipSuccess) {
@@ -124,6 +102,40 @@ public:
     }
 
 private:
+    // The oldest kept buffer of the size, where it is idle.
+    bool take(int dev, size_t size, void **out) {
+        std::lock_guard<std::mutex> g(mu);
+        for (auto it = kept.begin(); it != kept.end(); ++it) {
+            if (it->dev != dev || it->bytes != size) continue;
+            if (it->freed > idle[dev]) return false;                 // (so are the later ones)
+            live[it->p] = Live{size, dev};
+            *out = it->p;
+            total -= size;
+            kept.erase(it);
+            return true;
+        }
+        return false;
+    }
+
+    // Takes the smallest kept buffer of the device out, to be freed for the wait, where a buffer of the size is kept and the wait is
+    // worth it.
+    bool give_back(int dev, size_t size, Kept *back, uint64_t *upto) {
+        std::lock_guard<std::mutex> g(mu);
+        auto found = kept.end(), least = kept.end();
+        for (auto it = kept.begin(); it != kept.end(); ++it) {
+            if (it->dev != dev) continue;
+            if (it->bytes == size && found == kept.end()) found = it;
+            if (least == kept.end() || it->bytes < least->bytes) least = it;
+        }
+        if (found == kept.end()) return false;
+        if (found->waits >= waits && total + size <= POOL_TOTAL_MAX && kept.size() < POOL_COUNT_MAX) return false;
+        *back = *least;
+        *upto = frees;
+        total -= least->bytes;
+        kept.erase(least);
+        return true;
+    }
+
     hipError_t fresh_or_release(size_t bytes, void **out) {
         hipError_t e = hipMalloc(out, bytes);
         if (e != hipErrorOutOfMemory) return e;
