@@ -94,8 +94,8 @@ __device__ __forceinline__ void row_load_fast(f32x4 (&v)[ROW_U], const float *x,
 __device__ __forceinline__ void row_load_clamped(f32x4 (&v)[ROW_U], const float *x, int V, int stage, int tid) {
 #pragma unroll
     for (int u = 0; u < ROW_U; u++) {
-        const int j = min(((stage * ROW_U + u) * ROW_BLOCK + tid) << 2, V - 4);
-        v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(x + j));
+        const unsigned j = (unsigned)min(((stage * ROW_U + u) * ROW_BLOCK + tid) << 2, V - 4);
+        v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(reinterpret_cast<const char *>(x) + j * 4u));   // (bytes of a row: below 2^21)
     }
 }
 // A row whose length is no multiple of four: its last block was loaded from where the row's last four elements start, and
@@ -788,9 +788,10 @@ __device__ __forceinline__ void topk_row_body(SampleArgs &a) {
         // rows) in the last place, which are kept out of the loop (so that the loop's stages are all of one kind).
         auto examine = [&](f32x4 (&v)[ROW_U], int t) {
             const int st = stage_at(t);
-            if (st == last && nfull > 0) row_place_last(v, V, st, tid);   // (a row of one stage that it does not fill: placed above)
-            if (st == last) row_stage<G::WCAP, true>(v, tw, twkey, list, count, st, tid, V, want, W);   // wave-uniform
-            else row_stage<G::WCAP, false>(v, tw, twkey, list, count, st, tid, V, want, W);
+            if (st == last) {                                        // wave-uniform
+                if (nfull > 0) row_place_last(v, V, st, tid);        // (a row of one stage that it does not fill: placed above)
+                row_stage<G::WCAP, true>(v, tw, twkey, list, count, st, tid, V, want, W);
+            } else row_stage<G::WCAP, false>(v, tw, twkey, list, count, st, tid, V, want, W);
         };
         int s = 0;
         if (nstage > 3) {                                            // (place 1 is the row's last stage, places 0 and 2 are whole)
