@@ -65,7 +65,8 @@ int born_rocm_device_name(int32_t device, char *buf, int64_t buf_len);
 
 /* Device buffers — Born's RawTensor is host-only (internal/tensor/raw.go:42-46,139-141); these give the Go
  * layer its DeviceBuffer handle.  Copies are enqueued on `stream` and are synchronous with respect to the host
- * when the host pointer is pageable. */
+ * when the host pointer is pageable.  Up to 256 MiB of freed buffers (each of at most 32 MiB) are kept for the next allocation
+ * of their size; one is handed out again only after the device was waited for since its free, as hipFree would. */
 int born_rocm_alloc(int64_t bytes, void **dev_ptr);
 int born_rocm_free(void *dev_ptr);
 int born_rocm_h2d(void *dst_dev, const void *src_host, int64_t bytes, void *stream);
