@@ -21,6 +21,10 @@ constexpr int WAVE = 64;
 // no more alignment than that on this part, and a wave's 1024 bytes then touch nine 128-byte lines in place of eight.  (Such
 // rows one logit at a time, one load in flight: 96 rows of 100 003 under settings of their own took 160.7 us; like this 96.7.)
 typedef float row_f32x4 __attribute__((ext_vector_type(4), aligned(4)));
+// Rows that start 16-byte aligned; others are read by 128-bit loads where they are long (each kernel says from where on).
+__host__ __device__ __forceinline__ bool rows_aligned(const float *logits, long long stride) {
+    return (stride & 3) == 0 && (((unsigned long long)logits) & 15) == 0;
+}
 
 // Pointers into LDS (and, where a pointer travels in a struct, into global memory) that keep their address space through structs and calls that are not inlined: a plain
 // pointer there makes the compiler fall back to flat loads, stores and atomics, which are slower than their

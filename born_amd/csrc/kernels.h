@@ -64,6 +64,9 @@ struct SampleArgs {
     // RN(1 / T) when the three-instruction division shortcut equals the correctly rounded y / T for every y it is
     // applied to (division.cpp decides, on the host), else 0: the kernels then divide
     float rcp_T;
+    // set by the launcher of the three-sweep kernels: how many blocks of four logits of a row they read by 128-bit loads (V / 4, or 0
+    // for short rows that are not aligned)
+    int row_blocks;
 };
 
 // division.cpp
@@ -99,6 +102,7 @@ struct SpecArgs {
     unsigned long long *run_mass; // [B][SPEC_CHUNKS][1024] residual mass of each thread's run of ids
     int *status;
     int mass_shift;
+    int wide;                     // set by the launcher: the rows are read by 128-bit loads
 };
 
 // C[M,N] = A[M,K] * B (+ bias[N]); B is [N,K] (b_transposed, the weight of a linear layer) or [K,N].

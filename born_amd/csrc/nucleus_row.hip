@@ -59,7 +59,7 @@ typedef row_f32x4 nuc_f32x4;
 
 struct NucRow {                               // uniform per workgroup
     const float *x;
-    int V;
+    int V, n4;                                // n4: the blocks of four that are read by 128-bit loads
     bool penal, degenerate;
     bool masked = false;                      // the visitor replaces every seen logit by `skip`; the seen ids are visited apart
     float skip = 0.0f;
@@ -96,8 +96,8 @@ __device__ __forceinline__ float nuc_reciprocal(float T) {
 }
 
 // Visits every element of the row with its penalised logit: four at a time as f4(id of the first, y[4]), in stages of
-// U float4 per thread, the next stage's loads in flight while this one is visited; what is left over one at a time as
-// f1(id, y).
+// U float4 per thread, the next stage's loads in flight while this one is visited; what is left over (and every element of a
+// short row that is not aligned) one at a time as f1(id, y).
 // AHEAD: the row's partial last stage is loaded ahead like the whole ones (3 % faster on short rows, where the few
 // blocks left over are a third of the row; measured slower on long ones and in the single-sweep kernel).
 // `pre` runs once before the first element is visited, with the first stage's loads already in flight (work that
@@ -107,8 +107,14 @@ struct NucNoPre {
 };
 // NT: the row is read once (non-temporal loads: measured 6 % faster for a single sweep); a kernel that sweeps the row
 // again wants it to stay in the caches.
-template <bool NT>
-__device__ __forceinline__ nuc_f32x4 nuc_load4(const nuc_f32x4 *p) {
+// Block i of the row.  512 threads (two rows to a CU: 128 registers a lane, all of them in use): a 32-bit offset from the row's
+// uniform address; with a 64-bit address per load in flight the sampling kernel spilled nine registers (1024 x 152 064, top-p alone:
+// 315.7 us, 313.1 like this).  With 1024 threads it is the offsets that spill, in the instance without the early request.
+static_assert(WIDE_MAX_VOCAB < (1 << 30), "a row's bytes fit 32 bits");
+template <int NUC_BLOCK, bool NT>
+__device__ __forceinline__ nuc_f32x4 nuc_load4(const float *x, int i) {
+    const nuc_f32x4 *p = NUC_BLOCK == 512 ? reinterpret_cast<const nuc_f32x4 *>(reinterpret_cast<const char *>(x) + (unsigned)i * 16u)
+                                          : reinterpret_cast<const nuc_f32x4 *>(x) + i;
     return NT ? __builtin_nontemporal_load(p) : *p;
 }
 // PLAIN: the caller knows that the row has no penalties (a loop of its own without the penalty code: the visitor's
@@ -155,26 +161,25 @@ __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 
         if (!PLAIN && r.penal && ((bm[j >> 5] >> (j & 31)) & 1u)) y = r.masked ? r.skip : penalise_seen(y, r.rep, r.counts, j, r.freq, r.pres);
         f1(j, y);
     };
-    const int n4 = r.V >> 2;
+    const int n4 = r.n4;
     constexpr int NUC_U = NucGeom<NUC_BLOCK>::U;
     if constexpr (!AHEAD) {
         const int nfull = n4 / (NUC_U * NUC_BLOCK);
-        const nuc_f32x4 *x4 = reinterpret_cast<const nuc_f32x4 *>(r.x);
         if (nfull > 0) {
             // Two stages a turn, each loaded while the other is visited, so that no register is copied; the last
             // one or two stages in a loop of their own.
             nuc_f32x4 va[NUC_U], vb[NUC_U];
 #pragma unroll
-            for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(x4 + u * NUC_BLOCK + tid);
+            for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NUC_BLOCK, NT>(r.x, u * NUC_BLOCK + tid);
             pre();
             int s = 0;
             for (; s + 2 < nfull; s += 2) {
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4<NT>(x4 + ((s + 1) * NUC_U + u) * NUC_BLOCK + tid);
+                for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4<NUC_BLOCK, NT>(r.x, ((s + 1) * NUC_U + u) * NUC_BLOCK + tid);
 #pragma unroll
                 for (int u = 0; u < NUC_U; u++) visit4(va[u], ((s * NUC_U + u) * NUC_BLOCK + tid) << 2);
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(x4 + ((s + 2) * NUC_U + u) * NUC_BLOCK + tid);
+                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NUC_BLOCK, NT>(r.x, ((s + 2) * NUC_U + u) * NUC_BLOCK + tid);
 #pragma unroll
                 for (int u = 0; u < NUC_U; u++) visit4(vb[u], (((s + 1) * NUC_U + u) * NUC_BLOCK + tid) << 2);
             }
@@ -183,18 +188,17 @@ __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 
                 for (int u = 0; u < NUC_U; u++) visit4(va[u], ((s * NUC_U + u) * NUC_BLOCK + tid) << 2);
                 if (++s >= nfull) break;
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(x4 + (s * NUC_U + u) * NUC_BLOCK + tid);
+                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NUC_BLOCK, NT>(r.x, (s * NUC_U + u) * NUC_BLOCK + tid);
             }
         } else {
             pre();
         }
         for (int i = nfull * NUC_U * NUC_BLOCK + tid; i < n4; i += NUC_BLOCK) {
-            const nuc_f32x4 q = nuc_load4<NT>(x4 + i);
+            const nuc_f32x4 q = nuc_load4<NUC_BLOCK, NT>(r.x, i);
             visit4(q, i << 2);
         }
     } else {
         const int nst = (n4 + NUC_U * NUC_BLOCK - 1) / (NUC_U * NUC_BLOCK);      // stages, the last one whole or partial
-        const nuc_f32x4 *x4 = reinterpret_cast<const nuc_f32x4 *>(r.x);
         if (nst > 0) {
             // Loads are unconditional, of a block index clamped to the row's last block (a load under a condition makes
             // the compiler wait for every load in flight); only the visits of the last stage ask whether the block exists.
@@ -205,12 +209,12 @@ __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 
                 for (int u = 0; u < NUC_U; u++) va[u] = first[u];
             } else {
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(x4 + min(u * NUC_BLOCK + tid, lastb));
+                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NUC_BLOCK, NT>(r.x, min(u * NUC_BLOCK + tid, lastb));
             }
             pre();
             for (int s = 0; s + 1 < nst; s++) {
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4<NT>(x4 + min(((s + 1) * NUC_U + u) * NUC_BLOCK + tid, lastb));
+                for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4<NUC_BLOCK, NT>(r.x, min(((s + 1) * NUC_U + u) * NUC_BLOCK + tid, lastb));
 #pragma unroll
                 for (int u = 0; u < NUC_U; u++) visit4(va[u], ((s * NUC_U + u) * NUC_BLOCK + tid) << 2);
 #pragma unroll
@@ -232,11 +236,10 @@ __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 
 // CUs idle are otherwise a memory latency each.
 template <int NUC_BLOCK, bool NT>
 __device__ __forceinline__ void nuc_request_first(const NucRow &r, nuc_f32x4 (&first)[NucGeom<NUC_BLOCK>::U]) {
-    const int n4 = r.V >> 2;
+    const int n4 = r.n4;
     if (n4 > 0) {
-        const nuc_f32x4 *x4 = reinterpret_cast<const nuc_f32x4 *>(r.x);
 #pragma unroll
-        for (int u = 0; u < NucGeom<NUC_BLOCK>::U; u++) first[u] = nuc_load4<NT>(x4 + min(u * NUC_BLOCK + (int)threadIdx.x, n4 - 1));
+        for (int u = 0; u < NucGeom<NUC_BLOCK>::U; u++) first[u] = nuc_load4<NUC_BLOCK, NT>(r.x, min(u * NUC_BLOCK + (int)threadIdx.x, n4 - 1));
     }
 }
 // Visits every element of the row as f(id, penalised logit).
@@ -306,6 +309,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     NucRow r;
     r.x = a.logits + (long long)row * a.row_stride;
     r.V = V;
+    r.n4 = a.row_blocks;
     r.T = cfg_T;
     r.rcp = cfg_rcp;
     r.rep = cfg_rep;
@@ -957,6 +961,7 @@ __global__ __launch_bounds__(NUC_BLOCK, 4) void token_logprob_kernel(SampleArgs 
     NucRow r;
     r.x = a.logits + (long long)row * a.row_stride;
     r.V = V;
+    r.n4 = V >> 2;
     r.T = a.T;
     r.rep = a.rep;
     r.scale = 0.0f;
@@ -1172,8 +1177,15 @@ int device_cu_count() {
 
 // A batch of at most this many bytes of logits is re-read from the L2s by sweeps 2 and 3 (eight L2s of 4 MiB).
 constexpr long long NUC_L2_RESIDENT_BYTES = 16ll << 20;
+// Rows that start at any four bytes are read by 128-bit loads from this length on: a shorter one leaves most lanes without such a
+// load and reads its ragged end after it, a second round trip to memory (22 x 101: 11.6 us one logit at a time, 12.8 by 128-bit loads;
+// 600 x 1001 27.1 and 28.2; 2039 27.1 and 26.0; 8191 35.8 and 28.1).
+constexpr int NUC_LOADS4_FROM = 1536;
+static int row_blocks(const SampleArgs &a) { return a.V >= NUC_LOADS4_FROM || rows_aligned(a.logits, a.row_stride) ? a.V >> 2 : 0; }
 template <int BLOCK>
-static void launch_nucleus_of(const SampleArgs &a, hipStream_t st, const RowConfigs *rows) {
+static void launch_nucleus_of(const SampleArgs &args, hipStream_t st, const RowConfigs *rows) {
+    SampleArgs a = args;
+    a.row_blocks = row_blocks(args);
     const dim3 gr((unsigned)a.B), bl(BLOCK);
     const size_t lds = nucleus_lds_bytes_of<BLOCK>(a.V);
     if (rows) {
@@ -1194,7 +1206,9 @@ static bool nucleus_two_per_cu(const SampleArgs &a, bool two_per_cu) {
 }
 // The rows without a top-k cut and the general kernel's rows of a batch with per-row configurations: one launch where
 // the former would get a workgroup of 1024 threads anyway, else the two kernels one after the other.
-hipError_t launch_nucleus_and_general_rows(const SampleArgs &a, hipStream_t st, const RowConfigs &rows, bool two_per_cu) {
+hipError_t launch_nucleus_and_general_rows(const SampleArgs &args, hipStream_t st, const RowConfigs &rows, bool two_per_cu) {
+    SampleArgs a = args;
+    a.row_blocks = row_blocks(args);
     if (nucleus_two_per_cu(a, two_per_cu)) {
         const hipError_t e = launch_nucleus_row(a, st, &rows, two_per_cu);
         if (e != hipSuccess) return e;
