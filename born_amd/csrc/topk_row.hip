@@ -50,6 +50,11 @@
 
 namespace born {
 
+enum { ROW_ALIGNED, ROW_ANY, ROW_SHORT };     // how the rows are read (topk_row_body)
+// Rows of any start are read by 128-bit loads from this length on, with 1024 threads to a row and with 512.
+constexpr int ROW_LOADS4_FROM = 7168, ROW512_LOADS4_FROM = 3072;
+static_assert(ROW_LOADS4_FROM <= 8192, "a shorter row is one stage, of 512 threads too");
+
 #define BORN_ROW_BLOCK 1024
 #include "topk_row_impl.h"
 #undef BORN_ROW_BLOCK
@@ -67,56 +72,63 @@ hipError_t launch_cand_rows(const SampleArgs &a, const float *thr, const unsigne
 }
 
 
-template <bool VEC, bool LOCAL>
-static void launch_topk_row_as(const SampleArgs &a, hipStream_t st, const RowConfigs *rows, bool two_per_cu) {
+template <int MODE, bool LOCAL>
+static void launch_topk_row_as(const SampleArgs &a, hipStream_t st, const RowConfigs *rows, bool boosts, bool two) {
     const dim3 gr((unsigned)a.B), bl(ROW_BLOCK);
+    if (two) {
+        hipLaunchKernelGGL((row512::topk_row_kernel<MODE, LOCAL, 0>), gr, dim3(row512::ROW_BLOCK), row512::row_pool_bytes<0>(), st, a);
+        return;
+    }
+    if (rows)
+        hipLaunchKernelGGL((topk_row_rows_kernel<MODE, LOCAL>), gr, bl, row_pool_bytes<1>(), st, a, *rows);
+    else if (a.top_k > TOPK_SMALL_K || boosts)
+        hipLaunchKernelGGL((topk_row_kernel<MODE, LOCAL, 1>), gr, bl, row_pool_bytes<1>(), st, a);
+    else
+        hipLaunchKernelGGL((topk_row_kernel<MODE, LOCAL, 0>), gr, bl, row_pool_bytes<0>(), st, a);
+}
+
+template <int MODE>
+static void launch_topk_row_mode(const SampleArgs &a, hipStream_t st, const RowConfigs *rows, bool boosts, bool two) {
+    if (a.local_counts) launch_topk_row_as<MODE, true>(a, st, rows, boosts, two);
+    else launch_topk_row_as<MODE, false>(a, st, rows, boosts, two);
+}
+
+hipError_t launch_topk_row(const SampleArgs &a, hipStream_t st, const RowConfigs *rows, bool two_per_cu) {
     // (penalties that raise logits add seen ids to the candidates: the instance with room for 1024 of them)
     const bool boosts = a.history && (a.rep < 1.0f || ((a.hist_counts || a.local_counts) && (a.freq < 0.0f || a.pres < 0.0f)));
     // More rows than CUs: a CU holds one 1024-thread workgroup of this kernel at a time, so the rows beyond the first
     // round would wait for a CU to come free; with 512 threads two rows share a CU, and one row's finish (one wave, no
     // memory traffic) runs beside the other's stream.  The instance for top_k <= 128 only: its LDS fits twice.
-    if (!rows && a.top_k <= TOPK_SMALL_K && !boosts && (two_per_cu || a.B > device_cu_count())) {
-        hipLaunchKernelGGL((row512::topk_row_kernel<VEC, LOCAL, 0>), gr, dim3(row512::ROW_BLOCK), row512::row_pool_bytes<0>(), st, a);
-        return;
-    }
-    if (rows)
-        hipLaunchKernelGGL((topk_row_rows_kernel<VEC, LOCAL>), gr, bl, row_pool_bytes<1>(), st, a, *rows);
-    else if (a.top_k > TOPK_SMALL_K || boosts)
-        hipLaunchKernelGGL((topk_row_kernel<VEC, LOCAL, 1>), gr, bl, row_pool_bytes<1>(), st, a);
-    else
-        hipLaunchKernelGGL((topk_row_kernel<VEC, LOCAL, 0>), gr, bl, row_pool_bytes<0>(), st, a);
-}
-
-hipError_t launch_topk_row(const SampleArgs &a, hipStream_t st, const RowConfigs *rows, bool two_per_cu) {
-    if (a.V >= 4) {                                                  // a row holds a 128-bit load
-        if (a.local_counts) launch_topk_row_as<true, true>(a, st, rows, two_per_cu); else launch_topk_row_as<true, false>(a, st, rows, two_per_cu);
-    } else {
-        if (a.local_counts) launch_topk_row_as<false, true>(a, st, rows, two_per_cu); else launch_topk_row_as<false, false>(a, st, rows, two_per_cu);
-    }
+    const bool two = !rows && a.top_k <= TOPK_SMALL_K && !boosts && (two_per_cu || a.B > device_cu_count());
+    if (rows_aligned(a.logits, a.row_stride)) launch_topk_row_mode<ROW_ALIGNED>(a, st, rows, boosts, two);
+    else if (a.V >= (two ? ROW512_LOADS4_FROM : ROW_LOADS4_FROM)) launch_topk_row_mode<ROW_ANY>(a, st, rows, boosts, two);
+    else launch_topk_row_mode<ROW_SHORT>(a, st, rows, boosts, two);
     return hipGetLastError();
 }
 
 // The LDS pools are dynamic allocations beyond 64 KiB: every instance is told so once.
-template <bool VEC, bool LOCAL>
+template <int MODE, bool LOCAL>
 static hipError_t configure_topk_row_as() {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(topk_row_kernel<VEC, LOCAL, 0>), hipFuncAttributeMaxDynamicSharedMemorySize,
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(topk_row_kernel<MODE, LOCAL, 0>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)row_pool_bytes<0>());
     if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(topk_row_kernel<VEC, LOCAL, 1>), hipFuncAttributeMaxDynamicSharedMemorySize,
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(topk_row_kernel<MODE, LOCAL, 1>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)row_pool_bytes<1>());
     if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(topk_row_rows_kernel<VEC, LOCAL>), hipFuncAttributeMaxDynamicSharedMemorySize,
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(topk_row_rows_kernel<MODE, LOCAL>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)row_pool_bytes<1>());
     if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(row512::topk_row_kernel<VEC, LOCAL, 0>),
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(row512::topk_row_kernel<MODE, LOCAL, 0>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)row512::row_pool_bytes<0>());
     return e;
 }
 hipError_t configure_topk_row() {
-    hipError_t e = configure_topk_row_as<true, false>();
-    if (e == hipSuccess) e = configure_topk_row_as<true, true>();
-    if (e == hipSuccess) e = configure_topk_row_as<false, false>();
-    if (e == hipSuccess) e = configure_topk_row_as<false, true>();
+    hipError_t e = configure_topk_row_as<ROW_ALIGNED, false>();
+    if (e == hipSuccess) e = configure_topk_row_as<ROW_ALIGNED, true>();
+    if (e == hipSuccess) e = configure_topk_row_as<ROW_ANY, false>();
+    if (e == hipSuccess) e = configure_topk_row_as<ROW_ANY, true>();
+    if (e == hipSuccess) e = configure_topk_row_as<ROW_SHORT, false>();
+    if (e == hipSuccess) e = configure_topk_row_as<ROW_SHORT, true>();
     return e;
 }
 

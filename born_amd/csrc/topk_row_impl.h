@@ -65,14 +65,14 @@ __device__ __forceinline__ int row_margin(int k) { return k <= TOPK_SMALL_K ? 16
 typedef row_f32x4 f32x4;
 
 // row_load_any: one stage of ROW_U consecutive blocks of ROW_BLOCK float4 in row order, for the row's ragged end
-// and anything past the end (-inf fill).  Used by the sweeps of the exact selection and by rows of less than one 128-bit
-// load.
-template <bool VEC>
+// and anything past the end (-inf fill).  Used by the sweeps of the exact selection and by rows of any start that end in
+// their first stage.
+template <bool WIDE>
 __device__ __forceinline__ void row_load_any(f32x4 (&v)[ROW_U], const float *x, int V, int stage, int tid) {
 #pragma unroll
     for (int u = 0; u < ROW_U; u++) {
         const int j = ((stage * ROW_U + u) * ROW_BLOCK + tid) * 4;
-        if (VEC && j + 3 < V) {
+        if (WIDE && j + 3 < V) {
             v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(x + j));
         } else {
 #pragma unroll
@@ -88,18 +88,18 @@ __device__ __forceinline__ void row_load_fast(f32x4 (&v)[ROW_U], const float *x,
         v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(x) + ((stage * ROW_U + u) * ROW_BLOCK + tid));
 }
 
-// Block indices clamped into the row: a stage that reaches past the row's end (or lies wholly beyond it) re-reads the
-// row's last four elements instead of branching around its loads, so that the loads of later stages can stay in flight (a
-// load under a condition makes the compiler wait for every load in flight).  V >= 4 (VEC).
-__device__ __forceinline__ void row_load_clamped(f32x4 (&v)[ROW_U], const float *x, int V, int stage, int tid) {
+// The place of every load clamped into the row: a stage that reaches past the row's end (or lies wholly beyond it) re-reads
+// the row's last load at `end` instead of branching around its loads, so that the loads of later stages can stay in flight
+// (a load under a condition makes the compiler wait for every load in flight).
+__device__ __forceinline__ void row_load_clamped(f32x4 (&v)[ROW_U], const float *x, int end, int stage, int tid) {
 #pragma unroll
     for (int u = 0; u < ROW_U; u++) {
-        const unsigned j = (unsigned)min(((stage * ROW_U + u) * ROW_BLOCK + tid) << 2, V - 4);
+        const unsigned j = (unsigned)min(((stage * ROW_U + u) * ROW_BLOCK + tid) << 2, end);
         v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(reinterpret_cast<const char *>(x) + j * 4u));   // (bytes of a row: below 2^21)
     }
 }
-// A row whose length is no multiple of four: its last block was loaded from where the row's last four elements start, and
-// goes to its place here (what lies past the end is masked by whoever looks at the stage).
+// A row of any start whose length is no multiple of four: its last block was loaded from where the row's last four elements
+// start, and goes to its place here (what lies past the end is masked by whoever looks at the stage).
 __device__ __forceinline__ void row_place_last(f32x4 (&v)[ROW_U], int V, int stage, int tid) {
     const int over = (4 - V) & 3;                                    // elements of the last block past the row's end
     if (__builtin_expect(over == 0, 1)) return;                      // uniform
@@ -307,11 +307,11 @@ __device__ __forceinline__ u32 row_pick(const u32 *wthr, int need) {
 
 // Visits every element of the row as f(id, logit), in row order, the loads of one stage in flight while the stage
 // before it is visited.
-template <bool VEC, class F>
+template <bool WIDE, class F>
 __device__ __forceinline__ void row_foreach(const float *x, int V, int tid, F f) {
     const int n4 = (V + 3) >> 2;
     const int nstage = ((n4 + ROW_BLOCK - 1) / ROW_BLOCK + ROW_U - 1) / ROW_U;
-    const int nfull = VEC ? (V >> 2) / (ROW_U * ROW_BLOCK) : 0;
+    const int nfull = WIDE ? (V >> 2) / (ROW_U * ROW_BLOCK) : 0;
     f32x4 va[ROW_U], vb[ROW_U];
     auto visit = [&](const f32x4 (&v)[ROW_U], int stage) {
 #pragma unroll
@@ -336,14 +336,14 @@ __device__ __forceinline__ void row_foreach(const float *x, int V, int tid, F f)
         s = nfull;
     }
     for (; s < nstage; s++) {
-        row_load_any<VEC>(va, x, V, s, tid);
+        row_load_any<WIDE>(va, x, V, s, tid);
         visit(va, s);
     }
 }
 
 // Exact selection of the row's top_k rank keys for any input (every thread of the workgroup calls it).
 // pool: the workgroup's LDS pool; s_n, s_x: two shared ints.
-template <bool VEC, bool LOCAL, class G>
+template <bool WIDE, bool LOCAL, class G>
 __device__ __forceinline__ void row_select_exact(const SampleArgs &a, int row, const float *x, int hlen, const int *h, float u_row,
                                                  u64 *pool, int *s_n, int *s_x) {
     const int tid = threadIdx.x, V = a.V, k = a.top_k;
@@ -409,7 +409,7 @@ __device__ __forceinline__ void row_select_exact(const SampleArgs &a, int row, c
         {
             const u64 pf = prefix;
             const int pl = plen;
-            row_foreach<VEC>(x, V, tid, [&](int j, float xv) {
+            row_foreach<WIDE>(x, V, tid, [&](int j, float xv) {
                 const u64 key = rank_key(j, xv);
                 if (pl == 0 || (key >> (64 - pl)) == pf) atomicAdd(&hist[(u32)(key >> (64 - pl - db)) & (u32)(nb - 1)], 1u);
             });
@@ -460,7 +460,7 @@ __device__ __forceinline__ void row_select_exact(const SampleArgs &a, int row, c
     const u64 lo_key = plen == 64 ? prefix : prefix << (64 - plen);
     if (tid == 0) s_n[0] = 0;
     __syncthreads();
-    row_foreach<VEC>(x, V, tid, [&](int j, float xv) {
+    row_foreach<WIDE>(x, V, tid, [&](int j, float xv) {
         const u64 key = rank_key(j, xv);
         if (key >= lo_key) {
             const int pos = atomicAdd(&s_n[0], 1);
@@ -602,9 +602,17 @@ __device__ __forceinline__ void row_resolve_ties(const u64 *K, const u32 *Khi, c
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// MODE: how the rows are read.
+//   ROW_ALIGNED  Every row starts 16-byte aligned and its pitch is a multiple of four floats, so that the block that holds
+//                the row's last logit lies inside the pitch.
+//   ROW_ANY      Rows that start at any four bytes.  Their last four logits are read in that block's stead and moved into
+//                place (row_place_last), which would cost an aligned row 1 % (1 x 32 000 9.8 -> 9.9 us).
+//   ROW_SHORT    Such a row below ROW_LOADS4_FROM (one stage): one logit at a time, nothing requested ahead.  22 x 2039: 7.8 us,
+//                8.3 like ROW_ANY; 22 x 6001 9.4 and 9.6; 22 x 8191 9.4 and 9.2.  600 x 2039, 512 threads to a row: 14.5 and 14.9;
+//                4001 15.4 and 15.0.
 // LOCAL: the frequency / presence penalties are on and the kernel counts the occurrences itself (SampleArgs::local_counts).
 // KC: the instance's sizes (RowGeom).
-template <bool VEC, bool LOCAL, int KC>
+template <int MODE, bool LOCAL, int KC>
 __device__ __forceinline__ void topk_row_body(SampleArgs &a) {
     using G = RowGeom<KC>;
     extern __shared__ __align__(16) u64 row_pool[];                 // G::POOL words
@@ -658,14 +666,15 @@ __device__ __forceinline__ void topk_row_body(SampleArgs &a) {
     const int last = nstage - 1;
     // the stage examined in place t (a place past the last one: a stage past the row's end, whose loads all re-read
     // the row's last block)
-    auto stage_at = [&](int t) { return !VEC || nstage < 3 || t == 0 ? t : t == 1 ? last : t < nstage ? t - 1 : nstage; };
+    auto stage_at = [&](int t) { return nstage < 3 || t == 0 ? t : t == 1 ? last : t < nstage ? t - 1 : nstage; };
     f32x4 va[ROW_U], vb[ROW_U], vc[ROW_U];
-    if (VEC) {
-        row_load_clamped(va, x, V, 0, tid);
-        row_load_clamped(vb, x, V, stage_at(1), tid);                // in flight during the search for the first threshold
-        row_load_clamped(vc, x, V, stage_at(2), tid);
-    } else {
+    const int end = MODE == ROW_ALIGNED ? (V - 1) & ~3 : V - 4;      // where the row's last load starts
+    if (MODE == ROW_SHORT) {
         row_load_any<false>(va, x, V, 0, tid);
+    } else {
+        row_load_clamped(va, x, end, 0, tid);
+        row_load_clamped(vb, x, end, stage_at(1), tid);              // in flight during the search for the first threshold
+        row_load_clamped(vc, x, end, stage_at(2), tid);
     }
 
     if (tid == 0) {
@@ -708,13 +717,13 @@ __device__ __forceinline__ void topk_row_body(SampleArgs &a) {
     const int need = (k + aw - 1) / aw;                              // <= act, but for a top_k beyond the lanes that hold data: no threshold then
     {
         float lm = -INFINITY;
-        if (!VEC || nfull > 0) {                                     // (without 128-bit loads, elements past the end were filled with -inf)
+        if (MODE == ROW_SHORT || nfull > 0) {                        // (a short row's elements past the end were filled with -inf)
 #pragma unroll
             for (int u = 0; u < ROW_U; u++)
 #pragma unroll
                 for (int c = 0; c < 4; c++) lm = fmaxf(lm, va[u][c]);    // fmaxf drops NaN
         } else {                                                     // the row ends inside the first stage
-            if (VEC) row_place_last(va, V, 0, tid);
+            if (MODE == ROW_ANY) row_place_last(va, V, 0, tid);
 #pragma unroll
             for (int u = 0; u < ROW_U; u++)
 #pragma unroll
@@ -782,36 +791,36 @@ __device__ __forceinline__ void topk_row_body(SampleArgs &a) {
             zbw_of = twkey;
         }
     };
-    if (VEC) {
+    if (MODE != ROW_SHORT) {
         // va, vb, vc hold places s, s + 1, s + 2 of the order of examination: two stages stay in flight while one is
         // examined.  Only the row's last stage may reach past its end: it is examined under a mask, in place 1 or (short
         // rows) in the last place, which are kept out of the loop (so that the loop's stages are all of one kind).
         auto examine = [&](f32x4 (&v)[ROW_U], int t) {
             const int st = stage_at(t);
             if (st == last) {                                        // wave-uniform
-                if (nfull > 0) row_place_last(v, V, st, tid);        // (a row of one stage that it does not fill: placed above)
+                if (MODE == ROW_ANY && nfull > 0) row_place_last(v, V, st, tid);   // (a row of one stage that it does not fill: placed above)
                 row_stage<G::WCAP, true>(v, tw, twkey, list, count, st, tid, V, want, W);
             } else row_stage<G::WCAP, false>(v, tw, twkey, list, count, st, tid, V, want, W);
         };
         int s = 0;
         if (nstage > 3) {                                            // (place 1 is the row's last stage, places 0 and 2 are whole)
             row_stage<G::WCAP, false>(va, tw, twkey, list, count, 0, tid, V, want, W);
-            row_load_clamped(va, x, V, stage_at(3), tid);
-            row_place_last(vb, V, last, tid);
+            row_load_clamped(va, x, end, stage_at(3), tid);
+            if (MODE == ROW_ANY) row_place_last(vb, V, last, tid);
             row_stage<G::WCAP, true>(vb, tw, twkey, list, count, last, tid, V, want, W);
-            row_load_clamped(vb, x, V, stage_at(4), tid);
+            row_load_clamped(vb, x, end, stage_at(4), tid);
             row_stage<G::WCAP, false>(vc, tw, twkey, list, count, stage_at(2), tid, V, want, W);
-            row_load_clamped(vc, x, V, stage_at(5), tid);
+            row_load_clamped(vc, x, end, stage_at(5), tid);
             s = 3;
             tighten();
         }
         while (s + 3 < nstage) {                                     // (places s .. s + 2 < nstage - 1: never the row's last stage)
             row_stage<G::WCAP, false>(va, tw, twkey, list, count, stage_at(s), tid, V, want, W);
-            row_load_clamped(va, x, V, stage_at(s + 3), tid);
+            row_load_clamped(va, x, end, stage_at(s + 3), tid);
             row_stage<G::WCAP, false>(vb, tw, twkey, list, count, stage_at(s + 1), tid, V, want, W);
-            row_load_clamped(vb, x, V, stage_at(s + 4), tid);
+            row_load_clamped(vb, x, end, stage_at(s + 4), tid);
             row_stage<G::WCAP, false>(vc, tw, twkey, list, count, stage_at(s + 2), tid, V, want, W);
-            row_load_clamped(vc, x, V, stage_at(s + 5), tid);
+            row_load_clamped(vc, x, end, stage_at(s + 5), tid);
             s += 3;
             tighten();
         }
@@ -820,7 +829,7 @@ __device__ __forceinline__ void topk_row_body(SampleArgs &a) {
         if (s + 1 < nstage) examine(vb, s + 1);
         if (s + 2 < nstage) examine(vc, s + 2);
     } else {
-        // a row of less than one 128-bit load: one stage, then one raise of the threshold
+        // one stage, then one raise of the threshold
         row_stage<G::WCAP, false>(va, tw, twkey, list, count, 0, tid, V, want, W);
         tighten();
     }
@@ -1000,7 +1009,7 @@ __device__ __forceinline__ void topk_row_body(SampleArgs &a) {
     ROW_STAMP(3);
     ok = ok && s_valid >= k;
     if (!ok) {                                                       // wave-uniform, workgroup-uniform
-        (row_select_exact<VEC, LOCAL, G>)(a, row, x, hlen, h, u_row, pool, &s_n, s_x);
+        (row_select_exact<MODE != ROW_SHORT, LOCAL, G>)(a, row, x, hlen, h, u_row, pool, &s_n, s_x);
         return;
     }
 
@@ -1254,14 +1263,14 @@ __global__ __launch_bounds__(ROW_BLOCK) void cand_row_kernel(SampleArgs a, const
 
 #endif
 
-template <bool VEC, bool LOCAL, int KC>
+template <int MODE, bool LOCAL, int KC>
 __global__ __launch_bounds__(ROW_BLOCK) void topk_row_kernel(SampleArgs a) {
-    (topk_row_body<VEC, LOCAL, KC>)(a);                              // (in parentheses: found by scope, not through the argument's namespace)
+    (topk_row_body<MODE, LOCAL, KC>)(a);                              // (in parentheses: found by scope, not through the argument's namespace)
 }
 #if BORN_ROW_BLOCK == 1024
 // The batch carries a configuration per row (row_config.h): the workgroup takes the row only if it is its own.  A row
 // may ask for any top_k the kernel serves, so these instances have the larger sizes.
-template <bool VEC, bool LOCAL>
+template <int MODE, bool LOCAL>
 __global__ __launch_bounds__(ROW_BLOCK) void topk_row_rows_kernel(SampleArgs a, RowConfigs rc) {
     bool invalid;
     if (!row_config(a, rc, (int)blockIdx.x, ROUTE_TOPK, invalid)) return;   // workgroup-uniform, before any barrier
@@ -1269,7 +1278,7 @@ __global__ __launch_bounds__(ROW_BLOCK) void topk_row_rows_kernel(SampleArgs a, 
         row_config_reject(a, (int)blockIdx.x);
         return;
     }
-    (topk_row_body<VEC, LOCAL, 1>)(a);
+    (topk_row_body<MODE, LOCAL, 1>)(a);
 }
 #endif
 
