@@ -17,7 +17,7 @@ static_assert(WIDE_BINS == WIDE_LIST_CAP, "the histogram scan and the list scan 
 struct WideCtx {
     const BORN_GLOBAL float *x;
     int V;
-    bool has_hist, count_mode;
+    bool vec, has_hist, count_mode;          // vec: the row is read by 128-bit loads
     float T, rcp, rep, m, scale, dcut;   // rcp: RN(1 / T) where the division shortcut is exact for T, else 0
     const unsigned *counts;  // occurrences of each id in the row's history (frequency / presence penalties), or null
     float freq, pres;
@@ -41,10 +41,11 @@ __device__ __forceinline__ float wide_z(const WideCtx &c, float y) {
     return canon(y / c.T);
 }
 
-// Visit every element of the row as (id, penalised logit).  The row is read in stages of WIDE_U float4 per thread, the
+// Visit every element of the row as (id, penalised logit).  The row (vec) is read in stages of WIDE_U float4 per thread, the
 // loads of the next stage in flight while this one is visited (the loop body has no branch around a load, so
 // the compiler can wait for exactly the stage it needs); what is left of the row is read block by block.
 constexpr int WIDE_U = 4;
+constexpr int WIDE_LOADS4_FROM = 4096;        // .. aligned or from here on; shorter ones element by element (22 x 2051: 26.6 us, 27.3 by 128-bit loads)
 typedef row_f32x4 wide_f32x4;
 
 __device__ __forceinline__ void wide_load_stage(wide_f32x4 (&v)[WIDE_U], const BORN_GLOBAL float *x, int stage, int tid) {
@@ -77,28 +78,36 @@ __device__ __forceinline__ void wide_visit_stage(const WideCtx &c, const wide_f3
 template <class F>
 __device__ __forceinline__ void wide_foreach(const WideCtx &c, F f) {
     const int tid = threadIdx.x;
-    const int n4 = c.V >> 2;
-    const int nfull = n4 / (WIDE_U * WIDE_BLOCK);              // whole stages
-    if (nfull > 0) {
-        wide_f32x4 va[WIDE_U], vb[WIDE_U];
-        wide_load_stage(va, c.x, 0, tid);
-        for (int s = 0; s + 1 < nfull; s++) {
-            wide_load_stage(vb, c.x, s + 1, tid);
-            wide_visit_stage(c, va, s, tid, f);
+    if (c.vec) {
+        const int n4 = c.V >> 2;
+        const int nfull = n4 / (WIDE_U * WIDE_BLOCK);              // whole stages
+        if (nfull > 0) {
+            wide_f32x4 va[WIDE_U], vb[WIDE_U];
+            wide_load_stage(va, c.x, 0, tid);
+            for (int s = 0; s + 1 < nfull; s++) {
+                wide_load_stage(vb, c.x, s + 1, tid);
+                wide_visit_stage(c, va, s, tid, f);
 #pragma unroll
-            for (int u = 0; u < WIDE_U; u++) va[u] = vb[u];
+                for (int u = 0; u < WIDE_U; u++) va[u] = vb[u];
+            }
+            wide_visit_stage(c, va, nfull - 1, tid, f);
         }
-        wide_visit_stage(c, va, nfull - 1, tid, f);
-    }
-    const BORN_GLOBAL wide_f32x4 *x4 = (const BORN_GLOBAL wide_f32x4 *)c.x;
-    for (int i = nfull * WIDE_U * WIDE_BLOCK + tid; i < n4; i += WIDE_BLOCK) {
-        const wide_f32x4 q = x4[i];
-        wide_visit4(c, q, i << 2, f);
-    }
-    for (int j = (n4 << 2) + tid; j < c.V; j += WIDE_BLOCK) {
-        float y = c.x[j];
-        if (c.has_hist && ((c.bm[j >> 5] >> (j & 31)) & 1u)) y = penalise_seen(y, c.rep, c.counts, j, c.freq, c.pres);
-        f(j, y);
+        const BORN_GLOBAL wide_f32x4 *x4 = (const BORN_GLOBAL wide_f32x4 *)c.x;
+        for (int i = nfull * WIDE_U * WIDE_BLOCK + tid; i < n4; i += WIDE_BLOCK) {
+            const wide_f32x4 q = x4[i];
+            wide_visit4(c, q, i << 2, f);
+        }
+        for (int j = (n4 << 2) + tid; j < c.V; j += WIDE_BLOCK) {
+            float y = c.x[j];
+            if (c.has_hist && ((c.bm[j >> 5] >> (j & 31)) & 1u)) y = penalise_seen(y, c.rep, c.counts, j, c.freq, c.pres);
+            f(j, y);
+        }
+    } else {
+        for (int j = tid; j < c.V; j += WIDE_BLOCK) {
+            float y = c.x[j];
+            if (c.has_hist && ((c.bm[j >> 5] >> (j & 31)) & 1u)) y = penalise_seen(y, c.rep, c.counts, j, c.freq, c.pres);
+            f(j, y);
+        }
     }
 }
 
@@ -328,6 +337,7 @@ __device__ __forceinline__ void wide_row(const SampleArgs &a, const int row, lds
     WideCtx c;
     c.x = (const BORN_GLOBAL float *)(a.logits + (long long)row * a.row_stride);
     c.V = V;
+    c.vec = V >= WIDE_LOADS4_FROM || rows_aligned(a.logits, a.row_stride);
     c.T = uniform_f32(a.T);
     c.rcp = uniform_f32(a.rcp_T);
     c.rep = uniform_f32(a.rep);

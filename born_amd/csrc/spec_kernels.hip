@@ -19,13 +19,16 @@ namespace born {
 
 constexpr int SPEC_BLOCK = 1024;
 constexpr int SPEC_NF4 = 8;                   // float4 per thread and array that the stats kernel keeps in registers
+// Rows that start at any four bytes are read by 128-bit loads from this length on (600 x 3 x 1001: 48.5 us one logit at a time, 49.9 by
+// 128-bit loads; 2039 55.6 and 53.1; 3001 62.6 and 56.2).
+constexpr int SPEC_LOADS4_FROM = 1536;
 constexpr int SPEC_RESIDENT_V = SPEC_NF4 * SPEC_BLOCK * 4;
 
 typedef row_f32x4 spec_f32x4;
 
 template <class F>
-__device__ __forceinline__ void spec_foreach(const float *x, int V, F f) {
-    const int tid = threadIdx.x, n4 = V >> 2;
+__device__ __forceinline__ void spec_foreach(const float *x, int V, bool wide, F f) {
+    const int tid = threadIdx.x, n4 = wide ? V >> 2 : 0;
     const spec_f32x4 *x4 = reinterpret_cast<const spec_f32x4 *>(x);
     for (int i = tid; i < n4; i += SPEC_BLOCK) {
         const spec_f32x4 q = x4[i];
@@ -37,7 +40,7 @@ __device__ __forceinline__ void spec_foreach(const float *x, int V, F f) {
 
 // One workgroup per (sequence, position, distribution): blockIdx.x = 2 * row + (0 target | 1 draft).  The two
 // distributions of a position are independent, and twice as many work items spread better over the CUs.
-// RESIDENT: V <= SPEC_RESIDENT_V.
+// RESIDENT: V <= SPEC_RESIDENT_V and a row that 128-bit loads suit (SpecArgs::wide).  TAIL: V may be no multiple of four.
 // z = canon(x / T); UNIT: T == 1, where the division is the identity and is not computed at all.
 template <bool UNIT>
 __device__ __forceinline__ float spec_z(float x, float T, float rcp) {
@@ -73,7 +76,7 @@ __device__ __forceinline__ u64 spec_usual_mass(float x, float m, float T, float 
     return qfix32(expneg_core(__builtin_amdgcn_fmed3f(z - m, -87.0f, 0.0f)), scale32);
 }
 
-template <bool RESIDENT, bool UNIT>
+template <bool RESIDENT, bool UNIT, bool TAIL>
 __global__ __launch_bounds__(SPEC_BLOCK) void spec_stats_kernel(SpecArgs a) {
     __shared__ BlockScratch scr;
     const int tid = threadIdx.x;
@@ -99,8 +102,9 @@ __global__ __launch_bounds__(SPEC_BLOCK) void spec_stats_kernel(SpecArgs a) {
     if (RESIDENT) {
         const int n4 = V >> 2;
         spec_f32x4 t[SPEC_NF4];
-        const int jt = (n4 << 2) + tid;                              // the row's last V % 4 logits, one per thread
-        const float last = jt < V ? x[jt] : -INFINITY;
+        const int jt = TAIL ? (n4 << 2) + tid : V;                   // the row's last V % 4 logits, one per thread
+        float last = -INFINITY;
+        if (TAIL && jt < V) last = x[jt];
         m = fmaxf(m, last);
 #pragma unroll
         for (int i = 0; i < SPEC_NF4; i++) {
@@ -125,7 +129,7 @@ __global__ __launch_bounds__(SPEC_BLOCK) void spec_stats_kernel(SpecArgs a) {
                     for (int c = 0; c < 4; c++) sum += spec_usual_mass<UNIT>(t[i][c], m, T, rcp, scale32);
                 }
             }
-            if (jt < V) sum += spec_usual_mass<UNIT>(last, m, T, rcp, scale32);
+            if (TAIL && jt < V) sum += spec_usual_mass<UNIT>(last, m, T, rcp, scale32);
         } else if (m > -INFINITY) {                                  // (uniform) m - z is a number: +inf for a masked logit, no mass
 #pragma unroll
             for (int i = 0; i < SPEC_NF4; i++) {
@@ -134,7 +138,7 @@ __global__ __launch_bounds__(SPEC_BLOCK) void spec_stats_kernel(SpecArgs a) {
                     for (int c = 0; c < 4; c++) sum += qfix(expneg(m - spec_z<UNIT>(t[i][c], T, rcp)), scale);
                 }
             }
-            if (jt < V) sum += qfix(expneg(m - spec_z<UNIT>(last, T, rcp)), scale);
+            if (TAIL && jt < V) sum += qfix(expneg(m - spec_z<UNIT>(last, T, rcp)), scale);
         } else {                                                     // nothing finite: (-inf) - (-inf) := 0 for every logit
 #pragma unroll
             for (int i = 0; i < SPEC_NF4; i++) {
@@ -143,12 +147,12 @@ __global__ __launch_bounds__(SPEC_BLOCK) void spec_stats_kernel(SpecArgs a) {
                     for (int c = 0; c < 4; c++) sum += qfix(emass(spec_z<UNIT>(t[i][c], T, rcp), m), scale);
                 }
             }
-            if (jt < V) sum += qfix(emass(spec_z<UNIT>(last, T, rcp), m), scale);
+            if (TAIL && jt < V) sum += qfix(emass(spec_z<UNIT>(last, T, rcp), m), scale);
         }
     } else {
-        spec_foreach(x, V, [&](float v) { m = fmaxf(m, spec_z<UNIT>(v, T, rcp)); });
+        spec_foreach(x, V, a.wide != 0, [&](float v) { m = fmaxf(m, spec_z<UNIT>(v, T, rcp)); });
         m = block_max_f32<SPEC_BLOCK>(m, &scr);
-        spec_foreach(x, V, [&](float v) { sum += qfix(emass(spec_z<UNIT>(v, T, rcp), m), scale); });
+        spec_foreach(x, V, a.wide != 0, [&](float v) { sum += qfix(emass(spec_z<UNIT>(v, T, rcp), m), scale); });
     }
     u64 Z;
     block_inclusive_scan_u64<SPEC_BLOCK>(sum, &scr, &Z);
@@ -370,21 +374,20 @@ __global__ __launch_bounds__(SPEC_BLOCK) void spec_pick_kernel(SpecArgs a) {
     }
 }
 
-hipError_t launch_spec_verify(const SpecArgs &a, hipStream_t st) {
-    const bool resident = a.V <= SPEC_RESIDENT_V;
-    const unsigned stats_grid = (unsigned)(2 * a.B * a.G + (a.bonus ? a.B : 0));
-    const dim3 sg(stats_grid), sb(SPEC_BLOCK);
-    if (resident) {
-        if (a.T == 1.0f)
-            hipLaunchKernelGGL((spec_stats_kernel<true, true>), sg, sb, 0, st, a);
-        else
-            hipLaunchKernelGGL((spec_stats_kernel<true, false>), sg, sb, 0, st, a);
-    } else {
-        if (a.T == 1.0f)
-            hipLaunchKernelGGL((spec_stats_kernel<false, true>), sg, sb, 0, st, a);
-        else
-            hipLaunchKernelGGL((spec_stats_kernel<false, false>), sg, sb, 0, st, a);
-    }
+template <bool RESIDENT, bool TAIL>
+static void launch_spec_stats(const SpecArgs &a, hipStream_t st) {
+    const dim3 sg((unsigned)(2 * a.B * a.G + (a.bonus ? a.B : 0))), sb(SPEC_BLOCK);
+    if (a.T == 1.0f) hipLaunchKernelGGL((spec_stats_kernel<RESIDENT, true, TAIL>), sg, sb, 0, st, a);
+    else hipLaunchKernelGGL((spec_stats_kernel<RESIDENT, false, TAIL>), sg, sb, 0, st, a);
+}
+
+hipError_t launch_spec_verify(const SpecArgs &args, hipStream_t st) {
+    SpecArgs a = args;
+    a.wide = a.V >= SPEC_LOADS4_FROM || ((a.V & 3) == 0 && rows_aligned(a.target, a.t_seq) && rows_aligned(a.draft, a.d_seq) &&
+                                       (!a.bonus || rows_aligned(a.bonus, a.b_seq)));
+    if (!a.wide || a.V > SPEC_RESIDENT_V) launch_spec_stats<false, false>(a, st);
+    else if (a.V & 3) launch_spec_stats<true, true>(a, st);
+    else launch_spec_stats<true, false>(a, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(spec_residual_kernel, dim3((unsigned)(a.B * SPEC_CHUNKS)), dim3(SPEC_BLOCK), 0, st, a);
