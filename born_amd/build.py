@@ -11,7 +11,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libborn_rocm.so")
 SOURCES = ["api.hip", "basic_kernels.hip", "topk_row.hip", "nucleus_row.hip", "sample_wide.hip", "spec_kernels.hip", "linear.hip", "gemm_split.hip", "tensor_ops.hip",
-           "division.cpp"]          # .cpp: host code only
+           "gemm_plan.cpp", "division.cpp"]          # .cpp: host code only
 
 # -ffp-contract=off and correctly rounded fp32 division: every floating-point step of the
 # fixed-point pipeline must be a single IEEE rounding, identical on host and device.

@@ -27,10 +27,8 @@
 // be lost - are noticed at the end (by non-finite results; by flags the pack keeps of its operand; by a scan of the
 // weights where either those flags or a result near zero make their magnitudes matter), and the wave recomputes its
 // block with fp32 matrix instructions (gemm_recompute), so such operands give what they always gave.
-#include <algorithm>
-#include <cmath>
-
 #include "gemm_epilogue.h"
+#include "gemm_plan.h"
 
 namespace born {
 
@@ -39,9 +37,6 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef u32 u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int SG = 32;                        // k-values of a group (two matrix instructions deep)
-constexpr int SG_BYTES = 6 * 1024;            // packed bytes of a group and a block of 32 rows
-constexpr int PACK_GROUPS = 4;                // groups a workgroup of the pack handles
 constexpr float SPLIT_BIG = 0x1p30f;          // against a partner up to this the loss stays below 2^-96 per product
 constexpr float SPLIT_SMALL_RESULT = 0x1p-60f;   // .. which a result at or above this does not feel
 
@@ -495,55 +490,6 @@ __global__ __launch_bounds__(64 * NW * KH) void gemm_split_kernel(SplitArgs s) {
     }
     static_assert(gemm_stage_bytes(NW * KH) <= (2 * A_STAGE + SW * W_STAGE) * 16, "the epilogue's stage");
     gemm_finish<EPI, 16, NW * KH>(g, fin, mfin, ncol, lds);
-}
-
-size_t gemm_split_workspace(int M, int K) {
-    const size_t ng = (size_t)(K + 2 * SG - 1) / (2 * SG) * 2, mb = (size_t)(M + 31) / 32;
-    const size_t bytes = ng * mb * SG_BYTES + 8 * SG_BYTES + mb * ((ng + PACK_GROUPS - 1) / PACK_GROUPS) * sizeof(uint2);   // (8 blocks: the last tile's copy may run on)
-    return (bytes + 255) / 256 * 256;
-}
-
-// The four tiles, and what one of them takes at K = 4096 on a part that is nearly idle and on one where every CU has one
-// (power: the clock falls from 2.4 to about 1.9 GHz), in microseconds.
-//   64 x 128   four waves' columns twice along K          70 .. 121   decode batches: no matrix work for padding
-//   128 x 128  four waves' columns twice along K         120 .. 180   few columns: tiles for all CUs
-//   128 x 256  eight waves' columns                      222 .. 317
-//   256 x 256  eight waves' columns                      405 .. 532   the most products per byte moved through LDS
-struct SplitTile {
-    int rows, cols;
-    float idle_us, busy_us;
-};
-constexpr SplitTile SPLIT_TILES[4] = {{64, 128, 70.f, 121.f}, {128, 128, 120.f, 180.f}, {128, 256, 222.f, 317.f}, {256, 256, 405.f, 532.f}};
-
-// Tile and slices of K with the least expected time: rounds of tiles over the CUs, each with about 8 us to fill and drain;
-// slices write and re-read partial products (about 4 TB/s) and cost one more launch.  Measured against the choice on
-// twenty shapes: within 15 % of the best of all of them (256 x 4096 -> 4096: 128 x 128 in four slices 61 us, 128 us unsplit,
-// 425 us as 256 x 256; 300 x 2528 -> 21539: 128 x 256 179 us, 64 x 128 212, 256 x 256 288).
-SplitPlan gemm_split_plan(int M, int N, int K) {
-    constexpr float CUS = 256.f;
-    SplitPlan best = {0, 1};
-    float least = INFINITY;
-    for (int t = 0; t < 4; t++) {
-        const SplitTile &T = SPLIT_TILES[t];
-        const float tiles = (float)((M + T.rows - 1) / T.rows) * (float)((N + T.cols - 1) / T.cols);
-        for (int slices = 1; slices <= 16 && (slices == 1 || K / slices >= 256); slices *= 2) {
-            if (slices > 1 && tiles * slices > 2.f * CUS) break;
-            const float wgs = tiles * slices, rounds = std::ceil(wgs / CUS);
-            const float share = std::min(1.f, wgs / CUS);
-            float us = rounds * ((T.idle_us + (T.busy_us - T.idle_us) * share) * ((float)K / 4096.f) / slices + 8.f);
-            if (slices > 1) us += 3.f + (float)M * (float)N * 4.f * (slices + 1) / 4e6f;
-            if (us < least) {
-                least = us;
-                best.tile = t;
-                best.slices = slices;
-            }
-        }
-    }
-    // whole pairs of groups to a slice, none of them empty
-    const int pairs = (K + 2 * SG - 1) / (2 * SG), per = (pairs + best.slices - 1) / best.slices;
-    best.slices = (pairs + per - 1) / per;
-    best.kslice = per * 2 * SG;
-    return best;
 }
 
 template <int IB, int NW, int KH, int SW, int EPI>

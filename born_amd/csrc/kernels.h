@@ -131,14 +131,9 @@ constexpr int LM_CAND_CAP = 4096;          // candidates a row's list holds
 constexpr int LM_SAMPLE_MAX = 1024;        // columns of the strided sample the thresholds come from
 constexpr int LM_CAND_TARGET = 1536;       // candidates per row the thresholds aim at (the count varies by about a third around it)
 hipError_t launch_gemm_f32(const GemmArgs &g, bool b_transposed, hipStream_t st);
-// The same product on the bf16 matrix cores at fp32 precision (gemm_split.hip).  A plan: which of its tiles, how many slices of K
-// (kslice values each).  `workspace` holds gemm_split_workspace(M, K) bytes, 256-byte aligned; g.ksplit > 1: as above.
-struct SplitPlan {
-    int tile, slices, kslice;
-};
-SplitPlan gemm_split_plan(int M, int N, int K);
+// The same product on the bf16 matrix cores (gemm_split.hip), where gemm_split_pays, in the tile of its plan (gemm_plan.h).
+// `workspace` holds gemm_split_workspace(M, K) bytes, 256-byte aligned; g.ksplit > 1: as above.
 hipError_t launch_gemm_split(const GemmArgs &g, bool b_transposed, int tile, void *workspace, hipStream_t st);
-size_t gemm_split_workspace(int M, int K);
 
 // Index map of an element-wise or shape operation over a (collapsed) result of nd dimensions: shape[d] and,
 // per operand, the element stride that result dimension d walks in it (0 where the operand is broadcast).

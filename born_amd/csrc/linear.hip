@@ -17,7 +17,7 @@
 // operand reads of 16 lanes cover all banks); within a group of 8 k-values lanes 0-31 feed k..k+3 and lanes
 // 32-63 feed k+4..k+7 to four consecutive MFMAs (the order of the k-sum is free, both operands use the same one).
 //
-// Products of 3 GFLOP and more over more than 32 rows go to the bf16 matrix cores instead (gemm_split.hip, split_pays below).
+// Products of 3 GFLOP and more over more than 32 rows go to the bf16 matrix cores instead (gemm_split.hip, gemm_split_pays).
 //
 // Workgroup ids are dealt round-robin to the 8 XCDs; the tile order makes the workgroups that share a tile
 // column of B (all M-tiles of that column) land on the same XCD back to back, so that B is fetched from HBM
@@ -27,6 +27,7 @@
 #include <vector>
 #include "dev_common.h"
 #include "gemm_epilogue.h"
+#include "gemm_plan.h"
 #include "kernels.h"
 
 namespace born {
@@ -564,15 +565,6 @@ static void launch_splitk_sum(const GemmArgs &g, hipStream_t st) {
     else hipLaunchKernelGGL(gemm_splitk_sum_kernel<0>, sg, sb, 0, st, g, mn);
 }
 
-// Whether the product goes to the bf16 matrix cores (gemm_split.hip).  They do an fp32 product's work about twice as fast,
-// after a launch that packs the left operand: below about 3 GFLOP the fp32 tiles, finer and split along K, are level
-// (64 x 4096 -> 4096, 2.1 GFLOP: 33 us against 28; 1024^3 24 against 32; 128 x 4096 -> 4096, 4.3: 72 against 41; 200 x 1056 ->
-// 8272, 3.5: 72 against 45); a batch of up to 32 rows is bound by reading the weights (32 x 4096 -> 32000: 118 against 130 us).
-// A caller that names the tile height keeps it.
-static bool split_pays(const GemmArgs &g) {
-    return !g.bm && g.M > 32 && 2.0 * (double)g.M * (double)g.N * (double)g.K >= 3e9;
-}
-
 hipError_t launch_gemm_f32(const GemmArgs &g, bool b_transposed, hipStream_t st) {
     int bm = g.bm ? g.bm : g.M <= 16 ? 16 : g.M <= 32 ? 32 : g.M <= 64 ? 64 : 128;
     // A product of few tiles leaves most of the device idle (1024 x 1024 x 1024 is 64 tiles of 128 x 128 for 256 CUs):
@@ -592,7 +584,7 @@ hipError_t launch_gemm_f32(const GemmArgs &g, bool b_transposed, hipStream_t st)
     const bool fast = g.vec_a && g.vec_b && g.K % GK == 0 && (b_transposed || (g.N % 4 == 0));
     if (g.cand && (!b_transposed || !g.thr || !g.cand_cnt || g.cand_cap <= 0)) return hipErrorInvalidValue;   // candidate epilogue: W[N,K] form only
     if (g.best && (!b_transposed || !g.tokens)) return hipErrorInvalidValue;                                    // argmax epilogue: W[N,K] form only
-    if (split_pays(g)) {
+    if (!g.bm && gemm_split_pays(g.M, g.N, g.K, g.ldb)) {                  // (a caller that names the tile height keeps it)
         const SplitPlan plan = gemm_split_plan(g.M, g.N, g.K);
         // the packed operand of a call takes 6 bytes a value of the workspace: rows in chunks that fit beside the partial products
         const long long chunk_max = plan.slices > 1 ? g.M : std::max<long long>(256, (long long)(GEMM_WS_MAX / 7) / ((g.K + 63) / 64 * 64) / 256 * 256);
