@@ -52,7 +52,7 @@ namespace born {
 
 enum { ROW_ALIGNED, ROW_ANY, ROW_SHORT };     // how the rows are read (topk_row_body)
 // Rows of any start are read by 128-bit loads from this length on, with 1024 threads to a row and with 512.
-constexpr int ROW_LOADS4_FROM = 7168, ROW512_LOADS4_FROM = 3072;
+constexpr int ROW_LOADS4_FROM = 8192, ROW512_LOADS4_FROM = 3584;
 static_assert(ROW_LOADS4_FROM <= 8192, "a shorter row is one stage, of 512 threads too");
 
 #define BORN_ROW_BLOCK 1024

@@ -608,8 +608,8 @@ __device__ __forceinline__ void row_resolve_ties(const u64 *K, const u32 *Khi, c
 //   ROW_ANY      Rows that start at any four bytes.  Their last four logits are read in that block's stead and moved into
 //                place (row_place_last), which would cost an aligned row 1 % (1 x 32 000 9.8 -> 9.9 us).
 //   ROW_SHORT    Such a row below ROW_LOADS4_FROM (one stage): one logit at a time, nothing requested ahead.  22 x 2039: 7.8 us,
-//                8.3 like ROW_ANY; 22 x 6001 9.4 and 9.6; 22 x 8191 9.4 and 9.2.  600 x 2039, 512 threads to a row: 14.5 and 14.9;
-//                4001 15.4 and 15.0.
+//                8.5 like ROW_ANY; 22 x 7169 9.6 and 10.0; 22 x 8191 9.6 and 9.5.  600 x 3073, 512 threads to a row: 15.4 and 15.8;
+//                4001 15.7 and 15.3.
 // LOCAL: the frequency / presence penalties are on and the kernel counts the occurrences itself (SampleArgs::local_counts).
 // KC: the instance's sizes (RowGeom).
 template <int MODE, bool LOCAL, int KC>

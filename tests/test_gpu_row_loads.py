@@ -6,8 +6,8 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-# around 1536 (three sweeps, verification), 3072 and 7168 (top-k with 512 and 1024 threads), 4096 (general kernel)
-LENGTHS = [1000, 1535, 1537, 3071, 3073, 4095, 4097, 7167, 7169]
+# around 1536 (three sweeps, verification), 3584 and 8192 (top-k with 512 and 1024 threads), 4096 (general kernel)
+LENGTHS = [1000, 1535, 1537, 3583, 3585, 4095, 4097, 8191, 8193]
 FORMS = [(0, 0), (1, 0), (0, 3), (2, 1)]                    # (floats in front of the first row, floats between rows beyond a multiple of 4)
 
 
