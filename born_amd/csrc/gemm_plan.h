@@ -8,12 +8,17 @@ constexpr int SG = 32;                        // k-values of a group (two matrix
 constexpr int SG_BYTES = 6 * 1024;            // packed bytes of a group and a block of 32 rows
 constexpr int PACK_GROUPS = 4;                // groups a workgroup of the pack handles
 
-// A plan: which of the tiles, how many slices of K (kslice values each).
+// The workspace of a stream (linear.hip): the packed operand and the partial products of the slices of K.
+constexpr size_t GEMM_WS_MAX = (size_t)64 << 20, GEMM_WS_MIN = (size_t)8 << 20;
+
+// A plan: which of the tiles, how many slices of K (kslice values each), how many rows at a time (M, or a multiple of the
+// tile's height; 0 where the fp32 tiles have the product after all).
 struct SplitPlan {
-    int tile, slices, kslice;
+    int tile, slices, kslice, rows;
 };
 bool gemm_split_pays(int M, int N, int K, long long ldb);
 SplitPlan gemm_split_plan(int M, int N, int K);
 size_t gemm_split_workspace(int M, int K);    // bytes of the packed operand and its flags, a multiple of 256
+size_t gemm_split_bytes(const SplitPlan &p, int rows, int N, int K);   // .. and of the partial products behind it
 
 }  // namespace born

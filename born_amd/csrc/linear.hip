@@ -422,7 +422,6 @@ __global__ __launch_bounds__(256) void gemm_splitk_sum_kernel(GemmArgs g, long l
 // one, kept until the process ends (calls on one stream are ordered, so they can share; calls on different streams cannot;
 // a buffer once handed out stays, so that a graph captured with it stays good).  Null when none can be had now (the stream
 // is being captured, too many streams, out of memory): the product is then computed without.
-constexpr size_t GEMM_WS_MAX = (size_t)64 << 20, GEMM_WS_MIN = (size_t)8 << 20;
 static float *gemm_workspace(hipStream_t st, size_t bytes) {
     struct Entry {
         int dev;
@@ -586,16 +585,13 @@ hipError_t launch_gemm_f32(const GemmArgs &g, bool b_transposed, hipStream_t st)
     if (g.best && (!b_transposed || !g.tokens)) return hipErrorInvalidValue;                                    // argmax epilogue: W[N,K] form only
     if (!g.bm && gemm_split_pays(g.M, g.N, g.K, g.ldb)) {                  // (a caller that names the tile height keeps it)
         const SplitPlan plan = gemm_split_plan(g.M, g.N, g.K);
-        // the packed operand of a call takes 6 bytes a value of the workspace: rows in chunks that fit beside the partial products
-        const long long chunk_max = plan.slices > 1 ? g.M : std::max<long long>(256, (long long)(GEMM_WS_MAX / 7) / ((g.K + 63) / 64 * 64) / 256 * 256);
-        const long long chunks = (g.M + chunk_max - 1) / chunk_max, rows = ((g.M + chunks - 1) / chunks + 255) / 256 * 256;
-        const long long most = std::min<long long>(rows, g.M);
-        const size_t packed = gemm_split_workspace((int)most, g.K);
-        float *ws = gemm_workspace(st, packed + (plan.slices > 1 ? (size_t)plan.slices * (size_t)g.M * (size_t)g.N * sizeof(float) : 0));
+        const int most = std::min(plan.rows, g.M);
+        const size_t packed = gemm_split_workspace(most, g.K);
+        float *ws = plan.rows ? gemm_workspace(st, gemm_split_bytes(plan, most, g.N, g.K)) : nullptr;
         if (ws) {
-            for (long long r0 = 0; r0 < g.M; r0 += rows) {
+            for (long long r0 = 0; r0 < g.M; r0 += plan.rows) {
                 GemmArgs gc = g;
-                gc.M = (int)std::min<long long>(rows, g.M - r0);
+                gc.M = (int)std::min<long long>(plan.rows, g.M - r0);
                 gc.a += r0 * g.lda;
                 if (g.c) gc.c += r0 * g.ldc;
                 if (g.best) gc.best += r0 * LM_BEST_PITCH;

@@ -9,6 +9,13 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 WRAPPER = """
 #include "gemm_plan.h"
+extern "C" long long budget() { return born::GEMM_WS_MAX; }
+// [tile, slices, kslice, rows, bytes]
+extern "C" void plan(int M, int N, int K, long long *out) {
+    const born::SplitPlan p = born::gemm_split_plan(M, N, K);
+    out[0] = p.tile; out[1] = p.slices; out[2] = p.kslice; out[3] = p.rows;
+    out[4] = p.rows ? born::gemm_split_bytes(p, p.rows < M ? p.rows : M, N, K) : 0;
+}
 extern "C" int pays(int M, int N, int K, long long ldb) { return born::gemm_split_pays(M, N, K, ldb); }
 """
 
@@ -20,6 +27,7 @@ def plan(tmp_path_factory):
     so, csrc = str(d / "libplan.so"), os.path.join(ROOT, "born_amd", "csrc")
     subprocess.check_call(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-I", csrc, os.path.join(csrc, "gemm_plan.cpp"), str(d / "wrapper.cpp"), "-o", so])
     lib = C.CDLL(so)
+    lib.budget.restype = C.c_longlong
     lib.pays.argtypes = [C.c_int, C.c_int, C.c_int, C.c_longlong]
     return lib
 
@@ -32,3 +40,45 @@ def test_pitches_beyond_32_bit_offsets_stay_on_the_fp32_tiles(plan):
         assert not plan.pays(64, 35_000_000, 64, ldb), ldb
     for ldb in range(2 ** 25 - 2, 2 ** 25 + 3):
         assert not plan.pays(64, 32000, 4096, ldb) or ldb <= most, ldb
+
+
+def _plan(plan, M, N, K):
+    out = (C.c_longlong * 5)()
+    plan.plan(M, N, K, out)
+    return dict(zip(("tile", "slices", "kslice", "rows", "bytes"), out))
+
+
+def test_plans_fit_the_workspace(plan):
+    """What a plan asks for fits, and few products stay on the fp32 tiles for it: none that the rows of a hidden layer or a head make."""
+    sizes = [33, 64, 65, 200, 256, 512, 708, 1024, 2048, 4096, 5000, 20001]
+    seen = left = 0
+    for M in sizes:
+        for N in (1, 130, 1000, 2048, 4096, 8192, 10386, 14336, 32000, 128256, 152064):
+            for K in (16, 61, 288, 1056, 2240, 3584, 4096, 8192, 14336, 65536, 160000):
+                if not plan.pays(M, N, K, K):
+                    continue
+                p = _plan(plan, M, N, K)
+                seen += 1
+                if p["rows"] == 0:
+                    left += K < 65536
+                    assert K >= 65536 or N <= 1000, (M, N, K)
+                    continue
+                assert 0 < p["bytes"] <= plan.budget(), (M, N, K, p)
+                assert p["rows"] == M or p["rows"] % (64, 128, 128, 256)[p["tile"]] == 0, (M, N, K, p)
+                # slices of whole pairs of groups that cover K, none of them empty
+                assert p["kslice"] % 64 == 0 and (p["slices"] - 1) * p["kslice"] < K <= p["slices"] * p["kslice"], (M, N, K, p)
+    assert seen > 700 and left < 25
+    for M, N, K in ((512, 4096, 4096), (1024, 4096, 4096), (2048, 4096, 4096), (256, 8192, 4096), (1024, 8192, 4096), (512, 14336, 4096),
+                    (512, 4096, 14336), (256, 4096, 14336), (708, 10386, 2240)):
+        assert _plan(plan, M, N, K)["rows"], (M, N, K)
+
+
+def test_products_whose_rows_come_in_chunks(plan):
+    """What tests/test_gpu_gemm_split.py multiplies in chunks of rows does come in chunks, with and without slices of K."""
+    p = _plan(plan, 2900, 2600, 4096)
+    assert p["slices"] == 1 and 1 < -(-2900 // p["rows"]) <= 3, p
+    p = _plan(plan, 1900, 2600, 8192)
+    assert 0 < p["rows"] < 1900, p
+    p = _plan(plan, 700, 4096, 8192)
+    assert p["slices"] > 1 and p["rows"] < 700, p
+    assert _plan(plan, 64, 4096, 200000)["rows"] == 0

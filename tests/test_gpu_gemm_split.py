@@ -106,10 +106,38 @@ def test_fused_heads_see_the_plain_head(rocm, lin):  # noqa: F811
 
 def test_rows_in_chunks(rocm, lin):  # noqa: F811
     """A left operand whose packed form exceeds the workspace is multiplied in chunks of rows."""
-    M, K, N = 1900, 8192, 130
+    M, K, N = 1900, 8192, 2600                             # (tests/test_gemm_plan.py holds it to more than one)
     rng = np.random.default_rng(3)
     x = rng.standard_normal((M, K), dtype=np.float32)
     w = rng.standard_normal((N, K), dtype=np.float32)
     got = _gpu_linear(rocm, lin, x, w, None)
     exact = x.astype(np.float64) @ w.T.astype(np.float64)
     assert np.all(np.abs(got - exact) <= _bound(x, w, None, K))
+
+
+# (tests/test_gemm_plan.py holds these to more than one chunk: rows without slices of K, and with them)
+@pytest.mark.parametrize("shape", [(2900, 2600, 4096), (700, 4096, 8192)])
+def test_every_epilogue_in_chunks_of_rows(rocm, lin, shape):  # noqa: F811
+    """The rows of every chunk, as the same rows alone give them: a chunk's offsets into the results, the greedy keys and the
+    candidates' thresholds, counters and lists."""
+    from tests.test_gpu_linear import _fused_vs_unfused
+    M, N, K = shape
+    rng = np.random.default_rng(M)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    w = rng.standard_normal((N, K), dtype=np.float32) * np.float32(1.5 / np.sqrt(K))
+    bias = np.float32(0.3) * rng.standard_normal(N, dtype=np.float32)
+    layer = lin.Linear(K, N, rocm.DeviceBuffer.from_numpy(w), rocm.DeviceBuffer.from_numpy(bias))
+    dx, logits = rocm.DeviceBuffer.from_numpy(x), rocm.DeviceBuffer(M * N * 4)
+    layer.Forward(dx, (M, K), logits)
+    got = logits.to_numpy(np.float32, (M, N))
+    rows = np.unique(np.concatenate([np.arange(0, M, 97), [255, 256, 257, 511, 512, 1023, 1024, 1535, 1536, M - 1]]))
+    rows = rows[rows < M]
+    exact = x[rows].astype(np.float64) @ w.T.astype(np.float64) + bias[None, :]
+    assert np.all(np.abs(got[rows] - exact) <= _bound(x[rows], w, bias, K))
+    s, a, b = rocm.NewSampler(max_batch=M, max_vocab=N), rocm.DeviceBuffer(4 * M), rocm.DeviceBuffer(4 * M)
+    s.Argmax(logits, M, N, a)
+    lin.ForwardArgmax(s, layer, dx, (M, K), b)
+    assert np.array_equal(a.to_numpy(np.int32, (M,)), b.to_numpy(np.int32, (M,)))
+    s.Close()
+    hist = rng.integers(0, N, size=(M, 8)).astype(np.int32)
+    _fused_vs_unfused(rocm, lin, x, w, bias, rocm.SamplerConfig(Temperature=0.7, TopK=20, TopP=0.9, RepetitionPenalty=1.15), hist)
