@@ -23,11 +23,10 @@
 // column of B (all M-tiles of that column) land on the same XCD back to back, so that B is fetched from HBM
 // once and re-read from that XCD's L2.
 #include <algorithm>
-#include <mutex>
-#include <vector>
 #include "dev_common.h"
 #include "gemm_epilogue.h"
 #include "gemm_plan.h"
+#include "gemm_workspace.h"
 #include "kernels.h"
 
 namespace born {
@@ -418,40 +417,10 @@ __global__ __launch_bounds__(256) void gemm_splitk_sum_kernel(GemmArgs g, long l
     }
 }
 
-// Workspace for partial products and packed operands: one small and one large buffer per (device, stream) that ever needed
-// one, kept until the process ends (calls on one stream are ordered, so they can share; calls on different streams cannot;
-// a buffer once handed out stays, so that a graph captured with it stays good).  Null when none can be had now (the stream
-// is being captured, too many streams, out of memory): the product is then computed without.
-static float *gemm_workspace(hipStream_t st, size_t bytes) {
-    struct Entry {
-        int dev;
-        hipStream_t st;
-        float *p[2];                                                 // GEMM_WS_MIN, GEMM_WS_MAX bytes
-    };
-    static std::mutex mu;
-    static std::vector<Entry> cache;
-    int dev = 0;
-    if (bytes > GEMM_WS_MAX || hipGetDevice(&dev) != hipSuccess) return nullptr;
-    std::lock_guard<std::mutex> lock(mu);
-    Entry *found = nullptr;
-    for (Entry &e : cache)
-        if (e.dev == dev && e.st == st) found = &e;
-    const int large = bytes > GEMM_WS_MIN;
-    if (found && (found->p[large] || found->p[1])) return found->p[large] ? found->p[large] : found->p[1];
-    if (!found && cache.size() >= 16) return nullptr;
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return nullptr;
-    float *p = nullptr;
-    if (hipMalloc((void **)&p, large ? GEMM_WS_MAX : GEMM_WS_MIN) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    if (!found) {
-        cache.push_back(Entry{dev, st, {nullptr, nullptr}});
-        found = &cache.back();
-    }
-    found->p[large] = p;
-    return p;
+// (never destroyed: a graph may end while the process does)
+static GemmWorkspaces &gemm_workspaces() {
+    static GemmWorkspaces *const all = new GemmWorkspaces;
+    return *all;
 }
 
 template <int EPI>
@@ -587,8 +556,8 @@ hipError_t launch_gemm_f32(const GemmArgs &g, bool b_transposed, hipStream_t st)
         const SplitPlan plan = gemm_split_plan(g.M, g.N, g.K);
         const int most = std::min(plan.rows, g.M);
         const size_t packed = gemm_split_workspace(most, g.K);
-        float *ws = plan.rows ? gemm_workspace(st, gemm_split_bytes(plan, most, g.N, g.K)) : nullptr;
-        if (ws) {
+        const GemmWorkspaces::Lease ws = plan.rows ? gemm_workspaces().take(st, gemm_split_bytes(plan, most, g.N, g.K)) : GemmWorkspaces::Lease();
+        if (ws.p) {
             for (long long r0 = 0; r0 < g.M; r0 += plan.rows) {
                 GemmArgs gc = g;
                 gc.M = (int)std::min<long long>(plan.rows, g.M - r0);
@@ -602,8 +571,8 @@ hipError_t launch_gemm_f32(const GemmArgs &g, bool b_transposed, hipStream_t st)
                 }
                 gc.ksplit = plan.slices > 1 ? plan.slices : 0;
                 gc.kslice = plan.kslice;
-                gc.ws = ws + packed / sizeof(float);
-                const hipError_t e = launch_gemm_split(gc, b_transposed, plan.tile, ws, st);
+                gc.ws = ws.p + packed / sizeof(float);
+                const hipError_t e = launch_gemm_split(gc, b_transposed, plan.tile, ws.p, st);
                 if (e != hipSuccess) return e;
                 if (gc.ksplit > 1) launch_splitk_sum(gc, st);
             }
@@ -614,17 +583,18 @@ hipError_t launch_gemm_f32(const GemmArgs &g, bool b_transposed, hipStream_t st)
     // A product of few tiles and a long K: the slices of K go to workgroups of their own, each writes a partial
     // product to the workspace, and one more launch adds them in order and does what the product's epilogue does.
     GemmArgs gs = g;
+    GemmWorkspaces::Lease partial;
     gs.ksplit = 0;
     if (grid < 128 && g.K >= 256 && (long long)g.M * g.N <= (long long)(GEMM_WS_MAX / sizeof(float) / 2)) {
         int slices = (int)std::min<long long>(std::min<long long>(16, 512 / grid), g.K / 128);   // (two workgroups to a CU)
         if (slices >= 2) {
             const int kslice = (((g.K + slices - 1) / slices + GK - 1) / GK) * GK;
             slices = (g.K + kslice - 1) / kslice;
-            float *ws = slices >= 2 ? gemm_workspace(st, (size_t)slices * (size_t)g.M * (size_t)g.N * sizeof(float)) : nullptr;
-            if (ws) {
+            if (slices >= 2) partial = gemm_workspaces().take(st, (size_t)slices * (size_t)g.M * (size_t)g.N * sizeof(float));
+            if (partial.p) {
                 gs.ksplit = slices;
                 gs.kslice = kslice;
-                gs.ws = ws;
+                gs.ws = partial.p;
             }
         }
     }

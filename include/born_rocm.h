@@ -263,9 +263,13 @@ int born_rocm_linear(const float *x, int64_t batch, int64_t in_features, int64_t
                      int64_t out_features, int64_t w_stride, const float *bias, float *out, int64_t out_stride,
                      void *stream);
 /* (born_rocm_matmul, born_rocm_linear and the fused heads below: a product of few output tiles and a long k is computed
- * in slices of k that are added in a fixed order, and a large product reads its left operand from a packed copy; the
- * first such call on a stream allocates the library's workspace for that stream, 8 or 64 MiB kept until the process
- * ends - outside a stream capture; a call under capture that finds no workspace computes the product without.) */
+ * in slices of k that are added in a fixed order, and a large product reads its left operand from a packed copy.  The
+ * library's workspace for that is a buffer of the stream, of 8 or 64 MiB, allocated by the stream's first such call and kept
+ * for the last sixteen streams that made one (hipStreamPerThread: one for each thread).  Any number of host threads may call
+ * on one stream.  Calls recorded into a graph get a buffer of the capture, which belongs to the graph and is given
+ * back after the graph and what was instantiated from it are destroyed: a graph instantiated more than once shares it, and
+ * its instances must not be replayed at the same time.  The bits of a result depend neither on the stream nor on
+ * whether the call was recorded, unless memory runs out: the product is then computed without a workspace.) */
 int born_rocm_matmul(const float *a, const float *b, float *c, int64_t m, int64_t k, int64_t n, int64_t lda,
                      int64_t ldb, int64_t ldc, void *stream);
 
