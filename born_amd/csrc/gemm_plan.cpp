@@ -10,10 +10,11 @@ namespace born {
 // after a launch that packs the left operand: below about 3 GFLOP the fp32 tiles, finer and split along K, are level
 // (64 x 4096 -> 4096, 2.1 GFLOP: 33 us against 28; 1024^3 24 against 32; 128 x 4096 -> 4096, 4.3: 72 against 41; 200 x 1056 ->
 // 8272, 3.5: 72 against 45); a batch of up to 32 rows is bound by reading the weights (32 x 4096 -> 32000: 118 against 130 us).
+// A sum of fewer than a dozen terms is more accurate on the fp32 tiles (gemm_split.hip), so K is 16 at least.
 // The kernel's loads reach 32 rows of the weights by 32-bit byte offsets: 31 ldb + 31 values of four bytes, and 32 bytes, stay below
 // 2^32 up to a pitch of 2^25.
 bool gemm_split_pays(int M, int N, int K, long long ldb) {
-    return M > 32 && ldb <= (1ll << 25) && 2.0 * (double)M * (double)N * (double)K >= 3e9;
+    return M > 32 && K >= 16 && ldb <= (1ll << 25) && 2.0 * (double)M * (double)N * (double)K >= 3e9;
 }
 
 size_t gemm_split_workspace(int M, int K) {

@@ -246,8 +246,10 @@ int born_rocm_spec_verify_bonus(born_sampler *s, const float *target, int64_t ta
 
 /* The logits producer, fp32 on the matrix cores (fp32 operands, fp32 accumulation; the order of the k-sum
  * differs from the reference's sequential loop, so results agree with it to rounding, not bit for bit).  Large
- * products run on the bf16 matrix cores at fp32 precision: each operand is the exact sum of three bf16 parts, and the
- * six products of parts that can reach an fp32 rounding of the product are accumulated in fp32.
+ * products (3 GFLOP and more, over more than 32 rows and k of at least 16) run on the bf16 matrix cores: each operand is the
+ * exact sum of three bf16 parts, and the six largest of the nine products of parts are accumulated in fp32.  Against fp64 a
+ * sum of a dozen terms or more is no less accurate for it, usually more; a sum of which all but one to four terms are
+ * zero is less (up to 1.6 times the error, root mean square).
  *
  * born_rocm_linear: out[batch, out_features] = x[batch, in_features] @ weight^T + bias, weight stored
  * [out_features, in_features] row-major as nn.Linear holds it, bias [out_features] or NULL: Linear.Forward,

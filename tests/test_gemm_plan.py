@@ -82,3 +82,7 @@ def test_products_whose_rows_come_in_chunks(plan):
     p = _plan(plan, 700, 4096, 8192)
     assert p["slices"] > 1 and p["rows"] < 700, p
     assert _plan(plan, 64, 4096, 200000)["rows"] == 0
+
+
+def test_sums_of_few_terms_stay_on_the_fp32_tiles(plan):
+    assert plan.pays(4096, 65536, 16, 16) and not plan.pays(4096, 65536, 15, 15)

@@ -2,7 +2,7 @@
 form at the edges of tiles and of K, slices of K, rows in chunks, and operands the three bf16 parts cannot hold.
 
 Tolerance: that of tests/test_gpu_linear.py, (4 sqrt(K) + 2) 2^-24 (sum |a| |b| + |bias|).  Three rounded bf16 parts hold an fp32
-value exactly and what the six products leave out is below 2^-26 |a b| a product, so the fp32 bound covers it.  Integer-valued
+value exactly and what the six products leave out is at most about 2^-24 |a b| a product, one of the bound's 4 sqrt(K) + 2 units.  Integer-valued
 operands whose partial sums stay below 2^24 are exact.
 """
 import numpy as np
@@ -33,6 +33,40 @@ def test_matches_fp64(rocm, lin, shape, form):  # noqa: F811
     # and no further off, overall, than a product of fp32 sums in blocks of two: half the ulps of sqrt(K / 2) additions
     rms = np.sqrt(np.mean((got - exact) ** 2) / np.mean(exact ** 2))
     assert rms <= 0.5 * np.sqrt(K / 2) * EPS + EPS, (shape, rms)
+
+
+WORST = np.float32(1 + 2.0 ** -8 - 2.0 ** -17)            # parts 1, 2^-8, -2^-17: what is left out of its square is the most
+
+
+def _operand(rng, family, rows, K):
+    if family == "positive":
+        return rng.random((rows, K), dtype=np.float32) + np.float32(0.5)
+    if family == "equal":
+        return np.full((rows, K), WORST)
+    if family == "equal, signed":
+        return WORST * rng.choice(np.array([-1, 1], np.float32), (rows, K))
+    x = rng.standard_normal((rows, K), dtype=np.float32)
+    return np.ldexp(x, rng.integers(-10, 11, (rows, K))).astype(np.float32) if family == "magnitudes" else x
+
+
+@pytest.mark.parametrize("K", [16, 64, 1000, 4096])
+@pytest.mark.parametrize("family", ["normal", "positive", "equal", "equal, signed", "magnitudes"])
+def test_error_is_no_larger_than_the_fp32_tiles(rocm, lin, family, K):  # noqa: F811
+    """The 2-norm of the error against fp64, beside that of the same rows 32 at a time, which the fp32 tiles multiply.  Two correct sums
+    of tens of thousands of results: 3 % for the sample."""
+    M = 64
+    N = int(3.05e9 / (2 * M * K))
+    rng = np.random.default_rng(K)
+    x, w = _operand(rng, family, M, K), _operand(rng, family, N, K)
+    layer, dx = lin.Linear(K, N, rocm.DeviceBuffer.from_numpy(w), None), rocm.DeviceBuffer.from_numpy(x)
+    one, two = rocm.DeviceBuffer(M * N * 4), rocm.DeviceBuffer(M * N * 4)
+    layer.Forward(dx, (M, K), one)
+    for r in (0, 32):
+        layer.Forward(dx.ptr + 4 * r * K, (32, K), two.ptr + 4 * r * N)
+    some = rng.choice(N, min(N, 2000), replace=False)
+    exact = x.astype(np.float64) @ w[some].T.astype(np.float64)
+    split, tiles = (np.sqrt(np.mean((b.to_numpy(np.float32, (M, N))[:, some] - exact) ** 2)) for b in (one, two))
+    assert split <= 1.03 * tiles, (split, tiles)
 
 
 @pytest.mark.parametrize("shape", [(70, 24000, 960), (300, 21539, 288)])
