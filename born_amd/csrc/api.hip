@@ -38,12 +38,6 @@ int hip_fail(hipError_t e, const char *what) {
         if (e__ != hipSuccess) return hip_fail(e__, #expr); \
     } while (0)
 
-// (never destroyed: a buffer may come back while the process ends)
-DevicePool &device_pool() {
-    static DevicePool *const pool = new DevicePool;
-    return *pool;
-}
-
 std::once_flag g_cfg_once;
 hipError_t g_cfg_err = hipSuccess;
 
@@ -200,7 +194,7 @@ int born_rocm_sampler_create(const born_sampler_config *cfg, int64_t max_batch, 
     const size_t rows = (size_t)max_batch, segs = rows * (size_t)s->S_max;
     hipError_t e = hipSuccess;
     auto alloc = [&](void **p, size_t bytes) {
-        if (e == hipSuccess) e = hipMalloc(p, bytes);
+        if (e == hipSuccess) e = device_malloc(p, bytes);
         if (e == hipSuccess) e = hipMemset(*p, 0, bytes);
     };
     alloc((void **)&s->arg_val, segs * sizeof(float));
@@ -241,7 +235,7 @@ int born_rocm_sampler_set_config(born_sampler *s, const born_sampler_config *cfg
     if (counts_history(c) && !s->hist_counts) {
         // the table of occurrence counts: allocated here, never inside a sampling call (which may be under graph capture)
         const size_t bytes = (size_t)s->max_batch * (size_t)s->max_vocab * sizeof(unsigned);
-        HIP_TRY(hipMalloc((void **)&s->hist_counts, bytes));
+        HIP_TRY(device_malloc(&s->hist_counts, bytes));
         HIP_TRY(hipMemset(s->hist_counts, 0, bytes));
     }
     s->cfg = c;
@@ -442,7 +436,7 @@ static int sample_impl(born_sampler *s, const float *logits, int64_t batch, int6
                         "capture; configure the handle with a frequency or presence penalty (born_rocm_sampler_set_config) beforehand");
         const size_t bytes = (size_t)s->max_batch * (size_t)s->max_vocab * sizeof(unsigned);
         HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
-        HIP_TRY(hipMalloc((void **)&s->hist_counts, bytes));
+        HIP_TRY(device_malloc(&s->hist_counts, bytes));
         HIP_TRY(hipMemset(s->hist_counts, 0, bytes));
     }
     a.hist_counts = table ? s->hist_counts : nullptr;
@@ -674,16 +668,16 @@ static int spec_verify_impl(born_sampler *s, const float *target, int64_t target
             *p = nullptr;
         }
         s->spec_rows = 0;
-        HIP_TRY(hipMalloc((void **)&s->sp_mp, (size_t)rows * sizeof(float)));
-        HIP_TRY(hipMalloc((void **)&s->sp_mq, (size_t)rows * sizeof(float)));
-        HIP_TRY(hipMalloc((void **)&s->sp_Zp, (size_t)rows * sizeof(unsigned long long)));
-        HIP_TRY(hipMalloc((void **)&s->sp_Zq, (size_t)rows * sizeof(unsigned long long)));
-        HIP_TRY(hipMalloc((void **)&s->sp_pd, (size_t)rows * sizeof(unsigned long long)));
-        HIP_TRY(hipMalloc((void **)&s->sp_qd, (size_t)rows * sizeof(unsigned long long)));
-        HIP_TRY(hipMalloc((void **)&s->sp_part, (size_t)rows * SPEC_CHUNKS * sizeof(unsigned long long)));
-        HIP_TRY(hipMalloc((void **)&s->sp_run, (size_t)rows * SPEC_CHUNKS * 1024 * sizeof(unsigned long long)));
-        HIP_TRY(hipMalloc((void **)&s->sp_mb, (size_t)rows * sizeof(float)));                 // rows >= batch
-        HIP_TRY(hipMalloc((void **)&s->sp_Zb, (size_t)rows * sizeof(unsigned long long)));
+        HIP_TRY(device_malloc(&s->sp_mp, (size_t)rows * sizeof(float)));
+        HIP_TRY(device_malloc(&s->sp_mq, (size_t)rows * sizeof(float)));
+        HIP_TRY(device_malloc(&s->sp_Zp, (size_t)rows * sizeof(unsigned long long)));
+        HIP_TRY(device_malloc(&s->sp_Zq, (size_t)rows * sizeof(unsigned long long)));
+        HIP_TRY(device_malloc(&s->sp_pd, (size_t)rows * sizeof(unsigned long long)));
+        HIP_TRY(device_malloc(&s->sp_qd, (size_t)rows * sizeof(unsigned long long)));
+        HIP_TRY(device_malloc(&s->sp_part, (size_t)rows * SPEC_CHUNKS * sizeof(unsigned long long)));
+        HIP_TRY(device_malloc(&s->sp_run, (size_t)rows * SPEC_CHUNKS * 1024 * sizeof(unsigned long long)));
+        HIP_TRY(device_malloc(&s->sp_mb, (size_t)rows * sizeof(float)));                 // rows >= batch
+        HIP_TRY(device_malloc(&s->sp_Zb, (size_t)rows * sizeof(unsigned long long)));
         s->spec_rows = rows;
     }
     SpecArgs a;
@@ -855,7 +849,7 @@ int born_rocm_linear_sample(born_sampler *s, const float *x, int64_t batch, int6
         void *got[4] = {nullptr, nullptr, nullptr, nullptr};
         hipError_t e = hipSuccess;
         for (int i = 0; i < 4 && e == hipSuccess; i++) {
-            e = hipMalloc(&got[i], bytes[i]);
+            e = device_malloc(&got[i], bytes[i]);
             if (e == hipSuccess) e = hipMemset(got[i], 0, bytes[i]);
         }
         if (e != hipSuccess) {

@@ -23,6 +23,7 @@
 #include <mutex>
 #include <vector>
 
+#include "device_pool.h"
 #include "gemm_plan.h"
 
 namespace born {
@@ -82,7 +83,7 @@ class GemmWorkspaces {
         Relaxed relaxed;
         give_back();
         void *p = nullptr;
-        if (hipMalloc(&p, bytes) == hipSuccess) return p;
+        if (device_malloc(&p, bytes) == hipSuccess) return p;
         (void)hipGetLastError();
         return nullptr;
     }
@@ -108,7 +109,7 @@ public:
             int dev = 0;
             hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
             if (bytes > GEMM_WS_MAX || hipGetDevice(&dev) != hipSuccess) return Lease();
-            if (hipStreamIsCapturing(st, &status) != hipSuccess) {
+            if (st && hipStreamIsCapturing(st, &status) != hipSuccess) {   // (the null stream is never captured)
                 (void)hipGetLastError();
                 return Lease();
             }

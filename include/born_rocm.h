@@ -66,7 +66,10 @@ int born_rocm_device_name(int32_t device, char *buf, int64_t buf_len);
 /* Device buffers — Born's RawTensor is host-only (internal/tensor/raw.go:42-46,139-141); these give the Go
  * layer its DeviceBuffer handle.  Copies are enqueued on `stream` and are synchronous with respect to the host
  * when the host pointer is pageable.  Up to 256 MiB of freed buffers (each of at most 32 MiB) are kept for the next allocation
- * of their size; one is handed out again only after the device was waited for since its free, as hipFree would. */
+ * of their size; one is handed out again only after the device was waited for since its free, as hipFree would.  All of them go
+ * back to the device when the library finds memory short, and all but 16 MiB when the last buffer handed out is freed.  Under a stream capture an
+ * allocation that hipMalloc would refuse can therefore succeed, and a buffer freed while a graph still uses it can be another's
+ * before the graph is replayed (where hipFree would unmap it): keep what a graph uses until the graph is destroyed. */
 int born_rocm_alloc(int64_t bytes, void **dev_ptr);
 int born_rocm_free(void *dev_ptr);
 int born_rocm_h2d(void *dst_dev, const void *src_host, int64_t bytes, void *stream);

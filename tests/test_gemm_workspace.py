@@ -14,7 +14,7 @@ HIP = r"""
 #include <mutex>
 #include <set>
 #include <vector>
-enum hipError_t { hipSuccess, hipErrorOutOfMemory, hipErrorUnknown };
+enum hipError_t { hipSuccess, hipErrorOutOfMemory, hipErrorInvalidValue, hipErrorUnknown };
 enum hipStreamCaptureStatus { hipStreamCaptureStatusNone, hipStreamCaptureStatusActive, hipStreamCaptureStatusInvalidated };
 enum hipStreamCaptureMode { hipStreamCaptureModeGlobal, hipStreamCaptureModeThreadLocal, hipStreamCaptureModeRelaxed };
 enum { hipUserObjectNoDestructorSync = 1, hipGraphUserObjectMove = 1 };
