@@ -66,10 +66,10 @@ static void order() {
 // The last buffer that comes back, of whatever size, takes all but 16 MiB of the kept ones with it, the oldest first.
 static void last() {
     DevicePool p;
-    void *large = get(p, (size_t)100 << 20), *a = get(p, 10 << 20), *b = get(p, 3000);
-    CHECK(p.free(a) == hipSuccess && p.free(b) == hipSuccess && hip_live.size() == 3);
+    void *large = get(p, (size_t)100 << 20), *tiny = get(p, 1), *a = get(p, 10 << 20), *b = get(p, 3000);
+    CHECK(p.free(tiny) == hipSuccess && p.free(a) == hipSuccess && p.free(b) == hipSuccess && hip_live.size() == 4);
     p.waited();
-    CHECK(get(p, 3000) == b);                             // kept, and waited for
+    CHECK(get(p, 3000) == b && hip_freed.back() == tiny); // kept, and waited for: the smallest one's free
     CHECK(p.free(b) == hipSuccess && p.free(b) != hipSuccess);
     void *c = get(p, 12 << 20);
     CHECK(p.free(c) == hipSuccess && hip_live.size() == 4);
