@@ -24,8 +24,8 @@
 //     16 x 16 form sustains 1.9 PFLOP/s where the 32 x 32 form sustains 1.7.
 //   * C tiles are 32 IB x 32 NW: IB blocks of 32 rows per wave, NW waves side by side.
 //
-// Bound by power: at 256 x 4096 -> 128256 the matrix pipes are busy in three quarters of the cycles at a clock that has fallen
-// to 1.9 GHz.  Measured against the fp32 tiles of linear.hip (us): 256 x 4096 -> 128256 2060 -> 1065 (253 TFLOP/s of
+// Bound by power: at 256 x 4096 -> 128256 the matrix pipes are busy in 76 % of the cycles at a clock that has fallen from 2.4 to
+// 1.9 GHz, and a bare loop of the instruction on random operands does no more than 1.9 PFLOP/s.  Measured against the fp32 tiles of linear.hip (us): 256 x 4096 -> 128256 2060 -> 1065 (253 TFLOP/s of
 // fp32 work, 1.5 PFLOP/s of bf16), 128 x 4096 -> 32000 280 -> 174, 64 x 4096 -> 32000 160 -> 126, 2048^3 137 -> 88.
 //
 // Values outside what bf16 parts can hold - an infinity or NaN anywhere, magnitudes below 2^-100 whose third part would
@@ -193,6 +193,8 @@ __device__ __forceinline__ void load_to_lds(const char *base, u32 off, u32 lds) 
 // matrix: the packed operand is zero there, or the column is not stored).  A workgroup has NW x KH waves: NW side by
 // side along N, and KH of each of those take turns along K (KH = 2: two waves share a SIMD also where a narrow tile is all a
 // CU gets: one's loads, splits and waits under the other's matrix instructions).  SW: stages of weights in LDS.
+// (One instance, the 256 x 256 tile over [K,N] weights value by value, has two registers in scratch; a 128 x 256 tile without them is
+// slower all the same: 256 x 4096 @ 4096 x 128257 1116 us against 1235.)
 template <bool BT, bool VEC, int IB, int NW, int KH, int SW, int EPI>
 __global__ __launch_bounds__(64 * NW * KH) void gemm_split_kernel(SplitArgs s) {
     constexpr int AC = (IB * 6 + NW - 1) / NW;                       // 1 KiB pieces of A's groups each wave copies (some twice)

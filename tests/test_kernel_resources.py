@@ -11,7 +11,9 @@ from born_amd import _capi
 LLVM = "/opt/rocm/llvm/bin"
 
 #: kernel -> a pattern of its mangled names
-HOT = {"sampling without a top-k cut": r"nucleus_row_kernelILi\d+E", "the same, a row's own settings": r"nucleus_row_rows_kernelILi\d+E"}
+HOT = {"sampling without a top-k cut": r"nucleus_row_kernelILi\d+E", "the same, a row's own settings": r"nucleus_row_rows_kernelILi\d+E",
+       "top-k sampling": r"topk_row(_rows)?_kernelILi\d+E", "token log-probabilities": "token_logprob", "verification": "spec_",
+       "softmax": "softmax_", "large products, weights of a linear layer": r"gemm_split_kernelILb1E", "fp32 products": r"gemm_f32_"}
 
 
 @pytest.fixture(scope="module")
