@@ -401,7 +401,9 @@ static void launch_gemm_bm(const GemmArgs &g, int bm, hipStream_t st) {
 // The sum of the partial products of a split K, slice by slice in ascending order (so the result does not depend on
 // which workgroup finished first), plus the bias; then what the product's own epilogue would have done with the
 // result (EPI as in the tiles' epilogues: stored, offered as its row's largest, or listed as a candidate), so that the
-// fused forms of a head see the very numbers its plain form stores.
+// fused forms of a head see the very numbers its plain form stores.  A wave's 64 columns are one row's but where it ends: one atomic
+// for them all (head and sampling step of 512 rows x 1408 -> 4000, where a third of the logits are candidates: 237 us with an atomic for
+// each, 94 like this; the fp32 tiles unsplit, whose epilogue stages its candidates, 222).
 template <int EPI>
 __global__ __launch_bounds__(256) void gemm_splitk_sum_kernel(GemmArgs g, long long mn) {
     const float *__restrict__ ws = g.ws;
@@ -411,9 +413,38 @@ __global__ __launch_bounds__(256) void gemm_splitk_sum_kernel(GemmArgs g, long l
         const int row = (int)(i / g.N);
         const int col = (int)(i - (long long)row * g.N);
         const float val = g.bias ? sum + g.bias[col] : sum;
-        if (EPI == 0) g.c[(long long)row * g.ldc + col] = val;
-        else if (EPI == 1) gemm_offer_key(g.best, row, gemm_argmax_key(val, col));
-        else gemm_offer_candidate(g, row, col, val, g.thr[row]);
+        if (EPI == 0) {
+            g.c[(long long)row * g.ldc + col] = val;
+            continue;
+        }
+        const int row0 = __builtin_amdgcn_readfirstlane(row);
+        if (__all(row == row0)) {                                    // (nearly always: 64 columns of one row)
+            if (EPI == 1) {
+                u64 key = gemm_argmax_key(val, col);
+                const u64 in = __ballot(true);
+                const int lane = (int)(threadIdx.x & (WAVE - 1));
+#pragma unroll
+                for (int o = 1; o < WAVE; o <<= 1) {
+                    const u64 k = gemm_shfl_xor_u64(key, o);
+                    if ((in >> (lane ^ o)) & 1ull) key = gemm_max_u64(key, k);
+                }
+                if (lane == (int)__builtin_ctzll(in) && key) gemm_offer_key(g.best, row0, key);
+            } else {
+                const bool pass = val >= g.thr[row0];                // a NaN never passes
+                const u64 m = __ballot(pass);
+                if (m) {
+                    const u32 rank = __builtin_amdgcn_mbcnt_hi((u32)(m >> 32), __builtin_amdgcn_mbcnt_lo((u32)m, 0u));
+                    u32 base = 0u;
+                    if (pass && rank == 0u) base = atomicAdd(&g.cand_cnt[(long long)row0 * LM_CAND_PITCH], (u32)__popcll(m));
+                    const u32 pos = (u32)__builtin_amdgcn_readlane((int)base, (int)__builtin_ctzll(m)) + rank;
+                    if (pass && pos < (u32)g.cand_cap) g.cand[(long long)row0 * g.cand_cap + pos] = make_uint2(__float_as_uint(val), (unsigned)col);
+                }
+            }
+        } else if (EPI == 1) {
+            gemm_offer_key(g.best, row, gemm_argmax_key(val, col));
+        } else {
+            gemm_offer_candidate(g, row, col, val, g.thr[row]);
+        }
     }
 }
 
