@@ -56,3 +56,21 @@ def test_every_result_keeps_its_precision(rocm, lin, kind, shape):  # noqa: F811
     err = np.abs(got - exact) - 2.0 ** -140 * K             # (products below the floats' range)
     bound = _bound(x, w[some], None, K)
     assert np.all(err <= bound), (kind, shape, np.argwhere(err > bound)[:3], (err / np.maximum(bound, 1e-300)).max())
+
+
+def test_values_cut_under_columns_far_above_their_scale(rocm, lin):  # noqa: F811
+    """A row of one large value that meets zeros and many equal ones 2^-32 of it, whose parts are cut (all alike, so that nothing averages out), against
+    columns whose later values are 256 times those their scale is made from: what is lost shows in results of any size, so they are summed again.
+    Sixteen units: sums of fp32 products in pieces of 512 are off by the walk of 128 roundings, three or four."""
+    M, N, K = 40, 33000, 4096                                # (K in one piece: a slice's partial sums are smaller)
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    w = rng.random((N, K), dtype=np.float32) * np.float32(0.09) + np.float32(1.9)
+    w[:, 64:] *= 256
+    w[:, 4000] = 0
+    rows, some = np.arange(1, M, 7), rng.choice(N, 1000, replace=False)
+    x[rows] = np.float32(1.007) * np.float32(2.0 ** -32)
+    x[rows, 4000] = 1
+    got = _gpu_linear(rocm, lin, x, w, None)[np.ix_(rows, some)]
+    exact = x[rows].astype(np.float64) @ w[some].T.astype(np.float64)
+    assert (np.abs(got - exact) / exact).max() <= 16 * 2.0 ** -24
