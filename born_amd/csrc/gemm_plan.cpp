@@ -25,7 +25,7 @@ int gemm_split_parts(int K) { return K >= 256 ? 2 : 3; }
 
 size_t gemm_split_workspace(int M, int K) {
     const size_t ng = (size_t)(K + 2 * SG - 1) / (2 * SG) * 2, mb = (size_t)(M + 31) / 32;
-    const size_t bytes = ng * mb * SG_BYTES + 8 * SG_BYTES + mb * ((ng + PACK_GROUPS - 1) / PACK_GROUPS) * 2 * sizeof(unsigned) + mb * 32 * 4 * sizeof(int);   // (8 blocks: the last tile's copy may run on)
+    const size_t bytes = ng * mb * SG_BYTES + 8 * SG_BYTES + mb * ((ng + PACK_GROUPS - 1) / PACK_GROUPS) * 2 * sizeof(unsigned) + mb * 32 * (4 * sizeof(int) + 1);   // (8 blocks: the last tile's copy may run on)
     return (bytes + 255) / 256 * 256;
 }
 
@@ -72,7 +72,7 @@ SplitPlan gemm_split_plan(int M, int N, int K) {
             const long long per = (pairs + want - 1) / want;
             const int slices = (int)((pairs + per - 1) / per);
             // rows at a time: as many tiles' as fit, shared out evenly
-            const double block = (double)(2 * pairs * SG_BYTES + (2 * pairs + PACK_GROUPS - 1) / PACK_GROUPS * 8 + 32 * 16) +
+            const double block = (double)(2 * pairs * SG_BYTES + (2 * pairs + PACK_GROUPS - 1) / PACK_GROUPS * 8 + 32 * 17) +
                                  (slices > 1 ? 32.0 * 4.0 * slices * (double)N : 0.0);
             const long long fit = (long long)((double)(GEMM_WS_MAX - 8 * SG_BYTES - 256) / block) * 32;
             long long rows = M;

@@ -258,10 +258,16 @@ int born_rocm_spec_verify_bonus(born_sampler *s, const float *target, int64_t ta
 
 /* The logits producer, fp32 on the matrix cores (fp32 operands, fp32 accumulation; the order of the k-sum
  * differs from the reference's sequential loop, so results agree with it to rounding, not bit for bit).  Large
- * products (3 GFLOP and more, over more than 32 rows and k of at least 16, or more than 16 rows and k of at least 2048) run on the 16-bit matrix cores: each operand is a sum of
- * two fp16 parts (k below 256: three bf16 parts), and the products of parts but the smallest are accumulated in fp32.  Against fp64 a
- * sum of a dozen terms or more is no less accurate for it, usually more; a sum of which all but one to four terms are
- * zero is less (2 to 3 times the error, root mean square: 2^-23.7 of the result).
+ * products (3 GFLOP and more, over more than 32 rows and k of at least 16, or more than 16 rows and k of at least 2048) run on the 16-bit matrix cores:
+ * each operand is a sum of 16-bit parts, and the products of parts but the smallest are accumulated in fp32.
+ *   k below 256: three bf16 parts, exact; what is left out is at most about 2^-24 of a product.
+ *   k of 256 and more: two fp16 parts, which hold a value to a unit in its 24th bit and leave out at most 2^-22 of a product; for
+ *   rows and columns for which that would show, three, exact, with 2^-34 of a product left out: rows of few terms (the square of the magnitudes' sum below 12 times
+ *   the sum of squares), rows of whole numbers of 12 to 22 bits (times any power of two), rows of which an eighth shares one significand of
+ *   more than 11 bits, and columns whose first 32 values add up to less than three times their largest.
+ * Sums of whole numbers below 2^24 are exact where the rows' are of at most 22 bits, and so are rows and columns that select (a power of
+ * two, all else zero).  Against fp64 the error of dense sums is no larger than the fp32 matrix cores' (2-norm; k = 256 0.4, 4096 0.5 of it); sums of
+ * some 12 to 100 terms that are spread over a long k are rounded twice in every group of 32 that holds one, and their error is up to twice theirs.
  *
  * born_rocm_linear: out[batch, out_features] = x[batch, in_features] @ weight^T + bias, weight stored
  * [out_features, in_features] row-major as nn.Linear holds it, bias [out_features] or NULL: Linear.Forward,

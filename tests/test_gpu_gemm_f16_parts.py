@@ -1,4 +1,5 @@
-"""Large products in two fp16 parts (born_amd/csrc/gemm_split.hip, K from 256 on): operands that their scales or their range do not fit.
+"""Large products in two fp16 parts (born_amd/csrc/gemm_split.hip, K from 256 on): operands that their scales or their range do not fit, and rows and
+columns for which two parts are not enough and which have to be whole.
 
 Tolerance: that of tests/test_gpu_linear.py, (4 sqrt(K) + 2) 2^-24 (sum |a| |b|), result by result.  Two parts hold a value to 2^-23 of it and leave
 2^-22 of a product out at most, 8 of the bound's more than 66 units together; values too small for that are looked after apart.
@@ -74,3 +75,93 @@ def test_values_cut_under_columns_far_above_their_scale(rocm, lin):  # noqa: F81
     got = _gpu_linear(rocm, lin, x, w, None)[np.ix_(rows, some)]
     exact = x[rows].astype(np.float64) @ w[some].T.astype(np.float64)
     assert (np.abs(got - exact) / exact).max() <= 16 * 2.0 ** -24
+
+
+# a tile of each height; ragged M, N and K, and K in slices (64 x 6100)
+WHOLE_SHAPES = [(20, 45001, 2048), (48, 130000, 257), (100, 15011, 1057), (130, 40004, 300), (270, 16000, 352), (64, 6100, 4096)]
+
+
+def _both_forms(rocm, lin, x, w):
+    yield _gpu_linear(rocm, lin, x, w, None)
+    yield _gpu_matmul(rocm, lin, x, np.ascontiguousarray(w.T))
+
+
+@pytest.mark.parametrize("shape", WHOLE_SHAPES)
+def test_rows_and_columns_that_select_are_exact(rocm, lin, shape):  # noqa: F811
+    """One power of two in a row: a row of the weights, bit for bit; one in a column: the activations."""
+    M, N, K = shape
+    rng = np.random.default_rng(K)
+    x, w = rng.standard_normal((M, K), dtype=np.float32), rng.standard_normal((N, K), dtype=np.float32)
+    rows, at = np.arange(1, M, 9), rng.integers(0, K, len(range(1, M, 9)))
+    x[rows] = 0
+    x[rows, at] = np.ldexp(np.float32(1), rng.integers(-3, 4, len(rows))).astype(np.float32) * rng.choice(np.array([-1, 1], np.float32), len(rows))
+    for got in _both_forms(rocm, lin, x, w):
+        assert np.array_equal(got[rows], w[:, at].T * x[rows, at][:, None])
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    cols, of = rng.choice(N, 700, replace=False), rng.integers(0, K, 700)
+    w[cols] = 0
+    w[cols, of] = np.float32(0.25)
+    for got in _both_forms(rocm, lin, x, w):
+        assert np.array_equal(got[:, cols], x[:, of] * np.float32(0.25))
+
+
+@pytest.mark.parametrize("shape", WHOLE_SHAPES)
+def test_a_product_of_two_whole_values_is_rounded_once(rocm, lin, shape):  # noqa: F811
+    """Rows of one term: six of nine products of parts, their small ones in a sum of their own that is off by 2^-11 of a unit."""
+    M, N, K = shape
+    rng = np.random.default_rng(K + 1)
+    x, w = np.zeros((M, K), np.float32), rng.standard_normal((N, K), dtype=np.float32)
+    at = rng.integers(0, K, M)
+    x[np.arange(M), at] = rng.standard_normal(M, dtype=np.float32)
+    for got in _both_forms(rocm, lin, x, w):
+        exact = x[np.arange(M), at].astype(np.float64)[:, None] * w[:, at].T.astype(np.float64)
+        assert np.all(np.abs(got - exact) <= 2.0 ** -24 * (1 + 2.0 ** -8) * np.abs(exact))
+
+
+@pytest.mark.parametrize("shape", WHOLE_SHAPES)
+def test_whole_numbers_are_exact(rocm, lin, shape):  # noqa: F811
+    """Sums below 2^24 of products whose factors both need their second part, and of factors of 22 bits."""
+    M, N, K = shape
+    rng = np.random.default_rng(K + 2)
+    x, w = rng.integers(-20, 21, (M, K)).astype(np.float32), rng.integers(-20, 21, (N, K)).astype(np.float32)
+    x[:, K // 2], w[:, K // 2] = rng.integers(2049, 2600, M), rng.integers(2049, 2600, N)
+    x[:, 7], w[:, 7] = rng.integers(2 ** 21, 2 ** 22, M), rng.integers(-1, 2, N)
+    assert (np.abs(x).astype(np.float64) @ np.abs(w[:2000]).T.astype(np.float64)).max() < 2.0 ** 24
+    want = (x.astype(np.float64) @ w.T.astype(np.float64)).astype(np.float32)
+    for got in _both_forms(rocm, lin, x, w):
+        assert np.array_equal(got, want)
+
+
+# what two fp16 parts lose most of: the product of the second parts; that, and a unit of either factor
+SIGNIFICANDS = [1 + 2.0 ** -11, 1 + 2.0 ** -11 - 3 * 2.0 ** -23]
+
+
+@pytest.mark.parametrize("K", [256, 1000, 4096])
+@pytest.mark.parametrize("family", ["equal", "signed", "powers", "4 terms", "12 terms"])
+@pytest.mark.parametrize("value", SIGNIFICANDS)
+def test_error_is_that_of_whole_operands(rocm, lin, family, value, K):  # noqa: F811
+    """The 2-norm of the error against fp64, beside that of the same rows 16 at a time, which the fp32 tiles multiply.  What two parts lose is
+    up to 8 units of 2^-24 here; two roundings to a group of 32 are a walk of sqrt(K / 16) / 3 units (rounded the same way by equal terms: one and a half of
+    it), and the result is rounded once."""
+    M, N = 64, int(3.1e9 / (2 * 64 * K))
+    rng = np.random.default_rng(K)
+    sign = lambda rows: rng.choice(np.array([-1, 1], np.float32), (rows, K))  # noqa: E731
+    x, w = np.full((M, K), np.float32(value)), np.full((N, K), np.float32(value))
+    if family == "signed":
+        x, w = x * sign(M), w * sign(N)
+    elif family == "powers":                                 # one significand, every value a power of two of its own
+        x, w = np.ldexp(x, rng.integers(-3, 4, (M, K))).astype(np.float32), np.ldexp(w, rng.integers(-3, 4, (N, K))).astype(np.float32)
+    elif family != "equal":
+        keep = np.argsort(rng.random((M, K)), axis=1)[:, int(family.split()[0]):]
+        np.put_along_axis(x, keep, np.float32(0), 1)
+        w = rng.standard_normal((N, K), dtype=np.float32)
+    some = rng.choice(N, min(N, 2000), replace=False)
+    layer, dx = lin.Linear(K, N, rocm.DeviceBuffer.from_numpy(w), None), rocm.DeviceBuffer.from_numpy(x)
+    one, two = rocm.DeviceBuffer(M * N * 4), rocm.DeviceBuffer(M * N * 4)
+    layer.Forward(dx, (M, K), one)
+    for r in range(0, M, 16):
+        layer.Forward(dx.ptr + 4 * r * K, (16, K), two.ptr + 4 * r * N)
+    exact = x.astype(np.float64) @ w[some].T.astype(np.float64)
+    split, tiles = (np.sqrt(np.mean((b.to_numpy(np.float32, (M, N))[:, some] - exact) ** 2) / np.mean(exact ** 2)) for b in (one, two))
+    print(f"{family} {value} {K}: {split * 2 ** 24:.3f} {tiles * 2 ** 24:.3f} units")
+    assert split <= max(1.03 * tiles, (1 + np.sqrt(K / 16) / 2) * 2.0 ** -24), (split, tiles)
