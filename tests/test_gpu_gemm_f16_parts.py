@@ -37,6 +37,12 @@ def _operands(kind, rng, M, N, K):
         return x, w
     if kind == "few values in a column":                      # now and then small ones first
         return x, np.where(rng.random((N, K), dtype=np.float32) < 0.03, np.ldexp(w, rng.integers(-12, 1, (N, K))), 0).astype(np.float32)
+    if kind == "equal rows":                                  # a small result in one is small in all, some over values that are cut
+        x[:] = x[0]
+        w[:, 5::64] *= np.float32(2.0 ** -24)
+        return x, w
+    if kind == "signs and zeros":                             # results of zero by the score
+        return rng.integers(-1, 2, (M, K)).astype(np.float32), rng.integers(-1, 2, (N, K)).astype(np.float32) * np.float32(0.37)
     if kind == "columns that outgrow their scale":
         w[::1000, K - 3:] *= np.float32(2.0 ** 30)
         w[5::1000, K - 3:] *= np.float32(2.0 ** -30)
@@ -48,7 +54,7 @@ def _operands(kind, rng, M, N, K):
 
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("kind", ["few terms of every magnitude", "rows of a wide range", "one huge factor that meets zeros",
-                                  "columns that begin with zeros", "few values in a column", "columns that outgrow their scale", "units"])
+                                  "columns that begin with zeros", "few values in a column", "equal rows", "signs and zeros", "columns that outgrow their scale", "units"])
 def test_every_result_keeps_its_precision(rocm, lin, kind, shape):  # noqa: F811
     M, N, K = shape
     rng = np.random.default_rng(K)
