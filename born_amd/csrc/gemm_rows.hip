@@ -165,11 +165,22 @@ static void launch_gemm_rows_epi(const GemmArgs &g, hipStream_t st) {
     else launch_gemm_rows_as<4, EPI>(g, st);
 }
 
-// Up to four rows; eight read x as often as W and are slower (8 x 4096 -> 32 000 103 us, the tiles 88).  More than one row of many columns
-// and a short K stays with the tiles: a wave's adding over the lanes is then what it does (us, tiles and here, 2 and 4 rows: 320 -> 50 000 15.4
-// 16.0 and 17.9 24.7; 1024 -> 32 000 26.9 27.5 and 22.6 26.1).
+// Up to four rows; eight read x as often as W and are slower (8 x 4096 -> 32 000 103 us, the tiles 88).  A wave's adding over the lanes is what
+// many columns and a short K take, and lanes past a short K idle; the tiles have it where they are at their best, in one round of 256 or fewer (us, tiles
+// and here):
+//   one row, K a multiple of 32   K = 64, 12 000 columns 4.1 4.2, 20 000 4.1 4.9, 50 000 4.5 8.6, 152 064 9.7 27.6;   192, 20 000 5.4 5.2;
+//                                 256, 50 000 9.6 11.7, 100 000 20.7 21.9;   320, 30 000 8.0 7.8, 50 000 12.8 12.2;   384, 152 064 35.7 36.1
+//   other K (guarded tiles)       20, 18 000 5.2 4.6, 152 064 10.0 23.5;   100, 30 000 7.3 6.5, 50 000 8.4 9.0;   200, 100 000 22.3 21.3;   260, 152 064 33.8 32.8
+//   two rows and more             320, 50 000, 2 and 4 rows 15.4 16.0 and 17.9 24.7;   1024, 10 000 12.9 7.4 and 13.3 8.4, 50 000 32.2 29.9 and 32.7 33.9
+//   three and four                1024, 32 000 20.5 21.6 and 20.8 22.4;   2048, 32 000 39.9 40.4 and 40.6 43.1, 50 000 73.7 63.0 and 74.5 67.4;   4096, 32 000 87.2 78.1 and 87.3 82.4
 bool gemm_rows_takes(const GemmArgs &g, bool b_transposed) {
-    return b_transposed && !g.bm && g.M <= GEMM_ROWS_MAX && g.vec_a && g.vec_b && g.K % 4 == 0 && (g.M == 1 || g.K >= 1024 || g.N < ROWS_ALONE_FROM);
+    if (!b_transposed || g.bm || g.M > GEMM_ROWS_MAX || !g.vec_a || !g.vec_b || g.K % 4) return false;
+    if (g.M == 1) {
+        if (g.K % 32) return g.N < 24576 || (long long)g.K * 512 >= g.N;
+        return g.N < 16384 || g.K >= (g.N < 24576 ? 192 : 320);
+    }
+    if (g.N < ROWS_ALONE_FROM) return true;
+    return g.K >= (g.M > 2 && g.N > 24576 && g.N <= 32768 ? 3072 : 1024);
 }
 hipError_t launch_gemm_rows(const GemmArgs &g, hipStream_t st) {
     if (g.cand) launch_gemm_rows_epi<2>(g, st);

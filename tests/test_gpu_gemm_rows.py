@@ -71,3 +71,18 @@ def test_what_is_not_finite_stays_in_its_row_and_column(mods):
     assert np.array_equal(np.isnan(got), np.isnan(exact)) and np.array_equal(np.isposinf(got), np.isposinf(exact))
     ok = np.isfinite(exact)
     assert np.allclose(got[ok], exact[ok], rtol=0, atol=1e-3)
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 32, 16383), (1, 32, 16384), (1, 188, 24575), (1, 44, 24577), (1, 52, 24577), (1, 192, 16400), (1, 160, 16400), (1, 288, 40001),
+                                   (1, 320, 40001), (3, 1024, 24577), (4, 3068, 24580), (4, 3072, 24580), (3, 1024, 32769), (2, 1024, 30000)])
+def test_either_side_of_the_lines(mods, M, K, N):
+    """Where one row, or three and four, of many columns pass from the tiles to the waves: a chain of K at most, and the bias."""
+    L, S = mods
+    rng = np.random.default_rng(K + N)
+    w, b, layer = _layer(mods, rng, K, N)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    out = S.DeviceBuffer(4 * M * N)
+    layer.Forward(S.DeviceBuffer.from_numpy(x), (M, K), out)
+    exact = x.astype(np.float64) @ w.T.astype(np.float64) + b
+    bound = (K + 4) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T.astype(np.float64) + np.abs(b))
+    assert (np.abs(out.to_numpy(np.float32, (M, N)) - exact) <= bound).all()
