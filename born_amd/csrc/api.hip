@@ -352,6 +352,15 @@ int born_rocm_log_softmax(born_sampler *s, const float *logits, int64_t batch, i
     return BORN_ROCM_OK;
 }
 
+// While it lives this thread's allocations and waits are allowed beside a capture of another thread.
+struct LeavesCapturesAlone {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    ~LeavesCapturesAlone() {
+        if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
 // The handle's workspace for rows that are cut into parts (10 MiB; 90 us, which other handles do not pay).  A call under capture, or
 // without memory, has its rows by one workgroup each.  The allocation leaves captures of other threads alone.
 static void take_parts(born_sampler *s, hipStream_t st) {
@@ -361,8 +370,7 @@ static void take_parts(born_sampler *s, hipStream_t st) {
         return;
     }
     if (capturing != hipStreamCaptureStatusNone) return;
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    const LeavesCapturesAlone relaxed;
     const int parts = nucleus_workspace_parts(s->max_batch);
     if (device_malloc(&s->parts.p, nucleus_workspace_bytes(parts)) == hipSuccess) {
         s->parts.parts = parts;
@@ -371,7 +379,6 @@ static void take_parts(born_sampler *s, hipStream_t st) {
         s->parts.p = nullptr;
         s->no_parts = true;
     }
-    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
 }
 
 static int sample_impl(born_sampler *s, const float *logits, int64_t batch, int64_t vocab, int64_t row_stride,
@@ -531,7 +538,7 @@ int born_rocm_sample(born_sampler *s, const float *logits, int64_t batch, int64_
                        probs_out, nucleus_len_out, nucleus_ids_out, nucleus_probs_out, nucleus_cap, stream);
 }
 
-int born_rocm_token_logprobs(born_sampler *s, const float *logits, int64_t batch, int64_t vocab, int64_t row_stride,
+static int token_logprobs_at(born_sampler *s, float temperature, const float *logits, int64_t batch, int64_t vocab, int64_t row_stride,
                              const int32_t *history, const int32_t *hist_len, int64_t hist_stride, const int32_t *tokens,
                              float *logprobs_out, void *stream) {
     int rc = check_logits("token_logprobs", s, logits, batch, vocab, row_stride);
@@ -551,7 +558,7 @@ int born_rocm_token_logprobs(born_sampler *s, const float *logits, int64_t batch
     a.history = history;
     a.hist_len = hist_len;
     a.hist_stride = history ? hist_stride : 0;
-    a.T = s->cfg.temperature;
+    a.T = temperature;
     a.rep = s->cfg.repetition_penalty;
     a.status = s->status;
     a.counters = s->counters;
@@ -572,6 +579,12 @@ int born_rocm_token_logprobs(born_sampler *s, const float *logits, int64_t batch
     return BORN_ROCM_OK;
 }
 
+int born_rocm_token_logprobs(born_sampler *s, const float *logits, int64_t batch, int64_t vocab, int64_t row_stride,
+                             const int32_t *history, const int32_t *hist_len, int64_t hist_stride, const int32_t *tokens,
+                             float *logprobs_out, void *stream) {
+    return token_logprobs_at(s, s ? s->cfg.temperature : 1.0f, logits, batch, vocab, row_stride, history, hist_len, hist_stride, tokens, logprobs_out, stream);
+}
+
 // Terms of so few rows are written to pinned host memory by the kernel itself (a word each over the bus); more come in one copy.
 // 64 rows: the copies into pageable memory of terms and status that this replaces were two waits of about 15 us.
 constexpr int64_t LOSS_DIRECT_ROWS = 256;
@@ -581,14 +594,20 @@ int born_rocm_cross_entropy(born_sampler *s, const float *logits, int64_t batch,
     if (!s || !loss_out) return fail(BORN_ROCM_ERR_ARGUMENT, "sampler: cross_entropy: null handle or output");
     const int rc_args = check_logits("token_logprobs", s, logits, batch, classes, classes);
     if (rc_args) return rc_args;
+    if (!targets) return fail(BORN_ROCM_ERR_ARGUMENT, "sampler: cross_entropy: null targets");
+    hipStream_t st = (hipStream_t)stream;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (st) HIP_TRY(hipStreamIsCapturing(st, &capturing));
+    if (capturing != hipStreamCaptureStatusNone)
+        return fail(BORN_ROCM_ERR_UNSUPPORTED, "sampler: cross_entropy: the call waits for its stream, which a capture does not allow");
+    const LeavesCapturesAlone relaxed;                               // (the pinned memory, and the wait)
     if (!s->host_terms && hipHostMalloc((void **)&s->host_terms, (size_t)s->max_batch * sizeof(float)) != hipSuccess) {
         s->host_terms = nullptr;
         return hip_fail(hipGetLastError(), "cross_entropy: pinned memory");
     }
     const bool direct = batch <= LOSS_DIRECT_ROWS;
-    hipStream_t st = (hipStream_t)stream;
     float *const terms = direct ? s->host_terms : s->arg_val;        // (arg_val: at least a float per row, free outside argmax)
-    const int rc = born_rocm_token_logprobs(s, logits, batch, classes, classes, nullptr, nullptr, 0, targets, terms, stream);
+    const int rc = token_logprobs_at(s, 1.0f, logits, batch, classes, classes, nullptr, nullptr, 0, targets, terms, stream);
     if (rc) return rc;
     if (!direct) HIP_TRY(hipMemcpyAsync(s->host_terms, terms, (size_t)batch * sizeof(float), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));

@@ -213,8 +213,8 @@ int born_rocm_token_logprobs(born_sampler *s, const float *logits, int64_t batch
                              float *logprobs_out, void *stream);
 
 /* Mean of the negated log-probabilities of `targets` (int32 [batch] on the device), summed in fp32 in row order:
- * CrossEntropyLoss.Forward, internal/nn/cross_entropy.go:37-90, whole.  `loss_out` is host memory; the call waits for the stream.
- * A target outside [0, classes): BORN_ROCM_ERR_DATA.  The first call on a handle allocates 4 bytes of pinned host memory per row of max_batch. */
+ * CrossEntropyLoss.Forward, internal/nn/cross_entropy.go:37-90, whole: of the logits as they are, whatever the handle's temperature.  `loss_out` is host
+ * memory; the call waits for the stream (one under capture: BORN_ROCM_ERR_UNSUPPORTED).  A target outside [0, classes): BORN_ROCM_ERR_DATA.  The first call on a handle allocates 4 bytes of pinned host memory per row of max_batch. */
 int born_rocm_cross_entropy(born_sampler *s, const float *logits, int64_t batch, int64_t classes, const int32_t *targets,
                             float *loss_out, void *stream);
 
