@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "device_pool.h"
+#include "handle_workspace.h"
 #include "kernels.h"
 
 using namespace born;
@@ -352,35 +353,6 @@ int born_rocm_log_softmax(born_sampler *s, const float *logits, int64_t batch, i
     return BORN_ROCM_OK;
 }
 
-// While it lives this thread's allocations and waits are allowed beside a capture of another thread.
-struct LeavesCapturesAlone {
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-    ~LeavesCapturesAlone() {
-        if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
-    }
-};
-
-// The handle's workspace for rows that are cut into parts (10 MiB; 90 us, which other handles do not pay).  A call under capture, or
-// without memory, has its rows by one workgroup each.  The allocation leaves captures of other threads alone.
-static void take_parts(born_sampler *s, hipStream_t st) {
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (st && hipStreamIsCapturing(st, &capturing) != hipSuccess) {
-        (void)hipGetLastError();
-        return;
-    }
-    if (capturing != hipStreamCaptureStatusNone) return;
-    const LeavesCapturesAlone relaxed;
-    const int parts = nucleus_workspace_parts(s->max_batch);
-    if (device_malloc(&s->parts.p, nucleus_workspace_bytes(parts)) == hipSuccess) {
-        s->parts.parts = parts;
-    } else {
-        (void)hipGetLastError();
-        s->parts.p = nullptr;
-        s->no_parts = true;
-    }
-}
-
 static int sample_impl(born_sampler *s, const float *logits, int64_t batch, int64_t vocab, int64_t row_stride,
                        const int32_t *history, const int32_t *hist_len, int64_t hist_stride, const float *uniforms,
                        const born_sampler_row_configs *per_row, int32_t *tokens_out, float *probs_out, int32_t *nucleus_len_out, int32_t *nucleus_ids_out,
@@ -518,7 +490,11 @@ static int sample_impl(born_sampler *s, const float *logits, int64_t batch, int6
             a.rcp_T = s->div_rcp;
         }
         if (launched == 2u) {
-            if (!s->parts.p && !s->no_parts && !s->fixed_workspace && nucleus_wants_parts(a, s->path == 2)) take_parts(s, st);
+            // (the workspace of rows that are cut into parts: 10 MiB and 90 us, which other handles do not pay; without it a workgroup takes a row)
+            if (!s->parts.p && !s->fixed_workspace && nucleus_wants_parts(a, s->path == 2)) {
+                s->parts.parts = nucleus_workspace_parts(s->max_batch);
+                take_once(st, nucleus_workspace_bytes(s->parts.parts), &s->parts.p, &s->no_parts);
+            }
             keep_first(launch_nucleus_row(a, st, nullptr, s->path == 2, s->parts));
         } else {
             keep_first(launch_sample_wide(a, st));

@@ -140,9 +140,10 @@ int born_rocm_log_softmax(born_sampler *s, const float *logits, int64_t batch, i
  *   nucleus outputs (all three NULL, or all three set with nucleus_cap > 0): the first
  *   min(n, nucleus_cap) survivors of each row in rank order; produced when 1 <= top_k <= 4096
  *   (nucleus_len_out[b] = -1 otherwise).
- * Rows of 49152 logits and more without a top-k cut, fewer than half as many as the device has compute units, are shared by several
- * workgroups through up to 10 MiB of the handle's, which the first such call outside a capture allocates; where there is none,
- * a workgroup takes a row, with the same results. */
+ * Rows without a top-k cut of 65536 logits and more, up to half as many as the device has compute units (of 49152 and more: an
+ * eighth as many), are shared by several workgroups through up to 10 MiB of the handle's, which the first such call outside a
+ * capture allocates; where there is none - under capture, or without memory - a workgroup takes a row, with the same results.  (Not those of
+ * born_rocm_sample_rows, nor with a history of more than 4096 tokens, a min-p bound, a frequency or presence penalty, or another kernel selection.) */
 int born_rocm_sample(born_sampler *s, const float *logits, int64_t batch, int64_t vocab, int64_t row_stride,
                      const int32_t *history, const int32_t *hist_len, int64_t hist_stride,
                      const float *uniforms, int32_t *tokens_out, float *probs_out,

@@ -100,3 +100,57 @@ def test_ids_outside_the_vocabulary_are_reported(rocm):
             with pytest.raises(Exception):
                 s.Status()
             s.Close()
+
+
+def test_captures_before_and_after_the_workspace(oracle, rocm):
+    """A handle's first such call under capture (a workgroup to a row: nothing is allocated), then an eager one (which allocates), then one captured
+    with the workspace; every replay of either graph, with eager calls between, gives the oracle's."""
+    import ctypes as C
+    from born_amd import _capi
+    hip = C.CDLL("libamdhip64.so")
+    rng = np.random.default_rng(6)
+    B, V, T, p = 5, 70001, 0.9, 0.95
+    xh = (2 * rng.standard_normal((B, V))).astype(np.float32)
+    x, u = rocm.DeviceBuffer.from_numpy(xh), rocm.DeviceBuffer(4 * B)
+    tok, pr = rocm.DeviceBuffer(4 * B), rocm.DeviceBuffer(4 * B)
+    s = rocm.NewSampler(rocm.SamplerConfig(Temperature=T, TopP=p), max_batch=B, max_vocab=V)
+    stream = C.c_void_p()
+    assert hip.hipStreamCreate(C.byref(stream)) == 0
+
+    def capture():
+        graph, graph_exec = C.c_void_p(), C.c_void_p()
+        assert hip.hipStreamBeginCapture(stream, 0) == 0
+        try:
+            s.Sample(x, B, V, None, None, u, tok, pr, stream=stream)
+        finally:
+            rc = hip.hipStreamEndCapture(stream, C.byref(graph))
+        assert rc == 0 and graph.value, "the capture was invalidated"
+        assert hip.hipGraphInstantiate(C.byref(graph_exec), graph, None, None, C.c_size_t(0)) == 0
+        return graph, graph_exec
+
+    def check(run):
+        uh = rng.random(B).astype(np.float32)
+        for buf, h in ((u, uh), (tok, np.full(B, -7, np.int32)), (pr, np.full(B, -1, np.float32))):
+            _capi.check(_capi.lib().born_rocm_h2d(buf.ptr, h.ctypes.data, h.nbytes, None))
+        run()
+        assert hip.hipStreamSynchronize(stream) == 0
+        s.Status()
+        want = oracle.sample(xh, uh, T, 0, p, 1.0, None, mode=oracle.MODE_FIXED)
+        assert np.array_equal(tok.to_numpy(np.int32, (B,)), want["tokens"])
+        assert np.array_equal(pr.to_numpy(np.uint32, (B,)), want["probs"].view(np.uint32))
+
+    graphs = [capture()]
+    replay = lambda g: check(lambda: hip.hipGraphLaunch(g[1], stream))  # noqa: E731
+    replay(graphs[0])
+    eager = lambda: check(lambda: s.Sample(x, B, V, None, None, u, tok, pr, stream=stream))  # noqa: E731
+    eager()
+    graphs.append(capture())
+    for _ in range(3):
+        for g in graphs:
+            replay(g)
+            eager()
+    for graph, graph_exec in graphs:
+        hip.hipGraphExecDestroy(graph_exec)
+        hip.hipGraphDestroy(graph)
+    hip.hipStreamDestroy(stream)
+    s.Close()
