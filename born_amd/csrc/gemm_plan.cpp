@@ -32,24 +32,25 @@ size_t gemm_split_workspace(int M, int K) {
 // The four tiles, and what one of them takes at K = 4096 on a part that is nearly idle and on one where every CU has one
 // (power: the clock falls), in microseconds; what a round of tiles takes besides, to fill and drain; and what slices of K take: a launch, and
 // writing and reading the partial products again.  Two parts, then three: two parts' fitted to 44 shapes in every tile and up to 16 slices (the
-// choice is within 1 % of the best of them on average, 19 % at worst: 88 x 2144 -> 11475).
+// choice is within 1 % of the best of them on average, 19 % at worst: 88 x 2144 -> 11475).  Three parts have a K below 256, so they are not sliced; their
+// times are those of a K of 4096 in proportion.
 //   64 x 128   four waves' columns twice along K    decode batches: no matrix work for padding
 //   128 x 128  four waves' columns twice along K    few columns: tiles for all CUs
 //   128 x 256  eight waves' columns
 //   256 x 256  eight waves' columns                 the most products per byte moved through LDS
 constexpr int SPLIT_TILES = 4, SPLIT_ROWS[SPLIT_TILES] = {64, 128, 128, 256}, SPLIT_COLS[SPLIT_TILES] = {128, 128, 256, 256};
 struct SplitTimes {
-    float idle_us[SPLIT_TILES], busy_us[SPLIT_TILES], round_us, slices_us, slices_bytes_per_us;
+    float idle_us[SPLIT_TILES], busy_us[SPLIT_TILES], round_us;
 };
-constexpr SplitTimes SPLIT_TIMES[2] = {{{44.f, 80.f, 170.f, 198.f}, {66.f, 114.f, 208.f, 390.f}, 4.f, 0.2f, 3.3e6f},
-                                       {{70.f, 120.f, 222.f, 405.f}, {121.f, 180.f, 317.f, 532.f}, 8.f, 3.f, 4e6f}};
+constexpr SplitTimes SPLIT_TIMES[2] = {{{44.f, 80.f, 170.f, 198.f}, {66.f, 114.f, 208.f, 390.f}, 4.f}, {{70.f, 120.f, 222.f, 405.f}, {121.f, 180.f, 317.f, 532.f}, 8.f}};
+constexpr float SLICES_US = 0.2f, SLICES_BYTES_PER_US = 3.3e6f;
 
 size_t gemm_split_bytes(const SplitPlan &p, int rows, int N, int K) {
     return gemm_split_workspace(rows, K) + (p.slices > 1 ? (size_t)p.slices * (size_t)rows * (size_t)N * sizeof(float) : 0);
 }
 
 // Tile, slices of K and rows at a time with the least expected time, among those whose packed operand and partial products fit the
-// workspace: rounds of tiles over the CUs, each with about 8 us to fill and drain; slices write and re-read partial products
+// workspace: rounds of tiles over the CUs, each with 4 us (three parts 8) to fill and drain; slices write and re-read partial products
 // and cost one more launch; a product whose rows do not fit at once is as many products, each with its own
 // launches.  (256 x 4096 -> 4096: 128 x 128 in four slices 48 us, 128 x 256 in eight 51; 300 x 2528 -> 21539: 128 x 256 145 us, 64 x
 // 128 172, 256 x 256 191.)  A choice that would not fit gives way to one that does (us, the fp32 tiles): 512 x 4096 -> 4096
@@ -88,7 +89,7 @@ SplitPlan gemm_split_plan(int M, int N, int K) {
                 const float wgs = tiles(m) * want, rounds = std::ceil(wgs / CUS);
                 const float share = std::min(1.f, wgs / CUS);
                 float us = rounds * ((T.idle_us[t] + (T.busy_us[t] - T.idle_us[t]) * share) * ((float)K / 4096.f) / want + T.round_us);
-                if (slices > 1) us += T.slices_us + (float)m * (float)N * 4.f * (want + 1) / T.slices_bytes_per_us;
+                if (slices > 1) us += SLICES_US + (float)m * (float)N * 4.f * (want + 1) / SLICES_BYTES_PER_US;
                 return us;
             };
             const long long chunks = (M + rows - 1) / rows, last = M - (chunks - 1) * rows;

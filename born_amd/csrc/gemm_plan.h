@@ -5,7 +5,7 @@
 namespace born {
 
 constexpr int SG = 32;                        // k-values of a group (two matrix instructions deep)
-constexpr int SG_BYTES = 6 * 1024;            // packed bytes of a group and a block of 32 rows, in three parts (two take 4 KiB of it)
+constexpr int SG_BYTES = 6 * 1024;            // packed bytes of a group and a block of 32 rows, in three parts (two of fp16: 4 KiB, and 2 KiB of what they leave)
 constexpr int PACK_GROUPS = 4;                // groups a workgroup of the pack handles
 
 // The workspace of a stream (linear.hip): the packed operand and the partial products of the slices of K.

@@ -2,7 +2,7 @@
 //
 // A wave owns four rows of W (columns of C) and walks along K with 128-bit loads that do not stay in the caches, two stages of
 // 2 x 256 values of each row in two register sets, so that one is in flight while the other is multiplied; x comes through the L1 (16 KiB for
-// one row of 4096).  No LDS, no barrier and few registers: about twenty waves a CU keep 200 KiB in flight.  The fp32 tiles
+// one row of 4096).  No LDS and no barrier: twelve waves a CU (131 registers with one row) keep 100 to 200 KiB in flight.  The fp32 tiles
 // (linear.hip) have a workgroup of four waves per CU there and a barrier every 32 values of K.  Waves start at different
 // places along K, since rows a large power of two apart would crowd the same memory channels.
 // Few columns: the four waves of a workgroup share a group of them and each takes a quarter of K.

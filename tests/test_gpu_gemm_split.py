@@ -1,9 +1,10 @@
-"""The large products on the bf16 matrix cores (born_amd/csrc/gemm_split.hip) against fp64 products: every tile and load
-form at the edges of tiles and of K, slices of K, rows in chunks, and operands the three bf16 parts cannot hold.
+"""The large products on the 16-bit matrix cores (born_amd/csrc/gemm_split.hip) against fp64 products: every tile and load
+form at the edges of tiles and of K, slices of K, rows in chunks, and operands the parts cannot hold.  (What two fp16 parts, K of 256 and more, lose
+and when: tests/test_gpu_gemm_f16_parts.py.)
 
 Tolerance: that of tests/test_gpu_linear.py, (4 sqrt(K) + 2) 2^-24 (sum |a| |b| + |bias|).  Three rounded bf16 parts hold an fp32
-value exactly and what the six products leave out is at most about 2^-24 |a b| a product, one of the bound's 4 sqrt(K) + 2 units.  Integer-valued
-operands whose partial sums stay below 2^24 are exact.
+value exactly and what the six products leave out is at most about 2^-24 |a b| a product, one of the bound's 4 sqrt(K) + 2 units; two fp16 parts take
+eight.  Integer-valued operands whose partial sums stay below 2^24 are exact.
 """
 import numpy as np
 import pytest
@@ -35,7 +36,7 @@ def test_matches_fp64(rocm, lin, shape, form):  # noqa: F811
     assert rms <= 0.5 * np.sqrt(K / 2) * EPS + EPS, (shape, rms)
 
 
-WORST = np.float32(1 + 2.0 ** -8 - 2.0 ** -17)            # parts 1, 2^-8, -2^-17: what is left out of its square is the most
+WORST = np.float32(1 + 2.0 ** -8 - 2.0 ** -17)            # bf16 parts 1, 2^-8, -2^-17: what three leave out of its square is the most
 
 
 def _operand(rng, family, rows, K):
@@ -75,7 +76,7 @@ def test_integer_valued_operands_are_exact(rocm, lin, shape):  # noqa: F811
     rng = np.random.default_rng(5)
     x = rng.integers(-100, 101, (M, K)).astype(np.float32)
     w = rng.integers(-100, 101, (N, K)).astype(np.float32)
-    x[:, ::17] *= 513                                    # values that take two and three parts; every sum stays below 2^24
+    x[:, ::17] *= 513                                    # values that take two and three bf16 parts (two fp16 parts'); every sum stays below 2^24
     x[:, 1::3] = 0
     w[:, ::17] = np.sign(w[:, ::17])
     want = x.astype(np.float64) @ w.T.astype(np.float64)

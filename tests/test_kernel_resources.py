@@ -13,7 +13,12 @@ LLVM = "/opt/rocm/llvm/bin"
 #: kernel -> a pattern of its mangled names
 HOT = {"sampling without a top-k cut": r"nucleus_row_kernelILi\d+E", "the same, a row's own settings": r"nucleus_row_rows_kernelILi\d+E",
        "top-k sampling": r"topk_row(_rows)?_kernelILi\d+E", "token log-probabilities": "token_logprob", "verification": "spec_",
-       "softmax": "softmax_", "large products, weights of a linear layer": r"gemm_split_kernelILb1E", "fp32 products": r"gemm_f32_"}
+       "softmax": "softmax_", "large products, weights of a linear layer": r"gemm_split_kernelILb1E", "fp32 products": r"gemm_f32_",
+       "few rows of a linear layer": r"gemm_rows_kernel", "rows in parts: the sweeps": r"nucleus_parts_(max|masses|gather)", "the left operand's parts": r"gemm_split_pack"}
+
+#: kernels that keep some registers in scratch, outside their inner loops -> the most bytes a lane
+SOME = {"rows of every kind in one launch": (r"any_row_kernel", 276), "rows in parts: the draw": (r"nucleus_parts_draw", 8),
+        "large products, [K,N] weights": (r"gemm_split_kernelILb0E", 84)}
 
 
 @pytest.fixture(scope="module")
@@ -42,3 +47,9 @@ def test_no_scratch(kernels, kernel):
     assert of, "no such kernel in the library"
     bad = {n: k["private_segment_fixed_size"] for n, k in of.items() if k["private_segment_fixed_size"] or k["vgpr_spill_count"]}
     assert not bad, bad
+
+
+@pytest.mark.parametrize("kernel", SOME)
+def test_no_more_scratch(kernels, kernel):
+    of = {n: k["private_segment_fixed_size"] for n, k in kernels.items() if re.search(SOME[kernel][0], n)}
+    assert of and max(of.values()) <= SOME[kernel][1], of
