@@ -266,9 +266,9 @@ int born_rocm_spec_verify_bonus(born_sampler *s, const float *target, int64_t ta
  *   rows and columns for which that would show, three, exact, with 2^-34 of a product left out: rows of few terms (the square of the magnitudes' sum below 12 times
  *   the sum of squares), rows of whole numbers of 12 to 22 bits (times any power of two), rows of which an eighth shares one significand of
  *   more than 11 bits, and columns whose first 32 values add up to less than three times their largest.
- * Sums of whole numbers below 2^24 are exact where the rows' are of at most 22 bits, and so are rows and columns that select (a power of
+ * Sums of whole numbers below 2^24 are exact where no number has more than 22 bits, and so are rows and columns that select (a power of
  * two, all else zero).  Against fp64 the error of dense sums is no larger than the fp32 matrix cores' (2-norm; k = 256 0.4, 4096 0.5 of it); sums of
- * some 12 to 100 terms that are spread over a long k are rounded twice in every group of 32 that holds one, and their error is up to twice theirs.
+ * some 12 to 100 terms that are spread over a long k are rounded twice in every group of 32 that holds one, and their error is up to one and a half times theirs.
  *
  * born_rocm_linear: out[batch, out_features] = x[batch, in_features] @ weight^T + bias, weight stored
  * [out_features, in_features] row-major as nn.Linear holds it, bias [out_features] or NULL: Linear.Forward,

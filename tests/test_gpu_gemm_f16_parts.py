@@ -85,8 +85,9 @@ def test_values_cut_under_columns_far_above_their_scale(rocm, lin):  # noqa: F81
     assert (np.abs(got - exact) / exact).max() <= 16 * 2.0 ** -24
 
 
-# a tile of each height; ragged M, N and K, and K in slices (64 x 6100)
-WHOLE_SHAPES = [(20, 45001, 2048), (48, 130000, 257), (100, 15011, 1057), (130, 40004, 300), (270, 16000, 352), (64, 6100, 4096)]
+# every tile, by 128-bit loads and value by value; ragged M, N and K, and K in slices (64 x 6100, 128 x 6000)
+WHOLE_SHAPES = [(20, 45001, 2048), (48, 130000, 257), (100, 15011, 1057), (130, 40004, 300), (270, 16000, 352), (64, 6100, 4096),
+                (128, 6000, 4096), (128, 6001, 4099), (300, 40001, 517), (512, 20001, 513)]
 
 
 def _both_forms(rocm, lin, x, w):
@@ -173,3 +174,27 @@ def test_error_is_that_of_whole_operands(rocm, lin, family, value, K):  # noqa: 
     split, tiles = (np.sqrt(np.mean((b.to_numpy(np.float32, (M, N))[:, some] - exact) ** 2) / np.mean(exact ** 2)) for b in (one, two))
     print(f"{family} {value} {K}: {split * 2 ** 24:.3f} {tiles * 2 ** 24:.3f} units")
     assert split <= max(1.03 * tiles, (1 + np.sqrt(K / 16) / 2) * 2.0 ** -24), (split, tiles)
+
+
+@pytest.mark.parametrize("shape", [(48, 36000, 928), (140, 33000, 352), (300, 40001, 517), (260, 66000, 300)])
+def test_fused_heads_see_the_plain_head_s_whole_rows(rocm, lin, shape):  # noqa: F811
+    """Batches of which a tile is whole and others may not be: bit for bit the plain head's numbers."""
+    from tests.test_gpu_linear import _fused_vs_unfused
+    M, N, K = shape
+    rng = np.random.default_rng(M)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    x[3] = 0
+    x[3, 5], x[M - 1] = 2, np.round(1000 * x[M - 1])
+    w = rng.standard_normal((N, K), dtype=np.float32) * np.float32(1.5 / np.sqrt(K))
+    bias = np.float32(0.3) * rng.standard_normal(N, dtype=np.float32)
+    x[M - 1] /= 1024
+    hist = rng.integers(0, N, size=(M, 40)).astype(np.int32)
+    _fused_vs_unfused(rocm, lin, x, w, bias, rocm.SamplerConfig(Temperature=0.7, TopK=50, TopP=0.9, RepetitionPenalty=1.15), hist)
+    s = rocm.NewSampler(max_batch=M, max_vocab=N)
+    layer = lin.Linear(K, N, rocm.DeviceBuffer.from_numpy(w), rocm.DeviceBuffer.from_numpy(bias))
+    dx, logits, a, b = rocm.DeviceBuffer.from_numpy(x), rocm.DeviceBuffer(M * N * 4), rocm.DeviceBuffer(4 * M), rocm.DeviceBuffer(4 * M)
+    layer.Forward(dx, (M, K), logits)
+    s.Argmax(logits, M, N, a)
+    lin.ForwardArgmax(s, layer, dx, (M, K), b)
+    assert np.array_equal(a.to_numpy(np.int32, (M,)), b.to_numpy(np.int32, (M,)))
+    s.Close()

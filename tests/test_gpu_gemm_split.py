@@ -4,7 +4,7 @@ and when: tests/test_gpu_gemm_f16_parts.py.)
 
 Tolerance: that of tests/test_gpu_linear.py, (4 sqrt(K) + 2) 2^-24 (sum |a| |b| + |bias|).  Three rounded bf16 parts hold an fp32
 value exactly and what the six products leave out is at most about 2^-24 |a b| a product, one of the bound's 4 sqrt(K) + 2 units; two fp16 parts take
-eight.  Integer-valued operands whose partial sums stay below 2^24 are exact.
+eight.  Integer-valued operands of up to 22 bits whose partial sums stay below 2^24 are exact.
 """
 import numpy as np
 import pytest
