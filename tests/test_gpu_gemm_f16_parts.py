@@ -198,3 +198,22 @@ def test_fused_heads_see_the_plain_head_s_whole_rows(rocm, lin, shape):  # noqa:
     lin.ForwardArgmax(s, layer, dx, (M, K), b)
     assert np.array_equal(a.to_numpy(np.int32, (M,)), b.to_numpy(np.int32, (M,)))
     s.Close()
+
+
+@pytest.mark.parametrize("shape", [(64, 24000, 1024), (100, 15011, 1057), (128, 12000, 1024), (300, 16000, 1024)])
+def test_sums_of_nothing_but_tiny_products(rocm, lin, shape):  # noqa: F811
+    """Values far below their row's and column's largest, none of which is cut, where those largest meet zeros: the accumulators do not hold such sums."""
+    M, N, K = shape
+    rng = np.random.default_rng(K)
+    x, w = rng.standard_normal((M, K), dtype=np.float32), np.zeros((N, K), np.float32)
+    rows = np.arange(2, M, 3)
+    sized = lambda *s: (1 + rng.random(s, dtype=np.float32)) * rng.choice(np.array([-1, 1], np.float32), s)  # noqa: E731
+    w[:, ::16] = 1
+    w[:, [41, 700]] = np.float32(2.0 ** -18) * sized(N, 2)
+    x[rows] = 0
+    x[rows, 300] = 1
+    x[np.ix_(rows, [41, 700])] = np.float32(2.0 ** -25) * sized(len(rows), 2)
+    for got in _both_forms(rocm, lin, x, w):
+        exact = x[rows].astype(np.float64) @ w.T.astype(np.float64)
+        err = np.abs(got[rows] - exact) / _bound(x[rows], w, None, K)
+        assert err.max() <= 1, err.max()
