@@ -43,6 +43,11 @@ def _operands(kind, rng, M, N, K):
         return x, w
     if kind == "signs and zeros":                             # results of zero by the score
         return rng.integers(-1, 2, (M, K)).astype(np.float32), rng.integers(-1, 2, (N, K)).astype(np.float32) * np.float32(0.37)
+    if kind == "late large values":                          # the tiles that begin before them are done again
+        w[:, K // 2:] *= 1000
+        return x, w
+    if kind == "heavy tails":
+        return x, w / np.maximum(np.abs(rng.standard_normal((N, K), dtype=np.float32)), np.float32(1e-6))
     if kind == "columns that outgrow their scale":
         w[::1000, K - 3:] *= np.float32(2.0 ** 30)
         w[5::1000, K - 3:] *= np.float32(2.0 ** -30)
@@ -54,7 +59,7 @@ def _operands(kind, rng, M, N, K):
 
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("kind", ["few terms of every magnitude", "rows of a wide range", "one huge factor that meets zeros",
-                                  "columns that begin with zeros", "few values in a column", "equal rows", "signs and zeros", "columns that outgrow their scale", "units"])
+                                  "columns that begin with zeros", "few values in a column", "equal rows", "signs and zeros", "late large values", "heavy tails", "columns that outgrow their scale", "units"])
 def test_every_result_keeps_its_precision(rocm, lin, kind, shape):  # noqa: F811
     M, N, K = shape
     rng = np.random.default_rng(K)
@@ -217,3 +222,20 @@ def test_sums_of_nothing_but_tiny_products(rocm, lin, shape):  # noqa: F811
         exact = x[rows].astype(np.float64) @ w.T.astype(np.float64)
         err = np.abs(got[rows] - exact) / _bound(x[rows], w, None, K)
         assert err.max() <= 1, err.max()
+
+
+@pytest.mark.parametrize("shape", [(64, 24000, 1024), (100, 15011, 1057), (128, 12000, 1024), (300, 16000, 1024)])
+def test_columns_that_outgrow_their_scale_lose_nothing(rocm, lin, shape):  # noqa: F811
+    """The 2-norm of the error of columns whose second half is 1000 times their first, beside that of the same columns reversed, which begin with their
+    largest: both are sums of the same products in groups of 32, one and a half walks of their roundings at most."""
+    M, N, K = shape
+    rng = np.random.default_rng(K)
+    x, w = rng.standard_normal((M, K), dtype=np.float32), rng.standard_normal((N, K), dtype=np.float32)
+    w[:, K // 2:] *= 1000
+    some = rng.choice(N, 2000, replace=False)
+    exact = x.astype(np.float64) @ w[some].T.astype(np.float64)
+    size = np.sqrt(np.mean(exact ** 2))
+    rms = lambda got: np.sqrt(np.mean((got[:, some] - exact) ** 2)) / size  # noqa: E731
+    late, early = rms(_gpu_linear(rocm, lin, x, w, None)), rms(_gpu_linear(rocm, lin, x[:, ::-1].copy(), w[:, ::-1].copy(), None))
+    print(f"{shape}: {late * 2 ** 24:.2f} and {early * 2 ** 24:.2f} units")
+    assert late <= 1.3 * early and late <= (1 + np.sqrt(K / 16) / 2) * 2.0 ** -24, (late, early)
