@@ -155,6 +155,26 @@ __device__ __forceinline__ u64 qfix32(float e, float scale32) {
     const u32 lo = (u32)(__builtin_amdgcn_fractf(t) * 4294967296.0f);
     return ((u64)hi << 32) | (u64)lo;
 }
+// The same integer masses, summed in fp64 by additions that round towards zero.  A sum that begins at 2^(52 - S) has a last place of 2^-S, so that
+// each addition adds trunc(e * 2^S) * 2^-S, as long as what is added stays below 2^(52 - S) (or equal to it): two instructions a logit where the integer
+// parts and their sum take seven.  Only fp64 rounding is switched (fp32 has its own mode bits), from mass_sum_begin to mass_sum_end.  The additions are
+// asm volatile and the values pass through the switches, so that no addition of theirs leaves, and no fp64 operation on the values given to
+// a switch enters; the code between has no other fp64 arithmetic.
+__device__ __forceinline__ double mass_sum_start(int S) { return __longlong_as_double((long long)(1023 + 52 - S) << 52); }
+__device__ __forceinline__ void mass_sum_begin(double &a) { asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 3" : "+v"(a)); }
+__device__ __forceinline__ void mass_sum_begin(double &a, double &b) { asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 3" : "+v"(a), "+v"(b)); }
+__device__ __forceinline__ void mass_sum_add(double &acc, float e) {
+    const double x = (double)e;
+    asm volatile("v_add_f64 %0, %0, %1" : "+v"(acc) : "v"(x));
+}
+__device__ __forceinline__ void mass_sum_end(double &a) { asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 0" : "+v"(a)); }
+template <int N>
+__device__ __forceinline__ void mass_sum_end(double (&a)[N], double (&b)[N]) {
+    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 0" : "+v"(a[0]), "+v"(b[0]));
+#pragma unroll
+    for (int i = 1; i < N; i++) asm volatile("" : "+v"(a[i]), "+v"(b[i]));   // (in order after the switch)
+}
+__device__ __forceinline__ u64 mass_sum_of(double acc, double start) { return (u64)__double_as_longlong(acc) - (u64)__double_as_longlong(start); }
 __device__ __forceinline__ float mass_scale(int S) { return __uint_as_float((u32)(S + 127) << 23); }
 
 // ---- built-in uniform stream ------------------------------------------------
