@@ -5,8 +5,8 @@
 //            the penalised logit, so no division is needed yet): m = z(max), and the span of d = m - z.
 //   sweep 2  integer masses trunc(expneg(d) * 2^S) accumulated into 4096 bins that cover exactly that span
 //            (u64 LDS atomics), then an inclusive scan: cumulative mass in rank order, bin by bin.
-//   targets  the top-p cut target ceil(p * Z) and the draw target each fall into one bin; the draw's bin is
-//            predicted from the interval the nucleus mass must lie in, so one gather usually serves both.
+//   targets  the top-p cut target ceil(p * Z) falls into one bin, the draw's into one of the few that the interval of
+//            the nucleus's mass allows: one gather serves both.
 //   sweep 3  gather: a compare of the penalised logit against the wanted bins' value ranges (widened, so
 //            that it can only over-select) stages about 1 % of the row in per-wave LDS lists (ballot + lane
 //            rank); the staged entries are then classified exactly.
@@ -285,7 +285,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     extern __shared__ __align__(16) u64 nuc_dyn[];
     __shared__ BlockScratch scr;
     __shared__ int s_n, s_over, s_nseen;
-    __shared__ u64 s_win, s_mass, s_slot0[4];
+    __shared__ u64 s_win, s_mass, s_slot0[2];
     __shared__ u32 s_wcount[NUC_WAVES];
 
     u64 *const mass = nuc_dyn;                                                   // [NUC_BINS] masses, then cumulative
@@ -455,7 +455,8 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     //   +inf, y >= 2^100        not in such a row (the maximum is below 2^90).
     // Beyond d = 80 the specified mass is 0, and so is trunc(exp(x) * 2^S) down to the clamp (S <= 61).  A seen id's
     // stored logit may exceed the penalised maximum: clamped to x = 0, some mass that the correction takes out again.
-    const float scale32 = r.scale * 2.3283064365386963e-10f, nsbin = -r.sbin;
+    const float nsbin = -r.sbin;
+    const float scale32 = r.scale * 2.3283064365386963e-10f;
     auto lin_z = [&](float y) { return r.T == 1.0f ? y : nuc_z_shortcut<ANY_T>(r, y); };
     auto lin_put = [&](float z, auto minus) {
         const float x = z - r.m;
@@ -465,16 +466,6 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     };
     typedef std::integral_constant<bool, false> Plus;
     typedef std::integral_constant<bool, true> Minus;
-    if (lin && r.penal) {
-        // The histogram is a sum of integers modulo 2^64: sweep 2 adds every id's stored logit, so each seen id's stored
-        // logit is taken out (by the same arithmetic, to the bit) and its penalised logit put in, here, in any order.
-#pragma unroll
-        for (int k = 0; k < NUC_SEEN; k++)
-            if (seen_id[k] >= 0) {
-                lin_put(lin_z(seen_raw[k]), Minus());
-                lin_put(lin_z(seen_y[k]), Plus());
-            }
-    }
 
     BORN_STAMP(a, row, 2);
 #if defined(BORN_NUC_STOP_AFTER) && BORN_NUC_STOP_AFTER == 1
@@ -484,6 +475,16 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
 #endif
     // ---- sweep 2: integer masses by bin
     if (lin) {
+        if (r.penal) {
+            // The histogram is a sum of integers modulo 2^64: the sweep adds every id's stored logit, so each seen id's stored
+            // logit is taken out (by the same arithmetic, to the bit) and its penalised logit put in, here, in any order.
+#pragma unroll
+            for (int k = 0; k < NUC_SEEN; k++)
+                if (seen_id[k] >= 0) {
+                    lin_put(lin_z(seen_raw[k]), Minus());
+                    lin_put(lin_z(seen_y[k]), Plus());
+                }
+        }
         if (r.T == 1.0f) sweep_plain(Cached(), [&](int, float y) { lin_put(y, Plus()); }, first);
         else sweep_plain(Cached(), [&](int, float y) { lin_put(nuc_z_shortcut<ANY_T>(r, y), Plus()); }, first);
     } else if (r.T == 1.0f && !r.degenerate) {
@@ -532,67 +533,35 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     lds_barrier();
     const u64 *cum = mass;
 
-    // ---- the bins to gather: the top-p cut's, and the draw's predicted from the interval [tp, cum[bp]]
+    // ---- the bins to gather: the top-p cut's, w0, and those that the draw may fall into, w1 to w2.  The mass of the nucleus lies in
+    // [tp, cum[w0]], which bounds the draw's target.  All of w1 .. w2 are few logits: what lies strictly between them adds up to at most the
+    // mass of bin w0, and each of its logits has at least the mass of any in w0 (w2 <= w0), so there are no more of them than w0 holds.
+    // (Before, up to two such bins, else the cut's alone and two more sweeps of the row for a draw elsewhere.  us, then and now: 96 x 100 003, settings
+    // per row, 78 and 49 (50 where every row's draw was in those two bins); 256 x 128 256 of twenty likely tokens, top-p 0.9, 131 and 82; 100 x 300 23.6 and 12.1.)
     const bool cut = cfg_p < 1.0f;
     u64 tp = Zk;
     int w0, w1, w2;
-    bool unpredicted = false;                                        // the draw's bin could not be narrowed down to two
     if (cut) {
         tp = top_p_target(cfg_p, Zk);
         w0 = nuc_first_reaching(cum, tp);
         const u64 hi = cum[w0] < Zk ? cum[w0] : Zk;
         w1 = nuc_first_reaching(cum, draw_target(u, tp));
         w2 = nuc_first_reaching(cum, draw_target(u, hi));
-        unpredicted = w2 - w1 > 1;
-        if (unpredicted) w1 = w2 = w0;
     } else {
         w0 = w1 = w2 = nuc_first_reaching(cum, draw_target(u, Zk));
     }
-    // Where that prediction gives up (a peaked row: the cut's bin holds so much of the mass that the draw may fall
-    // anywhere, and a draw outside the gathered bins costs further sweeps of the row), a small nucleus is gathered
-    // whole, every bin down to the cut's: the draw then needs no predicted bin.  A bin's mass over the smallest mass a
-    // logit in it can have bounds the number of its logits.
-    bool whole = false;
-    if (unpredicted && !r.degenerate && w0 < NUC_BINS - 1) {
-        const float per_bin = 1.44269504f / r.sbin;                  // bin b holds d < (b + 1) / sbin: masses above scale * 2^-((b + 1) * per_bin)
-        if (__builtin_amdgcn_exp2f(-(float)(w0 + 1) * per_bin) * r.scale >= 1024.0f) {   // (integer truncation is then below 0.1 %)
-            float bound = 0.0f;
-#pragma unroll
-            for (int t = 0; t < NUC_PER; t++) {
-                const int b = tid * NUC_PER + t;
-                if (b <= w0) {
-                    const u64 mb = cum[b] - (b ? cum[b - 1] : 0ull);
-                    bound += (float)mb / (__builtin_amdgcn_exp2f(-(float)(b + 1) * per_bin) * r.scale * 0.98f);
-                }
-            }
-            // (summed in sixteenths, each thread's share rounded up)
-            const u32 total = block_sum_u32<NUC_BLOCK, true>((u32)fminf(ceilf(bound * 16.0f), 1048576.0f), &scr);
-            whole = total <= (u32)(16 * NUC_CAP / 2);                 // (half the capacity: the lists are per wave, the logits fall as they may)
-        }
-    }
-    if (whole) w1 = w2 = w0;
 
     BORN_STAMP(a, row, 4);
     // ---- sweep 3: stage the logits inside the wanted bins' ranges, then classify them exactly
     {
+        // The cut's bin, and above it (w2 <= w0) the draw's; one interval where the two meet.
         float lo0, hi0, lo1, hi1, lo2, hi2;
         nuc_range(r, w0, lo0, hi0);
         nuc_range(r, w1, lo1, hi1);
         nuc_range(r, w2, lo2, hi2);
-        if (whole) hi0 = hi1 = hi2 = INFINITY;                       // every bin down to the cut's
-        // The three value ranges as disjoint intervals in ascending order, overlapping ones merged (the draw's two bins
-        // are neighbours, and often the cut's bin is one of them): most rows test one or two intervals per logit.
-        // An unused interval is (+inf, -inf), which only a NaN passes (as it passes a real one: classified below).
-        if (lo1 < lo0) { float t = lo0; lo0 = lo1; lo1 = t; t = hi0; hi0 = hi1; hi1 = t; }
-        if (lo2 < lo1) { float t = lo1; lo1 = lo2; lo2 = t; t = hi1; hi1 = hi2; hi2 = t; }
-        if (lo1 < lo0) { float t = lo0; lo0 = lo1; lo1 = t; t = hi0; hi0 = hi1; hi1 = t; }
-        int nint = 3;
-        if (!(lo1 > hi0)) { hi0 = fmaxf(hi0, hi1); lo1 = lo2; hi1 = hi2; lo2 = INFINITY; hi2 = -INFINITY; nint--; }
-        if (nint == 3 ? !(lo2 > hi1) : !(lo1 > hi0)) {
-            if (nint == 3) { hi1 = fmaxf(hi1, hi2); lo2 = INFINITY; hi2 = -INFINITY; }
-            else { hi0 = fmaxf(hi0, hi1); lo1 = INFINITY; hi1 = -INFINITY; }
-            nint--;
-        }
+        lo1 = lo2;
+        const bool one = !(lo1 > hi0);
+        if (one) hi0 = fmaxf(hi0, hi1);
         uint2 *list = stage + wave_id() * NUC_WCAP;
         // The wave's running count of staged entries lives in LDS, not in a register of every lane: the row visitor
         // lets different lanes of a wave sit out different visits (the row's last whole float4 blocks end inside a
@@ -619,28 +588,23 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         if (lin) {
             // (the stored logits; a seen id's stored logit that passes is dropped below, its penalised logit is offered
             // here under the id with the top bit set)
-            if (nint == 1) {
+            if (one) {
                 sweep_plain(Streamed(), [&](int j, float y) { append(!(y < lo0) & !(y > hi0), y, j); }, first);
             } else {
-                sweep_plain(Streamed(), [&](int j, float y) {
-                    append((!(y < lo0) & !(y > hi0)) | (!(y < lo1) & !(y > hi1)) | (!(y < lo2) & !(y > hi2)), y, j);
-                }, first);
+                sweep_plain(Streamed(), [&](int j, float y) { append((!(y < lo0) & !(y > hi0)) | (!(y < lo1) & !(y > hi1)), y, j); }, first);
             }
             if (r.penal) {
 #pragma unroll
                 for (int k = 0; k < NUC_SEEN; k++)
                     if (seen_id[k] >= 0) {
                         const float y = seen_y[k];
-                        append((!(y < lo0) & !(y > hi0)) | (!(y < lo1) & !(y > hi1)) | (!(y < lo2) & !(y > hi2)), y,
-                               (int)((u32)seen_id[k] | 0x80000000u));
+                        append((!(y < lo0) & !(y > hi0)) | (!(y < lo1) & !(y > hi1)), y, (int)((u32)seen_id[k] | 0x80000000u));
                     }
             }
-        } else if (nint == 1) {
+        } else if (one) {
             sweep(Streamed(), [&](int j, float y) { append(!(y < lo0) & !(y > hi0), y, j); }, NucNoPre(), first);
         } else {
-            sweep(Streamed(), [&](int j, float y) {
-                append((!(y < lo0) & !(y > hi0)) | (!(y < lo1) & !(y > hi1)) | (!(y < lo2) & !(y > hi2)), y, j);
-            }, NucNoPre(), first);
+            sweep(Streamed(), [&](int j, float y) { append((!(y < lo0) & !(y > hi0)) | (!(y < lo1) & !(y > hi1)), y, j); }, NucNoPre(), first);
         }
         const u32 count = __hip_atomic_load(wcount, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
         if (count > (u32)NUC_WCAP && lane_id() == 0) s_over = 1;
@@ -659,7 +623,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
                 const float z = nuc_z(r, __uint_as_float(c.x));
                 const float d = nuc_d(r, z);
                 const int b = nuc_bin(r, d);
-                const int slot = stale ? -1 : whole ? (b <= w0 ? 0 : -1) : b == w0 ? 0 : b == w1 ? 1 : b == w2 ? 2 : -1;
+                const int slot = stale ? -1 : b == w0 ? 0 : b >= w1 && b <= w2 ? 1 : -1;
                 if (slot >= 0) {
                     take = true;
                     key = make_key64(z, (int)c.y);
@@ -755,8 +719,8 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         const u64 target = phase == 0 ? tp : draw_target(u, Zp);
         const int b = phase == 0 ? w0 : nuc_first_reaching(cum, target);
         u64 base = b ? cum[b - 1] : 0ull;
-        const int slot = !listed ? -1 : whole ? (b <= w0 ? 0 : -1) : b == w0 ? 0 : b == w1 ? 1 : b == w2 ? 2 : -1;
-        if (whole && slot == 0) base = 0ull;                         // the list starts at the row's maximum
+        const int slot = !listed ? -1 : b == w0 ? 0 : b >= w1 && b <= w2 ? 1 : -1;
+        if (slot == 1) base = w1 ? cum[w1 - 1] : 0ull;               // (listed from w1 on)
         if (slot < 0) {
             u64 prefix = 0ull;
             int plen = 0;
