@@ -14,7 +14,7 @@ LLVM = "/opt/rocm/llvm/bin"
 HOT = {"sampling without a top-k cut": r"nucleus_row_kernelILi\d+E", "the same, a row's own settings": r"nucleus_row_rows_kernelILi\d+E",
        "top-k sampling": r"topk_row(_rows)?_kernelILi\d+E", "token log-probabilities": "token_logprob", "verification": "spec_",
        "softmax": "softmax_", "large products, weights of a linear layer": r"gemm_split_kernelILb1E", "fp32 products": r"gemm_f32_",
-       "few rows of a linear layer": r"gemm_rows_kernel", "rows in parts: the sweeps": r"nucleus_parts_(max|masses|gather)", "the left operand's parts": r"gemm_split_pack"}
+       "few rows of a linear layer": r"gemm_rows_kernel", "small products": r"gemm_small_kernel", "rows in parts: the sweeps": r"nucleus_parts_(max|masses|gather)", "the left operand's parts": r"gemm_split_pack"}
 
 #: kernels that keep some registers in scratch, outside their inner loops -> the most bytes a lane
 SOME = {"rows of every kind in one launch": (r"any_row_kernel", 276), "rows in parts: the draw": (r"nucleus_parts_draw", 8),
