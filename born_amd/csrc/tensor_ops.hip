@@ -20,6 +20,16 @@ __device__ __forceinline__ float tensor_apply(float x, float y) {
 
 constexpr int TOPS_BLOCK = 256;
 
+// n / d for n < 2^31 by a multiplication and a shift (Granlund and Montgomery, 1994).
+struct FastDiv {
+    u32 m, s;
+    explicit FastDiv(u32 d) : m(0), s(0) {                           // (host)
+        while ((1ull << s) < d) s++;
+        m = (u32)((((1ull << s) - d) << 32) / d + 1);
+    }
+    __device__ __forceinline__ u32 operator()(u32 n) const { return (__umulhi(n, m) + n) >> s; }
+};
+
 // Same shape, both operands contiguous: 128-bit accesses, one pass.
 template <int OP>
 __global__ __launch_bounds__(TOPS_BLOCK) void binary_flat_kernel(const float *a, const float *b, float *out, long long n,
@@ -106,6 +116,30 @@ __global__ __launch_bounds__(TOPS_BLOCK) void binary_general_kernel(TensorIndexA
             ob += idx * t.sb[d];
         }
         out[i] = tensor_apply<OP>(a[oa], b[ob]);
+    }
+}
+
+// The same for three dimensions (a bias per channel of images: [N,C,H,W] and [1,C,1,1]) whose results 31 bits count: no division, and
+// N4 results along the last dimension at once, four where its extent is a multiple of four (operands of any start by 128-bit loads).
+// [64,32,24,24] + [1,32,1,1] 8.1 -> 4.0 us, [64,64,8,8] 4.5 -> 2.4.
+template <int OP, int N4>
+__global__ __launch_bounds__(TOPS_BLOCK) void binary_three_kernel(const float *a, const float *b, float *out, u32 items, FastDiv by_inner, FastDiv by_middle, u32 inner,
+                                                                  u32 middle, long long sa0, long long sa1, int sa2, long long sb0, long long sb1, int sb2) {
+    const u32 i = blockIdx.x * (u32)TOPS_BLOCK + threadIdx.x;        // (inner: items of the last dimension)
+    if (i >= items) return;
+    const u32 row = by_inner(i), c = (i - row * inner) * N4, x = by_middle(row), y = row - x * middle;
+    const float *pa = a + x * sa0 + y * sa1 + c * (long long)sa2, *pb = b + x * sb0 + y * sb1 + c * (long long)sb2;
+    if constexpr (N4 == 1) {
+        out[i] = tensor_apply<OP>(*pa, *pb);
+    } else {
+        row_f32x4 va, vb, v;
+        if (sa2) va = *reinterpret_cast<const row_f32x4 *>(pa);
+        else va = row_f32x4{*pa, *pa, *pa, *pa};
+        if (sb2) vb = *reinterpret_cast<const row_f32x4 *>(pb);
+        else vb = row_f32x4{*pb, *pb, *pb, *pb};
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = tensor_apply<OP>(va[k], vb[k]);
+        *reinterpret_cast<row_f32x4 *>(out + (long long)i * 4) = v;
     }
 }
 
@@ -248,6 +282,31 @@ __global__ __launch_bounds__(TOPS_BLOCK) void maxpool2d_kernel(const float *in, 
     }
 }
 
+// The same where 31 bits count the results: found without dividing; KS: the window's size, its loads in flight together (0: any).
+template <int KS>
+__global__ __launch_bounds__(TOPS_BLOCK) void maxpool2d_counted_kernel(const float *in, float *out, u32 total, FastDiv by_plane, FastDiv by_row,
+                                                                       u32 plane, u32 WO, long long HW, int W, int ksize, int stride) {
+    const u32 i = blockIdx.x * (u32)TOPS_BLOCK + threadIdx.x;
+    if (i >= total) return;
+    const u32 n = by_plane(i), at = i - n * plane, oh = by_row(at), ow = at - oh * WO;
+    const float *ip = in + n * HW + (long long)oh * stride * W + (long long)ow * stride;
+    float best = -1e38f;
+    if constexpr (KS > 0) {
+        float v[KS * KS];
+#pragma unroll
+        for (int k = 0; k < KS * KS; k++) v[k] = ip[(long long)(k / KS) * W + k % KS];
+#pragma unroll
+        for (int k = 0; k < KS * KS; k++) best = v[k] > best ? v[k] : best;
+    } else {
+        for (int kh = 0; kh < ksize; kh++)
+            for (int kw = 0; kw < ksize; kw++) {
+                const float v = ip[(long long)kh * W + kw];
+                if (v > best) best = v;
+            }
+    }
+    out[i] = best;
+}
+
 hipError_t launch_conv2d(const float *in, const float *ker, float *out, int N, int C, int H, int W, int CO, int KH, int KW,
                          int HO, int WO, int stride, int padding, hipStream_t st);
 hipError_t launch_maxpool2d(const float *in, float *out, long long planes, int H, int W, int HO, int WO, int ksize, int stride,
@@ -287,6 +346,16 @@ static void launch_binary_op(const TensorIndexArgs &t, const float *a, const flo
         const long long items = rows * strips;
         hipLaunchKernelGGL(binary_rowcol_kernel<OP>, dim3((unsigned)(items > 65536 ? 65536 : items)), dim3(TOPS_BLOCK), 0, st,
                            a, b, out, rows, cols, ars, t.sa[t.nd - 1], brs, t.sb[t.nd - 1]);
+    } else if (t.nd == 3 && t.n < (1ll << 31) && t.sa[2] <= 1 && t.sb[2] <= 1) {
+        const bool four = (t.shape[2] & 3) == 0;
+        const u32 inner = (u32)(four ? t.shape[2] / 4 : t.shape[2]), middle = (u32)t.shape[1], items = (u32)(four ? t.n / 4 : t.n);
+        const dim3 grid((items + TOPS_BLOCK - 1) / TOPS_BLOCK), block(TOPS_BLOCK);
+        if (four)
+            hipLaunchKernelGGL((binary_three_kernel<OP, 4>), grid, block, 0, st, a, b, out, items, FastDiv(inner), FastDiv(middle), inner, middle, t.sa[0], t.sa[1],
+                               (int)t.sa[2], t.sb[0], t.sb[1], (int)t.sb[2]);
+        else
+            hipLaunchKernelGGL((binary_three_kernel<OP, 1>), grid, block, 0, st, a, b, out, items, FastDiv(inner), FastDiv(middle), inner, middle, t.sa[0], t.sa[1],
+                               (int)t.sa[2], t.sb[0], t.sb[1], (int)t.sb[2]);
     } else {
         hipLaunchKernelGGL(binary_general_kernel<OP>, dim3(tensor_grid(t.n)), dim3(TOPS_BLOCK), 0, st, t, a, b, out);
     }
@@ -401,6 +470,82 @@ __global__ __launch_bounds__(TOPS_BLOCK) void conv2d_group_kernel(const float *_
     }
 }
 
+// The same for square kernels of 3 and 5 without padding, where 31 bits count the positions: a row of the patch is a 128-bit load and
+// one more (96 bits for 3), a channel's patch is loaded while the one before is summed, and a position is found without dividing.
+// us, conv2d_group_kernel and here: [64,1,28,28] * [32,1,5,5] 8.0 4.3, [64,32,12,12] * [64,32,5,5] 31.5 20.1, [1,32,12,12] * [64,32,5,5] 22.1 10.8,
+// [256,32,30,30] * [64,32,5,5] 655 348 (17.7 G products and sums at 51 T a second), [32,16,32,32] * [32,16,3,3] 14.9 10.9.  A wave alone on its SIMD issues
+// a vector instruction every eight clocks, so output channels per lane trade loads against waves: [64,32,12,12] has one wave a SIMD with four (26.8 us), two with
+// two, and with one its loads are the limit (26.3).  Kernel values in LDS, read by broadcasts, 20.4; by lane and v_readlane 18.6, but 520 for 348 above.
+typedef float tensor_f32x3 __attribute__((ext_vector_type(3), aligned(4)));
+template <int KT, int COG>
+__global__ __launch_bounds__(TOPS_BLOCK) void conv2d_square_kernel(const float *__restrict__ in, const float *__restrict__ ker, float *__restrict__ out,
+                                                                   int C, int H, int W, int CO, int stride, u32 P, FastDiv by_plane, FastDiv by_row, u32 plane, u32 WO) {
+    constexpr int KK = KT * KT;
+    const u32 p = min(blockIdx.x * (u32)TOPS_BLOCK + threadIdx.x, P - 1u);
+    const int co0 = (int)blockIdx.y * COG;
+    const u32 n = by_plane(p), at = p - n * plane, oh = by_row(at), ow = at - oh * WO;
+    const long long HW = (long long)H * W, ksz = (long long)C * KK;
+    const float *const ip = in + (long long)n * C * HW + (long long)oh * stride * W + ow * stride;
+    const float *kp[COG];                                            // uniform: the kernel values come through scalar loads
+#pragma unroll
+    for (int g = 0; g < COG; g++) kp[g] = ker + min(co0 + g, CO - 1) * ksz;   // (a channel past the last: computed, not stored)
+
+    auto load = [&](int c, float (&x)[KK]) {
+#pragma unroll
+        for (int kh = 0; kh < KT; kh++) {
+            const float *const rowp = ip + c * HW + (long long)kh * W;
+            if constexpr (KT == 3) {
+                const tensor_f32x3 v = *reinterpret_cast<const tensor_f32x3 *>(rowp);
+#pragma unroll
+                for (int kw = 0; kw < 3; kw++) x[kh * KT + kw] = v[kw];
+            } else {
+                const row_f32x4 v = *reinterpret_cast<const row_f32x4 *>(rowp);
+#pragma unroll
+                for (int kw = 0; kw < 4; kw++) x[kh * KT + kw] = v[kw];
+                x[kh * KT + 4] = rowp[4];
+            }
+        }
+    };
+    float sum[COG];
+#pragma unroll
+    for (int g = 0; g < COG; g++) sum[g] = 0.0f;
+    auto add = [&](int c, const float (&x)[KK]) {
+#pragma unroll
+        for (int t = 0; t < KK; t++)
+#pragma unroll
+            for (int g = 0; g < COG; g++) sum[g] += kp[g][c * KK + t] * x[t];
+    };
+    float x[KK], y[KK];
+    load(0, x);
+    int c = 0;
+    for (; c + 2 < C; c += 2) {
+        load(c + 1, y);
+        add(c, x);
+        load(c + 2, x);
+        add(c + 1, y);
+    }
+    if (c + 1 < C) {
+        load(c + 1, y);
+        add(c, x);
+        add(c + 1, y);
+    } else {
+        add(c, x);
+    }
+    if (blockIdx.x * (u32)TOPS_BLOCK + threadIdx.x < P) {
+#pragma unroll
+        for (int g = 0; g < COG; g++)
+            if (co0 + g < CO) out[((long long)n * CO + co0 + g) * plane + at] = sum[g];
+    }
+}
+template <int KT, int COG>
+static hipError_t launch_conv2d_square(long long blocks, hipStream_t st, const float *in, const float *ker, float *out, int C, int H, int W, int CO, int HO, int WO,
+                                       int stride, u32 P) {
+    const u32 plane = (u32)HO * (u32)WO;
+    hipLaunchKernelGGL((conv2d_square_kernel<KT, COG>), dim3((unsigned)blocks, (unsigned)((CO + COG - 1) / COG)), dim3(TOPS_BLOCK), 0, st, in, ker, out, C, H, W,
+                       CO, stride, P, FastDiv(plane), FastDiv((u32)WO), plane, (u32)WO);
+    return hipGetLastError();
+}
+
 template <int KWT, bool SQUARE>
 static void launch_conv2d_group(int cog, dim3 block, long long blocks, int CO, hipStream_t st, const float *in, const float *ker, float *out, int N,
                                 int C, int H, int W, int KH, int KW, int HO, int WO, int stride, int padding) {
@@ -417,6 +562,17 @@ hipError_t launch_conv2d(const float *in, const float *ker, float *out, int N, i
     // (2048 on the device) to hide the loads behind
     const long long waves1 = blocks * (TOPS_BLOCK / 64) * CO;
     const int cog = waves1 >= 4 * 2048 ? 4 : waves1 >= 2 * 2048 ? 2 : 1;
+    if (KH == KW && (KW == 3 || KW == 5) && padding == 0 && P < (1ll << 31) && CO <= 65535) {
+        // (waves of one channel a lane, us with one, two and four: 560 5.1 7.3 9.9, 1400 10.4 12.3 17.6, 1984 5.8 6.2 8.3, 3200 6.6 5.7 6.6, 4096 26.3 20.1 26.8,
+        // 14 464 22.0 13.2 10.9, 18 432 6.0 4.5 4.3)
+        const int per = waves1 >= 8192 ? 4 : waves1 >= 3072 ? 2 : 1;
+        if (KW == 5 && per == 4) return launch_conv2d_square<5, 4>(blocks, st, in, ker, out, C, H, W, CO, HO, WO, stride, (u32)P);
+        if (KW == 5 && per == 2) return launch_conv2d_square<5, 2>(blocks, st, in, ker, out, C, H, W, CO, HO, WO, stride, (u32)P);
+        if (KW == 5) return launch_conv2d_square<5, 1>(blocks, st, in, ker, out, C, H, W, CO, HO, WO, stride, (u32)P);
+        if (per == 4) return launch_conv2d_square<3, 4>(blocks, st, in, ker, out, C, H, W, CO, HO, WO, stride, (u32)P);
+        if (per == 2) return launch_conv2d_square<3, 2>(blocks, st, in, ker, out, C, H, W, CO, HO, WO, stride, (u32)P);
+        return launch_conv2d_square<3, 1>(blocks, st, in, ker, out, C, H, W, CO, HO, WO, stride, (u32)P);
+    }
     if (blocks <= 0x7FFFFFFFll && (CO + cog - 1) / cog <= 65535) {
         const dim3 block(TOPS_BLOCK);
         if (KW == 3 && KH == 3) launch_conv2d_group<3, true>(cog, block, blocks, CO, st, in, ker, out, N, C, H, W, KH, KW, HO, WO, stride, padding);
@@ -434,6 +590,17 @@ hipError_t launch_conv2d(const float *in, const float *ker, float *out, int N, i
 }
 hipError_t launch_maxpool2d(const float *in, float *out, long long planes, int H, int W, int HO, int WO, int ksize, int stride,
                             hipStream_t st) {
+    const long long total = planes * HO * WO;
+    if (total < (1ll << 31)) {
+        const dim3 grid((unsigned)((total + TOPS_BLOCK - 1) / TOPS_BLOCK)), block(TOPS_BLOCK);
+        const u32 plane = (u32)HO * (u32)WO;
+        const FastDiv by_plane(plane), by_row((u32)WO);
+        const long long HW = (long long)H * W;
+        if (ksize == 2) hipLaunchKernelGGL(maxpool2d_counted_kernel<2>, grid, block, 0, st, in, out, (u32)total, by_plane, by_row, plane, (u32)WO, HW, W, ksize, stride);
+        else if (ksize == 3) hipLaunchKernelGGL(maxpool2d_counted_kernel<3>, grid, block, 0, st, in, out, (u32)total, by_plane, by_row, plane, (u32)WO, HW, W, ksize, stride);
+        else hipLaunchKernelGGL(maxpool2d_counted_kernel<0>, grid, block, 0, st, in, out, (u32)total, by_plane, by_row, plane, (u32)WO, HW, W, ksize, stride);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(maxpool2d_kernel, dim3(tensor_grid(planes * HO * WO)), dim3(TOPS_BLOCK), 0, st, in, out, planes, H, W, HO, WO,
                        ksize, stride);
     return hipGetLastError();
