@@ -208,6 +208,10 @@ typedef row_f32x4 sm_f32x4;
 // canon() without its last step (-0 -> +0 only matters where z is turned into a sort key)
 __device__ __forceinline__ float sm_canon(float z) { return fminf((z != z) ? -INFINITY : z, 3.402823466e+38f); }
 
+// A row whose maximum is a number below the largest, as nearly all rows: of a logit x, d = x - m <= 0, the mass is that of exp(clamp(d, -87, 0)) (a median
+// of three, which makes a NaN -87; beyond d = -80, where the specified mass is 0, exp(d) 2^S is below 1), without a test of x.
+__device__ __forceinline__ bool sm_usual(float m) { return m > -INFINITY && m < 3.402823466e+38f; }
+
 // fl32(fl64(e) / Zd).  The quotient by a reciprocal is within two units of the fp64 quotient's last place, so the two
 // round to the same fp32 unless the product lies that close to the middle between two fp32 values (or the result is
 // subnormal in fp32): only then is the division itself carried out.
@@ -232,6 +236,7 @@ __global__ __launch_bounds__(TPR == 64 ? 256 : TPR) void softmax_resident_kernel
     const float *x = logits + (long long)row * stride;
     float *o = out + (long long)row * V;
     float v[U][4];
+    float mx = -INFINITY;
 #pragma unroll
     for (int u = 0; u < U; u++) {
         const int j = (u * TPR + t) * 4;
@@ -241,28 +246,52 @@ __global__ __launch_bounds__(TPR == 64 ? 256 : TPR) void softmax_resident_kernel
             for (int c = 0; c < 4; c++) v[u][c] = f[c];
         } else {
 #pragma unroll
-            for (int c = 0; c < 4; c++) v[u][c] = j + c < V ? x[j + c] : 0.0f;
+            for (int c = 0; c < 4; c++) v[u][c] = j + c < V ? x[j + c] : -INFINITY;
         }
     }
-    float mx = -INFINITY;
 #pragma unroll
     for (int u = 0; u < U; u++)
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            v[u][c] = sm_canon(v[u][c]);
-            if ((u * TPR + t) * 4 + c < V) mx = fmaxf(mx, v[u][c]);
-        }
-    const float m = TPR == 64 ? wave_max_f32(mx) : block_max_f32<BLOCK>(mx, &scr);
+        for (int c = 0; c < 4; c++) mx = fmaxf(mx, v[u][c]);         // (a NaN never is the larger)
+    const float m = sm_canon(TPR == 64 ? wave_max_f32(mx) : block_max_f32<BLOCK>(mx, &scr));
     const float scale = mass_scale(S);
     u64 acc = 0;
+    if (sm_usual(m)) {                                               // (uniform)
+        // A thread's masses in one fp64 sum where 1024 lanes have the row (more than 8192 logits: the sum holds 2^(52 - S) of them, which they are at
+        // most), a load's four in one where 256 lanes have it (more than 2048).
+        constexpr int SUMS = TPR == 1024 ? 1 : U;
+        double sum[SUMS];
+        const double start = mass_sum_start(S);
+        if (TPR > 64) {
 #pragma unroll
-    for (int u = 0; u < U; u++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const float e = emass(v[u][c], m);
-            if ((u * TPR + t) * 4 + c < V) acc += qfix(e, scale);
-            if (!LOG) v[u][c] = e;
+            for (int u = 0; u < SUMS; u++) sum[u] = start;
+            mass_sum_begin(sum);
         }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const float d = v[u][c] - m, e = expneg_core(__builtin_amdgcn_fmed3f(d, -87.0f, 0.0f));
+                if (TPR > 64) mass_sum_add(sum[SUMS == 1 ? 0 : u], e);
+                else acc += qfix32(e, scale * 2.3283064365386963e-10f);
+                v[u][c] = LOG ? fmaxf(v[u][c], -INFINITY) : d >= -80.0f ? e : 0.0f;   // (a NaN's z is -inf)
+            }
+        if (TPR > 64) {
+            mass_sum_end(sum);
+#pragma unroll
+            for (int u = 0; u < SUMS; u++) acc += mass_sum_of(sum[u], start);
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                v[u][c] = sm_canon(v[u][c]);
+                const float e = emass(v[u][c], m);
+                if ((u * TPR + t) * 4 + c < V) acc += qfix(e, scale);
+                if (!LOG) v[u][c] = e;
+            }
+    }
     u64 Z;
     if (TPR == 64) Z = wave_sum_u64(acc);
     else block_inclusive_scan_u64<BLOCK>(acc, &scr, &Z);
@@ -356,16 +385,28 @@ __global__ __launch_bounds__(1024) void softmax_sweep_kernel(const float *__rest
     float mx = -INFINITY;
     sweep([&](int, const sm_f32x4 &q) {
 #pragma unroll
-        for (int c = 0; c < 4; c++) mx = fmaxf(mx, sm_canon(q[c]));
+        for (int c = 0; c < 4; c++) mx = fmaxf(mx, q[c]);
     });
-    for (int j = (n4 << 2) + tid; j < V; j += 1024) mx = fmaxf(mx, sm_canon(x[j]));
-    const float m = block_max_f32<1024>(mx, &scr);
+    for (int j = (n4 << 2) + tid; j < V; j += 1024) mx = fmaxf(mx, x[j]);
+    const float m = sm_canon(block_max_f32<1024>(mx, &scr));
     const float scale = mass_scale(S);
     u64 acc = 0;
-    sweep([&](int, const sm_f32x4 &q) {
+    if (sm_usual(m)) {                                               // (uniform)
+        const double start = mass_sum_start(S);                      // (a thread's logits in whole blocks are at most 2^(52 - S))
+        double sum = start;
+        mass_sum_begin(sum);
+        sweep([&](int, const sm_f32x4 &q) {
 #pragma unroll
-        for (int c = 0; c < 4; c++) acc += qfix(emass(sm_canon(q[c]), m), scale);
-    });
+            for (int c = 0; c < 4; c++) mass_sum_add(sum, expneg_core(__builtin_amdgcn_fmed3f(q[c] - m, -87.0f, 0.0f)));
+        });
+        mass_sum_end(sum);
+        acc = mass_sum_of(sum, start);
+    } else {
+        sweep([&](int, const sm_f32x4 &q) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) acc += qfix(emass(sm_canon(q[c]), m), scale);
+        });
+    }
     for (int j = (n4 << 2) + tid; j < V; j += 1024) acc += qfix(emass(sm_canon(x[j]), m), scale);
     u64 Z;
     block_inclusive_scan_u64<1024>(acc, &scr, &Z);

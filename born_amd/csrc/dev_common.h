@@ -169,6 +169,18 @@ __device__ __forceinline__ void mass_sum_add(double &acc, float e) {
 }
 __device__ __forceinline__ void mass_sum_end(double &a) { asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 0" : "+v"(a)); }
 template <int N>
+__device__ __forceinline__ void mass_sum_begin(double (&a)[N]) {
+    mass_sum_begin(a[0]);
+#pragma unroll
+    for (int i = 1; i < N; i++) asm volatile("" : "+v"(a[i]));       // (in order after the switch)
+}
+template <int N>
+__device__ __forceinline__ void mass_sum_end(double (&a)[N]) {
+    mass_sum_end(a[0]);
+#pragma unroll
+    for (int i = 1; i < N; i++) asm volatile("" : "+v"(a[i]));
+}
+template <int N>
 __device__ __forceinline__ void mass_sum_end(double (&a)[N], double (&b)[N]) {
     asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 0" : "+v"(a[0]), "+v"(b[0]));
 #pragma unroll

@@ -34,3 +34,37 @@ def test_verification(oracle, V, T):
         s.Close()
         want = oracle.spec_verify(np.ascontiguousarray(t[:, :G]), d, tok, ua, ur, temperature=T, mode=oracle.MODE_FIXED, bonus=np.ascontiguousarray(t[:, G]))
         assert np.array_equal(got["n_accepted"], want["n_accepted"]) and np.array_equal(got["next_token"], want["next_token"]), off
+
+
+@pytest.mark.parametrize("V", [64, 256, 2047, 2048, 2049, 4096, 8191, 8192, 8193, 16383, 16384, 16385, 32767, 32768, 32769, 65535, 65536, 100001])
+def test_softmax(oracle, V):
+    """Rows of equal logits (each sum as full as it gets), of masses that truncate, with NaNs, infinities of both signs and zeros: the masses' sum is the
+    oracle's to the bit in softmax, and log-softmax is the specified expression of it within the rounding of its logarithm."""
+    from born_amd import sampler as S
+    rng = np.random.default_rng(V)
+    x = np.zeros((7, V), np.float32)
+    x[1] = -3.0
+    x[2] = -(60 * rng.random(V)).astype(np.float32)
+    x[3], x[4] = 3 * rng.standard_normal(V), 3 * rng.standard_normal(V)
+    x[3, ::5], x[3, 1::7], x[3, 2] = np.nan, -np.inf, -3e38
+    x[4, V // 2] = np.inf
+    x[5] = -np.inf
+    x[6, 1:] = -100 - rng.random(V - 1)
+    s = S.NewSampler(max_batch=7, max_vocab=V)
+    d, o = S.DeviceBuffer.from_numpy(x), S.DeviceBuffer(x.nbytes)
+    z = np.minimum(np.where(np.isnan(x), -np.inf, x), np.float32(3.402823466e38)).astype(np.float32)
+    m = z.max(1)
+    with np.errstate(invalid="ignore", over="ignore"):
+        dist = np.where(z == m[:, None], np.float32(0), (m[:, None] - z).astype(np.float32)).astype(np.float32)
+    e = oracle.expneg(dist).astype(np.float64)
+    S2 = 62 - int(V).bit_length()
+    Z = np.array([float(sum(int(v) for v in np.trunc(row * 2.0 ** S2))) for row in e]) * 2.0 ** -S2
+    s.Softmax(d, 7, V, o)
+    assert np.array_equal(o.to_numpy(np.uint32, x.shape), (e / Z[:, None]).astype(np.float32).view(np.uint32))
+    s.Softmax(d, 7, V, o, log=True)
+    got = o.to_numpy(np.float32, x.shape)
+    with np.errstate(invalid="ignore"):
+        want = ((z.astype(np.float64) - m[:, None].astype(np.float64)) - np.log(Z)[:, None]).astype(np.float32)
+    same = (got == want) | (np.abs(got - want) <= 2.0 ** -23 * np.abs(want)) | (np.isnan(got) & np.isnan(want))   # (the logarithm's last place)
+    assert same.all()
+    s.Close()
