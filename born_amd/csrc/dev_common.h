@@ -167,6 +167,14 @@ __device__ __forceinline__ void mass_sum_add(double &acc, float e) {
     const double x = (double)e;
     asm volatile("v_add_f64 %0, %0, %1" : "+v"(acc) : "v"(x));
 }
+// trunc(e * 2^S) by itself, for S <= 51 and e <= 1: the 52 places that the addition leaves behind the leading one of `start` (three instructions).
+// Between mass_sum_begin and mass_sum_end as well.
+__device__ __forceinline__ u64 mass_of(float e, const double &start) {
+    const double x = (double)e;
+    double y;
+    asm volatile("v_add_f64 %0, %1, %2" : "=v"(y) : "v"(start), "v"(x));
+    return (u64)__double_as_longlong(y) & 0xFFFFFFFFFFFFFull;
+}
 __device__ __forceinline__ void mass_sum_end(double &a) { asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 2, 2), 0" : "+v"(a)); }
 template <int N>
 __device__ __forceinline__ void mass_sum_begin(double (&a)[N]) {

@@ -198,8 +198,17 @@ __global__ __launch_bounds__(PARTS_BLOCK, 4) void nucleus_parts_masses_kernel(Sa
             lds_barrier();
         }
     };
-    if (r.T == 1.0f) nuc_foreach<PARTS_BLOCK, false, true, true>(r, bm, [&](int, float y) { put(y, false); }, prologue);
-    else nuc_foreach<PARTS_BLOCK, false, true, true>(r, bm, [&](int, float y) { put(nuc_z_shortcut<true>(r, y), false); }, prologue);
+    static_assert(PARTS_FROM >= 1024, "mass_of's shift");
+    double start = mass_sum_start(a.mass_shift);
+    mass_sum_begin(start);
+    auto add = [&](float z) {
+        const float x = z - r.m;
+        const u64 q = mass_of(expneg_core(__builtin_amdgcn_fmed3f(x, -87.0f, 0.0f)), start);
+        atomicAdd(&mass[(int)__builtin_amdgcn_fmed3f(x * nsbin, 0.0f, (float)(NUC_BINS - 1))], q);
+    };
+    if (r.T == 1.0f) nuc_foreach<PARTS_BLOCK, false, true, true>(r, bm, [&](int, float y) { add(y); }, prologue);
+    else nuc_foreach<PARTS_BLOCK, false, true, true>(r, bm, [&](int, float y) { add(nuc_z_shortcut<true>(r, y)); }, prologue);
+    mass_sum_end(start);
     __syncthreads();
     const long long part = (long long)blockIdx.x * pa.parts + blockIdx.y;
     u64 *const out = pa.bins + part * NUC_BINS, *const sums = pa.runs + part * PARTS_RUNS;
@@ -311,22 +320,12 @@ __global__ __launch_bounds__(PARTS_BLOCK, 4) void nucleus_parts_gather_kernel(Sa
     nuc_range(r, w0.bin, lo0, hi0);
     nuc_range(r, w1.bin, unused, hi1);
     nuc_range(r, w2.bin, lo1, unused);
-    uint2 *const list = stage + wave_id() * WCAP;
-    u32 *const wcount = &s_wcount[wave_id()];
-    if (l == 0) __hip_atomic_store(wcount, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-    auto append = [&](float y, int j) {
-        const bool pass = (!(y < lo0) & !(y > hi0)) | (!(y < lo1) & !(y > hi1));
-        const u64 mk = __ballot(pass);
-        if (mk) {                                                    // (the wave's count is in LDS: lanes may sit out a visit)
-            const u32 base = __hip_atomic_load(wcount, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-            if (pass) {
-                const u32 rank = __builtin_amdgcn_mbcnt_hi((u32)(mk >> 32), __builtin_amdgcn_mbcnt_lo((u32)mk, 0u));
-                if (base + rank < (u32)WCAP) list[base + rank] = make_uint2(__float_as_uint(y), (u32)j);
-                if (rank == 0u) __hip_atomic_store(wcount, base + (u32)__popcll(mk), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-            }
-        }
-    };
-    nuc_foreach<PARTS_BLOCK, true, true, true>(r, bm, [&](int j, float y) { append(y, j); }, NucNoPre(), first);
+    const NucList staged{stage + wave_id() * WCAP, &s_wcount[wave_id()]};
+    staged.clear();
+    auto wanted = [&](float y) { return nuc_within(y, lo0, hi0) | nuc_within(y, lo1, hi1); };
+    auto append = [&](float y, int j) { staged.append<WCAP>(wanted(y), y, j); };
+    nuc_foreach4<PARTS_BLOCK, true, true, true>(r, bm, [&](int j, const float (&y)[4]) { staged.append4<WCAP>(wanted, y, j); },
+                                                [&](int j, float y) { append(y, j); }, NucNoPre(), first);
     if (r.penal) {
 #pragma unroll
         for (int k = 0; k < PARTS_SEEN; k++)
@@ -337,14 +336,14 @@ __global__ __launch_bounds__(PARTS_BLOCK, 4) void nucleus_parts_gather_kernel(Sa
     lds_barrier();
     const long long part = (long long)row * pa.parts + blockIdx.y;
     ulonglong2 *const out = pa.list + part * PARTS_LIST;
-    const u32 count = __hip_atomic_load(wcount, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    const u32 count = staged.size();
     if (count > (u32)WCAP && l == 0) s_over = 1;
     for (int e0 = 0; e0 < (int)min(count, (u32)WCAP); e0 += WAVE) {
         const int e = e0 + l;
         bool take = false;
         u64 key = 0ull, qs = 0ull;
         if (e < (int)min(count, (u32)WCAP)) {
-            uint2 c = list[e];
+            uint2 c = staged.at[e];
             bool stale = false;                                      // a seen id's stored logit
             if (r.penal) {
                 if (c.y & 0x80000000u) c.y &= 0x7FFFFFFFu;
@@ -387,7 +386,7 @@ __global__ __launch_bounds__(PARTS_BLOCK, 4) void nucleus_parts_gather_kernel(Sa
 __device__ __forceinline__ bool nucleus_parts_draw(const SampleArgs &a, const PartsArgs &pa, float u) {
     extern __shared__ __align__(16) u64 nuc_dyn[];                   // [PARTS_CAP] keys by bucket, then keys and masses in rank order
     __shared__ BlockScratch scr;
-    __shared__ u64 s_win, s_mass, s_slot0[4];
+    __shared__ u64 s_win[2], s_mass[2], s_slot0[4];
     __shared__ u32 s_start[PARTS_ROW_MAX + 1], s_top[2], s_low[2];
     __shared__ __align__(16) u32 s_count[256], s_at[256];
     __shared__ int s_over;
@@ -398,7 +397,7 @@ __device__ __forceinline__ bool nucleus_parts_draw(const SampleArgs &a, const Pa
     const u64 tp = of.tp, Zk = of.Zk, before[2] = {of.before[0], of.before[1]};
     const int draw = of.draw;
     const float m = of.m;
-    if (tid == 0) s_win = 0ull;
+    if (tid < 2) s_win[tid] = 0ull;
     if (tid < 256) s_count[tid] = 0u;
     if (tid < 2) {
         s_top[tid] = 0u;
@@ -484,22 +483,20 @@ __device__ __forceinline__ bool nucleus_parts_draw(const SampleArgs &a, const Pa
     __syncthreads();
     if (tid < n) mine = incl - s_slot0[myslot];                      // the mass at and above this entry in its bin
 
-    // ---- the cut, then the draw: the first entry in rank order at which the cumulative mass reaches the target
+    // ---- the cut, then the draw: the first entry in rank order at which the cumulative mass reaches the target, which its own mass crosses
     u64 Zp = Zk, tokkey = 0ull;
     for (int phase = cut ? 0 : 1; phase < 2; phase++) {
         const u64 target = phase == 0 ? tp : draw_target(u, Zp);
         const int slot = phase == 0 ? 0 : draw;
         const u64 base = slot ? before[1] : before[0];
-        if (myslot == slot && base + mine >= target) atomicMax(&s_win, mykey);
+        if (myslot == slot && base + mine >= target && base + (mine - q) < target) {
+            s_win[phase] = mykey;
+            s_mass[phase] = base + mine;
+        }
         __syncthreads();
-        const u64 win = s_win;
-        if (myslot == slot && mykey == win) s_mass = base + mine;
-        __syncthreads();
-        if (phase == 0) Zp = s_mass;
+        const u64 win = s_win[phase];
+        if (phase == 0) Zp = s_mass[0];
         else tokkey = win;
-        __syncthreads();
-        if (tid == 0) s_win = 0ull;
-        __syncthreads();
         if (win == 0ull) break;                                      // inconsistent masses: cannot happen
     }
     if (tid == 0) {

@@ -161,8 +161,8 @@ __global__ __launch_bounds__(NUC_BLOCK, 4) void token_logprob_kernel(SampleArgs 
         if (z > mt) raise(z);
         st += (double)term(z, mt);
     };
-    if (r.penal) nuc_foreach4<NUC_BLOCK, true, false, false>(r, bm, four, one, build_bitmap);
-    else nuc_foreach4<NUC_BLOCK, true, false, true>(r, bm, four, one, build_bitmap);
+    if (r.penal) nuc_foreach4<NUC_BLOCK, true, false, false, false>(r, bm, four, one, build_bitmap);
+    else nuc_foreach4<NUC_BLOCK, true, false, true, false>(r, bm, four, one, build_bitmap);
 
     const float m = block_max_f32<NUC_BLOCK>(mt, &scr);
     double part = mt == m ? st : st * exp((double)mt - (double)m);   // a thread without elements: st = 0

@@ -10,9 +10,9 @@
 //   sweep 3  gather: a compare of the penalised logit against the wanted bins' value ranges (widened, so
 //            that it can only over-select) stages about 1 % of the row in per-wave LDS lists (ballot + lane
 //            rank); the staged entries are then classified exactly.
-//   resolve  the gathered entries are put in rank order by counting, one scan of their masses gives every entry
+//   resolve  the gathered entries are put in rank order through buckets, one scan of their masses gives every entry
 //            the mass at and above it within its bin (a short list: summed directly); the first entry in rank
-//            order whose cumulative mass reaches a target is found with an LDS max.
+//            order whose cumulative mass reaches a target is the one whose own mass crosses it.
 // A wanted bin too full for the lists (heavy ties, masked rows) is refined in place by a radix descent over
 // the rank keys of that bin, 11 bits per sweep.
 // In the usual row (a maximum of ordinary size, a temperature whose division has the three-instruction shortcut, no
@@ -34,6 +34,7 @@ namespace born {
 // 512 (two workgroups per CU: one row's sweeps that wait for memory overlap the other's sweep that computes; for
 // batches of more rows than the device has CUs). The geometry below follows from it.
 constexpr int NUC_BINS = 4096;
+constexpr int NUC_DIRECT = 32;                // listed entries that sum what ranks above them directly
 template <int BLOCK>
 struct NucGeom {
     static_assert(BLOCK == 512 || BLOCK == 1024, "threads per row");
@@ -98,21 +99,27 @@ struct NucNoPre {
 };
 // NT: the row is read once (non-temporal loads: measured 6 % faster for a single sweep); a kernel that sweeps the row
 // again wants it to stay in the caches.
-// Block i of the row.  512 threads (two rows to a CU: 128 registers a lane, all of them in use): a 32-bit offset from the row's
-// uniform address; with a 64-bit address per load in flight the sampling kernel spilled nine registers (1024 x 152 064, top-p alone:
-// 315.7 us, 313.1 like this).  With 1024 threads it is the offsets that spill, in the instance without the early request.
+// The block of four logits `off` bytes behind block b of the row.  x and b are uniform: the row's address and the stage's are added in scalar registers,
+// and a lane holds one 32-bit offset for all its loads (512 threads: 88 registers, 128 with an offset per load).
 static_assert(WIDE_MAX_VOCAB < (1 << 30), "a row's bytes fit 32 bits");
-template <int NUC_BLOCK, bool NT>
-__device__ __forceinline__ nuc_f32x4 nuc_load4(const float *x, int i) {
-    const nuc_f32x4 *p = NUC_BLOCK == 512 ? reinterpret_cast<const nuc_f32x4 *>(reinterpret_cast<const char *>(x) + (unsigned)i * 16u)
-                                          : reinterpret_cast<const nuc_f32x4 *>(x) + i;
+template <bool NT>
+__device__ __forceinline__ nuc_f32x4 nuc_load4(const float *x, int b, u32 off) {
+    const nuc_f32x4 *p = reinterpret_cast<const nuc_f32x4 *>(reinterpret_cast<const char *>(x) + (u32)b * 16u + off);
     return NT ? __builtin_nontemporal_load(p) : *p;
+}
+// This thread's block of the workgroup's blocks from b on, or the row's last block beyond it.
+template <bool NT>
+__device__ __forceinline__ nuc_f32x4 nuc_load4_clamped(const float *x, int b, int last) {
+    const int from = min(b, last);
+    return nuc_load4<NT>(x, from, min((u32)threadIdx.x, (u32)(last - from)) * 16u);
 }
 // PLAIN: the caller knows that the row has no penalties (a loop of its own without the penalty code: the visitor's
 // test of r.penal at every visit cost the single-sweep kernel 5 %).
+// LOADS_FIRST: a stage's loads are issued before the visits of the one before, not among them, where the compiler spilled registers for them; off for
+// the sweep of token_logprob_kernel, which they held up (1024 x 152 064: 103 us, 100 without).
 // FIRST (AHEAD instances only): `first` holds the row's first stage, requested earlier with nuc_request_first.
 struct NucNoFirst {};
-template <int NUC_BLOCK, bool NT = false, bool AHEAD = false, bool PLAIN = false, class F4, class F1, class PRE = NucNoPre,
+template <int NUC_BLOCK, bool NT = false, bool AHEAD = false, bool PLAIN = false, bool LOADS_FIRST = true, class F4, class F1, class PRE = NucNoPre,
           class FIRST = NucNoFirst>
 __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 f4, F1 f1, PRE pre = PRE(),
                                              const FIRST &first = FIRST()) {
@@ -160,17 +167,20 @@ __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 
             // Two stages a turn, each loaded while the other is visited, so that no register is copied; the last
             // one or two stages in a loop of their own.
             nuc_f32x4 va[NUC_U], vb[NUC_U];
+            const u32 off = (u32)tid * 16u;
 #pragma unroll
-            for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NUC_BLOCK, NT>(r.x, u * NUC_BLOCK + tid);
+            for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(r.x, u * NUC_BLOCK, off);
             pre();
             int s = 0;
             for (; s + 2 < nfull; s += 2) {
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4<NUC_BLOCK, NT>(r.x, ((s + 1) * NUC_U + u) * NUC_BLOCK + tid);
+                for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4<NT>(r.x, ((s + 1) * NUC_U + u) * NUC_BLOCK, off);
+                if (LOADS_FIRST) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int u = 0; u < NUC_U; u++) visit4(va[u], ((s * NUC_U + u) * NUC_BLOCK + tid) << 2);
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NUC_BLOCK, NT>(r.x, ((s + 2) * NUC_U + u) * NUC_BLOCK + tid);
+                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(r.x, ((s + 2) * NUC_U + u) * NUC_BLOCK, off);
+                if (LOADS_FIRST) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int u = 0; u < NUC_U; u++) visit4(vb[u], (((s + 1) * NUC_U + u) * NUC_BLOCK + tid) << 2);
             }
@@ -179,13 +189,13 @@ __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 
                 for (int u = 0; u < NUC_U; u++) visit4(va[u], ((s * NUC_U + u) * NUC_BLOCK + tid) << 2);
                 if (++s >= nfull) break;
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NUC_BLOCK, NT>(r.x, (s * NUC_U + u) * NUC_BLOCK + tid);
+                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(r.x, (s * NUC_U + u) * NUC_BLOCK, off);
             }
         } else {
             pre();
         }
         for (int i = nfull * NUC_U * NUC_BLOCK + tid; i < n4; i += NUC_BLOCK) {
-            const nuc_f32x4 q = nuc_load4<NUC_BLOCK, NT>(r.x, i);
+            const nuc_f32x4 q = nuc_load4<NT>(r.x, 0, (u32)i * 16u);
             visit4(q, i << 2);
         }
     } else {
@@ -200,12 +210,13 @@ __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 
                 for (int u = 0; u < NUC_U; u++) va[u] = first[u];
             } else {
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NUC_BLOCK, NT>(r.x, min(u * NUC_BLOCK + tid, lastb));
+                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4_clamped<NT>(r.x, u * NUC_BLOCK, lastb);
             }
             pre();
             for (int s = 0; s + 1 < nst; s++) {
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4<NUC_BLOCK, NT>(r.x, min(((s + 1) * NUC_U + u) * NUC_BLOCK + tid, lastb));
+                for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4_clamped<NT>(r.x, ((s + 1) * NUC_U + u) * NUC_BLOCK, lastb);
+                if (LOADS_FIRST) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int u = 0; u < NUC_U; u++) visit4(va[u], ((s * NUC_U + u) * NUC_BLOCK + tid) << 2);
 #pragma unroll
@@ -230,7 +241,7 @@ __device__ __forceinline__ void nuc_request_first(const NucRow &r, nuc_f32x4 (&f
     const int n4 = r.n4;
     if (n4 > 0) {
 #pragma unroll
-        for (int u = 0; u < NucGeom<NUC_BLOCK>::U; u++) first[u] = nuc_load4<NUC_BLOCK, NT>(r.x, min(u * NUC_BLOCK + (int)threadIdx.x, n4 - 1));
+        for (int u = 0; u < NucGeom<NUC_BLOCK>::U; u++) first[u] = nuc_load4_clamped<NT>(r.x, u * NUC_BLOCK, n4 - 1);
     }
 }
 // Visits every element of the row as f(id, penalised logit).
@@ -241,6 +252,56 @@ __device__ __forceinline__ void nuc_foreach(const NucRow &r, const u32 *bm, F f,
         for (int t = 0; t < 4; t++) f(j + t, y[t]);
     }, f, pre, first);
 }
+
+// A wave's list of the logits that a sweep wants, (bits, id) each, at most `cap`; what would go beyond is only counted.  The count lives in LDS, not in a register
+// of every lane: the row visitor lets lanes of a wave sit out visits (the row's last whole blocks of four end inside a wave, its
+// ragged tail starts again at lane 0), and a lane that missed an append must not reuse a position.  LDS operations of one wave complete in order.
+// (Relaxed atomic accesses: re-read at every visit as a volatile would be, but they keep the LDS address space, where a volatile access became a flat one
+// that waits for the row's loads in flight.)
+// The lanes whose y is in [lo, hi] or a NaN, as a mask in scalar registers.
+__device__ __forceinline__ u64 nuc_within(float y, float lo, float hi) {
+    constexpr int UGE = 11, ULE = 13;                                // (the compare's predicates: true for a NaN)
+    return __builtin_amdgcn_fcmpf(y, lo, UGE) & __builtin_amdgcn_fcmpf(y, hi, ULE);
+}
+struct NucList {
+    uint2 *at;
+    u32 *count;
+    __device__ __forceinline__ void clear() const {
+        if (lane_id() == 0) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    }
+    __device__ __forceinline__ u32 size() const { return __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT); }
+    // mk: the lanes whose logit is wanted
+    template <int CAP>
+    __device__ __forceinline__ void append(u64 mk, float y, int j) const {
+        if (mk) {                                                    // uniform over the lanes that take part in this visit
+            const u32 base = size();
+            put<CAP>(mk, base, y, j);
+            __hip_atomic_store(count, base + (u32)__popcll(mk), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);   // (every lane the same)
+        }
+    }
+    // Four logits of a lane: one branch for the wave's 256, one read of the count.  (A test and a branch per logit were 5 vector instructions
+    // and a wait for the compare.)
+    template <int CAP, class P>
+    __device__ __forceinline__ void append4(P wanted, const float (&y)[4], int j) const {
+        const u64 mk[4] = {wanted(y[0]), wanted(y[1]), wanted(y[2]), wanted(y[3])};
+        if (mk[0] | mk[1] | mk[2] | mk[3]) {
+            u32 base = size();
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                if (mk[t]) {
+                    put<CAP>(mk[t], base, y[t], j + t);
+                    base += (u32)__popcll(mk[t]);
+                }
+            }
+            __hip_atomic_store(count, base, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        }
+    }
+    template <int CAP>
+    __device__ __forceinline__ void put(u64 mk, u32 base, float y, int j) const {
+        const u32 pos = base + __builtin_amdgcn_mbcnt_hi((u32)(mk >> 32), __builtin_amdgcn_mbcnt_lo((u32)mk, 0u));
+        if (__builtin_amdgcn_inverse_ballot_w64(mk) && pos < (u32)CAP) at[pos] = make_uint2(__float_as_uint(y), (u32)j);
+    }
+};
 
 // smallest bin whose inclusive cumulative mass reaches target (the last bin if none does); called by whole waves.
 // Two rounds of 64 lanes: which run of 64 bins, then which bin of the run (a binary search is twelve dependent LDS reads).
@@ -285,8 +346,8 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     extern __shared__ __align__(16) u64 nuc_dyn[];
     __shared__ BlockScratch scr;
     __shared__ int s_n, s_over, s_nseen;
-    __shared__ u64 s_win, s_mass, s_slot0[2];
-    __shared__ u32 s_wcount[NUC_WAVES];
+    __shared__ u64 s_win[2], s_mass[2], s_slot0[2];
+    __shared__ u32 s_wcount[NUC_WAVES], s_top[2], s_low[2];
 
     u64 *const mass = nuc_dyn;                                                   // [NUC_BINS] masses, then cumulative
     uint2 *const stage = reinterpret_cast<uint2 *>(nuc_dyn + NUC_BINS);          // [NUC_WAVES][NUC_WCAP] (logit bits, id)
@@ -334,7 +395,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         if (tid == 0) {
             s_n = 0;
             s_over = 0;
-            s_win = 0ull;
+            s_win[0] = s_win[1] = 0ull;
             s_nseen = 0;
         }
         lds_barrier();
@@ -485,8 +546,20 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
                     lin_put(lin_z(seen_y[k]), Plus());
                 }
         }
-        if (r.T == 1.0f) sweep_plain(Cached(), [&](int, float y) { lin_put(y, Plus()); }, first);
-        else sweep_plain(Cached(), [&](int, float y) { lin_put(nuc_z_shortcut<ANY_T>(r, y), Plus()); }, first);
+        if (a.mass_shift > 51) {                                     // (short rows)
+            sweep_plain(Cached(), [&](int, float y) { lin_put(lin_z(y), Plus()); }, first);
+        } else {
+            double start = mass_sum_start(a.mass_shift);
+            mass_sum_begin(start);
+            auto put = [&](float z) {
+                const float x = z - r.m;
+                const u64 q = mass_of(expneg_core(__builtin_amdgcn_fmed3f(x, -87.0f, 0.0f)), start);
+                atomicAdd(&mass[(int)__builtin_amdgcn_fmed3f(x * nsbin, 0.0f, (float)(NUC_BINS - 1))], q);
+            };
+            if (r.T == 1.0f) sweep_plain(Cached(), [&](int, float y) { put(y); }, first);
+            else sweep_plain(Cached(), [&](int, float y) { put(nuc_z_shortcut<ANY_T>(r, y)); }, first);
+            mass_sum_end(start);
+        }
     } else if (r.T == 1.0f && !r.degenerate) {
         sweep(Cached(), [&](int, float y) {
             float z = y;                                             // a logit of ordinary magnitude is its own canonical form
@@ -562,51 +635,33 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         lo1 = lo2;
         const bool one = !(lo1 > hi0);
         if (one) hi0 = fmaxf(hi0, hi1);
-        uint2 *list = stage + wave_id() * NUC_WCAP;
-        // The wave's running count of staged entries lives in LDS, not in a register of every lane: the row visitor
-        // lets different lanes of a wave sit out different visits (the row's last whole float4 blocks end inside a
-        // wave, its ragged tail starts again at lane 0), and a lane that missed an append must not reuse a position.
-        // Whichever lane appends first in a visit advances the count; LDS operations of one wave complete in order.
-        const int wid = wave_id();
-        // (relaxed atomic accesses: re-read at every visit as a volatile would be, but they keep the LDS address space,
-        // where a volatile access became a flat one that waits for the row's loads in flight)
-        u32 *const wcount = &s_wcount[wid];
-        if (lane_id() == 0) __hip_atomic_store(wcount, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-        auto append = [&](bool pass, float y, int j) {
-            const u64 mk = __ballot(pass);
-            if (mk) {                                                // uniform over the lanes that take part in this visit
-                const u32 base = __hip_atomic_load(wcount, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-                if (pass) {
-                    const u32 rank = __builtin_amdgcn_mbcnt_hi((u32)(mk >> 32), __builtin_amdgcn_mbcnt_lo((u32)mk, 0u));
-                    const u32 pos = base + rank;
-                    if (pos < (u32)NUC_WCAP) list[pos] = make_uint2(__float_as_uint(y), (u32)j);
-                    if (rank == 0u) __hip_atomic_store(wcount, base + (u32)__popcll(mk), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-                }
-            }
+        const NucList staged{stage + wave_id() * NUC_WCAP, &s_wcount[wave_id()]};
+        staged.clear();
+        auto append = [&](u64 mk, float y, int j) { staged.template append<NUC_WCAP>(mk, y, j); };
+        auto in_one = [&](float y) { return nuc_within(y, lo0, hi0); };
+        auto in_either = [&](float y) { return nuc_within(y, lo0, hi0) | nuc_within(y, lo1, hi1); };
+        auto sweep_few = [&](auto wanted) {
+            nuc_foreach4<NUC_BLOCK, true, NUC_BLOCK == 1024, true>(r, bm, [&](int j, const float (&y)[4]) { staged.template append4<NUC_WCAP>(wanted, y, j); },
+                                                                   [&](int j, float y) { append(wanted(y), y, j); }, NucNoPre(), first);
         };
-        // (bitwise and / or of the compares: the short-circuit forms compiled to a nest of branches per logit)
         if (lin) {
             // (the stored logits; a seen id's stored logit that passes is dropped below, its penalised logit is offered
             // here under the id with the top bit set)
-            if (one) {
-                sweep_plain(Streamed(), [&](int j, float y) { append(!(y < lo0) & !(y > hi0), y, j); }, first);
-            } else {
-                sweep_plain(Streamed(), [&](int j, float y) { append((!(y < lo0) & !(y > hi0)) | (!(y < lo1) & !(y > hi1)), y, j); }, first);
-            }
+            if (one) sweep_few(in_one);
+            else sweep_few(in_either);
             if (r.penal) {
 #pragma unroll
                 for (int k = 0; k < NUC_SEEN; k++)
                     if (seen_id[k] >= 0) {
-                        const float y = seen_y[k];
-                        append((!(y < lo0) & !(y > hi0)) | (!(y < lo1) & !(y > hi1)), y, (int)((u32)seen_id[k] | 0x80000000u));
+                        append(in_either(seen_y[k]), seen_y[k], (int)((u32)seen_id[k] | 0x80000000u));
                     }
             }
         } else if (one) {
-            sweep(Streamed(), [&](int j, float y) { append(!(y < lo0) & !(y > hi0), y, j); }, NucNoPre(), first);
+            sweep(Streamed(), [&](int j, float y) { append(in_one(y), y, j); }, NucNoPre(), first);
         } else {
-            sweep(Streamed(), [&](int j, float y) { append((!(y < lo0) & !(y > hi0)) | (!(y < lo1) & !(y > hi1)), y, j); }, NucNoPre(), first);
+            sweep(Streamed(), [&](int j, float y) { append(in_either(y), y, j); }, NucNoPre(), first);
         }
-        const u32 count = __hip_atomic_load(wcount, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        const u32 count = staged.size();
         if (count > (u32)NUC_WCAP && lane_id() == 0) s_over = 1;
         const int cw = (int)min(count, (u32)NUC_WCAP);
         for (int e0 = 0; e0 < cw; e0 += WAVE) {
@@ -614,7 +669,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
             bool take = false;
             u64 key = 0ull, qs = 0ull;
             if (e < cw) {
-                uint2 c = list[e];
+                uint2 c = staged.at[e];
                 bool stale = false;                                  // a seen id's stored logit
                 if (lin && r.penal) {
                     if (c.y & 0x80000000u) c.y &= 0x7FFFFFFFu;
@@ -659,14 +714,18 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     // ---- cumulative mass of every listed entry within its bin, in rank order.  The bins' value ranges are disjoint, so
     // the rank order of the whole list goes bin by bin: an entry counts the keys above its own (all distinct: the id is
     // part of the key) and moves to that place; one scan of the masses in that order gives every entry the mass at and
-    // above it, and where a bin begins the scan holds what the bins listed before it add up to.
-    u64 mykey = 0ull, mine = 0ull;                                   // inclusive mass at and above this entry in its bin
+    // above it, and where a bin begins the scan holds what the bins listed before it add up to.  128 buckets for the range of either slot (the draw's bins lie above
+    // the cut's): an entry counts the keys of its own bucket only.  Bound by the chain of LDS round trips.  (Against the whole list, then the
+    // targets by an LDS maximum and five barriers each: the resolve of the slowest row of 96 x 100 003 took 10 us, 3.8 so, of 1024 x 152 064 7.8 and 3.0;
+    // lists of 33 to 128 entries, summed directly before, 5.8 and 3.7.)
+    u64 mykey = 0ull, mine = 0ull, q = 0ull;                         // its own mass, and the mass at and above it in its bin
     int myslot = -1;
-    if (n <= 2 * WAVE) {
+    if (n <= NUC_DIRECT) {
         // (a short list: every entry sums the masses of its bin's entries at and above it; no barrier, no scan)
         if (tid < n) {
             mykey = fkey[tid];
             myslot = (int)(fq[tid] >> 62);
+            q = fq[tid] & 0x3FFFFFFFFFFFFFFFull;
             const ulonglong2 *k2 = reinterpret_cast<const ulonglong2 *>(fkey), *q2 = reinterpret_cast<const ulonglong2 *>(fq);
             for (int j = 0; j < n4; j += 4) {
                 const ulonglong2 ka = k2[j >> 1], kb = k2[(j >> 1) + 1], qa = q2[j >> 1], qb = q2[(j >> 1) + 1];
@@ -678,21 +737,59 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         }
     } else {
         u64 *const skey = reinterpret_cast<u64 *>(stage), *const sq = skey + NUC_CAP;       // the staging lists are spent
-        static_assert(2 * NUC_CAP <= NUC_WAVES * NUC_WCAP, "the ordered entries fit the staging lists' storage");
+        u32 *const count = reinterpret_cast<u32 *>(sq + NUC_CAP), *const at = count + 256;
+        static_assert(2 * NUC_CAP + 256 <= NUC_WAVES * NUC_WCAP, "the ordered entries and the buckets fit the staging lists' storage");
+        if (tid < 256) count[tid] = 0u;
+        if (tid < 2) {
+            s_top[tid] = 0u;
+            s_low[tid] = ~0u;
+        }
+        const u64 key = tid < n ? fkey[tid] : 0ull, kq = tid < n ? fq[tid] : 0ull;
+        const u32 z = (u32)(key >> 32);
+        const int in_slot = (int)(kq >> 62);
+        lds_barrier();
+        if ((tid & ~(WAVE - 1)) < n) {                               // wave-uniform
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const bool its = tid < n && in_slot == t;
+                const u32 most = wave_max_u32(its ? z : 0u), least = wave_min_u32(its ? z : ~0u);
+                if (lane_id() == 0) {
+                    atomicMax(&s_top[t], most);
+                    atomicMin(&s_low[t], least);
+                }
+            }
+        }
+        lds_barrier();
+        u32 bucket = 0u, pos = 0u;
         if (tid < n) {
-            const u64 key = fkey[tid];
-            int rank = 0;
-            // four keys a turn, read with two 128-bit LDS loads before any is used
+            const u32 range = s_top[in_slot] - s_low[in_slot];
+            const int sh = max(0, 25 - (int)__clz(range));           // (range >> sh) < 128
+            bucket = (in_slot ? 0u : 128u) + ((s_top[in_slot] - z) >> sh);
+            pos = atomicAdd(&count[bucket], 1u);
+        }
+        lds_barrier();
+        if (tid < WAVE) {
+            const uint4 c = reinterpret_cast<const uint4 *>(count)[tid];
+            const u32 four = c.x + c.y + c.z + c.w, ex = wave_inclusive_scan_u32(four) - four;
+            reinterpret_cast<uint4 *>(at)[tid] = make_uint4(ex, ex + c.x, ex + c.x + c.y, ex + c.x + c.y + c.z);
+        }
+        lds_barrier();
+        const u32 begin = tid < n ? at[bucket] : 0u;
+        if (tid < n) fkey[begin + pos] = key;                        // (by bucket; the keys that pad the list stay behind them)
+        lds_barrier();
+        if (tid < n) {
+            // four keys a turn, from a whole group of four on: those of earlier buckets count, those of later ones do not
+            const u32 end = begin + count[bucket];
+            u32 j = begin & ~3u, rank = j;
             const ulonglong2 *k2 = reinterpret_cast<const ulonglong2 *>(fkey);
-            for (int j = 0; j < n4; j += 4) {
+            for (; j < end; j += 4) {
                 const ulonglong2 ka = k2[j >> 1], kb = k2[(j >> 1) + 1];
-                rank += (int)(ka.x > key) + (int)(ka.y > key) + (int)(kb.x > key) + (int)(kb.y > key);
+                rank += (u32)(ka.x > key) + (u32)(ka.y > key) + (u32)(kb.x > key) + (u32)(kb.y > key);
             }
             skey[rank] = key;
-            sq[rank] = fq[tid];
+            sq[rank] = kq;
         }
         __syncthreads();
-        u64 q = 0ull;
         if (tid < n) {
             mykey = skey[tid];
             const u64 w = sq[tid];
@@ -705,8 +802,6 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         __syncthreads();
         if (tid < n) mine = incl - s_slot0[myslot];
     }
-    __syncthreads();                                                 // the lists may be overwritten from here on
-
     // ---- the cut, then the draw: each is the first element in rank order of one bin at which the cumulative
     // mass reaches a target.  A bin that is listed is resolved from `mine`; any other bin (the lists overflowed:
     // heavy ties, masked rows; or the draw's bin was not the predicted one) by a radix descent over the rank
@@ -722,6 +817,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         const int slot = !listed ? -1 : b == w0 ? 0 : b >= w1 && b <= w2 ? 1 : -1;
         if (slot == 1) base = w1 ? cum[w1 - 1] : 0ull;               // (listed from w1 on)
         if (slot < 0) {
+            __syncthreads();                                         // (the lists are overwritten)
             u64 prefix = 0ull;
             int plen = 0;
             for (;;) {
@@ -802,24 +898,23 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
             myslot = -1;
             if (tid < nb) {
                 mykey = fkey[tid];
+                q = fq[tid];
                 myslot = 0;
                 for (int j = 0; j < nb; j++)
                     if (fkey[j] >= mykey) mine += fq[j];
             }
             __syncthreads();
         }
-        // first entry in rank order (largest key) of the bin at which base + cumulative reaches target
+        // the first entry in rank order at which base + cumulative reaches the target: the one whose own mass crosses it
         const int sl = slot < 0 ? 0 : slot;
-        if (myslot == sl && base + mine >= target) atomicMax(&s_win, mykey);
+        if (myslot == sl && base + mine >= target && base + (mine - q) < target) {
+            s_win[phase] = mykey;
+            s_mass[phase] = base + mine;
+        }
         __syncthreads();
-        const u64 win = s_win;
-        if (myslot == sl && mykey == win) s_mass = base + mine;
-        __syncthreads();
-        if (phase == 0) Zp = s_mass;
+        const u64 win = s_win[phase];
+        if (phase == 0) Zp = s_mass[0];
         else tokkey = win;
-        __syncthreads();
-        if (tid == 0) s_win = 0ull;
-        __syncthreads();
         if (win == 0ull) break;                                      // inconsistent histogram: cannot happen
     }
     BORN_STAMP(a, row, 6);

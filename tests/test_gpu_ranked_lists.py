@@ -1,0 +1,34 @@
+"""Rows without a top-k cut whose wanted bins hold equal logits: lists around the 32 entries that are summed directly, the 1024 or 512 that fit, and beyond;
+rows around the 1024 logits from which a bin's masses are added in fp64; rows in parts.  Against the oracle's fixed-point layer, bit for bit."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("path", [0, 2])                    # 2: 512 threads to a row
+@pytest.mark.parametrize("p", [0.6, 1.0])
+@pytest.mark.parametrize("V,ties", [(1023, 31), (1023, 33), (1024, 32), (1056, 33), (2048, 128), (8193, 129), (16400, 511), (16400, 513), (30000, 1023), (40001, 1025),
+                                    (66001, 300), (66001, 1100)])
+def test_lists_of_equal_logits(oracle, V, ties, p, path):
+    from born_amd import sampler as S
+    rng = np.random.default_rng(V + ties)
+    B = 6
+    levels = -(-V // ties)
+    values = np.sort(rng.standard_normal(levels)).astype(np.float32)
+    x = np.stack([rng.permutation(values[np.arange(V) // ties]) for _ in range(B)])
+    x[1] *= 0.01                                            # masses that hardly differ
+    x[2, rng.choice(V, V // 2, replace=False)] = -np.inf
+    x[3] += 1e-4 * rng.standard_normal(V).astype(np.float32)  # nearly equal: many entries to a bucket, or many buckets
+    u = rng.random(B).astype(np.float32)
+    u[0], u[4] = 0, 1 - 2.0 ** -24
+    hist = rng.integers(0, V, (B, 40)).astype(np.int32)
+    for T, rep in ((1.0, 1.0), (0.7, 1.3)):
+        s = S.NewSampler(S.SamplerConfig(Temperature=T, TopP=p, RepetitionPenalty=rep), max_batch=B, max_vocab=V)
+        s.SetPath(path)
+        got = S.sample_host(s, x, u, hist)
+        s.Status()
+        s.Close()
+        want = oracle.sample(x, u, T, 0, p, rep, hist, mode=oracle.MODE_FIXED)
+        assert np.array_equal(got["tokens"], want["tokens"])
+        assert np.array_equal(got["probs"].view(np.uint32), want["probs"].view(np.uint32))
