@@ -23,14 +23,17 @@ constexpr int PARTS_ROW_MAX = 32;             // parts of a row
 constexpr int PARTS_SEEN = 4;                 // seen ids a thread keeps: histories of at most 4096 tokens
 constexpr int PARTS_TOTAL = 256;              // of a batch, at most
 constexpr int PARTS_LEAST = 4096;             // logits of a part, about: one 128-bit load per thread
-// Logits of a row, and from where on two parts pay, not only eight and more.  us, one workgroup to a row and parts, top-p 0.95 at T = 0.8:
-//               1 row        32           85           128
-//     49 999    26.6 24.0    30.3 27.9    37.7 33.7    37.6 35.7
-//     57 000    28.0 24.0    32.2 28.2    34.5 34.6    35.7 37.1
-//     66 001    31.4 24.4    40.9 28.9    38.1 35.8    45.1 40.3
-//    152 064    53.8 26.2    63.6 36.0    67.5 51.4    71.0 62.6
-// (32 000, before the draw's buckets: 20.4 22.6, 23.5 26.4, 27.5 29.4, 27.9 31.1.)  Four launches, chains of memory and LDS round trips each.
-constexpr int PARTS_FROM = 49152, PARTS_FEW_FROM = 65536, PARTS_MANY = 8;
+// Parts pay where the logits that a row's own workgroup is spared, V - V / parts, reach a number; two parts, whose batch keeps the device busy either way, only
+// from twice the row.  us, one workgroup to a row and parts, top-p 0.95 at T = 0.8 (rows, and so parts: 1 of 32, 32 of 8, 42 of 6, 64 of 4, 85 of 3, 128 of 2):
+//               1            32           42           64           85           128
+//     57 000    24.7 24.0    25.5 25.3    25.5 25.3    25.6 25.4    (not cut: 25.6)
+//     66 001    26.4 24.2    27.8 26.3    27.6 26.8    27.7 28.6    28.5 30.5    28.7 34.6
+//     80 000    28.8 24.3    30.1 26.2    30.1 27.6    29.9 29.2    30.2 31.3    32.1 38.1
+//    100 003    34.1 24.4    35.2 27.0    34.7 28.8    34.8 30.8    36.5 35.1    39.7 44.4
+//    152 064    45.0 25.2    46.1 29.1    46.5 31.5    48.2 37.6    50.9 44.6    53.4 56.1
+//    250 000    66.5 25.4    66.9 32.5    73.7 40.4    76.8 49.9    78.6 60.6    83.7 79.6
+// Four launches, chains of memory and LDS round trips each.
+constexpr int PARTS_FROM = 49152, PARTS_SPARED = 60000, PARTS_TWO_FROM = 196608;
 static_assert(PARTS_RUNS == WAVE, "one lane per run, one per bin of a run");
 static_assert(PARTS_ROW_MAX * PARTS_RUN <= 2 * PARTS_BLOCK && PARTS_ROW_MAX <= WAVE, "sums over parts");
 
@@ -553,7 +556,8 @@ static int parts_of(const SampleArgs &a, bool two_per_cu, int most) {
     if (two_per_cu || a.V < PARTS_FROM || a.hist_counts || a.hist_stride > PARTS_SEEN * PARTS_BLOCK) return 0;
     if (a.dcut != 80.0f) return 0;                                   // (a min-p bound is for the one-workgroup body)
     const int parts = std::min(std::min(std::min(most, device_cu_count()) / a.B, PARTS_ROW_MAX), a.V / PARTS_LEAST);
-    return a.V < PARTS_FEW_FROM && parts < PARTS_MANY ? 0 : parts;
+    if (parts < 2 || a.V - a.V / parts < PARTS_SPARED || (parts == 2 && a.V < PARTS_TWO_FROM)) return 0;
+    return parts;
 }
 bool nucleus_wants_parts(const SampleArgs &a, bool two_per_cu) { return parts_of(a, two_per_cu, PARTS_TOTAL) >= 2; }
 static bool parts_plan(const SampleArgs &a, bool two_per_cu, const NucleusWorkspace &ws, PartsArgs &pa) {

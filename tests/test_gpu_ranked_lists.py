@@ -32,3 +32,20 @@ def test_lists_of_equal_logits(oracle, V, ties, p, path):
         want = oracle.sample(x, u, T, 0, p, rep, hist, mode=oracle.MODE_FIXED)
         assert np.array_equal(got["tokens"], want["tokens"])
         assert np.array_equal(got["probs"].view(np.uint32), want["probs"].view(np.uint32))
+
+
+@pytest.mark.parametrize("B,V", [(3, 64285), (3, 64286), (64, 79999), (64, 80000), (85, 89999), (85, 90000), (128, 196607), (128, 196608)])
+def test_rows_around_the_shortest_that_are_cut(oracle, B, V):
+    from born_amd import sampler as S
+    rng = np.random.default_rng(B + V)
+    x = (2 * rng.standard_normal((4, V))).astype(np.float32)
+    x = np.concatenate([x] * (B // 4 + 1))[:B]
+    u = rng.random(B).astype(np.float32)
+    s = S.NewSampler(S.SamplerConfig(Temperature=0.8, TopP=0.95), max_batch=B, max_vocab=V)
+    got = S.sample_host(s, x, u, None)
+    s.Status()
+    s.Close()
+    at = [0, 1, 2, B // 2, B - 1]
+    want = oracle.sample(x[at], u[at], 0.8, 0, 0.95, 1.0, None, mode=oracle.MODE_FIXED)
+    assert np.array_equal(got["tokens"][at], want["tokens"])
+    assert np.array_equal(got["probs"][at].view(np.uint32), want["probs"].view(np.uint32))
