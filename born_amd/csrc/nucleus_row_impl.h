@@ -22,6 +22,7 @@
 // the three reads of the row from HBM, not by the vector ALU.
 #pragma once
 #include <algorithm>
+#include <tuple>
 #include <type_traits>
 #include "dev_common.h"
 #include "finish.h"
@@ -119,6 +120,16 @@ __device__ __forceinline__ nuc_f32x4 nuc_load4_clamped(const float *x, int b, in
 // the sweep of token_logprob_kernel, which they held up (1024 x 152 064: 103 us, 100 without).
 // FIRST (AHEAD instances only): `first` holds the row's first stage, requested earlier with nuc_request_first.
 struct NucNoFirst {};
+// KEPT (512 threads): the row's first stages stay in registers from its first sweep on, which fills them (NucFill), and the sweeps after it read the rest.
+constexpr int NUC_KEPT = 2;
+template <int NUC_BLOCK>
+struct NucKept {
+    nuc_f32x4 v[NUC_KEPT * NucGeom<NUC_BLOCK>::U];
+};
+template <int NUC_BLOCK>
+struct NucFill {
+    NucKept<NUC_BLOCK> *kept;
+};
 template <int NUC_BLOCK, bool NT = false, bool AHEAD = false, bool PLAIN = false, bool LOADS_FIRST = true, class F4, class F1, class PRE = NucNoPre,
           class FIRST = NucNoFirst>
 __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 f4, F1 f1, PRE pre = PRE(),
@@ -168,10 +179,24 @@ __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 
             // one or two stages in a loop of their own.
             nuc_f32x4 va[NUC_U], vb[NUC_U];
             const u32 off = (u32)tid * 16u;
+            constexpr bool FILL = std::is_same<FIRST, NucFill<NUC_BLOCK>>::value, KEPT = FILL || std::is_same<FIRST, NucKept<NUC_BLOCK>>::value;
+            int s = KEPT && nfull > NUC_KEPT ? NUC_KEPT : 0;         // the first stage that is loaded
+            if constexpr (FILL) {
+                if (s)
 #pragma unroll
-            for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(r.x, u * NUC_BLOCK, off);
+                    for (int k = 0; k < NUC_KEPT * NUC_U; k++) first.kept->v[k] = nuc_load4<NT>(r.x, k * NUC_BLOCK, off);
+            }
+#pragma unroll
+            for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(r.x, (s * NUC_U + u) * NUC_BLOCK, off);
             pre();
-            int s = 0;
+            if constexpr (KEPT) {
+                const NucKept<NUC_BLOCK> *kept;
+                if constexpr (FILL) kept = first.kept;
+                else kept = &first;
+                if (s)
+#pragma unroll
+                    for (int k = 0; k < NUC_KEPT * NUC_U; k++) visit4(kept->v[k], (k * NUC_BLOCK + tid) << 2);
+            }
             for (; s + 2 < nfull; s += 2) {
 #pragma unroll
                 for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4<NT>(r.x, ((s + 1) * NUC_U + u) * NUC_BLOCK, off);
@@ -457,8 +482,12 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     // every element of the row as f(id, penalised logit): the sweep, then the seen ids when the sweep masked them
     // (1024 threads: the first stage of sweeps 2 and 3 is requested ahead, into `ahead`)
     constexpr bool REQ = REQUEST && NUC_BLOCK == 1024;
-    typename std::conditional<REQ, nuc_f32x4[NucGeom<NUC_BLOCK>::U], NucNoFirst>::type ahead;
+    // (512 threads: its first stages are kept)
+    constexpr bool KEEP = NUC_BLOCK == 512;
+    typename std::conditional<REQ, nuc_f32x4[NucGeom<NUC_BLOCK>::U], typename std::conditional<KEEP, NucKept<NUC_BLOCK>, NucNoFirst>::type>::type ahead;
+    const NucNoFirst none;
     auto &first = ahead;
+    auto &requested = std::get<REQ ? 0 : 1>(std::tie(ahead, none));  // (the sweeps of rows that are not usual keep nothing)
     auto sweep = [&](auto nt, auto f, auto pre, const auto &first) {
         nuc_foreach<NUC_BLOCK, decltype(nt)::value, NUC_BLOCK == 1024>(r, bm, f, pre, first);
         if (r.masked) {
@@ -482,7 +511,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         sweep(Cached(), [&](int j, float y) {
             mx = fmaxf(mx, y);
             if ((j & 3) == 0) mn = fminf(mn, y > -3.402823466e+38f ? y : INFINITY);
-        }, prologue, NucNoFirst());
+        }, prologue, std::get<KEEP ? 0 : 1>(std::make_tuple(NucFill<NUC_BLOCK>{reinterpret_cast<NucKept<NUC_BLOCK> *>(&ahead)}, none)));
         // (sweep 2's first stage travels while the row's maximum is found; the barriers until then order LDS traffic only)
         if constexpr (REQ) nuc_request_first<NUC_BLOCK, false>(r, ahead);
         mx = block_max_f32<NUC_BLOCK, true>(mx, &scr);
@@ -569,19 +598,19 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
             }
             const float d = r.m - z;
             atomicAdd(&mass[nuc_bin(r, d)], qfix(expneg(d, r.dcut), r.scale));
-        }, NucNoPre(), first);
+        }, NucNoPre(), requested);
     } else if (r.rcp != 0.0f && !r.degenerate) {
         sweep(Cached(), [&](int, float y) {
             float z = nuc_z_shortcut<ANY_T>(r, y);
             if (!nuc_ordinary(y)) z = nuc_z(r, y);                   // zeros, masked (-inf) and other unusual logits: the division
             const float d = r.m - z;
             atomicAdd(&mass[nuc_bin(r, d)], qfix(expneg(d, r.dcut), r.scale));
-        }, NucNoPre(), first);
+        }, NucNoPre(), requested);
     } else {
         sweep(Cached(), [&](int, float y) {
             const float d = nuc_d(r, nuc_z(r, y));
             atomicAdd(&mass[nuc_bin(r, d)], qfix(expneg(d, r.dcut), r.scale));
-        }, NucNoPre(), first);
+        }, NucNoPre(), requested);
     }
     // (sweep 3's first stage travels while the bins are summed and the wanted ones found)
     if constexpr (REQ) nuc_request_first<NUC_BLOCK, true>(r, ahead);
@@ -657,9 +686,9 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
                     }
             }
         } else if (one) {
-            sweep(Streamed(), [&](int j, float y) { append(in_one(y), y, j); }, NucNoPre(), first);
+            sweep(Streamed(), [&](int j, float y) { append(in_one(y), y, j); }, NucNoPre(), requested);
         } else {
-            sweep(Streamed(), [&](int j, float y) { append(in_either(y), y, j); }, NucNoPre(), first);
+            sweep(Streamed(), [&](int j, float y) { append(in_either(y), y, j); }, NucNoPre(), requested);
         }
         const u32 count = staged.size();
         if (count > (u32)NUC_WCAP && lane_id() == 0) s_over = 1;
