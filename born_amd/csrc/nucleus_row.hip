@@ -13,11 +13,11 @@
 namespace born {
 
 // (at most 128 registers either way: 512 threads are launched two workgroups to a CU)
-// REQUEST: see the body; off for a batch small enough to be re-read from the L2s, where there is no memory latency to
-// hide and holding the requested stage in registers only costs (64 x 32 000: 21.1 us with it, 20.8 without).
-template <int BLOCK, bool COUNTED, bool REQUEST = true>
+// KEEP: see the body; off for a batch small enough to be re-read from the L2s, where the stage held in registers costs more than its loads
+// (64 x 32 000: 16.9 us with it, 16.7 without; 100 x 300 12.1 and 11.8; but 256 x 128 256 61.7 and 63.4, 200 x 50 257 29.4 and 30.0).
+template <int BLOCK, bool COUNTED, bool KEEP = true>
 __global__ __launch_bounds__(BLOCK, 4) void nucleus_row_kernel(SampleArgs a) {
-    nucleus_row_body<BLOCK, COUNTED, REQUEST>(a, a.T, a.top_p, a.rep, a.dcut, a.freq, a.pres, a.rcp_T);
+    nucleus_row_body<BLOCK, COUNTED, KEEP>(a, a.T, a.top_p, a.rep, a.dcut, a.freq, a.pres, a.rcp_T);
 }
 // The batch carries a configuration per row (row_config.h): the workgroup takes the row only if it is its own.
 template <int BLOCK, bool COUNTED>

@@ -22,7 +22,6 @@
 // the three reads of the row from HBM, not by the vector ALU.
 #pragma once
 #include <algorithm>
-#include <tuple>
 #include <type_traits>
 #include "dev_common.h"
 #include "finish.h"
@@ -118,13 +117,13 @@ __device__ __forceinline__ nuc_f32x4 nuc_load4_clamped(const float *x, int b, in
 // test of r.penal at every visit cost the single-sweep kernel 5 %).
 // LOADS_FIRST: a stage's loads are issued before the visits of the one before, not among them, where the compiler spilled registers for them; off for
 // the sweep of token_logprob_kernel, which they held up (1024 x 152 064: 103 us, 100 without).
-// FIRST (AHEAD instances only): `first` holds the row's first stage, requested earlier with nuc_request_first.
+// FIRST (AHEAD instances only): `first` holds the row's first stage, requested earlier with nuc_request_first, or
+// (NucKept) its first stages, kept in registers from the first sweep on, which fills them (NucFill).
 struct NucNoFirst {};
-// KEPT (512 threads): the row's first stages stay in registers from its first sweep on, which fills them (NucFill), and the sweeps after it read the rest.
-constexpr int NUC_KEPT = 2;
 template <int NUC_BLOCK>
 struct NucKept {
-    nuc_f32x4 v[NUC_KEPT * NucGeom<NUC_BLOCK>::U];
+    static constexpr int STAGES = NUC_BLOCK == 512 ? 2 : 1;
+    nuc_f32x4 v[STAGES * NucGeom<NUC_BLOCK>::U];
 };
 template <int NUC_BLOCK>
 struct NucFill {
@@ -171,7 +170,8 @@ __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 
         f1(j, y);
     };
     const int n4 = r.n4;
-    constexpr int NUC_U = NucGeom<NUC_BLOCK>::U;
+    constexpr int NUC_U = NucGeom<NUC_BLOCK>::U, NUC_KEPT = NucKept<NUC_BLOCK>::STAGES;
+    constexpr bool FILL = std::is_same<FIRST, NucFill<NUC_BLOCK>>::value, KEPT = FILL || std::is_same<FIRST, NucKept<NUC_BLOCK>>::value;
     if constexpr (!AHEAD) {
         const int nfull = n4 / (NUC_U * NUC_BLOCK);
         if (nfull > 0) {
@@ -179,7 +179,6 @@ __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 
             // one or two stages in a loop of their own.
             nuc_f32x4 va[NUC_U], vb[NUC_U];
             const u32 off = (u32)tid * 16u;
-            constexpr bool FILL = std::is_same<FIRST, NucFill<NUC_BLOCK>>::value, KEPT = FILL || std::is_same<FIRST, NucKept<NUC_BLOCK>>::value;
             int s = KEPT && nfull > NUC_KEPT ? NUC_KEPT : 0;         // the first stage that is loaded
             if constexpr (FILL) {
                 if (s)
@@ -230,15 +229,29 @@ __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 
             // the compiler wait for every load in flight); only the visits of the last stage ask whether the block exists.
             nuc_f32x4 va[NUC_U], vb[NUC_U];
             const int lastb = n4 - 1;
-            if constexpr (!std::is_same<FIRST, NucNoFirst>::value) {
+            int s = 0;
+            if constexpr (FILL) {
+#pragma unroll
+                for (int u = 0; u < NUC_U; u++) first.kept->v[u] = nuc_load4_clamped<NT>(r.x, u * NUC_BLOCK, lastb);
+            }
+            if constexpr (!KEPT && !std::is_same<FIRST, NucNoFirst>::value) {
 #pragma unroll
                 for (int u = 0; u < NUC_U; u++) va[u] = first[u];
             } else {
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4_clamped<NT>(r.x, u * NUC_BLOCK, lastb);
+                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4_clamped<NT>(r.x, ((KEPT ? 1 : 0) * NUC_U + u) * NUC_BLOCK, lastb);
             }
             pre();
-            for (int s = 0; s + 1 < nst; s++) {
+            if constexpr (KEPT) {
+                const NucKept<NUC_BLOCK> *kept;
+                if constexpr (FILL) kept = first.kept;
+                else kept = &first;
+#pragma unroll
+                for (int u = 0; u < NUC_U; u++)
+                    if (u * NUC_BLOCK + tid < n4) visit4(kept->v[u], (u * NUC_BLOCK + tid) << 2);
+                s = 1;
+            }
+            for (; s + 1 < nst; s++) {
 #pragma unroll
                 for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4_clamped<NT>(r.x, ((s + 1) * NUC_U + u) * NUC_BLOCK, lastb);
                 if (LOADS_FIRST) __builtin_amdgcn_sched_barrier(0);
@@ -247,10 +260,12 @@ __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 
 #pragma unroll
                 for (int u = 0; u < NUC_U; u++) va[u] = vb[u];
             }
+            if (!KEPT || nst > 1) {
 #pragma unroll
-            for (int u = 0; u < NUC_U; u++) {
-                const int i = ((nst - 1) * NUC_U + u) * NUC_BLOCK + tid;
-                if (i < n4) visit4(va[u], i << 2);
+                for (int u = 0; u < NUC_U; u++) {
+                    const int i = ((nst - 1) * NUC_U + u) * NUC_BLOCK + tid;
+                    if (i < n4) visit4(va[u], i << 2);
+                }
             }
         } else {
             pre();
@@ -361,8 +376,10 @@ __device__ __forceinline__ void nuc_range(const NucRow &r, int w, float &ylo, fl
 // COUNTED: a frequency or presence penalty is on (the table of occurrence counts is read for ids the history holds);
 // its own instance, so that the usual one carries none of it.
 // ANY_T: cfg_rcp is the reciprocal of a temperature that the host has not tried the three-instruction quotient on.
-// REQUEST (1024 threads only): the first stage of sweeps 2 and 3 is requested before the reductions between the sweeps.
-template <int NUC_BLOCK, bool COUNTED, bool REQUEST = true, bool ANY_T = false>
+// KEEP: the row's first stages (64 KiB: two of 512 threads, one of 1024) stay in registers from sweep 1 on.  The sweeps are bound by the row's three reads, of which
+// two are that much shorter, and begin without a wait.  (Before, sweeps 2 and 3 had their first stage requested ahead with 1024 threads.  us, then and now:
+// 256 x 128 256 63.4 and 61.7; with 512 threads 1024 x 152 064 299.8 and 280.7, 512 x 50 257 51.3 and 44.7.)
+template <int NUC_BLOCK, bool COUNTED, bool KEEP = true, bool ANY_T = false>
 __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const float cfg_T, const float cfg_p, const float cfg_rep,
                                                  const float cfg_dcut, const float cfg_freq, const float cfg_pres,
                                                  const float cfg_rcp) {
@@ -480,14 +497,11 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         }
     };
     // every element of the row as f(id, penalised logit): the sweep, then the seen ids when the sweep masked them
-    // (1024 threads: the first stage of sweeps 2 and 3 is requested ahead, into `ahead`)
-    constexpr bool REQ = REQUEST && NUC_BLOCK == 1024;
-    // (512 threads: its first stages are kept)
-    constexpr bool KEEP = NUC_BLOCK == 512;
-    typename std::conditional<REQ, nuc_f32x4[NucGeom<NUC_BLOCK>::U], typename std::conditional<KEEP, NucKept<NUC_BLOCK>, NucNoFirst>::type>::type ahead;
-    const NucNoFirst none;
-    auto &first = ahead;
-    auto &requested = std::get<REQ ? 0 : 1>(std::tie(ahead, none));  // (the sweeps of rows that are not usual keep nothing)
+    typename std::conditional<KEEP, NucKept<NUC_BLOCK>, NucNoFirst>::type kept;
+    auto fill = [&]() {
+        if constexpr (KEEP) return NucFill<NUC_BLOCK>{&kept};
+        else return NucNoFirst();
+    };
     auto sweep = [&](auto nt, auto f, auto pre, const auto &first) {
         nuc_foreach<NUC_BLOCK, decltype(nt)::value, NUC_BLOCK == 1024>(r, bm, f, pre, first);
         if (r.masked) {
@@ -511,10 +525,8 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         sweep(Cached(), [&](int j, float y) {
             mx = fmaxf(mx, y);
             if ((j & 3) == 0) mn = fminf(mn, y > -3.402823466e+38f ? y : INFINITY);
-        }, prologue, std::get<KEEP ? 0 : 1>(std::make_tuple(NucFill<NUC_BLOCK>{reinterpret_cast<NucKept<NUC_BLOCK> *>(&ahead)}, none)));
-        // (sweep 2's first stage travels while the row's maximum is found; the barriers until then order LDS traffic only)
-        if constexpr (REQ) nuc_request_first<NUC_BLOCK, false>(r, ahead);
-        mx = block_max_f32<NUC_BLOCK, true>(mx, &scr);
+        }, prologue, fill());
+            mx = block_max_f32<NUC_BLOCK, true>(mx, &scr);
         mn = -block_max_f32<NUC_BLOCK, true>(-mn, &scr);
         r.m = uniform_f32(nuc_z(r, mx));
         r.degenerate = r.m == -INFINITY;                             // nothing finite: every d is 0 by definition
@@ -576,7 +588,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
                 }
         }
         if (a.mass_shift > 51) {                                     // (short rows)
-            sweep_plain(Cached(), [&](int, float y) { lin_put(lin_z(y), Plus()); }, first);
+            sweep_plain(Cached(), [&](int, float y) { lin_put(lin_z(y), Plus()); }, kept);
         } else {
             double start = mass_sum_start(a.mass_shift);
             mass_sum_begin(start);
@@ -585,8 +597,8 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
                 const u64 q = mass_of(expneg_core(__builtin_amdgcn_fmed3f(x, -87.0f, 0.0f)), start);
                 atomicAdd(&mass[(int)__builtin_amdgcn_fmed3f(x * nsbin, 0.0f, (float)(NUC_BINS - 1))], q);
             };
-            if (r.T == 1.0f) sweep_plain(Cached(), [&](int, float y) { put(y); }, first);
-            else sweep_plain(Cached(), [&](int, float y) { put(nuc_z_shortcut<ANY_T>(r, y)); }, first);
+            if (r.T == 1.0f) sweep_plain(Cached(), [&](int, float y) { put(y); }, kept);
+            else sweep_plain(Cached(), [&](int, float y) { put(nuc_z_shortcut<ANY_T>(r, y)); }, kept);
             mass_sum_end(start);
         }
     } else if (r.T == 1.0f && !r.degenerate) {
@@ -598,22 +610,20 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
             }
             const float d = r.m - z;
             atomicAdd(&mass[nuc_bin(r, d)], qfix(expneg(d, r.dcut), r.scale));
-        }, NucNoPre(), requested);
+        }, NucNoPre(), kept);
     } else if (r.rcp != 0.0f && !r.degenerate) {
         sweep(Cached(), [&](int, float y) {
             float z = nuc_z_shortcut<ANY_T>(r, y);
             if (!nuc_ordinary(y)) z = nuc_z(r, y);                   // zeros, masked (-inf) and other unusual logits: the division
             const float d = r.m - z;
             atomicAdd(&mass[nuc_bin(r, d)], qfix(expneg(d, r.dcut), r.scale));
-        }, NucNoPre(), requested);
+        }, NucNoPre(), kept);
     } else {
         sweep(Cached(), [&](int, float y) {
             const float d = nuc_d(r, nuc_z(r, y));
             atomicAdd(&mass[nuc_bin(r, d)], qfix(expneg(d, r.dcut), r.scale));
-        }, NucNoPre(), requested);
+        }, NucNoPre(), kept);
     }
-    // (sweep 3's first stage travels while the bins are summed and the wanted ones found)
-    if constexpr (REQ) nuc_request_first<NUC_BLOCK, true>(r, ahead);
     lds_barrier();
     BORN_STAMP(a, row, 3);
 #if defined(BORN_NUC_STOP_AFTER) && BORN_NUC_STOP_AFTER == 2
@@ -671,7 +681,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         auto in_either = [&](float y) { return nuc_within(y, lo0, hi0) | nuc_within(y, lo1, hi1); };
         auto sweep_few = [&](auto wanted) {
             nuc_foreach4<NUC_BLOCK, true, NUC_BLOCK == 1024, true>(r, bm, [&](int j, const float (&y)[4]) { staged.template append4<NUC_WCAP>(wanted, y, j); },
-                                                                   [&](int j, float y) { append(wanted(y), y, j); }, NucNoPre(), first);
+                                                                   [&](int j, float y) { append(wanted(y), y, j); }, NucNoPre(), kept);
         };
         if (lin) {
             // (the stored logits; a seen id's stored logit that passes is dropped below, its penalised logit is offered
@@ -686,9 +696,9 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
                     }
             }
         } else if (one) {
-            sweep(Streamed(), [&](int j, float y) { append(in_one(y), y, j); }, NucNoPre(), requested);
+            sweep(Streamed(), [&](int j, float y) { append(in_one(y), y, j); }, NucNoPre(), kept);
         } else {
-            sweep(Streamed(), [&](int j, float y) { append(in_either(y), y, j); }, NucNoPre(), requested);
+            sweep(Streamed(), [&](int j, float y) { append(in_either(y), y, j); }, NucNoPre(), kept);
         }
         const u32 count = staged.size();
         if (count > (u32)NUC_WCAP && lane_id() == 0) s_over = 1;
