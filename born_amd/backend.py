@@ -10,6 +10,7 @@ with the reference's panic text ("add: shapes not compatible for broadcasting: .
 
 """
 import ctypes as C
+import functools
 import math
 
 import numpy as np
@@ -22,10 +23,14 @@ class BackendPanic(SamplerPanic):
     """What the Go layer would panic with."""
 
 
+# A program's operations come with the same few shapes at every pass: their arrays, which the library only reads, and the shapes of results are
+# worked out once each (a pass of an MNIST network of 64 images: 143 us, 153 when every operation made its own).
+@functools.lru_cache(maxsize=1024)
 def _shape_arr(shape):
     return (C.c_int64 * max(len(shape), 1))(*shape)
 
 
+@functools.lru_cache(maxsize=1024)
 def _broadcast(a, b):
     """The shape of an element-wise result of two shapes of one length; None where the library is asked (and says what is wrong)."""
     if len(a) != len(b) or not a:
@@ -43,7 +48,7 @@ class DeviceTensor:
 
     def __init__(self, buf, shape):
         self.buf = buf
-        self.shape = tuple(int(d) for d in shape)
+        self.shape = tuple(map(int, shape))
 
     @classmethod
     def from_numpy(cls, a):
@@ -132,7 +137,7 @@ class ROCmBackend:
                                                 int(stride), int(padding), out.buf.ptr, oshape, stream))
         except SamplerPanic as e:
             raise BackendPanic(str(e)) from None
-        out.shape = tuple(oshape[i] for i in range(4))
+        out.shape = tuple(oshape)
         return out
 
     def MaxPool2D(self, input, kernelSize, stride, stream=None):
@@ -145,11 +150,11 @@ class ROCmBackend:
                                                    out.buf.ptr, oshape, stream))
         except SamplerPanic as e:
             raise BackendPanic(str(e)) from None
-        out.shape = tuple(oshape[i] for i in range(4))
+        out.shape = tuple(oshape)
         return out
 
     def Reshape(self, t, new_shape, stream=None):
-        new_shape = tuple(int(d) for d in new_shape)
+        new_shape = tuple(map(int, new_shape))
         out = DeviceTensor.empty(new_shape)
         try:
             _check(_capi.lib().born_rocm_reshape(t.buf.ptr, _shape_arr(t.shape), len(t.shape), _shape_arr(new_shape), len(new_shape),
