@@ -118,12 +118,12 @@ __device__ __forceinline__ nuc_f32x4 nuc_load4_clamped(const float *x, int b, in
 // LOADS_FIRST: a stage's loads are issued before the visits of the one before, not among them, where the compiler spilled registers for them; off for
 // the sweep of token_logprob_kernel, which they held up (1024 x 152 064: 103 us, 100 without).
 // FIRST (AHEAD instances only): `first` holds the row's first stage, requested earlier with nuc_request_first, or
-// (NucKept) its first stages, kept in registers from the first sweep on, which fills them (NucFill).
+// (NucKept) its first blocks, kept in registers from the first sweep on, which fills them (NucFill).
 struct NucNoFirst {};
 template <int NUC_BLOCK>
 struct NucKept {
-    static constexpr int STAGES = NUC_BLOCK == 512 ? 2 : 1;
-    nuc_f32x4 v[STAGES * NucGeom<NUC_BLOCK>::U];
+    static constexpr int LOADS = NUC_BLOCK == 512 ? 10 : NucGeom<NUC_BLOCK>::U;   // of a thread: what the 128 registers of a lane leave (1024: a stage)
+    nuc_f32x4 v[LOADS];
 };
 template <int NUC_BLOCK>
 struct NucFill {
@@ -170,55 +170,56 @@ __device__ __forceinline__ void nuc_foreach4(const NucRow &r, const u32 *bm, F4 
         f1(j, y);
     };
     const int n4 = r.n4;
-    constexpr int NUC_U = NucGeom<NUC_BLOCK>::U, NUC_KEPT = NucKept<NUC_BLOCK>::STAGES;
+    constexpr int NUC_U = NucGeom<NUC_BLOCK>::U, NUC_KEPT = NucKept<NUC_BLOCK>::LOADS;
     constexpr bool FILL = std::is_same<FIRST, NucFill<NUC_BLOCK>>::value, KEPT = FILL || std::is_same<FIRST, NucKept<NUC_BLOCK>>::value;
     if constexpr (!AHEAD) {
-        const int nfull = n4 / (NUC_U * NUC_BLOCK);
+        const int kept_blocks = KEPT && n4 >= (NUC_KEPT + NUC_U) * NUC_BLOCK ? NUC_KEPT * NUC_BLOCK : 0;
+        const int nfull = (n4 - kept_blocks) / (NUC_U * NUC_BLOCK);
         if (nfull > 0) {
             // Two stages a turn, each loaded while the other is visited, so that no register is copied; the last
             // one or two stages in a loop of their own.
             nuc_f32x4 va[NUC_U], vb[NUC_U];
             const u32 off = (u32)tid * 16u;
-            int s = KEPT && nfull > NUC_KEPT ? NUC_KEPT : 0;         // the first stage that is loaded
+            int s = 0;
             if constexpr (FILL) {
-                if (s)
+                if (kept_blocks)
 #pragma unroll
-                    for (int k = 0; k < NUC_KEPT * NUC_U; k++) first.kept->v[k] = nuc_load4<NT>(r.x, k * NUC_BLOCK, off);
+                    for (int k = 0; k < NUC_KEPT; k++) first.kept->v[k] = nuc_load4<NT>(r.x, k * NUC_BLOCK, off);
             }
 #pragma unroll
-            for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(r.x, (s * NUC_U + u) * NUC_BLOCK, off);
+            for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(r.x, kept_blocks + (s * NUC_U + u) * NUC_BLOCK, off);
             pre();
             if constexpr (KEPT) {
                 const NucKept<NUC_BLOCK> *kept;
                 if constexpr (FILL) kept = first.kept;
                 else kept = &first;
-                if (s)
+                if (kept_blocks)
 #pragma unroll
-                    for (int k = 0; k < NUC_KEPT * NUC_U; k++) visit4(kept->v[k], (k * NUC_BLOCK + tid) << 2);
+                    for (int k = 0; k < NUC_KEPT; k++) visit4(kept->v[k], (k * NUC_BLOCK + tid) << 2);
             }
             for (; s + 2 < nfull; s += 2) {
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4<NT>(r.x, ((s + 1) * NUC_U + u) * NUC_BLOCK, off);
+                for (int u = 0; u < NUC_U; u++) vb[u] = nuc_load4<NT>(r.x, kept_blocks + ((s + 1) * NUC_U + u) * NUC_BLOCK, off);
                 if (LOADS_FIRST) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) visit4(va[u], ((s * NUC_U + u) * NUC_BLOCK + tid) << 2);
+                for (int u = 0; u < NUC_U; u++) visit4(va[u], (kept_blocks + (s * NUC_U + u) * NUC_BLOCK + tid) << 2);
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(r.x, ((s + 2) * NUC_U + u) * NUC_BLOCK, off);
+                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(r.x, kept_blocks + ((s + 2) * NUC_U + u) * NUC_BLOCK, off);
                 if (LOADS_FIRST) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) visit4(vb[u], (((s + 1) * NUC_U + u) * NUC_BLOCK + tid) << 2);
+                for (int u = 0; u < NUC_U; u++) visit4(vb[u], (kept_blocks + ((s + 1) * NUC_U + u) * NUC_BLOCK + tid) << 2);
             }
             for (;;) {
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) visit4(va[u], ((s * NUC_U + u) * NUC_BLOCK + tid) << 2);
+                for (int u = 0; u < NUC_U; u++) visit4(va[u], (kept_blocks + (s * NUC_U + u) * NUC_BLOCK + tid) << 2);
                 if (++s >= nfull) break;
 #pragma unroll
-                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(r.x, (s * NUC_U + u) * NUC_BLOCK, off);
+                for (int u = 0; u < NUC_U; u++) va[u] = nuc_load4<NT>(r.x, kept_blocks + (s * NUC_U + u) * NUC_BLOCK, off);
             }
         } else {
             pre();
         }
-        for (int i = nfull * NUC_U * NUC_BLOCK + tid; i < n4; i += NUC_BLOCK) {
+        for (int i = kept_blocks + nfull * NUC_U * NUC_BLOCK + tid; i < n4; i += NUC_BLOCK) {
             const nuc_f32x4 q = nuc_load4<NT>(r.x, 0, (u32)i * 16u);
             visit4(q, i << 2);
         }
@@ -376,9 +377,9 @@ __device__ __forceinline__ void nuc_range(const NucRow &r, int w, float &ylo, fl
 // COUNTED: a frequency or presence penalty is on (the table of occurrence counts is read for ids the history holds);
 // its own instance, so that the usual one carries none of it.
 // ANY_T: cfg_rcp is the reciprocal of a temperature that the host has not tried the three-instruction quotient on.
-// KEEP: the row's first stages (64 KiB: two of 512 threads, one of 1024) stay in registers from sweep 1 on.  The sweeps are bound by the row's three reads, of which
+// KEEP: the row's first logits (80 KiB of them with 512 threads, 64 with 1024) stay in registers from sweep 1 on.  The sweeps are bound by the row's three reads, of which
 // two are that much shorter, and begin without a wait.  (Before, sweeps 2 and 3 had their first stage requested ahead with 1024 threads.  us, then and now:
-// 256 x 128 256 63.4 and 61.7; with 512 threads 1024 x 152 064 299.8 and 280.7, 512 x 50 257 51.3 and 44.7.)
+// 256 x 128 256 63.4 and 61.7; with 512 threads 1024 x 152 064 299.8 and 276.4, 281.1 with 64 KiB, 512 x 50 257 51.3 and 43.5.)
 template <int NUC_BLOCK, bool COUNTED, bool KEEP = true, bool ANY_T = false>
 __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const float cfg_T, const float cfg_p, const float cfg_rep,
                                                  const float cfg_dcut, const float cfg_freq, const float cfg_pres,
