@@ -4,18 +4,22 @@
 // is wave c % NW's, and the waves' sums are added in order through LDS at the end.  Operands go from memory straight into
 // the matrix instructions' registers, a chunk ahead: no staging, no barrier before the end, one launch; rows may start at any four
 // bytes, and only the last chunk of K asks where K ends.  The tiles (linear.hip) have 16 to 128 rows of 128 columns, slices of K in a launch of
-// their own that another one adds, and loads of one value where K or a pitch is odd.  Each wave's sum is shorter than a tile's: 2-norm against fp64
-// 1.9e-7 at K = 784, theirs 2.3e-7 in slices and 5.0e-7 unsliced.
+// their own that another one adds, and loads of one value where K or a pitch is odd.
 //
-// us, tiles and here: linear 64 x 784 -> 512 12.3 5.0, 64 x 512 -> 128 8.0 4.4, 64 x 128 -> 10 4.3 3.5 (a launch after another: 3.4), 1000 x 784 -> 512 29.6 16.8,
-// 179 x 686 -> 226 15.4 5.2; matmul 64 x 1024 x 128 9.5 5.5, 64 x 128 x 10 8.9 3.8, 94 x 3212 x 101 19.0 11.9.  Bound by the loads' latency and, from
+// An accumulator is one chain of fp32 additions.  The tiles have up to sixteen slices' of it, K / 128 and 512 / tiles at most, so a wave has four here, for k modulo four:
+// sixteen chains or more wherever the tiles have more than four, in the squares of 32 one a wave where they have not (their registers: 1000 x 3 -> 4001 15.6 us, 20.3 with four).
+// 2-norm against fp64, tiles and here (one accumulator a wave in brackets): 64 x 784 -> 512 2.3e-7 1.2e-7 (2.0e-7), 64 x 2048 -> 1024 2.2e-7 1.6e-7 (2.9e-7),
+// 497 x 1568 -> 232 2.3e-7 1.9e-7 (3.6e-7), 94 x 3211 x 101 2.8e-7 2.0e-7 (3.7e-7), 2000 x 2000 -> 100 2.9e-7 2.1e-7 (4.1e-7), 3 x 100 003 -> 252 1.5e-6 1.0e-6 (1.9e-6); the times are the same.
+//
+// us, tiles and here: linear 64 x 784 -> 512 12.1 5.2, 64 x 512 -> 128 8.0 4.5, 64 x 128 -> 10 4.3 3.6 (a launch after another: 3.4), 1000 x 784 -> 512 29.3 16.9,
+// 179 x 686 -> 226 15.4 5.2; matmul 64 x 1024 x 128 9.5 5.8, 64 x 128 x 10 8.9 3.6, 94 x 3211 x 101 20.0 12.0.  Bound by the loads' latency and, from
 // about 200 million products on, by the L2s: a square of 32 rows reads 8 bytes for 64 products.
 #include "gemm_epilogue.h"
 
 namespace born {
 
 // T: 16-row blocks of the square's side.  U: 128-bit loads of an operand's row per lane and chunk.  NW: waves.
-template <bool BT, int T, int U, int NW, int EPI>
+template <bool BT, int T, int U, int NW, int ACC, int EPI>
 __global__ __launch_bounds__(NW * WAVE) void gemm_small_kernel(GemmArgs g) {
     constexpr int L = 16, SIDE = T * L, G = 16, CHUNK = U * G;       // tile side; k-values per load, per chunk
     extern __shared__ __align__(16) unsigned char small_lds[];       // [NW - 1][T * T][WAVE] accumulators, then the epilogue's stage
@@ -70,9 +74,9 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_small_kernel(GemmArgs g) {
             }
         }
     };
-    f32x4 acc[T][T];
+    f32x4 sum[ACC][T][T];                                            // (four: of the k-values that are 0, 1, 2, 3 modulo four)
 #pragma unroll
-    for (int i = 0; i < T * T; i++) acc[i / T][i % T] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < ACC * T * T; i++) sum[i / (T * T)][i / T % T][i % T] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto multiply = [&](const Chunk &x) {
 #pragma unroll
         for (int u = 0; u < U; u++)
@@ -81,7 +85,7 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_small_kernel(GemmArgs g) {
 #pragma unroll
                 for (int r = 0; r < T; r++)
 #pragma unroll
-                    for (int c = 0; c < T; c++) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.a[u][r][i], x.b[u][c][i], acc[r][c], 0, 0, 0);
+                    for (int c = 0; c < T; c++) sum[i % ACC][r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.a[u][r][i], x.b[u][c][i], sum[i % ACC][r][c], 0, 0, 0);
     };
     if (wave < chunks) {
         Chunk x, y;
@@ -94,6 +98,13 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_small_kernel(GemmArgs g) {
             x = y;
         }
         multiply(x);
+    }
+    f32x4 acc[T][T];
+#pragma unroll
+    for (int i = 0; i < T * T; i++) {
+        const int r = i / T, c = i % T;
+        if constexpr (ACC == 4) acc[r][c] = (sum[0][r][c] + sum[1][r][c]) + (sum[2][r][c] + sum[3][r][c]);
+        else acc[r][c] = sum[0][r][c];
     }
     f32x4 *const part = reinterpret_cast<f32x4 *>(small_lds);
     if (wave) {
@@ -109,22 +120,24 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_small_kernel(GemmArgs g) {
     gemm_finish<EPI, L, 1>(g, acc, m0, n0, small_lds + (NW - 1) * T * T * WAVE * sizeof(f32x4));
 }
 
-template <bool BT, int T, int U, int NW, int EPI>
+template <bool BT, int T, int U, int NW, int ACC, int EPI>
 static void launch_small_as(const GemmArgs &g, long long tiles, hipStream_t st) {
     const size_t lds = (size_t)(NW - 1) * T * T * 256 * sizeof(float) + (EPI == 2 ? gemm_stage_bytes(1) : 0);
-    hipLaunchKernelGGL((gemm_small_kernel<BT, T, U, NW, EPI>), dim3((unsigned)((tiles + NUM_XCD - 1) / NUM_XCD * NUM_XCD)), dim3(NW * WAVE), lds, st, g);
+    hipLaunchKernelGGL((gemm_small_kernel<BT, T, U, NW, ACC, EPI>), dim3((unsigned)((tiles + NUM_XCD - 1) / NUM_XCD * NUM_XCD)), dim3(NW * WAVE), lds, st, g);
 }
 static long long small_tiles(const GemmArgs &g, int side) { return (long long)((g.M + side - 1) / side) * ((g.N + side - 1) / side); }
 // us by form (side 16 with one, four and eight waves; side 32): 1000 x 300 -> 200, 819 squares of 16, 6.5 7.4 7.4 7.1;   130 x 1920 -> 1383, 783, 28.8 29.3
 // 28.4 18.4;   17 x 352 -> 6317, 790, 9.0 9.0 9.5 6.7;   310 x 320 -> 576, 720, 6.5 6.4 7.8 7.7;   497 x 1568 -> 232, 480, 17.8 14.9 15.0 16.1;   3000 x 100 -> 50, 752,
 // 4.1 4.2 5.3 5.5;   64 x 784 -> 512, 128, 9.0 5.3 5.1 9.9;   64 x 964 x 23, 8, 13.2 6.2 5.6 11.6.
 template <bool BT, int EPI>
-static void launch_small_epi(const GemmArgs &g, hipStream_t st) {
+static void launch_small_epi(const GemmArgs &g, long long tiles, hipStream_t st) {
     const long long t16 = small_tiles(g, 16);
-    if (t16 > 840 || (t16 > 600 && g.K > 340)) launch_small_as<BT, 2, 2, 4, EPI>(g, small_tiles(g, 32), st);
-    else if (g.K <= 64) launch_small_as<BT, 1, 4, 1, EPI>(g, t16, st);
-    else if (g.K <= 256 || t16 > 384) launch_small_as<BT, 1, 4, 4, EPI>(g, t16, st);
-    else launch_small_as<BT, 1, 4, 8, EPI>(g, t16, st);
+    if (t16 > 840 || (t16 > 600 && g.K > 340)) {
+        if (g.K < 640 || tiles > 102) launch_small_as<BT, 2, 2, 4, 1, EPI>(g, small_tiles(g, 32), st);
+        else launch_small_as<BT, 2, 2, 4, 4, EPI>(g, small_tiles(g, 32), st);
+    } else if (g.K <= 64) launch_small_as<BT, 1, 4, 1, 1, EPI>(g, t16, st);
+    else if (g.K <= 256 || t16 > 384) launch_small_as<BT, 1, 4, 4, 4, EPI>(g, t16, st);
+    else launch_small_as<BT, 1, 4, 8, 4, EPI>(g, t16, st);
 }
 
 // `tiles`: of the fp32 tiles (linear.hip).  Where their loads are guarded ones (us, theirs and here): 1000 x 784 -> 512 29.6 16.8, 2000 x 2000 -> 100 23.7 21.0,
@@ -138,11 +151,11 @@ bool gemm_small_takes(const GemmArgs &g, bool b_transposed, long long tiles) {
     if (g.N <= 64 && products <= 3e8) return g.K <= 2048 || small_tiles(g, 16) >= 128;
     return tiles < 128 && products <= 2.1e8 && (g.K <= 2048 || small_tiles(g, 16) >= 128);
 }
-hipError_t launch_gemm_small(const GemmArgs &g, bool b_transposed, hipStream_t st) {
-    if (!b_transposed) launch_small_epi<false, 0>(g, st);
-    else if (g.cand) launch_small_epi<true, 2>(g, st);
-    else if (g.best) launch_small_epi<true, 1>(g, st);
-    else launch_small_epi<true, 0>(g, st);
+hipError_t launch_gemm_small(const GemmArgs &g, bool b_transposed, long long tiles, hipStream_t st) {
+    if (!b_transposed) launch_small_epi<false, 0>(g, tiles, st);
+    else if (g.cand) launch_small_epi<true, 2>(g, tiles, st);
+    else if (g.best) launch_small_epi<true, 1>(g, tiles, st);
+    else launch_small_epi<true, 0>(g, tiles, st);
     return hipGetLastError();
 }
 

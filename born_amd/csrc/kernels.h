@@ -137,7 +137,7 @@ bool gemm_rows_takes(const GemmArgs &g, bool b_transposed);
 hipError_t launch_gemm_rows(const GemmArgs &g, hipStream_t st);
 // The same product where it is small (gemm_small.hip): where gemm_small_takes, given how many tiles it would be else.
 bool gemm_small_takes(const GemmArgs &g, bool b_transposed, long long tiles);
-hipError_t launch_gemm_small(const GemmArgs &g, bool b_transposed, hipStream_t st);
+hipError_t launch_gemm_small(const GemmArgs &g, bool b_transposed, long long tiles, hipStream_t st);
 // The same product on the 16-bit matrix cores (gemm_split.hip), where gemm_split_pays, in the tile of its plan (gemm_plan.h).
 // `workspace` holds gemm_split_workspace(M, K) bytes, 256-byte aligned; g.ksplit > 1: as above.
 hipError_t launch_gemm_split(const GemmArgs &g, bool b_transposed, int tile, void *workspace, hipStream_t st);

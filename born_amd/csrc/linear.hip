@@ -590,7 +590,7 @@ hipError_t launch_gemm_f32(const GemmArgs &g, bool b_transposed, hipStream_t st)
         return hipGetLastError();
     }
     if (gemm_small_takes(g, b_transposed, grid)) {
-        const hipError_t e = launch_gemm_small(g, b_transposed, st);
+        const hipError_t e = launch_gemm_small(g, b_transposed, grid, st);
         if (e != hipSuccess) return e;
         if (g.best) hipLaunchKernelGGL(argmax_keys_token_kernel, dim3((unsigned)((g.M + 255) / 256)), dim3(256), 0, st, g.best, g.tokens, g.M);
         return hipGetLastError();

@@ -43,6 +43,24 @@ def test_against_fp64(before, over):
             assert (got[:, N:] == 7).all(), (form, M, K, N)
 
 
+@pytest.mark.parametrize("M,K,N", [(64, 2048, 1024), (497, 1568, 232), (94, 3212, 101), (2000, 2000, 100), (400, 4097, 300), (911, 19590, 17), (3, 30001, 700)])
+def test_error_of_a_sum_in_sixteen_parts(M, K, N):
+    """No sum of the product is longer than K / 16 terms, as in the tiles' most slices.  A sum of L terms that are alike grows as sqrt(j), each addition rounds by
+    2^-24 / sqrt(3) of it at most, root mean square, so that sqrt(L / 6) 2^-24 is the most of a part's, and of the whole, 2-norm."""
+    from born_amd import _capi, sampler as S
+    rng = np.random.default_rng(K)
+    x, w = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((N, K)).astype(np.float32)
+    exact = x.astype(np.float64) @ w.T.astype(np.float64)
+    px, pw, pt, out = S.DeviceBuffer.from_numpy(x), S.DeviceBuffer.from_numpy(w), S.DeviceBuffer.from_numpy(np.ascontiguousarray(w.T)), S.DeviceBuffer(4 * M * N)
+    for form in ("linear", "matmul"):
+        if form == "linear":
+            _capi.check(_capi.lib().born_rocm_linear(px.ptr, M, K, K, pw.ptr, N, K, None, out.ptr, N, None))
+        else:
+            _capi.check(_capi.lib().born_rocm_matmul(px.ptr, pt.ptr, out.ptr, M, K, N, K, N, N, None))
+        err = np.linalg.norm(out.to_numpy(np.float32, (M, N)) - exact) / np.linalg.norm(exact)
+        assert err <= np.sqrt(K / 16 / 6) * 2.0 ** -24, (form, err)
+
+
 @pytest.mark.parametrize("M,K,N", [(5, 300, 300), (17, 256, 1001), (33, 352, 5000), (64, 1024, 200)])
 def test_the_fused_heads_see_the_plain_head_s_logits(oracle, M, K, N):
     from born_amd import linear as L, sampler as S
