@@ -1,4 +1,4 @@
-// Host side of the large products (gemm_split.hip): which go there, in which tiles and slices.
+// Host side of the products: which large ones go to gemm_split.hip, in which tiles and slices, and which small ones to gemm_small.hip.
 #include "gemm_plan.h"
 
 #include <algorithm>
@@ -101,6 +101,46 @@ SplitPlan gemm_split_plan(int M, int N, int K) {
         }
     }
     return best;
+}
+
+// ---- which small products go to gemm_small.hip, not to the fp32 tiles (linear.hip)
+// Where the tiles' loads are guarded ones.  us, tiles and here, linear and then matmul:
+//   a long K and few squares, a CU to each: the tiles' slices are on more of them
+//     1 square   3211 13.5 11.1, 16.9 10.8;   4097 15.2 16.7, 19.3 12.6;   8193 21.2 30.3, 28.2 21.6;   24 001 43 83, 61 55;   40 001 66 137, 96 94
+//     4          6001 17.9 16.7, 24.9 19.0;   8193 21.8 26.5, 31.3 23.4;   24 001 44 71, 68 57
+//     21         8193 31.2 30.8, 30.9 24.6;   12 001 39.6 43.7, 38.9 42.5
+//     42         12 001 43.8 44.6, 44.4 44.6;   20 001 64 71, 65 71;   126: 8193 36.2 30.9, 31.0 28.4;   169: 8193 48 31, 35 31, 12 001 67 45, 45 43
+//     288        4097 33.2 31.3, 34.7 32.5;   6001 40.5 38.7, 41.8 45.7 (the CUs' second round);   425: 4097 38.9 31.4, 30.6 30.9
+//     up to four rows, which are few lines here: 3 x 100 003 -> 10 148 138, 240 202, -> 252 257 176, 222 209, -> 700 282 206, 228 303;   3 x 30 001 -> 700 87 57, 75 73;   2 x 15 391 -> 18 30 36
+//     few columns of many rows, of which a tile wastes most: 911 x 19 590 -> 17 73 52, 92 56, 3415 x 35 508 -> 2 361 94, 502 108;   768 x 30 001 -> 9 97 65, 132 74
+//   large results of a short K, which the tiles store in whole lines where rows are a multiple of 16 bytes
+//     250 000 squares  8000 x 3 -> 8000 157 166, 143 198;   64 000: 4096 x 7 -> 4000 43 47, 39 56;   47 000: 3000 x 7 -> 4000 41 36, 37 43
+//     16 000 4096 x 20 -> 1000 18.8 17.2, 17.6 19.4;   32 000: 4096 x 50 -> 2000 33 34, 28 37;   8192: 4096 x 204 -> 500 20.4 25.2, 21.1 22.8, half the tiles' error (above 32 values here it is
+//     smaller than theirs)
+//     rows of odd length 16 000 1000 x 7 -> 4001 20.0 15.6, 18.5 18.2;   37 500 200 000 x 7 -> 33 68 40, 66 50
+static bool small_pays_guarded(int M, int N, int K, bool b_transposed) {
+    const long long squares = gemm_small_squares(M, N, 16);
+    if ((double)M * (double)N * (double)K > 5e8) return false;
+    if (N > 32 || M < 768) {
+        int k_max;
+        if (M <= 4 && (!b_transposed || squares == 1 || squares > 3)) k_max = b_transposed || squares <= 16 ? 131072 : 32768;
+        else if (b_transposed) k_max = squares < 4 ? 3584 : squares < 21 ? 6144 : squares < 42 ? 8448 : squares <= 256 ? 12288 : 4352;
+        else k_max = squares < 16 ? 24576 : squares <= 256 ? 8448 : 4352;
+        if (K > k_max) return false;
+    }
+    return N % 4 || squares <= (b_transposed ? 48000 : K > 32 ? 16384 : 3072);
+}
+// `tiles`: of the fp32 tiles.  whole: their loads need no guard.  Where K is a multiple of 32 and all aligned (us, theirs and here), columns that fill half a tile or less: 4096 x 1024 -> 64 21.1 13.1,
+// 2048 x 8192 -> 16 45 31, 512 x 4096 -> 64 16.8 17.0, 512 x 8192 -> 64 21.8 30.6, 1024 x 4096 -> 64 21.2 17.1, 1100 x 4096 -> 64 21.9 30.6, 1024 x 8192 -> 32 29.4 30.6; fewer tiles than would be left
+// unsliced: 64 x 2048 -> 1024 14.2 9.8, 308 x 1056 x 648 16.7 14.1, 89 x 1888 -> 1743 19.0 18.2, 64 x 4096 -> 4096 29.5 37.0, 55 x 64 x 1032 5.6 3.8, but few squares and a long
+// K, where slices put more CUs to work: 16 x 4096 -> 1000 13.2 16.8, 128 x 3072 -> 256 13.2 13.3, 128 x 4096 -> 256 15.1 16.7, 128 x 6144 -> 256 18.3 23.6.  More tiles: 2048 x 128 -> 512
+// 7.0 8.5, 7 x 320 -> 21 263 8.1 10.6.
+bool gemm_small_pays(int M, int N, int K, bool b_transposed, bool whole, long long tiles) {
+    if (!whole) return small_pays_guarded(M, N, K, b_transposed);
+    const double products = (double)M * (double)N * (double)K;
+    const long long squares = gemm_small_squares(M, N, 16);
+    if (N <= 64 && products <= 3e8) return K <= 2048 || (M >= 1024 && squares >= 128 && (N <= 16 || (K <= 4096 && squares <= 256)));
+    return tiles < 128 && products <= 2.1e8 && (K <= 2048 || (K <= 3072 && squares >= 128 && squares <= 256));
 }
 
 }  // namespace born

@@ -1,4 +1,5 @@
-// Which products go to the 16-bit matrix cores (gemm_split.hip), in which tiles and slices: host decisions without HIP.
+// Which products go to the 16-bit matrix cores (gemm_split.hip), in which tiles and slices, and which to the kernel of small ones (gemm_small.hip):
+// host decisions without HIP.
 #pragma once
 #include <cstddef>
 
@@ -21,5 +22,8 @@ bool gemm_split_pays(int M, int N, int K, long long ldb);
 SplitPlan gemm_split_plan(int M, int N, int K);
 size_t gemm_split_workspace(int M, int K);    // bytes of the packed operand and its flags, a multiple of 256
 size_t gemm_split_bytes(const SplitPlan &p, int rows, int N, int K);   // .. and of the partial products behind it
+
+inline long long gemm_small_squares(long long M, long long N, int side) { return ((M + side - 1) / side) * ((N + side - 1) / side); }
+bool gemm_small_pays(int M, int N, int K, bool b_transposed, bool whole, long long tiles);
 
 }  // namespace born

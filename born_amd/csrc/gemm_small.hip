@@ -15,6 +15,7 @@
 // 179 x 686 -> 226 15.4 5.2; matmul 64 x 1024 x 128 9.5 5.8, 64 x 128 x 10 8.9 3.6, 94 x 3211 x 101 20.0 12.0.  Bound by the loads' latency and, from
 // about 200 million products on, by the L2s: a square of 32 rows reads 8 bytes for 64 products.
 #include "gemm_epilogue.h"
+#include "gemm_plan.h"
 
 namespace born {
 
@@ -125,31 +126,25 @@ static void launch_small_as(const GemmArgs &g, long long tiles, hipStream_t st) 
     const size_t lds = (size_t)(NW - 1) * T * T * 256 * sizeof(float) + (EPI == 2 ? gemm_stage_bytes(1) : 0);
     hipLaunchKernelGGL((gemm_small_kernel<BT, T, U, NW, ACC, EPI>), dim3((unsigned)((tiles + NUM_XCD - 1) / NUM_XCD * NUM_XCD)), dim3(NW * WAVE), lds, st, g);
 }
-static long long small_tiles(const GemmArgs &g, int side) { return (long long)((g.M + side - 1) / side) * ((g.N + side - 1) / side); }
 // us by form (side 16 with one, four and eight waves; side 32): 1000 x 300 -> 200, 819 squares of 16, 6.5 7.4 7.4 7.1;   130 x 1920 -> 1383, 783, 28.8 29.3
 // 28.4 18.4;   17 x 352 -> 6317, 790, 9.0 9.0 9.5 6.7;   310 x 320 -> 576, 720, 6.5 6.4 7.8 7.7;   497 x 1568 -> 232, 480, 17.8 14.9 15.0 16.1;   3000 x 100 -> 50, 752,
 // 4.1 4.2 5.3 5.5;   64 x 784 -> 512, 128, 9.0 5.3 5.1 9.9;   64 x 964 x 23, 8, 13.2 6.2 5.6 11.6.
 template <bool BT, int EPI>
 static void launch_small_epi(const GemmArgs &g, long long tiles, hipStream_t st) {
-    const long long t16 = small_tiles(g, 16);
+    const long long t16 = gemm_small_squares(g.M, g.N, 16);
     if (t16 > 840 || (t16 > 600 && g.K > 340)) {
-        if (g.K < 640 || tiles > 102) launch_small_as<BT, 2, 2, 4, 1, EPI>(g, small_tiles(g, 32), st);
-        else launch_small_as<BT, 2, 2, 4, 4, EPI>(g, small_tiles(g, 32), st);
+        if (g.K < 640 || tiles > 102) launch_small_as<BT, 2, 2, 4, 1, EPI>(g, gemm_small_squares(g.M, g.N, 32), st);
+        else launch_small_as<BT, 2, 2, 4, 4, EPI>(g, gemm_small_squares(g.M, g.N, 32), st);
     } else if (g.K <= 64) launch_small_as<BT, 1, 4, 1, 1, EPI>(g, t16, st);
     else if (g.K <= 256 || t16 > 384) launch_small_as<BT, 1, 4, 4, 4, EPI>(g, t16, st);
     else launch_small_as<BT, 1, 4, 8, 4, EPI>(g, t16, st);
 }
 
-// `tiles`: of the fp32 tiles (linear.hip).  Where their loads are guarded ones (us, theirs and here): 1000 x 784 -> 512 29.6 16.8, 2000 x 2000 -> 100 23.7 21.0,
-// 900^3 33.4 34.2.  Where K is a multiple of 32 and all aligned, columns that fill half a tile or less: 4096 x 1024 -> 64 21.4 13.1; fewer tiles than would be left
-// unsliced: 64 x 2048 -> 1024 14.2 10.1, 308 x 1056 x 648 16.7 14.1, 89 x 1888 -> 1743 19.0 18.2, 64 x 4096 -> 4096 29.5 37.0, 55 x 64 x 1032 5.6 3.8, but few squares and a long
-// K, where slices put more CUs to work: 16 x 4096 -> 1000 13.2 16.8.  More tiles: 2048 x 128 -> 512 7.0 8.5, 7 x 320 -> 21 263 8.1 10.6.
+// `tiles`: of the fp32 tiles (linear.hip)
 bool gemm_small_takes(const GemmArgs &g, bool b_transposed, long long tiles) {
     if (g.bm) return false;                                          // (a caller that names the tile height keeps it)
-    const double products = (double)g.M * (double)g.N * (double)g.K;
-    if (!g.vec_a || !g.vec_b || g.K % 32 || (!b_transposed && g.N % 4)) return products <= 5e8;
-    if (g.N <= 64 && products <= 3e8) return g.K <= 2048 || small_tiles(g, 16) >= 128;
-    return tiles < 128 && products <= 2.1e8 && (g.K <= 2048 || small_tiles(g, 16) >= 128);
+    const bool whole = g.vec_a && g.vec_b && g.K % 32 == 0 && (b_transposed || g.N % 4 == 0);
+    return gemm_small_pays(g.M, g.N, g.K, b_transposed, whole, tiles);
 }
 hipError_t launch_gemm_small(const GemmArgs &g, bool b_transposed, long long tiles, hipStream_t st) {
     if (!b_transposed) launch_small_epi<false, 0>(g, tiles, st);

@@ -1,4 +1,4 @@
-"""Host decisions of the large products (born_amd/csrc/gemm_plan.cpp), without a GPU."""
+"""Host decisions of the products (born_amd/csrc/gemm_plan.cpp), without a GPU."""
 import ctypes as C
 import os
 import subprocess
@@ -17,6 +17,7 @@ extern "C" void plan(int M, int N, int K, long long *out) {
     out[4] = p.rows ? born::gemm_split_bytes(p, p.rows < M ? p.rows : M, N, K) : 0;
 }
 extern "C" int pays(int M, int N, int K, long long ldb) { return born::gemm_split_pays(M, N, K, ldb); }
+extern "C" int small(int M, int K, int N, int b_transposed, int whole, long long tiles) { return born::gemm_small_pays(M, N, K, b_transposed, whole, tiles); }
 """
 
 
@@ -86,3 +87,24 @@ def test_products_whose_rows_come_in_chunks(plan):
 
 def test_sums_of_few_terms_stay_on_the_fp32_tiles(plan):
     assert plan.pays(4096, 65536, 16, 16) and not plan.pays(4096, 65536, 15, 15)
+
+
+def test_a_long_k_of_few_squares_is_left_to_the_tiles_slices(plan):
+    """A square has one CU, the tiles' slices of K have up to sixteen each: wherever that was measured the faster."""
+    for M, K, N in ((16, 8193, 16), (64, 8193, 10), (40, 12001, 100), (200, 20001, 100), (757, 6001, 94), (64, 100003, 10)):
+        assert not plan.small(M, K, N, 1, 0, 16), (M, K, N)
+    for M, K, N in ((16, 40001, 16), (64, 20001, 64), (40, 12001, 100), (757, 6001, 94), (4, 100003, 700), (16, 1000001, 16)):
+        assert not plan.small(M, K, N, 0, 0, 16), (M, K, N)
+    for M, K, N in ((128, 4096, 256), (512, 8192, 64), (1100, 4096, 64), (16, 4096, 1000)):                     # K a multiple of 32
+        assert not plan.small(M, K, N, 1, 1, 64) and not plan.small(M, K, N, 0, 1, 64), (M, K, N)
+    for M, K, N in ((16, 3211, 16), (64, 6001, 10), (40, 8193, 100), (200, 12001, 200), (400, 4097, 300), (911, 19590, 17), (3, 100003, 252)):
+        assert plan.small(M, K, N, 1, 0, 16), (M, K, N)
+    for M, K, N in ((16, 24001, 16), (64, 16001, 10), (40, 8193, 100), (256, 6001, 256), (3, 30001, 700)):
+        assert plan.small(M, K, N, 0, 0, 16), (M, K, N)
+
+
+def test_large_results_of_a_short_k_are_left_to_the_tiles(plan):
+    for M, K, N in ((8000, 3, 8000), (4096, 7, 4000), (20000, 7, 2000)):
+        assert not plan.small(M, K, N, 1, 0, 4000) and not plan.small(M, K, N, 0, 0, 4000), (M, K, N)
+    assert not plan.small(4096, 20, 1000, 0, 0, 1024) and plan.small(4096, 20, 1000, 1, 0, 1024)
+    assert plan.small(1000, 7, 4001, 1, 0, 1024) and plan.small(200000, 7, 33, 0, 0, 1563)                      # rows of odd length
