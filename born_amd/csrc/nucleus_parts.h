@@ -171,23 +171,24 @@ __global__ __launch_bounds__(PARTS_BLOCK, 4) void nucleus_parts_max_kernel(Sampl
 }
 
 __global__ __launch_bounds__(PARTS_BLOCK, 4) void nucleus_parts_masses_kernel(SampleArgs a, PartsArgs pa) {
-    extern __shared__ __align__(16) u64 nuc_dyn[];                   // bins, seen ids, the bitmap
+    extern __shared__ __align__(16) u64 nuc_dyn[];                   // bins and the slots beyond them, seen ids, the bitmap
     __shared__ int s_n;
     u64 *const mass = nuc_dyn;
-    u32 *const list = reinterpret_cast<u32 *>(nuc_dyn + NUC_BINS), *const bm = list + PARTS_SEEN * PARTS_BLOCK;
+    u32 *const list = reinterpret_cast<u32 *>(nuc_dyn + NUC_BINS + NUC_BEYOND), *const bm = list + PARTS_SEEN * PARTS_BLOCK;
     const int tid = threadIdx.x;
     Part p = part_of(a, pa);
     if (!part_bins(p.r, pa)) return;                                 // workgroup-uniform
     const NucRow &r = p.r;
     const float scale32 = r.scale * 2.3283064365386963e-10f, nsbin = -r.sbin;
+    const float beyond = (float)(NUC_BINS - 1 + lane_id());          // (see nucleus_row_body)
+    auto bin = [&](float x) { return (int)__builtin_amdgcn_fmed3f(x * nsbin, 0.0f, beyond); };
     auto put = [&](float z, bool minus) {
-        const float x = z - r.m;
-        const u64 q = qfix32(expneg_core(__builtin_amdgcn_fmed3f(x, -87.0f, 0.0f)), scale32);
-        const int b = (int)__builtin_amdgcn_fmed3f(x * nsbin, 0.0f, (float)(NUC_BINS - 1));
-        atomicAdd(&mass[b], minus ? 0ull - q : q);
+        const float x = __builtin_amdgcn_fmed3f(z - r.m, -87.0f, 0.0f);
+        const u64 q = qfix32(expneg_core(x), scale32);
+        atomicAdd(&mass[bin(x)], minus ? 0ull - q : q);
     };
     auto prologue = [&]() {
-        for (int i = tid; i < NUC_BINS; i += PARTS_BLOCK) mass[i] = 0ull;
+        for (int i = tid; i < NUC_BINS + NUC_BEYOND; i += PARTS_BLOCK) mass[i] = 0ull;
         if (r.penal) {
             PartSeen seen;
             part_history(a, p, false, bm, list, &s_n, seen);         // (its barriers stand behind the bins' zeros)
@@ -205,9 +206,9 @@ __global__ __launch_bounds__(PARTS_BLOCK, 4) void nucleus_parts_masses_kernel(Sa
     double start = mass_sum_start(a.mass_shift);
     mass_sum_begin(start);
     auto add = [&](float z) {
-        const float x = z - r.m;
-        const u64 q = mass_of(expneg_core(__builtin_amdgcn_fmed3f(x, -87.0f, 0.0f)), start);
-        atomicAdd(&mass[(int)__builtin_amdgcn_fmed3f(x * nsbin, 0.0f, (float)(NUC_BINS - 1))], q);
+        const float x = __builtin_amdgcn_fmed3f(z - r.m, -87.0f, 0.0f);
+        const u64 q = mass_of(expneg_core(x), start);
+        atomicAdd(&mass[bin(x)], q);
     };
     if (r.T == 1.0f) nuc_foreach<PARTS_BLOCK, false, true, true>(r, bm, [&](int, float y) { add(y); }, prologue);
     else nuc_foreach<PARTS_BLOCK, false, true, true>(r, bm, [&](int, float y) { add(nuc_z_shortcut<true>(r, y)); }, prologue);
@@ -215,8 +216,10 @@ __global__ __launch_bounds__(PARTS_BLOCK, 4) void nucleus_parts_masses_kernel(Sa
     __syncthreads();
     const long long part = (long long)blockIdx.x * pa.parts + blockIdx.y;
     u64 *const out = pa.bins + part * NUC_BINS, *const sums = pa.runs + part * PARTS_RUNS;
+    u64 more = 0ull;
+    if (tid >= PARTS_BLOCK - WAVE) more = wave_inclusive_scan_u64(mass[NUC_BINS + lane_id()]);   // (one wave: its last lane has the last bin)
     for (int i = tid; i < NUC_BINS; i += PARTS_BLOCK) {              // a wave: a run of bins
-        const u64 q = mass[i];
+        const u64 q = mass[i] + (i == NUC_BINS - 1 ? more : 0ull);
         out[i] = q;
         const u64 s = wave_inclusive_scan_u64(q);
         if (lane_id() == WAVE - 1) sums[i / PARTS_RUN] = s;
@@ -525,7 +528,7 @@ __global__ __launch_bounds__(PARTS_BLOCK, 4) void nucleus_parts_draw_kernel(Samp
 }
 
 static size_t parts_max_lds(int len) { return sizeof(u32) * (size_t)(PARTS_SEEN * PARTS_BLOCK + (len + 31) / 32); }
-static size_t parts_masses_lds(int len) { return sizeof(u64) * NUC_BINS + parts_max_lds(len); }
+static size_t parts_masses_lds(int len) { return sizeof(u64) * (NUC_BINS + NUC_BEYOND) + parts_max_lds(len); }
 static size_t parts_gather_lds(int len) { return sizeof(u64) * NucGeom<PARTS_BLOCK>::WAVES * NucGeom<PARTS_BLOCK>::WCAP + parts_max_lds(len); }
 
 static size_t parts_bytes(size_t parts) {

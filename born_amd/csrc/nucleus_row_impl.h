@@ -34,6 +34,7 @@ namespace born {
 // 512 (two workgroups per CU: one row's sweeps that wait for memory overlap the other's sweep that computes; for
 // batches of more rows than the device has CUs). The geometry below follows from it.
 constexpr int NUC_BINS = 4096;
+constexpr int NUC_BEYOND = WAVE;              // slots behind the bins, which a lane's logits beyond the last bin take each for itself
 constexpr int NUC_DIRECT = 32;                // listed entries that sum what ranks above them directly
 template <int BLOCK>
 struct NucGeom {
@@ -392,7 +393,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     __shared__ u64 s_win[2], s_mass[2], s_slot0[2];
     __shared__ u32 s_wcount[NUC_WAVES], s_top[2], s_low[2];
 
-    u64 *const mass = nuc_dyn;                                                   // [NUC_BINS] masses, then cumulative
+    u64 *const mass = nuc_dyn;                                                   // [NUC_BINS] masses, then cumulative; [NUC_BEYOND] more until the scan, in the lists
     uint2 *const stage = reinterpret_cast<uint2 *>(nuc_dyn + NUC_BINS);          // [NUC_WAVES][NUC_WCAP] (logit bits, id)
     u64 *const fkey = nuc_dyn + NUC_BINS + NUC_WAVES * NUC_WCAP;                 // [NUC_CAP] rank keys of the gathered entries
     u64 *const fq = fkey + NUC_CAP;                                              // [NUC_CAP] mass | slot << 62
@@ -434,7 +435,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     auto prologue = [&]() {
         if (r.penal)
             for (int i = tid; i < ((V + 31) >> 5); i += NUC_BLOCK) bm[i] = 0u;
-        for (int i = tid; i < NUC_BINS; i += NUC_BLOCK) mass[i] = 0ull;
+        for (int i = tid; i < NUC_BINS + NUC_BEYOND; i += NUC_BLOCK) mass[i] = 0ull;
         if (tid == 0) {
             s_n = 0;
             s_over = 0;
@@ -560,12 +561,16 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     // stored logit may exceed the penalised maximum: clamped to x = 0, some mass that the correction takes out again.
     const float nsbin = -r.sbin;
     const float scale32 = r.scale * 2.3283064365386963e-10f;
+    // What lies beyond the bins (masked logits; all of a row far below one logit) goes to a slot behind them that is the lane's own, and from there to the last
+    // bin: LDS atomics of 64 lanes on one bin are done one after the other.  us, all in the last bin and now, rows of which a mask leaves a tenth, then ordinary rows:
+    // 8 x 50 257 53.2 21.7, 24.0 23.9; 64 x 32 000 37.7 17.5, 19.5 19.4; 128 x 152 064 146 51, 53 52; in parts 32 x 128 256 36.6 27.0, 27.0 27.0.
+    const float beyond = (float)(NUC_BINS - 1 + lane_id());
+    auto lin_bin = [&](float x) { return (int)__builtin_amdgcn_fmed3f(x * nsbin, 0.0f, beyond); };   // (x from -87 to 0; the bins end at -32 or above)
     auto lin_z = [&](float y) { return r.T == 1.0f ? y : nuc_z_shortcut<ANY_T>(r, y); };
     auto lin_put = [&](float z, auto minus) {
-        const float x = z - r.m;
-        const u64 q = qfix32(expneg_core(__builtin_amdgcn_fmed3f(x, -87.0f, 0.0f)), scale32);
-        const int b = (int)__builtin_amdgcn_fmed3f(x * nsbin, 0.0f, (float)(NUC_BINS - 1));
-        atomicAdd(&mass[b], decltype(minus)::value ? 0ull - q : q);
+        const float x = __builtin_amdgcn_fmed3f(z - r.m, -87.0f, 0.0f);
+        const u64 q = qfix32(expneg_core(x), scale32);
+        atomicAdd(&mass[lin_bin(x)], decltype(minus)::value ? 0ull - q : q);
     };
     typedef std::integral_constant<bool, false> Plus;
     typedef std::integral_constant<bool, true> Minus;
@@ -594,9 +599,9 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
             double start = mass_sum_start(a.mass_shift);
             mass_sum_begin(start);
             auto put = [&](float z) {
-                const float x = z - r.m;
-                const u64 q = mass_of(expneg_core(__builtin_amdgcn_fmed3f(x, -87.0f, 0.0f)), start);
-                atomicAdd(&mass[(int)__builtin_amdgcn_fmed3f(x * nsbin, 0.0f, (float)(NUC_BINS - 1))], q);
+                const float x = __builtin_amdgcn_fmed3f(z - r.m, -87.0f, 0.0f);
+                const u64 q = mass_of(expneg_core(x), start);
+                atomicAdd(&mass[lin_bin(x)], q);
             };
             if (r.T == 1.0f) sweep_plain(Cached(), [&](int, float y) { put(y); }, kept);
             else sweep_plain(Cached(), [&](int, float y) { put(nuc_z_shortcut<ANY_T>(r, y)); }, kept);
@@ -638,6 +643,14 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         for (int t = 0; t < NUC_PER; t++) {
             local += mass[tid * NUC_PER + t];
             v[t] = local;
+        }
+        static_assert(NUC_BEYOND == WAVE && NUC_BEYOND <= NUC_WAVES * NUC_WCAP, "a slot to each lane, in the lists' storage");
+        if (tid >= NUC_BLOCK - WAVE) {                               // (one wave: its last lane has the last bin)
+            const u64 more = wave_inclusive_scan_u64(mass[NUC_BINS + lane_id()]);
+            if (tid == NUC_BLOCK - 1) {
+                local += more;
+                v[NUC_PER - 1] = local;
+            }
         }
         const u64 excl = block_inclusive_scan_u64<NUC_BLOCK, true>(local, &scr, &Zk) - local;
 #pragma unroll

@@ -31,3 +31,38 @@ def test_draws(oracle, V, p, path):
     want = oracle.sample(x, u, 0.8, 0, p, 1.2, hist, mode=oracle.MODE_FIXED)
     assert np.array_equal(got["tokens"], want["tokens"])
     assert np.array_equal(got["probs"].view(np.uint32), want["probs"].view(np.uint32))
+
+
+@pytest.mark.parametrize("B,V", [(8, 50257), (300, 28676), (3, 100003)])    # 1024 and 512 threads to a row; rows in parts
+def test_logits_without_mass_do_not_queue(oracle, B, V):
+    """Rows of a mask that leaves one logit in ten, and rows of one logit far above the others: what lies beyond the bins of masses is added up apart, so that they take no
+    longer than rows of a model (2.2 times as long where all of it was added to one bin, and longer the longer the row)."""
+    import time
+
+    from born_amd import sampler as S
+    rng = np.random.default_rng(V)
+    plain = (2 * rng.standard_normal((B, V))).astype(np.float32)
+    masked = np.where(rng.random((B, V)) < 0.9, np.float32(-np.inf), plain)
+    peak = plain.copy()
+    peak[:, V // 2] += 60
+    u = rng.random(B).astype(np.float32)
+    for T in (1.0, 0.7):
+        s = S.NewSampler(S.SamplerConfig(Temperature=T, TopP=0.95), max_batch=B, max_vocab=V)
+        du, tok, prob = S.DeviceBuffer.from_numpy(u), S.DeviceBuffer(4 * B), S.DeviceBuffer(4 * B)
+        took = []
+        for x in (plain, masked, peak):
+            dx = S.DeviceBuffer.from_numpy(x)
+            best = np.inf
+            for _ in range(12):
+                s.Status()                                  # (waits)
+                t0 = time.perf_counter()
+                for _ in range(40):
+                    s.Sample(dx, B, V, None, None, du, tok, prob)
+                s.Status()
+                best = min(best, time.perf_counter() - t0)
+            took.append(best)
+            want = oracle.sample(x[:4], u[:4], T, 0, 0.95, 1.0, None, mode=oracle.MODE_FIXED)
+            assert np.array_equal(tok.to_numpy(np.int32, (B,))[:4], want["tokens"])
+            assert np.array_equal(prob.to_numpy(np.uint32, (B,))[:4], want["probs"].view(np.uint32))
+        s.Close()
+        assert max(took[1:]) <= 1.5 * took[0], took
