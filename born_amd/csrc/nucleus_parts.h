@@ -12,6 +12,7 @@
 //   draw     a workgroup per row puts the lists in rank order, finds the cut and draws.
 // Rows that are not "usual" (the same test as in the one-workgroup kernel, but any temperature: ANY_T) and lists that overflow
 // are the last launch's, which runs the one-workgroup body for them.  The bits are the same on every route: integer sums, and exact rank keys.
+#include "nucleus_plan.h"
 
 namespace born {
 
@@ -19,21 +20,8 @@ constexpr int PARTS_BLOCK = 1024;
 constexpr int PARTS_RUN = WAVE, PARTS_RUNS = NUC_BINS / PARTS_RUN;   // runs of bins
 constexpr int PARTS_LIST = 512;               // gathered entries of a part
 constexpr int PARTS_CAP = PARTS_BLOCK;        // of a row
-constexpr int PARTS_ROW_MAX = 32;             // parts of a row
 constexpr int PARTS_SEEN = 4;                 // seen ids a thread keeps: histories of at most 4096 tokens
 constexpr int PARTS_TOTAL = 256;              // of a batch, at most
-constexpr int PARTS_LEAST = 4096;             // logits of a part, about: one 128-bit load per thread
-// Parts pay where the logits that a row's own workgroup is spared, V - V / parts, reach a number; two parts, whose batch keeps the device busy either way, only
-// from twice the row.  us, one workgroup to a row and parts, top-p 0.95 at T = 0.8 (rows, and so parts: 1 of 32, 32 of 8, 42 of 6, 64 of 4, 85 of 3, 128 of 2):
-//               1            32           42           64           85           128
-//     57 000    24.7 24.0    25.5 25.3    25.5 25.3    25.6 25.4    (not cut: 25.6)
-//     66 001    26.4 24.2    27.8 26.3    27.6 26.8    27.7 28.6    28.5 30.5    28.7 34.6
-//     80 000    28.8 24.3    30.1 26.2    30.1 27.6    29.9 29.2    30.2 31.3    32.1 38.1
-//    100 003    34.1 24.4    35.2 27.0    34.7 28.8    34.8 30.8    36.5 35.1    39.7 44.4
-//    152 064    45.0 25.2    46.1 29.1    46.5 31.5    48.2 37.6    50.9 44.6    53.4 56.1
-//    250 000    66.5 25.4    66.9 32.5    73.7 40.4    76.8 49.9    78.6 60.6    83.7 79.6
-// Four launches, chains of memory and LDS round trips each.
-constexpr int PARTS_FROM = 49152, PARTS_SPARED = 60000, PARTS_TWO_FROM = 196608;
 static_assert(PARTS_RUNS == WAVE, "one lane per run, one per bin of a run");
 static_assert(PARTS_ROW_MAX * PARTS_RUN <= 2 * PARTS_BLOCK && PARTS_ROW_MAX <= WAVE, "sums over parts");
 
@@ -202,7 +190,7 @@ __global__ __launch_bounds__(PARTS_BLOCK, 4) void nucleus_parts_masses_kernel(Sa
             lds_barrier();
         }
     };
-    static_assert(PARTS_FROM >= 1024, "mass_of's shift");
+    static_assert(PARTS_SPARED >= 1024, "mass_of's shift");
     double start = mass_sum_start(a.mass_shift);
     mass_sum_begin(start);
     auto add = [&](float z) {
@@ -556,11 +544,9 @@ int nucleus_workspace_parts(int64_t max_batch) { return (int)std::min<int64_t>(P
 size_t nucleus_workspace_bytes(int parts) { return parts_bytes((size_t)parts); }
 // Whether a batch's rows are cut into parts, and into how many (below 2: not).
 static int parts_of(const SampleArgs &a, bool two_per_cu, int most) {
-    if (two_per_cu || a.V < PARTS_FROM || a.hist_counts || a.hist_stride > PARTS_SEEN * PARTS_BLOCK) return 0;
+    if (two_per_cu || a.hist_counts || a.hist_stride > PARTS_SEEN * PARTS_BLOCK) return 0;
     if (a.dcut != 80.0f) return 0;                                   // (a min-p bound is for the one-workgroup body)
-    const int parts = std::min(std::min(std::min(most, device_cu_count()) / a.B, PARTS_ROW_MAX), a.V / PARTS_LEAST);
-    if (parts < 2 || a.V - a.V / parts < PARTS_SPARED || (parts == 2 && a.V < PARTS_TWO_FROM)) return 0;
-    return parts;
+    return row_parts(a.V, a.B, std::min(most, device_cu_count()));
 }
 bool nucleus_wants_parts(const SampleArgs &a, bool two_per_cu) { return parts_of(a, two_per_cu, PARTS_TOTAL) >= 2; }
 static bool parts_plan(const SampleArgs &a, bool two_per_cu, const NucleusWorkspace &ws, PartsArgs &pa) {

@@ -34,8 +34,10 @@ def test_lists_of_equal_logits(oracle, V, ties, p, path):
         assert np.array_equal(got["probs"].view(np.uint32), want["probs"].view(np.uint32))
 
 
-@pytest.mark.parametrize("B,V", [(3, 64285), (3, 64286), (64, 79999), (64, 80000), (85, 89999), (85, 90000), (128, 196607), (128, 196608)])
+@pytest.mark.parametrize("B,V", [(3, 54165), (3, 54166), (32, 57141), (32, 57142), (42, 59998), (42, 59999), (51, 74998), (51, 74999), (64, 79998), (64, 79999), (85, 89998), (85, 89999),
+                                 (128, 196607), (128, 196608)])
 def test_rows_around_the_shortest_that_are_cut(oracle, B, V):
+    """The sizes of tests/test_nucleus_plan.py, which holds that one of each pair is cut."""
     from born_amd import sampler as S
     rng = np.random.default_rng(B + V)
     x = (2 * rng.standard_normal((4, V))).astype(np.float32)
