@@ -564,8 +564,9 @@ hipError_t launch_conv2d(const float *in, const float *ker, float *out, int N, i
     const int cog = waves1 >= 4 * 2048 ? 4 : waves1 >= 2 * 2048 ? 2 : 1;
     if (KH == KW && (KW == 3 || KW == 5) && padding == 0 && P < (1ll << 31) && CO <= 65535) {
         // (waves of one channel a lane, us with one, two and four: 560 5.1 7.3 9.9, 1400 10.4 12.3 17.6, 1984 5.8 6.2 8.3, 3200 6.6 5.7 6.6, 4096 26.3 20.1 26.8,
-        // 14 464 22.0 13.2 10.9, 18 432 6.0 4.5 4.3)
-        const int per = waves1 >= 8192 ? 4 : waves1 >= 3072 ? 2 : 1;
+        // 14 464 22.0 13.2 10.9, 18 432 6.0 4.5 4.3; never more than there are output channels: [693,32,32,32] * [1,32,5,5] 52 one, 78 four, [346,32,32,32] * [2,32,5,5]
+        // 34 two, 47 four)
+        const int per = waves1 >= 8192 && CO > 2 ? 4 : waves1 >= 3072 && CO > 1 ? 2 : 1;
         if (KW == 5 && per == 4) return launch_conv2d_square<5, 4>(blocks, st, in, ker, out, C, H, W, CO, HO, WO, stride, (u32)P);
         if (KW == 5 && per == 2) return launch_conv2d_square<5, 2>(blocks, st, in, ker, out, C, H, W, CO, HO, WO, stride, (u32)P);
         if (KW == 5) return launch_conv2d_square<5, 1>(blocks, st, in, ker, out, C, H, W, CO, HO, WO, stride, (u32)P);

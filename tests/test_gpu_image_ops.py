@@ -9,7 +9,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("N,C,H,W,CO,K,stride", [
     (1, 1, 5, 5, 1, 5, 1), (1, 1, 3, 3, 3, 3, 1), (3, 2, 7, 9, 5, 5, 1), (2, 3, 8, 8, 6, 3, 2), (5, 5, 12, 11, 7, 5, 3), (9, 4, 20, 20, 33, 5, 1), (40, 2, 20, 20, 21, 5, 1),
-    (64, 1, 28, 28, 32, 5, 1), (16, 3, 34, 34, 50, 3, 1), (17, 6, 30, 30, 11, 3, 1), (64, 32, 12, 12, 64, 5, 1)])
+    (64, 1, 28, 28, 32, 5, 1), (16, 3, 34, 34, 50, 3, 1), (17, 6, 30, 30, 11, 3, 1), (64, 32, 12, 12, 64, 5, 1), (270, 2, 32, 32, 1, 5, 1), (720, 1, 32, 32, 1, 3, 1),
+    (360, 1, 32, 32, 2, 5, 1), (320, 2, 32, 32, 2, 3, 1), (240, 2, 32, 32, 3, 5, 1)])
 def test_convolution(oracle, N, C, H, W, CO, K, stride):
     from born_amd import backend as BK
     rng = np.random.default_rng(N * 1000 + CO)
