@@ -10,7 +10,6 @@ with the reference's panic text ("add: shapes not compatible for broadcasting: .
 
 """
 import ctypes as C
-import functools
 import math
 
 import numpy as np
@@ -25,14 +24,36 @@ class BackendPanic(SamplerPanic):
 
 # A program's operations come with the same few shapes at every pass: their arrays, which the library only reads, and the shapes of results are
 # worked out once each (a pass of an MNIST network of 64 images: 143 us, 153 when every operation made its own).
-@functools.lru_cache(maxsize=1024)
+_arrays, _results = {}, {}
+_KEPT = 1024                                                         # of either, at most
+
+
+def _keep(kept, key, value):
+    try:
+        if len(kept) >= _KEPT:
+            kept.clear()
+        kept[key] = value
+    except TypeError:                                                # (a shape that was set to a list is not kept)
+        pass
+    return value
+
+
 def _shape_arr(shape):
-    return (C.c_int64 * max(len(shape), 1))(*shape)
+    try:
+        return _arrays[shape]
+    except (KeyError, TypeError):
+        return _keep(_arrays, shape, (C.c_int64 * max(len(shape), 1))(*shape))
 
 
-@functools.lru_cache(maxsize=1024)
 def _broadcast(a, b):
     """The shape of an element-wise result of two shapes of one length; None where the library is asked (and says what is wrong)."""
+    try:
+        return _results[a, b]
+    except (KeyError, TypeError):
+        return _keep(_results, (a, b), _broadcast_shape(a, b))
+
+
+def _broadcast_shape(a, b):
     if len(a) != len(b) or not a:
         return None
     out = []
