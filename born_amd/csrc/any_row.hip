@@ -2,9 +2,9 @@
 // single-pass body (topk_row_impl.h), the three-sweep body (nucleus_row_impl.h) or the general kernel's.
 //
 // Up to a row per CU.  As two launches, one for the rows with a small top-k and one for the others, each leaves the CUs of the
-// other's rows idle and a step takes the sum of the slowest row of either; in one it takes the larger.  Two launches and one, us, half
-// of the rows with a top-k of up to 100: 96 x 100 003 72.6 and 51.3, 8 x 32 000 41.0 and 26.2, 32 x 128 256 80.5 and 58.7,
-// 128 x 50 000 52.3 and 35.7 (with the three-sweep body of then; the first 41.2 now).  Bound by the slowest row's three sweeps on one CU.  (Registers are spilled in the general kernel's body,
+// other's rows idle and a step takes the sum of the slowest row of either; in one it takes the larger.  In one launch, us, half
+// of the rows with a top-k of up to 100 (two launches, with the three-sweep body of then, and one, with it and now): 96 x 100 003 72.6 51.3 40.4, 8 x 32 000 41.0 26.2 22.9, 32 x 128 256
+// 80.5 58.7 46.8, 128 x 50 000 52.3 35.7 28.2.  Bound by the slowest row's three sweeps on one CU.  (Registers are spilled in the general kernel's body,
 // as in nucleus_or_general_rows_kernel: the others take what they take alone.)  More rows than CUs keep the kernels of their own:
 // a CU holds one workgroup of this one, two of theirs.  Occurrence tables too: an instance with them would double the code.
 #include "nucleus_row_impl.h"

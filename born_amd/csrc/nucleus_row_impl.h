@@ -13,7 +13,7 @@
 //   resolve  the gathered entries are put in rank order through buckets, one scan of their masses gives every entry
 //            the mass at and above it within its bin (a short list: summed directly); the first entry in rank
 //            order whose cumulative mass reaches a target is the one whose own mass crosses it.
-// A wanted bin too full for the lists (heavy ties, masked rows) is refined in place by a radix descent over
+// A wanted bin too full for the lists (heavy ties) is refined in place by a radix descent over
 // the rank keys of that bin, 11 bits per sweep.
 // In the usual row (a maximum of ordinary size, a temperature whose division has the three-instruction shortcut, no
 // min-p bound, a history short enough to be listed) sweeps 2 and 3 read the logits as stored: no history bitmap, no
@@ -528,7 +528,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
             mx = fmaxf(mx, y);
             if ((j & 3) == 0) mn = fminf(mn, y > -3.402823466e+38f ? y : INFINITY);
         }, prologue, fill());
-            mx = block_max_f32<NUC_BLOCK, true>(mx, &scr);
+        mx = block_max_f32<NUC_BLOCK, true>(mx, &scr);
         mn = -block_max_f32<NUC_BLOCK, true>(-mn, &scr);
         r.m = uniform_f32(nuc_z(r, mx));
         r.degenerate = r.m == -INFINITY;                             // nothing finite: every d is 0 by definition
@@ -856,9 +856,8 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         if (tid < n) mine = incl - s_slot0[myslot];
     }
     // ---- the cut, then the draw: each is the first element in rank order of one bin at which the cumulative
-    // mass reaches a target.  A bin that is listed is resolved from `mine`; any other bin (the lists overflowed:
-    // heavy ties, masked rows; or the draw's bin was not the predicted one) by a radix descent over the rank
-    // keys of that bin, 11 bits per sweep, until its bucket fits the list.
+    // mass reaches a target.  Listed bins are resolved from `mine`; where the lists overflowed (heavy ties), each by a radix
+    // descent over the rank keys of its bin, 11 bits per sweep, until its bucket fits the list.
     r.masked = false;                                                // (the sweeps of a radix descent apply the penalties themselves)
     u64 Zp = Zk, tokkey = 0ull;
     u64 *const smass = reinterpret_cast<u64 *>(stage);               // [2048] sub-histogram of masses

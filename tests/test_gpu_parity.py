@@ -888,9 +888,8 @@ def test_three_sweep_kernel_seen_logits_above_the_penalised_maximum(oracle, rocm
 @pytest.mark.parametrize("V,peaks,lift", [(4096, 3, 14.0), (32000, 20, 9.0), (50000, 200, 6.0), (128256, 20, 9.0), (20000, 700, 7.0)])
 def test_three_sweep_kernel_peaked_rows_gather_the_nucleus_whole(oracle, rocm, V, peaks, lift, path):
     """Top-p alone on peaked rows (what a trained model emits): a few lifted logits carry nearly all of the mass, the
-    cut's bin holds so much of it that the draw's bin cannot be predicted, and the kernel gathers the whole nucleus
-    (every bin down to the cut's) when the bins' masses bound its size by half the list. From a handful of peaks to
-    more than the bound allows (the row then takes the older route), with and without penalties on the peaks
+    cut's bin holds so much of it that the draw may fall into any of many bins, all of which the kernel gathers with the
+    cut's. From a handful of peaks to more than the lists hold (the row then takes the radix descent), with and without penalties on the peaks
     themselves: bit-exact against the oracle."""
     rng = np.random.default_rng(V + peaks)
     B = 12
