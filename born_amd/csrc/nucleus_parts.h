@@ -168,7 +168,7 @@ __global__ __launch_bounds__(PARTS_BLOCK, 4) void nucleus_parts_masses_kernel(Sa
     if (!part_bins(p.r, pa)) return;                                 // workgroup-uniform
     const NucRow &r = p.r;
     const float scale32 = r.scale * 2.3283064365386963e-10f, nsbin = -r.sbin;
-    const float beyond = (float)(NUC_BINS - 1 + lane_id());          // (see nucleus_row_body)
+    const float beyond = (float)(NUC_BINS - 1 + (lane_id() & (NUC_BEYOND - 1)));          // (see nucleus_row_body)
     auto bin = [&](float x) { return (int)__builtin_amdgcn_fmed3f(x * nsbin, 0.0f, beyond); };
     auto put = [&](float z, bool minus) {
         const float x = __builtin_amdgcn_fmed3f(z - r.m, -87.0f, 0.0f);
@@ -205,7 +205,10 @@ __global__ __launch_bounds__(PARTS_BLOCK, 4) void nucleus_parts_masses_kernel(Sa
     const long long part = (long long)blockIdx.x * pa.parts + blockIdx.y;
     u64 *const out = pa.bins + part * NUC_BINS, *const sums = pa.runs + part * PARTS_RUNS;
     u64 more = 0ull;
-    if (tid >= PARTS_BLOCK - WAVE) more = wave_inclusive_scan_u64(mass[NUC_BINS + lane_id()]);   // (one wave: its last lane has the last bin)
+    if (tid == PARTS_BLOCK - 1) {                                    // (the last bin's)
+#pragma unroll
+        for (int i = 0; i < NUC_BEYOND; i++) more += mass[NUC_BINS + i];
+    }
     for (int i = tid; i < NUC_BINS; i += PARTS_BLOCK) {              // a wave: a run of bins
         const u64 q = mass[i] + (i == NUC_BINS - 1 ? more : 0ull);
         out[i] = q;

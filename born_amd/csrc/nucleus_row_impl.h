@@ -34,7 +34,7 @@ namespace born {
 // 512 (two workgroups per CU: one row's sweeps that wait for memory overlap the other's sweep that computes; for
 // batches of more rows than the device has CUs). The geometry below follows from it.
 constexpr int NUC_BINS = 4096;
-constexpr int NUC_BEYOND = WAVE;              // slots behind the bins, which a lane's logits beyond the last bin take each for itself
+constexpr int NUC_BEYOND = 16;                // slots behind the bins, for what lies beyond the last one
 constexpr int NUC_DIRECT = 32;                // listed entries that sum what ranks above them directly
 template <int BLOCK>
 struct NucGeom {
@@ -438,7 +438,8 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     auto prologue = [&]() {
         if (r.penal)
             for (int i = tid; i < ((V + 31) >> 5); i += NUC_BLOCK) bm[i] = 0u;
-        for (int i = tid; i < NUC_BINS + NUC_BEYOND; i += NUC_BLOCK) mass[i] = 0ull;
+        for (int i = tid; i < NUC_BINS; i += NUC_BLOCK) mass[i] = 0ull;
+        if (tid < NUC_BEYOND) mass[NUC_BINS + tid] = 0ull;
         if (tid == 0) {
             s_n = 0;
             s_over = 0;
@@ -564,10 +565,11 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
     // stored logit may exceed the penalised maximum: clamped to x = 0, some mass that the correction takes out again.
     const float nsbin = -r.sbin;
     const float scale32 = r.scale * 2.3283064365386963e-10f;
-    // What lies beyond the bins (masked logits; all of a row far below one logit) goes to a slot behind them that is the lane's own, and from there to the last
+    // What lies beyond the bins (masked logits; all of a row far below one logit) goes to the last bin or one of the slots behind it by lane, which the scan adds to the last
     // bin: LDS atomics of 64 lanes on one bin are done one after the other.  us, all in the last bin and now, rows of which a mask leaves a tenth, then ordinary rows:
-    // 8 x 50 257 53.2 21.7, 24.0 23.9; 64 x 32 000 37.7 17.5, 19.5 19.4; 128 x 152 064 146 51, 53 52; in parts 32 x 128 256 36.6 27.0, 27.0 27.0.
-    const float beyond = (float)(NUC_BINS - 1 + lane_id());
+    // 8 x 50 257 53.2 21.4, 24.0 23.9; 64 x 32 000 37.7 17.2, 19.1 18.9; 128 x 152 064 146 51, 53 52; 512 x 8191 23.8 14.8, 15.1 15.4; in parts 32 x 128 256 36.6 27.0, 27.0 27.0.
+    // (64 x 32 000 with 64 slots 17.1, with 8 17.7, 4 20.6.)
+    const float beyond = (float)(NUC_BINS - 1 + (lane_id() & (NUC_BEYOND - 1)));
     auto lin_bin = [&](float x) { return (int)__builtin_amdgcn_fmed3f(x * nsbin, 0.0f, beyond); };   // (x from -87 to 0; the bins end at -32 or above)
     auto lin_z = [&](float y) { return r.T == 1.0f ? y : nuc_z_shortcut<ANY_T>(r, y); };
     auto lin_put = [&](float z, auto minus) {
@@ -647,13 +649,11 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
             local += mass[tid * NUC_PER + t];
             v[t] = local;
         }
-        static_assert(NUC_BEYOND == WAVE && NUC_BEYOND <= NUC_WAVES * NUC_WCAP, "a slot to each lane, in the lists' storage");
-        if (tid >= NUC_BLOCK - WAVE) {                               // (one wave: its last lane has the last bin)
-            const u64 more = wave_inclusive_scan_u64(mass[NUC_BINS + lane_id()]);
-            if (tid == NUC_BLOCK - 1) {
-                local += more;
-                v[NUC_PER - 1] = local;
-            }
+        static_assert(NUC_BEYOND <= NUC_WAVES * NUC_WCAP, "in the lists' storage");
+        if (tid == NUC_BLOCK - 1) {
+#pragma unroll
+            for (int i = 0; i < NUC_BEYOND; i++) local += mass[NUC_BINS + i];
+            v[NUC_PER - 1] = local;
         }
         const u64 excl = block_inclusive_scan_u64<NUC_BLOCK, true>(local, &scr, &Zk) - local;
 #pragma unroll
@@ -682,6 +682,7 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
 
     BORN_STAMP(a, row, 4);
     // ---- sweep 3: stage the logits inside the wanted bins' ranges, then classify them exactly
+    bool listed;
     {
         // The cut's bin, and above it (w2 <= w0) the draw's; one interval where the two meet.
         float lo0, hi0, lo1, hi1, lo2, hi2;
@@ -720,45 +721,48 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         const u32 count = staged.size();
         if (count > (u32)NUC_WCAP && lane_id() == 0) s_over = 1;
         const int cw = (int)min(count, (u32)NUC_WCAP);
-        for (int e0 = 0; e0 < cw; e0 += WAVE) {
-            const int e = e0 + lane_id();
-            bool take = false;
-            u64 key = 0ull, qs = 0ull;
-            if (e < cw) {
-                uint2 c = staged.at[e];
-                bool stale = false;                                  // a seen id's stored logit
-                if (lin && r.penal) {
-                    if (c.y & 0x80000000u) c.y &= 0x7FFFFFFFu;
-                    else stale = (bm[c.y >> 5] >> (c.y & 31)) & 1u;
+        auto classify = [&]() {
+            for (int e0 = 0; e0 < cw; e0 += WAVE) {
+                const int e = e0 + lane_id();
+                bool take = false;
+                u64 key = 0ull, qs = 0ull;
+                if (e < cw) {
+                    uint2 c = staged.at[e];
+                    bool stale = false;                                  // a seen id's stored logit
+                    if (lin && r.penal) {
+                        if (c.y & 0x80000000u) c.y &= 0x7FFFFFFFu;
+                        else stale = (bm[c.y >> 5] >> (c.y & 31)) & 1u;
+                    }
+                    const float z = nuc_z(r, __uint_as_float(c.x));
+                    const float d = nuc_d(r, z);
+                    const int b = nuc_bin(r, d);
+                    const int slot = stale ? -1 : b == w0 ? 0 : b >= w1 && b <= w2 ? 1 : -1;
+                    if (slot >= 0) {
+                        take = true;
+                        key = make_key64(z, (int)c.y);
+                        qs = qfix(expneg(d, r.dcut), r.scale) | ((u64)slot << 62);
+                    }
                 }
-                const float z = nuc_z(r, __uint_as_float(c.x));
-                const float d = nuc_d(r, z);
-                const int b = nuc_bin(r, d);
-                const int slot = stale ? -1 : b == w0 ? 0 : b >= w1 && b <= w2 ? 1 : -1;
-                if (slot >= 0) {
-                    take = true;
-                    key = make_key64(z, (int)c.y);
-                    qs = qfix(expneg(d, r.dcut), r.scale) | ((u64)slot << 62);
-                }
-            }
-            const u64 mk = __ballot(take);
-            if (mk) {
-                int base = 0;
-                if (lane_id() == 0) base = atomicAdd(&s_n, __popcll(mk));
-                base = __builtin_amdgcn_readfirstlane(base);
-                if (take) {
-                    const int pos = base + (int)__builtin_amdgcn_mbcnt_hi((u32)(mk >> 32), __builtin_amdgcn_mbcnt_lo((u32)mk, 0u));
-                    if (pos < NUC_CAP) {
-                        fkey[pos] = key;
-                        fq[pos] = qs;
+                const u64 mk = __ballot(take);
+                if (mk) {
+                    int base = 0;
+                    if (lane_id() == 0) base = atomicAdd(&s_n, __popcll(mk));
+                    base = __builtin_amdgcn_readfirstlane(base);
+                    if (take) {
+                        const int pos = base + (int)__builtin_amdgcn_mbcnt_hi((u32)(mk >> 32), __builtin_amdgcn_mbcnt_lo((u32)mk, 0u));
+                        if (pos < NUC_CAP) {
+                            fkey[pos] = key;
+                            fq[pos] = qs;
+                        }
                     }
                 }
             }
-        }
+        };
+        classify();
+        __syncthreads();
+        listed = !s_over && s_n <= NUC_CAP;                          // the wanted bins fit the lists
     }
-    __syncthreads();
     BORN_STAMP(a, row, 5);
-    const bool listed = !s_over && s_n <= NUC_CAP;                   // the wanted bins fit the lists
     const int n = listed ? s_n : 0;
     const int n4 = (n + 3) & ~3;                                     // the list padded to whole groups of four ..
     if (tid >= n && tid < n4) {
