@@ -761,6 +761,17 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         classify();
         __syncthreads();
         listed = !s_over && s_n <= NUC_CAP;                          // the wanted bins fit the lists
+        if (!listed && !s_over && w1 < w0) {
+            // (uniform) Equal logits may make w1 and w2 themselves as full as w0.  Where w0's alone fit, they are listed, and the draw's bin is left to the descent
+            // (us, both by the descent and so: logits of steps of 0.07, 200 x 50 257 153 98, 32 x 32 000 131 90, 200 x 128 256 244 155)
+            w1 = w2 = w0;
+            __syncthreads();
+            if (tid == 0) s_n = 0;
+            __syncthreads();
+            classify();
+            __syncthreads();
+            listed = s_n <= NUC_CAP;
+        }
     }
     BORN_STAMP(a, row, 5);
     const int n = listed ? s_n : 0;
@@ -863,8 +874,8 @@ __device__ __forceinline__ void nucleus_row_body(const SampleArgs &a, const floa
         if (tid < n) mine = incl - s_slot0[myslot];
     }
     // ---- the cut, then the draw: each is the first element in rank order of one bin at which the cumulative
-    // mass reaches a target.  Listed bins are resolved from `mine`; where the lists overflowed (heavy ties), each by a radix
-    // descent over the rank keys of its bin, 11 bits per sweep, until its bucket fits the list.
+    // mass reaches a target.  Listed bins are resolved from `mine`; a bin that is not (heavy ties: the lists overflowed, or the cut's alone were gathered) by a radix
+    // descent over its rank keys, 11 bits per sweep, until its bucket fits the list.
     r.masked = false;                                                // (the sweeps of a radix descent apply the penalties themselves)
     u64 Zp = Zk, tokkey = 0ull;
     u64 *const smass = reinterpret_cast<u64 *>(stage);               // [2048] sub-histogram of masses

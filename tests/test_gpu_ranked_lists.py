@@ -51,3 +51,21 @@ def test_rows_around_the_shortest_that_are_cut(oracle, B, V):
     want = oracle.sample(x[at], u[at], 0.8, 0, 0.95, 1.0, None, mode=oracle.MODE_FIXED)
     assert np.array_equal(got["tokens"][at], want["tokens"])
     assert np.array_equal(got["probs"][at].view(np.uint32), want["probs"].view(np.uint32))
+
+
+@pytest.mark.parametrize("B,V,step,T,p", [(32, 50257, 30, 0.8, 0.95), (32, 50257, 30, 1.9, 0.9), (200, 32000, 30, 1.9, 0.9), (512, 8191, 3, 1.0, 0.6), (512, 2048, 3, 1.9, 0.9)])
+def test_levels_of_which_one_fits_the_list(oracle, B, V, step, T, p):
+    """Logits of a few hundred equal ones each: where the cut's fit the lists but not the draw's beside them, the cut's are listed: no row is left to the descent for both."""
+    from born_amd import sampler as S
+    rng = np.random.default_rng(V)
+    x = (np.round(step * rng.standard_normal((B, V))) * (2 / step)).astype(np.float32)
+    u = rng.random(B).astype(np.float32)
+    s = S.NewSampler(S.SamplerConfig(Temperature=T, TopP=p), max_batch=B, max_vocab=V)
+    got = S.sample_host(s, x, u, None)
+    s.Status()
+    counters = s.Counters()
+    s.Close()
+    want = oracle.sample(x, u, T, 0, p, 1.0, None, mode=oracle.MODE_FIXED)
+    assert np.array_equal(got["tokens"], want["tokens"])
+    assert np.array_equal(got["probs"].view(np.uint32), want["probs"].view(np.uint32))
+    assert counters["fallback_rows"] == 0, counters
