@@ -117,7 +117,7 @@ __device__ __forceinline__ nuc_f32x4 nuc_load4_clamped(const float *x, int b, in
 // PLAIN: the caller knows that the row has no penalties (a loop of its own without the penalty code: the visitor's
 // test of r.penal at every visit cost the single-sweep kernel 5 %).
 // LOADS_FIRST: a stage's loads are issued before the visits of the one before, not among them, where the compiler spilled registers for them; off for
-// the sweep of token_logprob_kernel, which they held up (1024 x 152 064: 103 us, 100 without).
+// the sweep of token_logprob_kernel, whose single rows it holds up (1 x 50 257: 10.2 us, 9.9 without; 1024 x 152 064 101.5 and 101.9).
 // FIRST (AHEAD instances only): `first` holds the row's first stage, requested earlier with nuc_request_first, or
 // (NucKept) its first blocks, kept in registers from the first sweep on, which fills them (NucFill).
 struct NucNoFirst {};
