@@ -125,22 +125,32 @@ static bool small_pays_guarded(int M, int N, int K, bool b_transposed) {
         int k_max;
         if (M <= 4 && (!b_transposed || squares == 1 || squares > 3)) k_max = b_transposed || squares <= 16 ? 131072 : 32768;
         else if (b_transposed) k_max = squares < 4 ? 3584 : squares < 21 ? 6144 : squares < 42 ? 8448 : squares <= 256 ? 12288 : 4352;
-        else k_max = squares < 16 ? 24576 : squares <= 256 ? 8448 : 4352;
+        else k_max = squares < 16 ? 24576 : squares <= 256 ? 10240 : 4352;
         if (K > k_max) return false;
     }
     return N % 4 || squares <= (b_transposed ? 48000 : K > 32 ? 16384 : 3072);
 }
-// `tiles`: of the fp32 tiles.  whole: their loads need no guard.  Where K is a multiple of 32 and all aligned (us, theirs and here), columns that fill half a tile or less: 4096 x 1024 -> 64 21.1 13.1,
-// 2048 x 8192 -> 16 45 31, 512 x 4096 -> 64 16.8 17.0, 512 x 8192 -> 64 21.8 30.6, 1024 x 4096 -> 64 21.2 17.1, 1100 x 4096 -> 64 21.9 30.6, 1024 x 8192 -> 32 29.4 30.6; fewer tiles than would be left
-// unsliced: 64 x 2048 -> 1024 14.2 9.8, 308 x 1056 x 648 16.7 14.1, 89 x 1888 -> 1743 19.0 18.2, 64 x 4096 -> 4096 29.5 37.0, 55 x 64 x 1032 5.6 3.8, but few squares and a long
-// K, where slices put more CUs to work: 16 x 4096 -> 1000 13.2 16.8, 128 x 3072 -> 256 13.2 13.3, 128 x 4096 -> 256 15.1 16.7, 128 x 6144 -> 256 18.3 23.6.  More tiles: 2048 x 128 -> 512
-// 7.0 8.5, 7 x 320 -> 21 263 8.1 10.6.
+// `tiles`: of the fp32 tiles.  whole: their loads need no guard, K a multiple of 32 and all aligned.  us, theirs and here:
+//   columns that fill half a tile or less  4096 x 1024 -> 64 21.1 13.1, 2048 x 8192 -> 16 45 31, 512 x 4096 -> 64 16.8 17.0, 512 x 8192 -> 64 21.8 30.6, 1024 x 4096 -> 64 21.2 17.1, 1100 x 4096 -> 64
+//                     21.9 30.6, 1024 x 8192 -> 32 29.4 30.6
+//   more than 128 tiles, which are left unsliced  2048 x 128 -> 512 7.0 8.5, 7 x 320 -> 21 263 8.1 10.6
+//   few squares and a long K, where slices put more CUs to work  16 x 4096 -> 1000 13.2 16.8;   128 squares: 3072 13.2 13.3, 4096 15.1 16.7;   148: 22 x 4096 -> 1170 16.0 16.7;   183: 6 x 4096 -> 2928
+//                     17.1 13.5;   250: 14 x 3616 -> 4000 18.6 15.4
+//   257 to 384, a second round of CUs  17 x 960 -> 2594 10.5 9.5, 12 x 1408 -> 4456 12.4 12.0, 17 x 1440 -> 2524 11.8 14.0, 32 x 1888 -> 2076 14.0 17.1, 18 x 3808 -> 2301 19.5 30.0;   more than 32 rows:
+//                     64 x 1408 -> 1410 15.6 12.9, 40 x 1664 -> 1604 15.6 14.4, 64 x 2016 -> 1108 14.6 17.9
+//   385 to 512, four waves each  128 x 1472 -> 901 17.1 12.9, 17 x 1792 -> 3701 15.3 15.1, 24 x 1888 -> 3100 16.3 16.8, 20 x 2112 -> 3648 16.8 17.9
+//   above             20 x 960 -> 4587 12.2 12.9, 17 x 1056 -> 4696 12.5 15.3, 100 x 1504 -> 1329 17.7 19.5;   from 600 on in squares of 32: 200 x 1280 -> 766 17.0 13.8, 17 x 1568 -> 5009 15.6 16.2;   which up to 16
+//                     rows fill half: 6 x 384 -> 8728 8.0 5.8, 6 x 672 -> 10 967 11.3 12.1, 8 x 1568 -> 11 388 18.0 23.2
 bool gemm_small_pays(int M, int N, int K, bool b_transposed, bool whole, long long tiles) {
     if (!whole) return small_pays_guarded(M, N, K, b_transposed);
     const double products = (double)M * (double)N * (double)K;
     const long long squares = gemm_small_squares(M, N, 16);
     if (N <= 64 && products <= 3e8) return K <= 2048 || (M >= 1024 && squares >= 128 && (N <= 16 || (K <= 4096 && squares <= 256)));
-    return tiles < 128 && products <= 2.1e8 && (K <= 2048 || (K <= 3072 && squares >= 128 && squares <= 256));
+    if (tiles >= 128 || products > 2.1e8) return false;
+    if (squares <= 256) return K <= (squares < 128 ? 2048 : squares < 144 ? 3072 : 4096);
+    if (squares <= 384) return K <= (M > 32 ? 1700 : 1400);
+    if (squares <= 512) return K <= 2048;
+    return K <= (M <= 16 ? 640 : squares <= 600 ? 1000 : 1700);
 }
 
 }  // namespace born

@@ -95,8 +95,10 @@ def test_a_long_k_of_few_squares_is_left_to_the_tiles_slices(plan):
         assert not plan.small(M, K, N, 1, 0, 16), (M, K, N)
     for M, K, N in ((16, 40001, 16), (64, 20001, 64), (40, 12001, 100), (757, 6001, 94), (4, 100003, 700), (16, 1000001, 16)):
         assert not plan.small(M, K, N, 0, 0, 16), (M, K, N)
-    for M, K, N in ((128, 4096, 256), (512, 8192, 64), (1100, 4096, 64), (16, 4096, 1000)):                     # K a multiple of 32
+    for M, K, N in ((128, 4096, 256), (512, 8192, 64), (1100, 4096, 64), (16, 4096, 1000), (17, 1440, 2524), (18, 3808, 2301), (64, 2016, 1108), (17, 1056, 4696), (8, 1568, 11388)):   # K a multiple of 32
         assert not plan.small(M, K, N, 1, 1, 64) and not plan.small(M, K, N, 0, 1, 64), (M, K, N)
+    for M, K, N in ((6, 4096, 2928), (14, 3616, 4000), (17, 960, 2594), (64, 1408, 1410), (128, 1472, 901), (200, 1280, 766), (6, 384, 8728), (64, 2048, 1024)):
+        assert plan.small(M, K, N, 1, 1, 64) and plan.small(M, K, N, 0, 1, 64), (M, K, N)
     for M, K, N in ((16, 3211, 16), (64, 6001, 10), (40, 8193, 100), (200, 12001, 200), (400, 4097, 300), (911, 19590, 17), (3, 100003, 252)):
         assert plan.small(M, K, N, 1, 0, 16), (M, K, N)
     for M, K, N in ((16, 24001, 16), (64, 16001, 10), (40, 8193, 100), (256, 6001, 256), (3, 30001, 700)):
