@@ -19,7 +19,7 @@
 
 namespace born {
 
-// T: 16-row blocks of the square's side.  U: 128-bit loads of an operand's row per lane and chunk.  NW: waves.
+// T: 16-row blocks of the square's side.  U: 128-bit loads of an operand's row per lane and chunk.  NW: waves.  ACC: accumulators of a wave, one or four.
 template <bool BT, int T, int U, int NW, int ACC, int EPI>
 __global__ __launch_bounds__(NW * WAVE) void gemm_small_kernel(GemmArgs g) {
     constexpr int L = 16, SIDE = T * L, G = 16, CHUNK = U * G;       // tile side; k-values per load, per chunk
